@@ -643,40 +643,66 @@ __global__ __launch_bounds__(256) void k_gemm_grouped(
     }
 }
 
-// One thread per particle: merge the 2*nseg sorted lists into the top T.
+// Merges a particle's nlist lists of T (score, view) entries into its topk
+// best: score descending, ties to the lower view index, unused places
+// (-inf, -1). One wavefront per particle: the lanes read the entries side by
+// side into lists of their own, then T rounds take the largest head. Entries
+// are ordered as 64-bit keys (score bits made monotonic, complemented index);
+// 0 stands for none. Bound by reading 8 B per entry. One thread per particle,
+// walking its entries alone, took 828 us for 150 particles x 2,048 entries
+// and 990 us for 5,000 x 1,664: whole searches of 1,173 -> 356 us (150
+// particles, 64^3 map) and 6,740 -> 5,522 us (5,000 particles, 128^3 map).
+__device__ __forceinline__ unsigned long long topk_key(float v, int id) {
+    const unsigned u = __float_as_uint(v + 0.f);   // -0 counts as 0
+    const unsigned o = (u & 0x80000000u) ? ~u : u | 0x80000000u;
+    return ((unsigned long long)o << 32) | (unsigned)~id;
+}
+
 template <int T>
-__global__ void k_topk_merge(const float* __restrict__ pscore, const int* __restrict__ pidx,
-                             int nlist, int64_t n, int topk, int* __restrict__ cand,
-                             float* __restrict__ cscore) {
-    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= n) return;
-    float best[T];
-    int bidx[T];
+__global__ __launch_bounds__(256) void k_topk_merge(const float* __restrict__ pscore,
+                                                    const int* __restrict__ pidx, int nlist,
+                                                    int64_t n, int topk, int* __restrict__ cand,
+                                                    float* __restrict__ cscore) {
+    const int64_t p = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (p >= n) return;   // a whole wavefront
+    const int lane = threadIdx.x & 63;
+    unsigned long long best[T];
 #pragma unroll
-    for (int q = 0; q < T; ++q) { best[q] = -INFINITY; bidx[q] = -1; }
+    for (int q = 0; q < T; ++q) best[q] = 0;
     const float* S = pscore + (size_t)p * nlist * T;
     const int* I = pidx + (size_t)p * nlist * T;
-    for (int e = 0; e < nlist * T; ++e) {
-        const float v = S[e];
+    for (int e = lane; e < nlist * T; e += 64) {
         const int id = I[e];
-        if (id >= 0 && (v > best[T - 1] || (v == best[T - 1] && bidx[T - 1] >= 0 && id < bidx[T - 1]) ||
-                        bidx[T - 1] < 0)) {
-            best[T - 1] = v;
-            bidx[T - 1] = id;
+        unsigned long long k = id >= 0 ? topk_key(S[e], id) : 0;
+        if (k > best[T - 1]) {
 #pragma unroll
-            for (int q = T - 1; q > 0; --q) {
-                const bool sw = bidx[q - 1] < 0 || best[q] > best[q - 1] ||
-                                (best[q] == best[q - 1] && bidx[q] < bidx[q - 1]);
-                if (sw) {
-                    const float tv = best[q]; best[q] = best[q - 1]; best[q - 1] = tv;
-                    const int ti = bidx[q]; bidx[q] = bidx[q - 1]; bidx[q - 1] = ti;
-                }
+            for (int q = 0; q < T; ++q) {   // insert, shifting the smaller ones down
+                const unsigned long long o = best[q];
+                best[q] = k > o ? k : o;
+                k = k > o ? o : k;
             }
         }
     }
-    for (int q = 0; q < topk; ++q) {
-        cand[p * topk + q] = bidx[q];
-        cscore[p * topk + q] = best[q];
+    for (int r = 0; r < topk; ++r) {
+        unsigned long long m = best[0];
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            const unsigned long long x = __shfl_xor(m, o, 64);
+            m = x > m ? x : m;
+        }
+        if (lane == 0) {
+            const unsigned o = (unsigned)(m >> 32);
+            cand[p * topk + r] = m ? (int)~(unsigned)m : -1;
+            cscore[p * topk + r] =
+                m ? __uint_as_float((o & 0x80000000u) ? o & 0x7fffffffu : ~o) : -INFINITY;
+        }
+        // one lane gives up its head (equal heads: the lowest lane)
+        const unsigned long long has = __ballot(m != 0 && best[0] == m);
+        if (has && lane == __builtin_ctzll(has)) {
+#pragma unroll
+            for (int q = 0; q + 1 < T; ++q) best[q] = best[q + 1];
+            best[T - 1] = 0;
+        }
     }
 }
 
@@ -1710,7 +1736,7 @@ int run_exhaustive(bsx_search* h, const uint16_t* A, int64_t nrows, int32_t* can
         hipLaunchKernelGGL((k_gemm_topk4<16>), grid, dim3(512), 0, s, A, h->d_lbf, h->Kp,
                            (int)h->nviews, tps, ntiles, (int)rblocks, nseg, h->d_pscore, h->d_pidx);
     BSX_HIP(hipGetLastError());
-    const unsigned mg = (unsigned)((nrows + 255) / 256);
+    const unsigned mg = (unsigned)((nrows + 3) / 4);
     if (T == 8)
         hipLaunchKernelGGL((k_topk_merge<8>), dim3(mg), dim3(256), 0, s, h->d_pscore, h->d_pidx,
                            4 * nseg, nrows, h->p.topk, cand_dev, score_dev);
@@ -1846,7 +1872,7 @@ int bsx_search_proposed(bsx_search* h, const int32_t* cls_dev, int32_t k, int32_
                                h->d_members, h->d_mcount, h->maxm, h->d_pscore, h->d_pidx);
         BSX_HIP(hipGetLastError());
     }
-    const unsigned mg = (unsigned)((n + 255) / 256);
+    const unsigned mg = (unsigned)((n + 3) / 4);
     if (T == 8)
         hipLaunchKernelGGL((k_topk_merge<8>), dim3(mg), dim3(256), 0, s, h->d_pscore, h->d_pidx, k,
                            n, h->p.topk, cand_dev, score_dev);

@@ -115,6 +115,33 @@ def test_gemm_topk_exact_on_bf16_rows(setup64, topk):
         assert np.all(np.diff(score[i]) <= 0)
 
 
+@pytest.mark.parametrize("npart,nview,repeat,topk", [(1, 3, 1, 8), (3, 5, 40, 8), (5, 300, 7, 16),
+                                                    (6, 700, 3, 3)])
+def test_topk_merge_ties_and_short_lists(setup64, npart, nview, repeat, topk):
+    """The merge of the per-segment lists orders candidates by score, ties
+    (here: repeated views, whose scores are equal bit for bit) by the lower
+    view index, and fills places beyond the number of views with -1 / -inf."""
+    n, R, bm, vol, ft, ps = setup64
+    rng = np.random.default_rng(nview)
+    base = search.view_matrices(synth.uniform_views(nview, rng))
+    mats = np.tile(base, (repeat, 1, 1))
+    say(f"merge particles={npart} views={len(mats)} topk={topk}")
+    s = search.Search(n, R, 1.5, topk=topk)
+    s.set_reference(ft, mats)
+    s.stage(ps.images[:npart].cuda().contiguous(), ps.parts[:npart])
+    cand, score = (t.cpu().numpy() for t in s.exhaustive())
+    one = search.Search(n, R, 1.5, topk=min(topk, 8) if nview <= 8 else topk)
+    one.set_reference(ft, base)
+    one.stage(ps.images[:npart].cuda().contiguous(), ps.parts[:npart])
+    bc, bs = (t.cpu().numpy() for t in one.exhaustive())
+    for i in range(npart):
+        want = [(float(v), c + nview * r) for v, c in zip(bs[i], bc[i]) if c >= 0 for r in range(repeat)]
+        want = sorted(want, key=lambda t: (-t[0], t[1]))[:topk]
+        assert list(cand[i][:len(want)]) == [c for _, c in want]
+        assert np.array_equal(score[i][:len(want)], np.float32([v for v, _ in want]))
+        assert np.all(cand[i][len(want):] == -1) and np.all(np.isneginf(score[i][len(want):]))
+
+
 def test_gemm_topk_row_blocks_and_k_steps():
     """The GEMM over more than one 256-row block (300 particles) and disk
     radii whose K = 2(Nd - 1), rounded up to 64, gives both odd and even
