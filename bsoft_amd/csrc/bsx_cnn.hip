@@ -31,6 +31,8 @@ __host__ __device__ inline uint16_t f_to_bf16(float f) {
     return (uint16_t)(u >> 16);
 }
 
+unsigned nblk(long n, int t = 256) { return (unsigned)std::min<long>((n + t - 1) / t, 1l << 30); }
+
 template <typename T> __device__ inline float ldw(const T* p, long i);
 template <> __device__ inline float ldw<float>(const float* p, long i) { return p[i]; }
 template <> __device__ inline float ldw<uint16_t>(const uint16_t* p, long i) { return bf16_to_f(p[i]); }
@@ -229,13 +231,443 @@ __global__ __launch_bounds__(256) void k_sgemm(int M, int N, int K, const float*
     }
 }
 
-// db[n] = sum_m g[m][n]
-__global__ void k_colsum(const float* __restrict__ g, int M, int N, float* __restrict__ db) {
-    const int n = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= N) return;
+// ------------------------------------------- FP32 training on matrix cores
+// The stride-2 layers (2-4), the fully connected layer and the pair scores
+// are contractions, run on v_mfma_f32_32x32x2_f32 (A: row lane & 31,
+// k lane >> 5; B: column lane & 31, k lane >> 5; FP32 products and sums, twice
+// the rate of scalar FP32 FMAs). An instruction takes 64 cycles for two
+// 4-byte LDS reads per lane, so neither LDS nor the gathers bound the
+// kernels; tiles are small so that the last layers still fill the chip.
+typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16;
+constexpr int TK = 16;   // k per LDS stage
+
+// Row of an accumulator register: D[8 (r / 4) + 4 (lane / 32) + r % 4][lane % 32].
+__device__ __forceinline__ int acc_row(int r, int lane) {
+    return 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+}
+
+// Conv weights [co][ci][tap] of layers 2-4 as [tap][ci][co] (forward) and
+// [tap][co][ci] (data gradient), so that the kernels below read them with
+// consecutive lanes; one launch for the three layers.
+struct PermLayers {
+    long woff[3], ofs[3];   // weights in the parameters, copies in the output
+    int cin[3], cout[3];
+};
+__global__ void k_perm_train(const float* __restrict__ P, PermLayers L, float* __restrict__ wf,
+                             float* __restrict__ wb) {
+    const int l = blockIdx.y;
+    const int ci = L.cin[l], co = L.cout[l];
+    const long n = (long)ci * co * 9;
+    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
+        const float v = P[L.woff[l] + i];
+        const int tap = (int)(i % 9), c = (int)((i / 9) % ci), o = (int)(i / (9l * ci));
+        wf[L.ofs[l] + ((long)tap * ci + c) * co + o] = v;
+        wb[L.ofs[l] + ((long)tap * co + o) * ci + c] = v;
+    }
+}
+
+// Implicit-GEMM convolution of a stride-2 layer, TC channels x TP positions
+// per workgroup, one 32 x 32 block per wave; k = (16 channels, tap).
+// BWD 0: y[b][n][yo][xo] = relu(bias[n] + sum W x), in = x (K channels, H x W),
+//   positions the Ho x Wo outputs.
+// BWD 1: dx[b][n][yi][xi] = (act > 0) sum W g (the ReLU backward of the layer
+//   below included), in = g (K channels, Ho x Wo). An input row 2 y receives
+//   tap 1 of output row y; row 2 y + 1 taps 0 and 2 of rows y + 1 and y: the
+//   four parities of (yi, xi) (blockIdx.z) are dense contractions over 1, 2, 2
+//   and 4 taps at Ho x Wo positions each.
+// Bound by the MFMA rate: at 512 x 32^2 inputs, 32-64-128-128 channels, 66 us
+// a layer forward and 63-97 us backward, 4.8 GFLOP each, 73 of 157 TFLOP/s
+// (direct FP32 kernels, one thread per output: 433 and 2,329 us a layer).
+template <int TC, int TP, bool BWD>
+__global__ __launch_bounds__(256) void k_conv32(const float* __restrict__ in, const float* __restrict__ Wt,
+                                                const float* __restrict__ bias,
+                                                const float* __restrict__ act,
+                                                float* __restrict__ out, int B, int K, int N, int H,
+                                                int W, int Ho, int Wo) {
+    static_assert(TC * TP == 4096, "four 32 x 32 blocks");
+    constexpr int RP = TP * TK / 256, RC = TC * TK / 256;   // loads per thread and stage
+    __shared__ float sp[2][TK][TP], sc[2][TK][TC];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wc = wave % (TC / 32), wp = wave / (TC / 32);
+    const int P = B * Ho * Wo, p0 = (int)blockIdx.x * TP;   // < 2^31: batch and input size are bounded
+    const int n0 = blockIdx.y * TC;
+    // the four-tap parity first: its workgroups run longest
+    const int par = BWD ? 3 - (int)blockIdx.z : 0;
+    const int py = par >> 1, px = par & 1;
+    const int ntx = BWD ? 1 + px : 3, ntap = BWD ? (1 + py) * ntx : 9;
+    const int ih = BWD ? Ho : H, iw = BWD ? Wo : W;
+    // this thread's position and channels of a stage
+    const int mp = tid % TP, kp = tid / TP * RP, mc = tid % TC, kc = tid / TC * RC;
+    const bool pok = p0 + mp < P;
+    const int pq = pok ? p0 + mp : 0;
+    const int x = pq % Wo, y = (pq / Wo) % Ho;
+    const long plane = (long)ih * iw;
+    const float* src = in + ((long)(pq / (Wo * Ho)) * K + kp) * plane;
+    const bool cok = n0 + mc < N;
+    const float* wsrc = Wt + (long)kc * N + n0 + mc;
+    float rp[RP], rc[RC];
+    int cb = 0, tap = 0;
+    auto load = [&]() {
+        int ky = tap / ntx, kx = tap - ky * ntx, iy, ix;
+        if (BWD) {
+            iy = y + (py && ky == 0);
+            ix = x + (px && kx == 0);
+            ky = py ? 2 * ky : 1;
+            kx = px ? 2 * kx : 1;
+        } else {
+            iy = 2 * y - 1 + ky;
+            ix = 2 * x - 1 + kx;
+        }
+        const bool ok = pok && iy >= 0 && iy < ih && ix >= 0 && ix < iw;
+        const float* s = src + cb * TK * plane + (ok ? (long)iy * iw + ix : 0);
+        const float* w = wsrc + ((long)(ky * 3 + kx) * K + cb * TK) * N;
+#pragma unroll
+        for (int j = 0; j < RP; ++j) rp[j] = ok ? s[j * plane] : 0.f;
+#pragma unroll
+        for (int j = 0; j < RC; ++j) rc[j] = cok ? w[(long)j * N] : 0.f;
+        if (++tap == ntap) { tap = 0; ++cb; }
+    };
+    auto store = [&](int buf) {
+#pragma unroll
+        for (int j = 0; j < RP; ++j) sp[buf][kp + j][mp] = rp[j];
+#pragma unroll
+        for (int j = 0; j < RC; ++j) sc[buf][kc + j][mc] = rc[j];
+    };
+    f32x16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    const int nst = K / TK * ntap;
+    load();
+    store(0);
+    __syncthreads();
+    for (int st = 0; st < nst; ++st) {
+        if (st + 1 < nst) load();
+        const int buf = st & 1;
+#pragma unroll
+        for (int k = 0; k < TK; k += 2)
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(sc[buf][k + (lane >> 5)][wc * 32 + (lane & 31)],
+                                                       sp[buf][k + (lane >> 5)][wp * 32 + (lane & 31)],
+                                                       acc, 0, 0, 0);
+        if (st + 1 < nst) store(buf ^ 1);
+        __syncthreads();
+    }
+    const int po = p0 + wp * 32 + (lane & 31);
+    if (po >= P) return;
+    const int xo = po % Wo, yo = (po / Wo) % Ho;
+    const long b = po / (Wo * Ho);
+    const long oplane = BWD ? (long)H * W : (long)Ho * Wo;
+    const long at = b * N * oplane + (BWD ? (long)(2 * yo + py) * W + 2 * xo + px : (long)yo * Wo + xo);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int n = n0 + wc * 32 + acc_row(r, lane);
+        if (n >= N) continue;
+        const long o = at + n * oplane;
+        if (BWD) out[o] = act[o] > 0.f ? acc[r] : 0.f;
+        else out[o] = fmaxf(acc[r] + bias[n], 0.f);
+    }
+}
+
+// Weight gradient of a stride-2 layer: partial sums over a share of the
+// B Ho Wo positions (blockIdx.z) of 64 output x 32 input channels for all 9
+// taps, part[z] = [tap][co][ci] and the bias gradient [co]. Each stage holds
+// 16 positions: g (64 channels) and the 9 shifted x (32 channels); waves are
+// 2 channel blocks x 2 halves of the positions, 9 accumulators each, so one
+// read of g serves 9 instructions. k_part_sum adds the shares in order.
+// 69 us a layer at the
+// sizes above (one workgroup per (co, ci), which read all of g and x each: 1,916 us).
+__global__ __launch_bounds__(256, 2) void k_conv32_dw(const float* __restrict__ g,
+                                                   const float* __restrict__ xin,
+                                                   float* __restrict__ part, int B, int Cin, int H,
+                                                   int W, int Cout, int Ho, int Wo) {
+    constexpr int NP = 16, LG = 65, LX = 33;
+    __shared__ float lds[NP * LG + 9 * NP * LX];
+    static_assert(sizeof(lds) >= 4 * 2 * 64 * 16, "one tap of the halves' exchange");
+    float* sg = lds;             // [pos][co]
+    float* sx = lds + NP * LG;   // [tap][pos][ci]
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wc = wave & 1, wh = wave >> 1;
+    const int co0 = blockIdx.x * 64, ci0 = blockIdx.y * 32;
+    const int P = B * Ho * Wo;
+    const int nst = (P + NP - 1) / NP;
+    const int per = (nst + (int)gridDim.z - 1) / (int)gridDim.z;
+    const int s0 = (int)blockIdx.z * per, s1 = min(nst, s0 + per);
+    const int mp = tid & 15, q = tid >> 4;   // position; g channels q + 16 j, x channels q, q + 16
+    const long oplane = (long)Ho * Wo, iplane = (long)H * W;
+    float rg[4], rx[2][9], gsum[4] = {0.f, 0.f, 0.f, 0.f};
+    auto load = [&](int st) {
+        const int p = st * NP + mp;
+        const bool pok = p < P;
+        const int pq = pok ? p : 0;
+        const int x = pq % Wo, y = (pq / Wo) % Ho;
+        const long b = pq / (Ho * Wo);
+        const float* gs = g + (b * Cout + co0 + q) * oplane + (long)y * Wo + x;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            rg[j] = (pok && co0 + q + 16 * j < Cout) ? gs[16l * j * oplane] : 0.f;
+        const float* xs = xin + (b * Cin + ci0 + q) * iplane;
+#pragma unroll
+        for (int t = 0; t < 9; ++t) {
+            const int iy = 2 * y - 1 + t / 3, ix = 2 * x - 1 + t % 3;
+            const bool ok = pok && iy >= 0 && iy < H && ix >= 0 && ix < W;
+            const long o = ok ? (long)iy * W + ix : 0;
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                rx[j][t] = (ok && ci0 + q + 16 * j < Cin) ? xs[16l * j * iplane + o] : 0.f;
+        }
+    };
+    f32x16 acc[9];
+#pragma unroll
+    for (int t = 0; t < 9; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[t][r] = 0.f;
+    if (s0 < s1) load(s0);
+    for (int st = s0; st < s1; ++st) {
+        __syncthreads();   // the stage before has been read
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            sg[mp * LG + q + 16 * j] = rg[j];
+            gsum[j] += rg[j];
+        }
+#pragma unroll
+        for (int t = 0; t < 9; ++t)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) sx[(t * NP + mp) * LX + q + 16 * j] = rx[j][t];
+        __syncthreads();
+        if (st + 1 < s1) load(st + 1);
+#pragma unroll
+        for (int k = 0; k < NP / 2; k += 2) {
+            const int p = wh * (NP / 2) + k + (lane >> 5);
+            const float a = sg[p * LG + wc * 32 + (lane & 31)];
+#pragma unroll
+            for (int t = 0; t < 9; ++t)
+                acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, sx[(t * NP + p) * LX + (lane & 31)],
+                                                              acc[t], 0, 0, 0);
+        }
+    }
+    float* out = part + (long)blockIdx.z * ((long)Cout * Cin * 9 + Cout);
+    // the second half of the positions joins the first, one tap at a time
+#pragma unroll
+    for (int t = 0; t < 9; ++t) {
+        __syncthreads();
+        if (wh == 1)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) lds[(wc * 16 + r) * 64 + lane] = acc[t][r];
+        __syncthreads();
+        if (wh == 0)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int co = co0 + wc * 32 + acc_row(r, lane), ci = ci0 + (lane & 31);
+                if (co < Cout && ci < Cin)
+                    out[((long)t * Cout + co) * Cin + ci] = acc[t][r] + lds[(wc * 16 + r) * 64 + lane];
+            }
+    }
+    if (blockIdx.y == 0) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            float v = gsum[j];
+            for (int o = 8; o > 0; o >>= 1) v += __shfl_xor(v, o, 16);
+            if (mp == 0 && co0 + q + 16 * j < Cout)
+                out[(long)Cout * Cin * 9 + co0 + q + 16 * j] = v;
+        }
+    }
+}
+
+// Four consecutive floats at float alignment (inputs may start anywhere).
+struct Float4u {
+    float v[4];
+};
+
+// First layer (one input channel, stride 1), forward: a thread holds the 3 x 6
+// window of 4 consecutive outputs and runs over 8 output channels (uniform
+// weights: scalar loads); bound by writing y.
+__global__ __launch_bounds__(256) void k_conv1_32(const float* __restrict__ x, const float* __restrict__ Wt,
+                                                  const float* __restrict__ bias, float* __restrict__ y,
+                                                  int B, int S, int Cout) {
+    const int quads = S * S / 4;
+    const long t = (long)blockIdx.x * 256 + threadIdx.x;
+    if (t >= (long)B * quads) return;
+    const long b = t / quads;
+    const int q = (int)(t - b * quads), yo = q / (S / 4), xo = (q - yo * (S / 4)) * 4;
+    float v[3][6];
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+        const int yi = yo - 1 + r;
+        const float* row = x + (b * S + yi) * S + xo;
+        const bool ok = yi >= 0 && yi < S;
+        Float4u x4 = {{0.f, 0.f, 0.f, 0.f}};
+        if (ok) x4 = *(const Float4u*)row;
+        v[r][0] = ok && xo > 0 ? row[-1] : 0.f;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) v[r][c + 1] = x4.v[c];
+        v[r][5] = ok && xo + 4 < S ? row[4] : 0.f;
+    }
+    const int c0 = blockIdx.y * 8, c1 = min(Cout, c0 + 8);
+    for (int co = c0; co < c1; ++co) {
+        float a[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) a[e] = bias[co];
+#pragma unroll
+        for (int k = 0; k < 9; ++k) {
+            const float w = Wt[co * 9 + k];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) a[e] = fmaf(w, v[k / 3][k % 3 + e], a[e]);
+        }
+        *(float4*)(y + ((b * Cout + co) * S + yo) * (long)S + xo) =
+            make_float4(fmaxf(a[0], 0.f), fmaxf(a[1], 0.f), fmaxf(a[2], 0.f), fmaxf(a[3], 0.f));
+    }
+}
+
+// First layer, weight and bias gradients: partial sums of `per` inputs per
+// workgroup (blockIdx.x), 32 output channels x 8 lanes that share a channel's
+// positions, 4 consecutive ones at a time; part[z] = [co][9] and [co]. Bound
+// by reading g.
+__global__ __launch_bounds__(256) void k_conv1_32_dw(const float* __restrict__ g,
+                                                     const float* __restrict__ x,
+                                                     float* __restrict__ part, int B, int S, int Cout,
+                                                     int per) {
+    const int co = blockIdx.y * 32 + (threadIdx.x >> 3), pg = threadIdx.x & 7;
+    const bool cok = co < Cout;
+    const int quads = S * S / 4;
+    float acc[10];
+#pragma unroll
+    for (int k = 0; k < 10; ++k) acc[k] = 0.f;
+    for (long b = (long)blockIdx.x * per; b < min((long)B, ((long)blockIdx.x + 1) * per); ++b) {
+        const float* gs = g + (b * Cout + (cok ? co : 0)) * (long)S * S;
+        for (int q = pg; q < quads; q += 8) {
+            const int yo = q / (S / 4), xo = (q - yo * (S / 4)) * 4;
+            const float4 g4 = *(const float4*)(gs + yo * S + xo);   // rows are multiples of 8 floats
+            const float gv[4] = {g4.x, g4.y, g4.z, g4.w};
+#pragma unroll
+            for (int r = 0; r < 3; ++r) {
+                const int yi = yo - 1 + r;
+                if (yi < 0 || yi >= S) continue;
+                const float* row = x + (b * S + yi) * S + xo;
+                const Float4u x4 = *(const Float4u*)row;
+                const float v[6] = {xo > 0 ? row[-1] : 0.f, x4.v[0], x4.v[1], x4.v[2], x4.v[3],
+                                    xo + 4 < S ? row[4] : 0.f};
+#pragma unroll
+                for (int c = 0; c < 3; ++c)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[3 * r + c] = fmaf(gv[e], v[c + e], acc[3 * r + c]);
+            }
+            acc[9] += (gv[0] + gv[1]) + (gv[2] + gv[3]);
+        }
+    }
+    float* out = part + (long)blockIdx.x * Cout * 10;
+#pragma unroll
+    for (int k = 0; k < 10; ++k) {
+        float v = acc[k];
+        for (int o = 4; o > 0; o >>= 1) v += __shfl_xor(v, o, 8);
+        if (pg == 0 && cok) out[k < 9 ? (long)co * 9 + k : (long)Cout * 9 + co] = v;
+    }
+}
+
+// out[i] = sum over nz shares of part[z][i], n values each, 16 groups of
+// shares per value (4 groups: 12 us a sum of 38 MB, 16: 8 us). taps > 1: the first nw values are [tap][co][ci] and go to
+// [co][ci][tap]; bias (or null) is added by column i % ncol.
+__global__ __launch_bounds__(1024) void k_part_sum(const float* __restrict__ part, int nz, long n, long nw,
+                                                  int taps, const float* __restrict__ bias, int ncol,
+                                                  float* __restrict__ out) {
+    __shared__ float red[16][64];
+    const int c = threadIdx.x & 63, grp = threadIdx.x >> 6;
+    const long i = (long)blockIdx.x * 64 + c;
     float s = 0.f;
-    for (int m = 0; m < M; ++m) s += g[(long)m * N + n];
-    db[n] = s;
+    if (i < n) {
+#pragma unroll 4
+        for (int z = grp; z < nz; z += 16) s += part[z * n + i];
+    }
+    red[grp][c] = s;
+    __syncthreads();
+    if (grp != 0 || i >= n) return;
+    float v = 0.f;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) v += red[q][c];
+    if (bias) v += bias[i % ncol];
+    const long per = taps > 1 ? nw / taps : 1;
+    out[taps > 1 && i < nw ? (i % per) * taps + i / per : i] = v;
+}
+
+// C[m][n] = sum_k A[m am + k ak] B[k bk + n bn] (+ bias[n]) in FP32 on matrix
+// cores, 64 x 64 per workgroup, blockIdx.z a share of K. One share: the result
+// goes to C; several: share z to C + z M N for k_part_sum (bias null). The fully
+// connected layer of 512 x 2048 -> 128 has 16 tiles only; its K is split so
+// that some 512 workgroups run.
+__global__ __launch_bounds__(256) void k_gemm32(int M, int N, int K, const float* __restrict__ A, long am,
+                                                long ak, const float* __restrict__ Bm, long bk, long bn,
+                                                const float* __restrict__ bias, float* __restrict__ Cm,
+                                                int kper) {
+    constexpr int LR = 65;
+    __shared__ float sa[2][TK][LR], sb[2][TK][LR];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wm = wave >> 1, wn = wave & 1;
+    const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
+    const int k0 = blockIdx.z * kper, k1 = min(K, k0 + kper);
+    // consecutive threads walk the dimension that is contiguous in memory
+    const bool ka = ak == 1, kb = bk == 1;
+    const int ar = ka ? tid >> 4 : tid & 63, ac = ka ? tid & 15 : tid >> 6;
+    const int br = kb ? tid >> 4 : tid & 63, bc = kb ? tid & 15 : tid >> 6;
+    float ra[4], rb[4];
+    auto load = [&](int kk) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int m = m0 + ar + (ka ? 16 * j : 0), k = kk + ac + (ka ? 0 : 4 * j);
+            ra[j] = (m < M && k < k1) ? A[m * am + k * ak] : 0.f;
+            const int n = n0 + br + (kb ? 16 * j : 0), q = kk + bc + (kb ? 0 : 4 * j);
+            rb[j] = (n < N && q < k1) ? Bm[q * bk + n * bn] : 0.f;
+        }
+    };
+    auto store = [&](int buf) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            sa[buf][ac + (ka ? 0 : 4 * j)][ar + (ka ? 16 * j : 0)] = ra[j];
+            sb[buf][bc + (kb ? 0 : 4 * j)][br + (kb ? 16 * j : 0)] = rb[j];
+        }
+    };
+    f32x16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    load(k0);
+    store(0);
+    __syncthreads();
+    for (int kk = k0, buf = 0; kk < k1; kk += TK, buf ^= 1) {
+        if (kk + TK < k1) load(kk + TK);
+#pragma unroll
+        for (int k = 0; k < TK; k += 2)
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(sa[buf][k + (lane >> 5)][wm * 32 + (lane & 31)],
+                                                       sb[buf][k + (lane >> 5)][wn * 32 + (lane & 31)],
+                                                       acc, 0, 0, 0);
+        if (kk + TK < k1) store(buf ^ 1);
+        __syncthreads();
+    }
+    const int n = n0 + wn * 32 + (lane & 31);
+    if (n >= N) return;
+    const float bv = bias ? bias[n] : 0.f;
+    float* C = Cm + (long)blockIdx.z * M * N;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int m = m0 + wm * 32 + acc_row(r, lane);
+        if (m < M) C[(long)m * N + n] = acc[r] + bv;
+    }
+}
+
+// db[n] = sum_m g[m][n]: 64 columns per workgroup, the rows over its 16 waves
+__global__ __launch_bounds__(1024) void k_colsum(const float* __restrict__ g, int M, int N,
+                                                 float* __restrict__ db) {
+    __shared__ float red[16][64];
+    const int c = threadIdx.x & 63, grp = threadIdx.x >> 6;
+    const int n = blockIdx.x * 64 + c;
+    float s = 0.f;
+    if (n < N) {
+#pragma unroll 4
+        for (int m = grp; m < M; m += 16) s += g[(long)m * N + n];
+    }
+    red[grp][c] = s;
+    __syncthreads();
+    if (grp != 0 || n >= N) return;
+    float v = 0.f;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) v += red[q][c];
+    db[n] = v;
 }
 
 // ------------------------------------------------------ softmax / top-k
@@ -352,18 +784,26 @@ __global__ __launch_bounds__(256) void k_row_topk(const float* __restrict__ logi
 }
 
 // --------------------------------------------- contrastive (embedding) head
+__device__ __forceinline__ float wave_add(float v) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    return v;
+}
+
 // Unit rows u = z / |z| of an n x d matrix (|z| floored at 1e-12); one
-// thread per row.
-__global__ void k_unit_rows(const float* __restrict__ z, long n, int d, float* __restrict__ u,
-                            float* __restrict__ nrm) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+// wavefront per row, so that rows are read and written with consecutive
+// lanes (one thread per row: 58 us for 4,096 x 128).
+__global__ __launch_bounds__(256) void k_unit_rows(const float* __restrict__ z, long n, int d,
+                                                   float* __restrict__ u, float* __restrict__ nrm) {
+    const long i = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
     if (i >= n) return;
     const float* r = z + i * d;
     float ss = 0.f;
-    for (int c = 0; c < d; ++c) ss = fmaf(r[c], r[c], ss);
-    const float nz = fmaxf(sqrtf(ss), 1e-12f), inv = 1.f / nz;
-    for (int c = 0; c < d; ++c) u[i * d + c] = r[c] * inv;
-    if (nrm) nrm[i] = nz;
+    for (int c = lane; c < d; c += 64) ss = fmaf(r[c], r[c], ss);
+    const float nz = fmaxf(sqrtf(wave_add(ss)), 1e-12f), inv = 1.f / nz;
+    for (int c = lane; c < d; c += 64) u[i * d + c] = r[c] * inv;
+    if (nrm && lane == 0) nrm[i] = nz;
 }
 
 // Softmax of the pair scores S (B x B, cosines) over temperature tau, by row
@@ -412,16 +852,19 @@ __global__ void k_pair_grad(const float* __restrict__ P, const float* __restrict
     if (j == 0 && loss_out) loss_out[i] = 0.5f * (lrow[i] + lcol[i]);
 }
 
-// Backward of u = z / |z|: dz = (du - (du . u) u) / |z|, one thread per row.
-__global__ void k_unit_rows_bwd(const float* __restrict__ du, const float* __restrict__ u,
-                                const float* __restrict__ nrm, long n, int d,
-                                float* __restrict__ dz) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+// Backward of u = z / |z|: dz = (du - (du . u) u) / |z|, one wavefront per row.
+__global__ __launch_bounds__(256) void k_unit_rows_bwd(const float* __restrict__ du,
+                                                       const float* __restrict__ u,
+                                                       const float* __restrict__ nrm, long n, int d,
+                                                       float* __restrict__ dz) {
+    const long i = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
     if (i >= n) return;
     float dot = 0.f;
-    for (int c = 0; c < d; ++c) dot = fmaf(du[i * d + c], u[i * d + c], dot);
+    for (int c = lane; c < d; c += 64) dot = fmaf(du[i * d + c], u[i * d + c], dot);
+    dot = wave_add(dot);
     const float inv = 1.f / nrm[i];
-    for (int c = 0; c < d; ++c) dz[i * d + c] = (du[i * d + c] - dot * u[i * d + c]) * inv;
+    for (int c = lane; c < d; c += 64) dz[i * d + c] = (du[i * d + c] - dot * u[i * d + c]) * inv;
 }
 
 __global__ void k_scale(float* __restrict__ x, long n, float a) {
@@ -454,7 +897,6 @@ __global__ void k_to_bf16(const float* __restrict__ p, uint16_t* __restrict__ q,
 // output channels, k = (tap, input channel) with the channel fastest, so
 // that 8 consecutive k are one 16-byte load from the NHWC input.
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
-typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16;
 constexpr int IM = 128, IN = 64, IK = 32, IROW = IK * 2 + 16;
 
 // y[b][yo][xo][co] = bf16(relu(bias + sum_{ky,kx} W[co][0][ky][kx] x[b][yo-1+ky][xo-1+kx]))
@@ -609,8 +1051,6 @@ __global__ void k_perm_fc(const float* __restrict__ W, int ncls, int C, int hw, 
     o[cls * F + (long)pos * C + c] = f_to_bf16(W[t]);
 }
 
-unsigned nblk(long n, int t = 256) { return (unsigned)std::min<long>((n + t - 1) / t, 1l << 30); }
-
 }  // namespace
 
 // ================================================================ host
@@ -628,6 +1068,12 @@ struct bsx_cnn {
     float* d_act[5] = {};      // activations 1..4 (index 1..4), logits at [0]
     float* d_gact[5] = {};
     float* d_loss = nullptr;
+    // training: conv weights of layers 2-4 reordered for k_conv32 (forward,
+    // data gradient), and the shares of split sums; sized for max_batch
+    float* d_wt[2] = {};
+    long wt_ofs[5] = {};
+    float* d_part = nullptr;
+    long part_cap = 0;
     long step = 0;
     // MFMA inference: permuted BF16 weights of layers 2-4 and the FC; NHWC
     // BF16 activations of layers 1-4 and FP32 logits, sized for chunks larger
@@ -657,6 +1103,9 @@ void free_cnn(bsx_cnn* h) {
         if (h->d_wi[i]) (void)hipFree(h->d_wi[i]);
         if (h->d_ib[i]) (void)hipFree(h->d_ib[i]);
     }
+    for (float* q : h->d_wt)
+        if (q) (void)hipFree(q);
+    if (h->d_part) (void)hipFree(h->d_part);
     if (h->d_ilog) (void)hipFree(h->d_ilog);
     if (h->d_nce) (void)hipFree(h->d_nce);
     if (h->d_match) (void)hipFree(h->d_match);
@@ -680,24 +1129,147 @@ struct Rng {
     double normal() { return sqrt(-2 * log(uniform())) * cos(2 * M_PI * uniform()); }
 };
 
+// Shares that a sum over `steps` stages is split into so that some 512
+// workgroups (two per CU) run, with at least 4 stages a share.
+int shares(long tiles, long steps) {
+    return (int)std::max<long>(1, std::min<long>((512 + tiles - 1) / tiles, steps / 4));
+}
+
+// The matrix-core kernels of a stride-2 layer take input channels in whole
+// 16-channel stages (the data gradient: output channels too); other channel
+// counts keep the direct kernels.
+bool conv32_ok(const bsx_cnn* h, int l) { return l >= 2 && h->ch[l - 1] % TK == 0 && h->ch[l] % TK == 0; }
+
+int reserve_part(bsx_cnn* h, long n, hipStream_t s) {
+    if (n <= h->part_cap) return BSX_OK;
+    if (h->d_part) {
+        BSX_HIP(hipStreamSynchronize(s));
+        (void)hipFree(h->d_part);
+    }
+    h->d_part = nullptr;
+    h->part_cap = 0;
+    BSX_HIP(hipMalloc(&h->d_part, sizeof(float) * n));
+    h->part_cap = n;
+    return BSX_OK;
+}
+
+// Shares of a k_gemm32 product, and the K range of each.
+int gemm32_shares(int M, int N, int K, int* kper) {
+    const int z = shares(((N + 63) / 64) * (long)((M + 63) / 64), (K + TK - 1) / TK);
+    *kper = ((K + z - 1) / z + TK - 1) / TK * TK;
+    return (K + *kper - 1) / *kper;
+}
+
+// Tiles and shares of a layer's weight gradient.
+dim3 dw_grid(const bsx_cnn* h, int l, int B) {
+    const int Cin = h->ch[l - 1], Cout = h->ch[l], Ho = h->hw[l];
+    if (l == 1) return dim3(1, (Cout + 31) / 32, std::min(B, 512));
+    const dim3 t((Cout + 63) / 64, (Cin + 31) / 32);
+    return dim3(t.x, t.y, shares((long)t.x * t.y, ((long)B * Ho * Ho + 15) / 16));
+}
+
+// One buffer for every split sum of a training step of B inputs (pairs: B / 2
+// pairs of them), so that the step allocates once.
+int reserve_training(bsx_cnn* h, int B, bool pairs, hipStream_t s) {
+    const int C = h->nclass, F = (int)h->feat;
+    long n = 0;
+    for (int l = 1; l <= 4; ++l)
+        if (l == 1 || conv32_ok(h, l))
+            n = std::max(n, ((long)h->ch[l] * h->ch[l - 1] * 9 + h->ch[l]) * dw_grid(h, l, B).z);
+    auto product = [&](int M, int N, int K) {
+        int kper;
+        const int nz = gemm32_shares(M, N, K, &kper);
+        if (nz > 1) n = std::max(n, (long)M * N * nz);
+    };
+    product(B, C, F);
+    product(C, F, B);
+    product(B, F, C);
+    if (pairs) {
+        product(B / 2, B / 2, C);
+        product(B / 2, C, B / 2);
+    }
+    return reserve_part(h, n, s);
+}
+
+// C = A B (+ bias) on k_gemm32, K split over shares where C has few tiles.
+int gemm32(bsx_cnn* h, int M, int N, int K, const float* A, long am, long ak, const float* B, long bk,
+           long bn, const float* bias, float* C, hipStream_t s) {
+    const dim3 g((N + 63) / 64, (M + 63) / 64);
+    int kper;
+    const int nz = gemm32_shares(M, N, K, &kper);
+    if (nz == 1) {
+        hipLaunchKernelGGL(k_gemm32, g, dim3(256), 0, s, M, N, K, A, am, ak, B, bk, bn, bias, C, K);
+        BSX_HIP(hipGetLastError());
+        return BSX_OK;
+    }
+    const long n = (long)M * N;
+    const int rc = reserve_part(h, n * nz, s);
+    if (rc) return rc;
+    hipLaunchKernelGGL(k_gemm32, dim3(g.x, g.y, nz), dim3(256), 0, s, M, N, K, A, am, ak, B, bk, bn,
+                       (const float*)nullptr, h->d_part, kper);
+    BSX_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_part_sum, dim3(nblk(n, 64)), dim3(1024), 0, s, h->d_part, nz, n, 0l, 1, bias, N, C);
+    BSX_HIP(hipGetLastError());
+    return BSX_OK;
+}
+
+// Fully connected layer of the forward pass; BF16 weights keep k_sgemm.
+int forward_fc(bsx_cnn* h, int B, const float* W, const float* bias, hipStream_t s) {
+    return gemm32(h, B, h->nclass, (int)h->feat, h->d_act[4], h->feat, 1, W, 1, h->feat, bias, h->d_act[0], s);
+}
+int forward_fc(bsx_cnn* h, int B, const uint16_t* W, const uint16_t* bias, hipStream_t s) {
+    const int F = (int)h->feat, C = h->nclass;
+    hipLaunchKernelGGL((k_sgemm<uint16_t>), dim3((C + 63) / 64, (B + 63) / 64), dim3(256), 0, s, B, C, F,
+                       h->d_act[4], (long)F, 1l, W, 1l, (long)F, bias, h->d_act[0], (long)C);
+    BSX_HIP(hipGetLastError());
+    return BSX_OK;
+}
+
+// Activations of the layers and the outputs d_act[0] for B inputs, with the
+// FP32 parameters (training) or their BF16 copies.
 template <typename TW>
 int forward(bsx_cnn* h, const float* x, int B, const TW* P, hipStream_t s) {
+    constexpr bool F32 = sizeof(TW) == 4;
     const float* in = x;
+    if (F32 && (conv32_ok(h, 2) || conv32_ok(h, 3) || conv32_ok(h, 4))) {
+        PermLayers L;
+        for (int l = 2; l <= 4; ++l) {
+            L.woff[l - 2] = h->woff[l - 1];
+            L.ofs[l - 2] = h->wt_ofs[l];
+            L.cin[l - 2] = h->ch[l - 1];
+            L.cout[l - 2] = h->ch[l];
+        }
+        hipLaunchKernelGGL(k_perm_train, dim3(256, 3), dim3(256), 0, s, (const float*)P, L, h->d_wt[0],
+                           h->d_wt[1]);
+        BSX_HIP(hipGetLastError());
+    }
     for (int l = 1; l <= 4; ++l) {
         const int Cin = h->ch[l - 1], Cout = h->ch[l], H = h->hw[l - 1], Ho = h->hw[l];
         const int stride = l == 1 ? 1 : 2;
-        const long tot = (long)B * (Cout / 4) * Ho * Ho;
-        hipLaunchKernelGGL((k_conv_fwd<TW>), dim3(nblk(tot)), dim3(256), 0, s, in, P + h->woff[l - 1],
-                           P + h->boff[l - 1], h->d_act[l], B, Cin, H, H, Cout, Ho, Ho, stride);
+        if (F32 && l == 1) {
+            hipLaunchKernelGGL(k_conv1_32, dim3(nblk((long)B * H * H / 4), (Cout + 7) / 8), dim3(256), 0, s,
+                               in, (const float*)P + h->woff[0], (const float*)P + h->boff[0],
+                               h->d_act[1], B, H, Cout);
+        } else if (F32 && conv32_ok(h, l)) {
+            const float* w = h->d_wt[0] + h->wt_ofs[l];
+            const float* bias = (const float*)P + h->boff[l - 1];
+            const long pos = (long)B * Ho * Ho;
+            if (Cout <= 32)
+                hipLaunchKernelGGL((k_conv32<32, 128, false>), dim3(nblk(pos, 128)), dim3(256), 0, s, in, w,
+                                   bias, (const float*)nullptr, h->d_act[l], B, Cin, Cout, H, H, Ho, Ho);
+            else
+                hipLaunchKernelGGL((k_conv32<64, 64, false>), dim3(nblk(pos, 64), (Cout + 63) / 64),
+                                   dim3(256), 0, s, in, w, bias, (const float*)nullptr, h->d_act[l], B,
+                                   Cin, Cout, H, H, Ho, Ho);
+        } else {
+            const long tot = (long)B * (Cout / 4) * Ho * Ho;
+            hipLaunchKernelGGL((k_conv_fwd<TW>), dim3(nblk(tot)), dim3(256), 0, s, in, P + h->woff[l - 1],
+                               P + h->boff[l - 1], h->d_act[l], B, Cin, H, H, Cout, Ho, Ho, stride);
+        }
         BSX_HIP(hipGetLastError());
         in = h->d_act[l];
     }
-    const int F = (int)h->feat, C = h->nclass;
-    dim3 g((C + 63) / 64, (B + 63) / 64);
-    hipLaunchKernelGGL((k_sgemm<TW>), g, dim3(256), 0, s, B, C, F, h->d_act[4], (long)F, 1l,
-                       P + h->woff[4], 1l, (long)F, P + h->boff[4], h->d_act[0], (long)C);
-    BSX_HIP(hipGetLastError());
-    return BSX_OK;
+    return forward_fc(h, B, P + h->woff[4], P + h->boff[4], s);
 }
 
 // Backpropagation from dL/dlogits in d_gact[0] (B rows) to the parameter
@@ -707,30 +1279,58 @@ int backward_body(bsx_cnn* h, const float* x, int B, hipStream_t s) {
     float* P = h->d_p;
     float* G = h->d_g;
     // FC: dW = dl^T x, db = colsum(dl), dx = dl W
-    {
-        dim3 g((F + 63) / 64, (C + 63) / 64);
-        hipLaunchKernelGGL((k_sgemm<float>), g, dim3(256), 0, s, C, F, B, h->d_gact[0], 1l, (long)C,
-                           h->d_act[4], (long)F, 1l, (const float*)nullptr, G + h->woff[4], (long)F);
-        BSX_HIP(hipGetLastError());
-        hipLaunchKernelGGL(k_colsum, dim3((C + 255) / 256), dim3(256), 0, s, h->d_gact[0], B, C,
-                           G + h->boff[4]);
-        BSX_HIP(hipGetLastError());
-        dim3 g2((F + 63) / 64, (B + 63) / 64);
-        hipLaunchKernelGGL((k_sgemm<float>), g2, dim3(256), 0, s, B, F, C, h->d_gact[0], (long)C, 1l,
-                           P + h->woff[4], (long)F, 1l, (const float*)nullptr, h->d_gact[4], (long)F);
-        BSX_HIP(hipGetLastError());
-    }
+    int rc = gemm32(h, C, F, B, h->d_gact[0], 1, C, h->d_act[4], F, 1, nullptr, G + h->woff[4], s);
+    if (rc) return rc;
+    hipLaunchKernelGGL(k_colsum, dim3((C + 63) / 64), dim3(1024), 0, s, h->d_gact[0], B, C, G + h->boff[4]);
+    BSX_HIP(hipGetLastError());
+    rc = gemm32(h, B, F, C, h->d_gact[0], C, 1, P + h->woff[4], F, 1, nullptr, h->d_gact[4], s);
+    if (rc) return rc;
+    bool masked = false;   // d_gact[l] already holds the gradient before the ReLU
     for (int l = 4; l >= 1; --l) {
         const int Cin = h->ch[l - 1], Cout = h->ch[l], H = h->hw[l - 1], Ho = h->hw[l];
         const int stride = l == 1 ? 1 : 2;
-        const long na = act_size(h, l, B);
-        hipLaunchKernelGGL(k_relu_bwd, dim3(nblk(na)), dim3(256), 0, s, h->d_gact[l], h->d_act[l], na);
-        BSX_HIP(hipGetLastError());
+        if (!masked) {
+            const long na = act_size(h, l, B);
+            hipLaunchKernelGGL(k_relu_bwd, dim3(nblk(na)), dim3(256), 0, s, h->d_gact[l], h->d_act[l], na);
+            BSX_HIP(hipGetLastError());
+        }
+        masked = false;
         const float* in = l == 1 ? x : h->d_act[l - 1];
-        hipLaunchKernelGGL(k_conv_bwd_weight, dim3(Cout, Cin + 1), dim3(256), 0, s, h->d_gact[l], in,
-                           G + h->woff[l - 1], G + h->boff[l - 1], B, Cin, H, H, Cout, Ho, Ho, stride);
+        const bool c32 = conv32_ok(h, l);
+        const long nw = (long)Cout * Cin * 9, n = nw + Cout;
+        if (l == 1 || c32) {
+            // weights and biases are neighbours in the parameter vector
+            const dim3 tiles = dw_grid(h, l, B);
+            const int nz = (int)tiles.z;
+            if ((rc = reserve_part(h, n * nz, s))) return rc;
+            if (l == 1)
+                hipLaunchKernelGGL(k_conv1_32_dw, dim3(nz, tiles.y), dim3(256), 0, s, h->d_gact[1], in,
+                                   h->d_part, B, H, Cout, (B + nz - 1) / nz);
+            else
+                hipLaunchKernelGGL(k_conv32_dw, tiles, dim3(256), 0, s, h->d_gact[l], in,
+                                   h->d_part, B, Cin, H, H, Cout, Ho, Ho);
+            BSX_HIP(hipGetLastError());
+            hipLaunchKernelGGL(k_part_sum, dim3(nblk(n, 64)), dim3(1024), 0, s, h->d_part, nz, n, nw,
+                               l == 1 ? 1 : 9, (const float*)nullptr, 1, G + h->woff[l - 1]);
+        } else {
+            hipLaunchKernelGGL(k_conv_bwd_weight, dim3(Cout, Cin + 1), dim3(256), 0, s, h->d_gact[l], in,
+                               G + h->woff[l - 1], G + h->boff[l - 1], B, Cin, H, H, Cout, Ho, Ho, stride);
+        }
         BSX_HIP(hipGetLastError());
-        if (l > 1) {
+        if (l > 1 && c32) {
+            const float* w = h->d_wt[1] + h->wt_ofs[l];
+            const long pos = (long)B * Ho * Ho;
+            if (Cin <= 32)
+                hipLaunchKernelGGL((k_conv32<32, 128, true>), dim3(nblk(pos, 128), 1, 4), dim3(256), 0, s,
+                                   h->d_gact[l], w, (const float*)nullptr, h->d_act[l - 1],
+                                   h->d_gact[l - 1], B, Cout, Cin, H, H, Ho, Ho);
+            else
+                hipLaunchKernelGGL((k_conv32<64, 64, true>), dim3(nblk(pos, 64), (Cin + 63) / 64, 4),
+                                   dim3(256), 0, s, h->d_gact[l], w, (const float*)nullptr,
+                                   h->d_act[l - 1], h->d_gact[l - 1], B, Cout, Cin, H, H, Ho, Ho);
+            BSX_HIP(hipGetLastError());
+            masked = true;
+        } else if (l > 1) {
             const long nx = (long)B * Cin * H * H;
             hipLaunchKernelGGL(k_conv_bwd_data, dim3(nblk(nx)), dim3(256), 0, s, h->d_gact[l],
                                P + h->woff[l - 1], h->d_gact[l - 1], B, Cin, H, H, Cout, Ho, Ho, stride);
@@ -901,6 +1501,10 @@ int bsx_cnn_create(bsx_cnn** out, int32_t in_size, const int32_t* channels, int3
         if ((e = hipMalloc(&h->d_act[l], sizeof(float) * n)) != hipSuccess) return fail(e, "activations");
         if ((e = hipMalloc(&h->d_gact[l], sizeof(float) * n)) != hipSuccess) return fail(e, "activations");
     }
+    for (int l = 2; l <= 4; ++l) h->wt_ofs[l] = l == 2 ? 0 : h->wt_ofs[l - 1] + (long)h->ch[l - 1] * h->ch[l - 2] * 9;
+    for (float*& q : h->d_wt)
+        if ((e = hipMalloc(&q, sizeof(float) * (h->wt_ofs[4] + (long)h->ch[4] * h->ch[3] * 9))) != hipSuccess)
+            return fail(e, "training weights");
     for (int l = 1; l < 4; ++l)
         if ((e = hipMalloc(&h->d_wi[l], sizeof(uint16_t) * h->ch[l + 1] * h->ch[l] * 9)) != hipSuccess)
             return fail(e, "inference weights");
@@ -960,7 +1564,8 @@ int bsx_cnn_gradients(bsx_cnn* h, const float* x_dev, const int32_t* labels_dev,
     BSX_REQUIRE(batch >= 1 && batch <= h->maxb, BSX_ERR_ARG,
                 "bsx_cnn_gradients: batch %d out of 1..%d", batch, h->maxb);
     hipStream_t s = (hipStream_t)stream;
-    int rc = forward<float>(h, x_dev, batch, h->d_p, s);
+    int rc = reserve_training(h, batch, false, s);
+    if (!rc) rc = forward<float>(h, x_dev, batch, h->d_p, s);
     if (!rc) rc = backward(h, x_dev, labels_dev, batch, s);
     if (rc) return rc;
     if (grad_dev)
@@ -1010,7 +1615,7 @@ int bsx_cnn_embed(bsx_cnn* h, const float* x_dev, int64_t n, float* emb_dev, voi
     hipStream_t s = (hipStream_t)stream;
     const int d = h->nclass;
     return infer_chunks(h, x_dev, n, s, "bsx_cnn_embed", [&](const float* lg, int64_t b0, int nb) {
-        hipLaunchKernelGGL(k_unit_rows, dim3(nblk(nb)), dim3(256), 0, s, lg, (long)nb, d,
+        hipLaunchKernelGGL(k_unit_rows, dim3(nblk(nb, 4)), dim3(256), 0, s, lg, (long)nb, d,
                            emb_dev + b0 * d, (float*)nullptr);
         BSX_HIP(hipGetLastError());
         return BSX_OK;
@@ -1083,16 +1688,15 @@ int bsx_cnn_pair_gradients(bsx_cnn* h, const float* x_dev, int32_t batch, float 
     float* P = S + (long)B * B;
     float* Q = P + (long)B * B;
     float* dS = Q + (long)B * B;
-    int rc = forward<float>(h, x_dev, B2, h->d_p, s);
+    int rc = reserve_training(h, B2, true, s);
+    if (!rc) rc = forward<float>(h, x_dev, B2, h->d_p, s);
     if (rc) return rc;
-    hipLaunchKernelGGL(k_unit_rows, dim3(nblk(B2)), dim3(256), 0, s, h->d_act[0], (long)B2, d, U, nrm);
+    hipLaunchKernelGGL(k_unit_rows, dim3(nblk(B2, 4)), dim3(256), 0, s, h->d_act[0], (long)B2, d, U, nrm);
     BSX_HIP(hipGetLastError());
     const float* Up = U;
     const float* Ur = U + (long)B * d;
     // S = Up Ur^T (cosines)
-    hipLaunchKernelGGL((k_sgemm<float>), dim3((B + 63) / 64, (B + 63) / 64), dim3(256), 0, s, B, B, d,
-                       Up, (long)d, 1l, Ur, 1l, (long)d, (const float*)nullptr, S, (long)B);
-    BSX_HIP(hipGetLastError());
+    if ((rc = gemm32(h, B, B, d, Up, d, 1, Ur, 1, d, nullptr, S, s))) return rc;
     const float it = 1.f / tau;
     hipLaunchKernelGGL(k_pair_softmax, dim3(B), dim3(256), 0, s, S, B, it, 0, P, lrl);
     hipLaunchKernelGGL(k_pair_softmax, dim3(B), dim3(256), 0, s, S, B, it, 1, Q, lrl + B);
@@ -1100,13 +1704,9 @@ int bsx_cnn_pair_gradients(bsx_cnn* h, const float* x_dev, int32_t batch, float 
                        lrl + B, dS, h->d_loss);
     BSX_HIP(hipGetLastError());
     // dUp = dS Ur, dUr = dS^T Up
-    dim3 gd((d + 63) / 64, (B + 63) / 64);
-    hipLaunchKernelGGL((k_sgemm<float>), gd, dim3(256), 0, s, B, d, B, dS, (long)B, 1l, Ur, (long)d,
-                       1l, (const float*)nullptr, dU, (long)d);
-    hipLaunchKernelGGL((k_sgemm<float>), gd, dim3(256), 0, s, B, d, B, dS, 1l, (long)B, Up, (long)d,
-                       1l, (const float*)nullptr, dU + (long)B * d, (long)d);
-    BSX_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_unit_rows_bwd, dim3(nblk(B2)), dim3(256), 0, s, dU, U, nrm, (long)B2, d,
+    if ((rc = gemm32(h, B, d, B, dS, B, 1, Ur, d, 1, nullptr, dU, s))) return rc;
+    if ((rc = gemm32(h, B, d, B, dS, 1, B, Up, d, 1, nullptr, dU + (long)B * d, s))) return rc;
+    hipLaunchKernelGGL(k_unit_rows_bwd, dim3(nblk(B2, 4)), dim3(256), 0, s, dU, U, nrm, (long)B2, d,
                        h->d_gact[0]);
     BSX_HIP(hipGetLastError());
     rc = backward_body(h, x_dev, B2, s);

@@ -97,6 +97,34 @@ def test_pair_gradients_match_oracle(S, ch, d, B):
         np.testing.assert_allclose(prob[i].cpu().numpy(), sm[cls[i].cpu().numpy()], rtol=1e-4)
 
 
+@pytest.mark.parametrize("S,ch,d,B", [
+    (8, (16, 16, 16, 16), 8, 3),       # one output position per last-layer image, one K stage
+    (24, (32, 48, 80, 16), 70, 5),     # odd output edges, ragged channel and output tiles
+    (16, (16, 96, 32, 144), 130, 33),  # more than one tile in every direction
+    (16, (8, 32, 64, 24), 12, 4),      # matrix-core and direct layers in one network
+])
+def test_pair_gradients_tile_edges(S, ch, d, B):
+    """Gradients of the matrix-core training kernels at the edges of their
+    tiles (channel counts, positions and batch that are no multiples of 16,
+    32 or 64) against the FP64 restatement, FP32 accumulation error only:
+    1e-4 of each parameter block's largest gradient."""
+    say(f"pairs S={S} ch={ch} dim={d} batch={B}")
+    net = EmbeddingNet(S, d, ch, max_batch=2 * B, seed=6)
+    x = np.random.default_rng(S + B).normal(size=(2 * B, S, S)).astype(np.float32)
+    xd = torch.as_tensor(x).cuda()
+    g, loss = net.pair_gradients(xd[:B], xd[B:], 0.2)
+    p = net.params().cpu().numpy().astype(np.float64)
+    L, og, olosses = cnn_ref.pair_loss_and_grad(p, x.astype(np.float64), B, 0.2, S, ch, d)
+    np.testing.assert_allclose(loss.cpu().numpy(), olosses, rtol=1e-5, atol=1e-5)
+    g = g.cpu().numpy()
+    off, n, feat, _ = cnn_ref.layout(S, ch, d)
+    for o, ob, c in off:
+        for a, b in ((o, ob), (ob, ob + c)):
+            assert np.abs(g[a:b] - og[a:b]).max() <= 1e-4 * np.abs(og[a:b]).max() + 1e-7
+    again, _ = net.pair_gradients(xd[:B], xd[B:], 0.2)
+    assert np.array_equal(g, again.cpu().numpy())      # sums in a fixed order
+
+
 @pytest.mark.parametrize("ch", [(8, 8, 16, 8), (32, 64, 32, 64)])
 def test_training_reduces_loss_and_bf16_inference(ch):
     """Adam memorises a fixed batch; BF16 inference (VALU path for small
