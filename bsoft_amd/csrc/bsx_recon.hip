@@ -16,7 +16,7 @@
 //                    accumulators (Bimage::fspace_pack_2D and
 //                    fspace_2D_interpolate, Bimage_reconstruct.cpp:25-174).
 // Finish (img_reconstruction_sum_weigh, mg_reconstruct.cpp:266-361):
-//   K4 k_weigh       sum of half sets, FP64 weighing, SNR FOM, centre shift
+//   K4 k_weigh_pairs sum of half sets, FP64 weighing, SNR FOM, centre shift
 //   K5 3 axis FFTs   inverse 3D transform, x 1/sqrt(N^3), real part.
 #include <cmath>
 #include <algorithm>
@@ -26,47 +26,12 @@
 #include <climits>
 #include <string>
 
-#include "bsx_fft_dev.h"
-#include "bsx_common.h"
+#include "bsx_insert.h"
 
 namespace bsx {
 int fft_axis_ex(float2* data, float* real_out, int nx, int ny, int nz, int64_t batch, int axis,
                 int sign, float scale, hipStream_t s);
 }
-
-using namespace bsx;
-
-// Device record of one particle, all derived quantities computed on the host
-// in double precision.
-struct alignas(16) PartDev {
-    double R[9];        // View::matrix (row-major d[i][j])
-    double invscale;    // (1/mag) / (ft * pixel_size)      fspace_pack_2D invscale
-    double phx, phy;    // 2 pi ori / ft                      phase_shift_to_origin
-    double rot[4];      // cos, sin of T phy and (T - ft) phy, T = ft / 8: the phase
-                        // steps between the rounds of a column thread
-    double c0, c20, c22, c2m2, c40;   // aberration weights   ctf.h:321-335
-    double fscale;      // 1 / (ft * pixel_size)              img_ctf_calculate freq_scale
-    double ew;          // Ewald offset lambda/2, 0 if off
-    double nyq[2];      // cos, sin of -ft phy: the phase factor of a Nyquist-row
-                        // mate is conj(sample's) times this
-    double hox, hoy;    // background-ellipse origin (image header)
-    long long src;      // index of the image in the caller's stack
-    float wp;           // particle weight incl. pad ratio
-    int half;           // accumulator set
-};
-
-struct ReconConst {
-    int N, ft, box, stride, interp, ctf_mode, fom, nhalves;   // ctf_mode 0 none 1 flip 2 apply 3 wiener
-    int merge, ewald, NT, pairs;                              // NT: 16^3 tiles per edge
-    // pairs: binned entries stand for a sample and its Friedel mate (value
-    // at v, conjugate at -v), folded into the volume by k_fold
-    double mins2, maxs2, mscale, shi2, wiener;
-    // z extent: a 2D map (breconstruct -TwoD) has one plane (nz = 1) and z
-    // real size 1 (particle_reconstruct sets the z sampling to 1,
-    // mg_reconstruct.cpp:117), which scales m_z and the resolution taper
-    double mscz;
-    int nz;
-};
 
 // ------------------------------------------------------------------- K1
 // Block-wide sums of 256 threads (FP64 and int).
@@ -92,12 +57,6 @@ __device__ __forceinline__ void block_sum256(double& a, double& b, int& c, int& 
     c = sc[0];
     d = sd[0];
     __syncthreads();
-}
-
-// Rescaled pixel value: the FP64 product and sum of Bimage::rescale
-// (Bimage_rescale.cpp:27-45) stored back as FP32.
-__device__ __forceinline__ float rescaled(float v, double2 r) {
-    return (float)((double)v * r.x + r.y);
 }
 
 // One workgroup per particle record: the background (mean of the pixels
@@ -204,855 +163,6 @@ __global__ __launch_bounds__(256) void k_background(const float* __restrict__ im
     }
 }
 
-// ------------------------------------------------------------------- K2
-// One workgroup: 2*LINES rows of one particle (rows y0 + 2j, y0 + 2j + 1 form
-// complex line j). Output: inter[p][x][y], x in [0, FT/2], y in [0, box).
-template <int FT, int LINES>
-__global__ __launch_bounds__(256) void k_rows(const float* __restrict__ imgs,
-                                              const PartDev* __restrict__ recs,
-                                              const float* __restrict__ bkg, int box,
-                                              int tiles_per_part, float2* __restrict__ inter,
-                                              const float2* __restrict__ twg,
-                                              const double2* __restrict__ resc) {
-    constexpr int T = FftThreads<FT>::value;
-    constexpr int G = 256 / T;
-    constexpr int NT = G * T;
-    constexpr int HX = FT / 2 + 1;
-    __shared__ __attribute__((aligned(16))) float2 lds[LINES * FT + FT];
-    float2* tw = lds + LINES * FT;
-    const int tid = threadIdx.x;
-    const int p = blockIdx.x / tiles_per_part;
-    const int y0 = (blockIdx.x % tiles_per_part) * 2 * LINES;
-    const float* img = imgs + (size_t)recs[p].src * box * box;
-    const float b = bkg[p];
-    for (int i = tid; i < FT; i += NT) tw[i] = twg[i];
-    // load: line j = rows (y0+2j, y0+2j+1), x < box from the image (rescaled
-    // when resc is given) minus the background, zero elsewhere (the padded
-    // region equals the background).
-    if (resc) {
-        const double2 rs = resc[p];
-        for (int idx = tid; idx < LINES * FT; idx += NT) {
-            const int j = idx / FT, x = idx - j * FT;
-            const int ya = y0 + 2 * j, yb = ya + 1;
-            float a = 0.f, c = 0.f;
-            if (x < box) {
-                if (ya < box) a = rescaled(img[(size_t)ya * box + x], rs) - b;
-                if (yb < box) c = rescaled(img[(size_t)yb * box + x], rs) - b;
-            }
-            lds[j * FT + x] = make_float2(a, c);
-        }
-    } else if ((box & 3) == 0) {
-        // rows y0 + 2j and y0 + 2j + 1 as float4 loads, written as four
-        // (a, c) pairs; x in [box, FT) zero
-        const int q4 = box >> 2;
-        for (int idx = tid; idx < LINES * q4; idx += NT) {
-            const int j = idx / q4, x4 = idx - j * q4;
-            const int ya = y0 + 2 * j, yb = ya + 1;
-            float4 a = make_float4(0.f, 0.f, 0.f, 0.f), c = a;
-            if (ya < box) {
-                a = *(const float4*)(img + (size_t)ya * box + 4 * x4);
-                a.x -= b; a.y -= b; a.z -= b; a.w -= b;
-            }
-            if (yb < box) {
-                c = *(const float4*)(img + (size_t)yb * box + 4 * x4);
-                c.x -= b; c.y -= b; c.z -= b; c.w -= b;
-            }
-            float4* d = (float4*)(lds + j * FT + 4 * x4);
-            d[0] = make_float4(a.x, c.x, a.y, c.y);
-            d[1] = make_float4(a.z, c.z, a.w, c.w);
-        }
-        const int zq = (FT - box) >> 1;   // float4 (two pairs) per line beyond the image
-        for (int idx = tid; idx < LINES * zq; idx += NT) {
-            const int j = idx / zq, x2 = idx - j * zq;
-            *(float4*)(lds + j * FT + box + 2 * x2) = make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-    } else {
-        for (int idx = tid; idx < LINES * FT; idx += NT) {
-            const int j = idx / FT, x = idx - j * FT;
-            const int ya = y0 + 2 * j, yb = ya + 1;
-            float a = 0.f, c = 0.f;
-            if (x < box) {
-                if (ya < box) a = img[(size_t)ya * box + x] - b;
-                if (yb < box) c = img[(size_t)yb * box + x] - b;
-            }
-            lds[j * FT + x] = make_float2(a, c);
-        }
-    }
-    __syncthreads();
-    const int g = tid / T, t = tid - g * T;
-#pragma unroll 1
-    for (int r0 = 0; r0 < LINES; r0 += G) FftLine<FT, -1, T>::run(lds + (r0 + g) * FT, tw, t);
-    // store: for each x in [0, FT/2], the 2*LINES consecutive rows
-    constexpr int ROWS = 2 * LINES;
-    float2* out = inter + (size_t)p * HX * box;
-    if ((box & 1) == 0) {
-        // rows y0 + 2j (A) and y0 + 2j + 1 (B) of column x as one 16-byte store
-        for (int idx = tid; idx < HX * LINES; idx += NT) {
-            const int x = idx / LINES, j = idx - x * LINES;
-            const int y = y0 + 2 * j;
-            if (y >= box) continue;
-            const float2 z = lds[j * FT + x];
-            const float2 zm = lds[j * FT + ((FT - x) & (FT - 1))];
-            *(float4*)(out + (size_t)x * box + y) =
-                make_float4(0.5f * (z.x + zm.x), 0.5f * (z.y - zm.y),
-                            0.5f * (z.y + zm.y), -0.5f * (z.x - zm.x));
-        }
-        return;
-    }
-    for (int idx = tid; idx < HX * ROWS; idx += NT) {
-        const int x = idx / ROWS, r = idx - x * ROWS;
-        const int y = y0 + r;
-        if (y >= box) continue;
-        const int j = r >> 1;
-        const float2 z = lds[j * FT + x];
-        const float2 zm = lds[j * FT + ((FT - x) & (FT - 1))];
-        float2 v;
-        if ((r & 1) == 0) v = make_float2(0.5f * (z.x + zm.x), 0.5f * (z.y - zm.y));   // A(x)
-        else v = make_float2(0.5f * (z.y + zm.y), -0.5f * (z.x - zm.x));              // B(x)
-        out[(size_t)x * box + y] = v;
-    }
-}
-
-// ------------------------------------------------------------------- K3
-// Accumulator layout: records of `stride` floats (sum w re, sum w im, sum w
-// [, sum w|F|^2, sum w^2]) in 16^3-voxel tiles; a tile is 4096 contiguous
-// records (48 KB lean). Key = half * NREC + record index, NREC = NT^3 * 4096,
-// so key >> 12 is the (half, tile) bin and key & 4095 the record in the tile.
-__host__ __device__ __forceinline__ long rec_index(long x, long y, long z, long NT) {
-    return ((((z >> 4) * NT + (y >> 4)) * NT + (x >> 4)) << 12) | ((z & 15) << 8) |
-           ((y & 15) << 4) | (x & 15);
-}
-
-// 32-bit forms for the insertion hot path (coordinates stay within a few
-// box sizes; record indices below 2^31 per half).
-__device__ __forceinline__ unsigned rec_index32(int x, int y, int z, int NT) {
-    return (unsigned)(((((z >> 4) * NT + (y >> 4)) * NT + (x >> 4)) << 12) | ((z & 15) << 8) |
-                      ((y & 15) << 4) | (x & 15));
-}
-__device__ __forceinline__ int wrap32(int c, int n) {
-    if (c >= 0 && c < n) return c;
-    if (c < 0 && c >= -n) return c + n;
-    if (c >= n && c < 2 * n) return c - n;
-    c %= n;
-    return c < 0 ? c + n : c;
-}
-
-// Periodic wrap (index_wrap, Bimage.h:418-426); the fast path covers the
-// in-range and single-step cases that the default geometry produces.
-__device__ __forceinline__ long wrapi(long c, long n) {
-    if (c >= 0 && c < n) return c;
-    if (c < 0 && c >= -n) return c + n;
-    if (c >= n && c < 2 * n) return c - n;
-    c %= n;
-    return c < 0 ? c + n : c;
-}
-
-enum { MODE_DIRECT = 0, MODE_FILL = 2 };
-
-// One emission: a contribution to the record `key`; `kk` is the sample row
-// (runs are merged only along unbroken k steps); `incl` marks samples the
-// reference inserts (decided from geometry alone, so the count and fill
-// passes agree exactly).
-struct Emit {
-    int key, kk, incl;
-    int bin;         // MODE_FILL: 1 = binned entry, 0 = added to the volume directly
-    float re, im, w, p, w2;
-};
-
-// Bins live in chunks of BSX_CHUNK entries taken from a pool while the fill
-// pass reserves them: a bin's reservation counter gives each entry a position,
-// position / BSX_CHUNK indexes the bin's chunk table, and the reservation that
-// holds a chunk's first position allocates it (one pool atomic, then a
-// compare-and-swap into the table) while the other writers of that chunk wait
-// for the table entry. No counting pass is needed: after the fill the counters are the bin
-// sizes, k_piece_scan turns them into work pieces, and k_bin_reset clears the
-// counters and the used table entries for the next batch. An entry whose
-// chunk cannot be had (table or pool exhausted) is added to the volume with
-// float atomics instead, so capacity only costs speed.
-#define BSX_CHUNK 4096
-#define BSX_SPIN_LIMIT 4096    // polls of a chunk-table entry before the atomic fallback
-
-// Fill-pass staging in LDS (nearest / weighted-nearest insertion without
-// Ewald): a workgroup appends its merged entries to a dense LDS list (one
-// 16-B record each; a wavefront takes its slots with one LDS atomic) and
-// counts them per bin in a small LDS hash table; at each flush one integer
-// atomic per (workgroup, bin) reserves the bin range (at most two chunks)
-// and the entries are written out.
-#define BSX_STAGE_CAP 512      // entries per flush: 2 rounds x 1 binned emission x 256 threads
-#define BSX_STAGE_HASH 128     // bins per flush (more fall back to direct reservations)
-static_assert(BSX_STAGE_CAP <= BSX_CHUNK, "a flushed bin range must span at most two chunks");
-static_assert(BSX_STAGE_CAP <= 1024 && BSX_STAGE_HASH <= 256, "list ranks take 10 bits, slots 8");
-
-struct Stage {
-    float4* ent;     // entries: (sum w re, sum w im, sum w, r) with r =
-                     // (hash slot << 22) | (rank in the bin << 12) | record in tile,
-                     // r = -1: slot taken by an entry reserved on its own
-    int* nent;       // entries in the list
-    int* hkey;       // bin per hash slot, -1 = free
-    int* hcnt;       // entries per hash slot
-    int4* hinfo;     // at a flush, per hash slot: reserved base, chunks of the
-                     // range start and end, bin
-    int on;
-    float2* ent2;    // FOM: (sum w|F|^2, sum w^2) of each entry, else null
-};
-
-struct BinCtx {
-    int* fill;       // per-bin reservation counters (bin sizes after the fill)
-    int* chunks;     // [nbins][maxc] pool chunk of each bin chunk, -1 = not yet, -2 = none
-    int* pool;       // [0] next free pool chunk, [1] fallback flags (1 table, 2 pool, 4 wait)
-    float4* bins;    // the pool: (re, im, w, record-in-tile) entries
-    float* acc;      // volume records (3 floats), target of the atomic fallback
-    int npool;       // chunks in the pool
-    int maxc;        // chunks per bin
-    Stage st;        // fill-pass staging (st.on = 0: reserve per wavefront)
-    float2* bins2;   // FOM: (sum w|F|^2, sum w^2) of each pool entry, else null
-    int stride;      // floats per volume record (3, or 5 with the FOM sums)
-};
-
-// Takes a pool chunk (-2 when the pool is exhausted) and installs it as chunk
-// ci of bin b unless one is there already; returns the installed value.
-__device__ __forceinline__ int chunk_take(const BinCtx& bc, int b, int ci) {
-    int nc = atomicAdd(bc.pool, 1);
-    if (nc >= bc.npool) nc = -2;
-    const int prev = atomicCAS(bc.chunks + (size_t)b * bc.maxc + ci, -1, nc);
-    return prev == -1 ? nc : prev;
-}
-
-// Called by the reservation holding position ci * BSX_CHUNK of bin b.
-__device__ __forceinline__ void chunk_alloc(const BinCtx& bc, int b, int ci) {
-    if (ci < bc.maxc) (void)chunk_take(bc, b, ci);
-}
-
-// Pool chunk of chunk ci of bin b once its allocator has installed it. A wait
-// past its bound installs a chunk itself (the allocator's chunk then goes
-// unused), so every writer of a bin chunk agrees on it. -1 selects the atomic
-// fallback (beyond the table or pool exhausted; then all writers of the chunk
-// fall back and the tile pass skips it).
-__device__ __forceinline__ int chunk_wait(const BinCtx& bc, int b, int ci) {
-    if (ci >= bc.maxc) {
-        atomicOr(bc.pool + 1, 1);
-        return -1;
-    }
-    const int* slot = bc.chunks + (size_t)b * bc.maxc + ci;
-    int c = -1;
-    for (int i = 0; i < BSX_SPIN_LIMIT && c == -1; ++i) {
-        c = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (c == -1) __builtin_amdgcn_s_sleep(2);
-    }
-    if (c == -1) {
-        atomicOr(bc.pool + 1, 4);
-        c = chunk_take(bc, b, ci);
-    }
-    if (c == -2) {
-        atomicOr(bc.pool + 1, 2);
-        return -1;
-    }
-    return c;
-}
-
-__device__ __forceinline__ void put_entry(const BinCtx& bc, int c, int pos, float re, float im,
-                                          float w, int key, float p = 0.f, float w2 = 0.f) {
-    if (c >= 0) {
-        const size_t e = (size_t)c * BSX_CHUNK + (pos & (BSX_CHUNK - 1));
-        bc.bins[e] = make_float4(re, im, w, __int_as_float(key & 4095));
-        if (bc.bins2) bc.bins2[e] = make_float2(p, w2);
-    } else {
-        float* rec = bc.acc + (size_t)(unsigned)key * bc.stride;
-        unsafeAtomicAdd(rec + 0, re);
-        unsafeAtomicAdd(rec + 1, im);
-        unsafeAtomicAdd(rec + 2, w);
-        if (bc.bins2) {
-            unsafeAtomicAdd(rec + 3, p);
-            unsafeAtomicAdd(rec + 4, w2);
-        }
-    }
-}
-
-// Resolves the (at most two) chunks of a reserved range [base, base + cnt):
-// allocations first, then waits, so that no allocator is held up behind a
-// wait of its own wavefront.
-__device__ __forceinline__ void range_chunks(const BinCtx& bc, int b, int base, int cnt,
-                                             bool any, int& c0, int& c1) {
-    const int i0 = base / BSX_CHUNK, i1 = (base + cnt - 1) / BSX_CHUNK;
-    if (any) {
-        if ((base & (BSX_CHUNK - 1)) == 0) chunk_alloc(bc, b, i0);
-        if (i1 != i0) chunk_alloc(bc, b, i1);
-    }
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    if (any) {
-        c0 = chunk_wait(bc, b, i0);
-        c1 = i1 != i0 ? chunk_wait(bc, b, i1) : c0;
-    }
-}
-
-// One entry into slot i of the workgroup's list (per-lane LDS atomics for
-// the bin table: measured faster here than grouping the lanes of a
-// wavefront by bin first).
-__device__ __forceinline__ void stage_entry(const BinCtx& bc, int i, int key, float re, float im,
-                                           float w, float p = 0.f, float w2 = 0.f) {
-    const int bin = (int)((unsigned)key >> 12);
-    int slot = -1;
-    int hs = (int)(((unsigned)bin * 2654435761u) >> 25) & (BSX_STAGE_HASH - 1);
-    for (int t = 0; t < BSX_STAGE_HASH; ++t) {
-        const int prev = atomicCAS(&bc.st.hkey[hs], -1, bin);
-        if (prev == -1 || prev == bin) { slot = hs; break; }
-        hs = (hs + 1) & (BSX_STAGE_HASH - 1);
-    }
-    const bool alone = slot < 0;   // table full: reserve this entry on its own
-    int pos = 0, c0 = -1, c1 = -1;
-    if (alone) pos = atomicAdd(bc.fill + bin, 1);
-    range_chunks(bc, bin, pos, 1, alone, c0, c1);
-    if (alone) {
-        put_entry(bc, c0, pos, re, im, w, key, p, w2);
-        bc.st.ent[i] = make_float4(0.f, 0.f, 0.f, __int_as_float(-1));
-        return;
-    }
-    const int rank = atomicAdd(&bc.st.hcnt[slot], 1);
-    bc.st.ent[i] = make_float4(re, im, w, __int_as_float((slot << 22) | (rank << 12) | (key & 4095)));
-    if (bc.st.ent2) bc.st.ent2[i] = make_float2(p, w2);
-}
-
-// The lanes with `out` set append their entries: dense slots from one LDS
-// atomic per wavefront (all lanes call this together).
-__device__ __forceinline__ void stage_append(const BinCtx& bc, bool out, int key, float re,
-                                            float im, float w, float p = 0.f, float w2 = 0.f) {
-    const unsigned long long m = __ballot(out);
-    if (m == 0) return;
-    const int lane = __lane_id();
-    const int leader = __builtin_ctzll(m);
-    int base = 0;
-    if (lane == leader) base = atomicAdd(bc.st.nent, __popcll(m));
-    base = __shfl(base, leader, 64);
-    if (out) stage_entry(bc, base + __popcll(m & ((1ull << lane) - 1ull)), key, re, im, w, p, w2);
-}
-
-// Workgroup-uniform: reserve every staged bin range, write the staged
-// entries, clear the list (r = -1: empty slot) and the table.
-__device__ __forceinline__ void stage_flush(const BinCtx& bc) {
-    __syncthreads();
-    const int tid = threadIdx.x;
-    int b = -1, cnt = 0, base = 0, c0 = -1, c1 = -1;
-    if (tid < BSX_STAGE_HASH) {
-        b = bc.st.hkey[tid];
-        if (b >= 0) {
-            cnt = bc.st.hcnt[tid];
-            base = atomicAdd(bc.fill + b, cnt);
-        }
-    }
-    range_chunks(bc, b, base, cnt, b >= 0, c0, c1);
-    if (b >= 0) bc.st.hinfo[tid] = make_int4(base, c0, c1, b);
-    __syncthreads();
-    const int n = *bc.st.nent;
-    for (int i = tid; i < n; i += blockDim.x) {
-        const float4 e = bc.st.ent[i];
-        const int pr = __float_as_int(e.w);
-        if (pr < 0) continue;
-        const int4 hi = bc.st.hinfo[pr >> 22];
-        const int pos = hi.x + ((pr >> 12) & 1023);
-        const int c = pos / BSX_CHUNK == hi.x / BSX_CHUNK ? hi.y : hi.z;
-        // full record key (bin from the hash slot) for the atomic fallback
-        const int key = (int)(((unsigned)hi.w << 12) | (unsigned)(pr & 4095));
-        const float2 e2 = bc.st.ent2 ? bc.st.ent2[i] : make_float2(0.f, 0.f);
-        put_entry(bc, c, pos, e.x, e.y, e.z, key, e2.x, e2.y);
-    }
-    __syncthreads();
-    if (tid < BSX_STAGE_HASH) {
-        bc.st.hkey[tid] = -1;
-        bc.st.hcnt[tid] = 0;
-    }
-    if (tid == 0) *bc.st.nent = 0;
-    __syncthreads();
-}
-
-// Row shifts of a wavefront (DPP, rows of 16 lanes): dpp_down<D> gives lane
-// i the value of lane i + D of its row, dpp_up1 that of lane i - 1; lanes
-// whose source lies outside the row read 0 (the merge conditions exclude
-// them).
-template <int D>
-__device__ __forceinline__ int dpp_down(int v) {
-    static_assert(D >= 1 && D <= 15, "row shift");
-    return __builtin_amdgcn_update_dpp(0, v, 0x100 + D, 0xF, 0xF, true);
-}
-template <int D>
-__device__ __forceinline__ float dpp_downf(float v) {
-    return __int_as_float(dpp_down<D>(__float_as_int(v)));
-}
-__device__ __forceinline__ int dpp_up1(int v) {
-    return __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, true);
-}
-
-// One step of the segmented suffix sum below: lane l takes lane l + D's sums
-// when both hold the same key and bin flag and their sample rows differ by D.
-// pk packs (row << 2) | (bin << 1) | incl.
-template <int D, int MG, bool FOM>
-__device__ __forceinline__ void merge_step(Emit& e, int& pk, int lg) {
-    if (D >= MG) return;
-    const int nk = dpp_down<D>(e.key);
-    const int np = dpp_down<D>(pk);
-    const float r0 = dpp_downf<D>(e.re);
-    const float r1 = dpp_downf<D>(e.im);
-    const float r2 = dpp_downf<D>(e.w);
-    float r3 = 0.f, r4 = 0.f;
-    if (FOM) {
-        r3 = dpp_downf<D>(e.p);
-        r4 = dpp_downf<D>(e.w2);
-    }
-    if (lg + D < MG && nk == e.key && ((np ^ pk) & 2) == 0 && abs((np >> 2) - e.kk) == D) {
-        pk |= np & 1;
-        e.re += r0;
-        e.im += r1;
-        e.w += r2;
-        if (FOM) { e.p += r3; e.w2 += r4; }
-    }
-}
-
-// Merges runs of equal keys inside aligned groups of MG <= 16 lanes (segmented
-// Hillis-Steele suffix sums over DPP row shifts); lanes l and l+d merge only if their keys are
-// equal and their sample rows differ by exactly d, so the samples between lie
-// on one straight segment and equal keys are contiguous (a periodic revisit
-// would need a segment longer than N-1 voxels, excluded on the host). The
-// first lane of each run then either adds to the volume with atomics
-// (MODE_DIRECT) or reserves a bin slot: lanes of a wavefront are grouped by
-// bin with ballots and one integer atomic per (wavefront, bin).
-template <int MG, bool FOM, int MODE, int FAST = 0>
-__device__ __forceinline__ void emit(float* __restrict__ acc, int stride, int merge, Emit e,
-                                     const BinCtx& bc) {
-    bool head = true;
-    if (MG > 1 && merge) {
-        const int lg = __lane_id() & (MG - 1);
-        // sample row, bin flag and inclusion in one word for the shifts
-        int pk = (e.kk * 4) | (e.bin << 1) | e.incl;
-        merge_step<1, MG, FOM>(e, pk, lg);
-        merge_step<2, MG, FOM>(e, pk, lg);
-        if (merge == 1) {   // runs may exceed 4 samples (merge 2: the host showed they do not)
-            merge_step<4, MG, FOM>(e, pk, lg);
-            merge_step<8, MG, FOM>(e, pk, lg);
-        }
-        e.incl = pk & 1;
-        const int prev_key = dpp_up1(e.key);
-        const int prev_pk = dpp_up1(pk);
-        head = !(lg != 0 && prev_key == e.key && ((prev_pk ^ pk) & 2) == 0 &&
-                 abs(e.kk - (prev_pk >> 2)) == 1);
-    }
-    const bool out0 = head && e.incl;
-    if (MODE == MODE_DIRECT || !e.bin) {
-        if (!out0) return;
-        float* rec = acc + (size_t)(unsigned)e.key * stride;
-        unsafeAtomicAdd(rec + 0, e.re);
-        unsafeAtomicAdd(rec + 1, e.im);
-        unsafeAtomicAdd(rec + 2, e.w);
-        if (FOM) {
-            unsafeAtomicAdd(rec + 3, e.p);
-            unsafeAtomicAdd(rec + 4, e.w2);
-        }
-        return;
-    }
-    const bool out = out0;   // lanes still here hold binned entries
-    if (FAST || bc.st.on) {
-        stage_append(bc, out, e.key, e.re, e.im, e.w, e.p, e.w2);
-        return;
-    }
-    // per wavefront: one reservation per bin, all issued before any chunk
-    // lookup waits on them
-    const int bin = (int)((unsigned)e.key >> 12);
-    const int lane = __lane_id();
-    unsigned long long active = __ballot(out);
-    int mybase = 0, myleader = lane, myrank = 0, mycnt = 0;
-    while (active) {
-        const int leader = __builtin_ctzll(active);
-        const int b0 = __shfl(bin, leader, 64);
-        const bool mine = out && bin == b0;
-        const unsigned long long m = __ballot(mine);
-        if (lane == leader) {
-            mycnt = __popcll(m);
-            mybase = atomicAdd(bc.fill + b0, mycnt);
-        }
-        if (mine) {
-            myleader = leader;
-            myrank = __popcll(m & ((1ull << lane) - 1ull));
-        }
-        active &= ~m;
-    }
-    int myc0 = -1, myc1 = -1;   // this lane leads its bin's group: resolve its chunks
-    range_chunks(bc, bin, mybase, mycnt, mycnt > 0, myc0, myc1);
-    const int base = __shfl(mybase, myleader, 64);
-    const int c0 = __shfl(myc0, myleader, 64);
-    const int c1 = __shfl(myc1, myleader, 64);
-    if (out) {
-        const int pos = base + myrank;
-        put_entry(bc, pos / BSX_CHUNK == base / BSX_CHUNK ? c0 : c1, pos, e.re, e.im, e.w, e.key,
-                  e.p, e.w2);
-    }
-}
-
-template <bool FOM>
-__device__ __forceinline__ Emit make_emit(unsigned key, int kk, bool incl, float fr, float fi,
-                                          double w, int bin) {
-    Emit e;
-    e.key = (int)key;
-    e.kk = kk;
-    e.incl = incl ? 1 : 0;
-    e.bin = bin;
-    if (!incl) w = 0;
-    e.re = (float)(fr * w);
-    e.im = (float)(fi * w);
-    e.w = (float)w;
-    e.p = FOM ? (float)(w * ((double)fr * fr + (double)fi * fi)) : 0.f;
-    e.w2 = FOM ? (float)(w * w) : 0.f;
-    return e;
-}
-
-// sin and cos of a double-precision angle: exact reduction to [-pi, pi] in
-// FP64, then FP32 evaluation (absolute error ~1e-7, below the FP32 rounding
-// the reference applies when it stores the shifted / CTF-multiplied values).
-__device__ __forceinline__ void sincos_red(double a, float* s, float* c) {
-    const double r = a - 6.283185307179586 * rint(a * 0.15915494309189535);
-    sincosf((float)r, s, c);
-}
-__device__ __forceinline__ float sin_red(double a) {
-    const double r = a - 6.283185307179586 * rint(a * 0.15915494309189535);
-    return sinf((float)r);
-}
-
-// Band, taper, phase shift and CTF of one sample (fspace_pack_2D :147-157,
-// phase_shift_to_origin, img_ctf_calculate): returns whether the sample is in
-// the resolution band, its weight and (unless counting) its value.
-// ph: the phase factor exp(i (h phx + k phy)) when the caller tracks it
-// (nullptr: evaluated here).
-template <int MODE>
-__device__ __forceinline__ bool sample_value(const ReconConst& K, const PartDev& P, bool active,
-                                             long h, long k, float2 F, double* s0, double* s1,
-                                             double* s2, double* w, float* fr, float* fi,
-                                             const float2* ph = nullptr) {
-    *s0 = (double)h * P.invscale;
-    *s1 = (double)k * P.invscale;
-    *s2 = *s0 * *s0 + *s1 * *s1;
-    const bool inband = active && *s2 >= K.mins2 && *s2 <= K.maxs2;
-    *w = 0;
-    *fr = 0.f;
-    *fi = 0.f;
-    if (!inband) return false;
-    double ww = P.wp;
-    // taper of the outermost shell: most wavefronts hold no such sample and
-    // skip it; FP32 square root (the weight is stored in FP32)
-    const double d = (K.maxs2 - *s2) * K.mscz;
-    if (__ballot(d < 1) != 0) {
-        if (d < 1) ww *= (double)__builtin_amdgcn_sqrtf((float)d);
-    }
-    *w = ww;
-    float sn, cs;
-    if (ph) {
-        cs = ph->x;
-        sn = ph->y;
-    } else {
-        sincos_red((double)h * P.phx + (double)k * P.phy, &sn, &cs);
-    }
-    float vr = F.x * cs - F.y * sn, vi = F.x * sn + F.y * cs;
-    if (K.ctf_mode) {
-        const double fx = (double)h * P.fscale, fy = (double)k * P.fscale;
-        const double cs2 = fx * fx + fy * fy;
-        float c = 0.f;
-        if (cs2 <= K.shi2) {
-            // chi = c0 + c2m2 s^2 sin 2a + c20 s^2 + c22 s^2 cos 2a + c40 s^4 with
-            // s^2 cos 2a = fx^2 - fy^2 and s^2 sin 2a = 2 fx fy (no division)
-            double dphi = P.c0;
-            dphi += P.c2m2 * (2 * fx * fy);
-            dphi += P.c20 * cs2;
-            dphi += P.c22 * (fx * fx - fy * fy);
-            dphi += P.c40 * cs2 * cs2;
-            if (K.ctf_mode == 1) {
-                // phase flip needs the sign only: sin chi < 0 iff the reduced
-                // angle lies in (-pi, 0)
-                const double r = dphi - 6.283185307179586 * rint(dphi * 0.15915494309189535);
-                c = (r < 0) ? -1.f : 1.f;
-            } else {
-                c = sin_red(dphi);
-                if (K.ctf_mode == 3) c = (float)((K.wiener + 1) * c / ((double)c * c + K.wiener));
-            }
-        }
-        vr *= c;
-        vi *= c;
-    }
-    *fr = vr;
-    *fi = vi;
-    return true;
-}
-
-// Interpolation of one sample at voxel coordinates m (fspace_2D_interpolate,
-// Bimage_reconstruct.cpp:25-88): nearest / weighted nearest / trilinear.
-template <int MG, bool FOM, int MODE, int FAST = 0>
-__device__ __forceinline__ void interp_emit(float* __restrict__ acc, const ReconConst& K,
-                                            const double m[3], bool inband, double w, float fr,
-                                            float fi, int kk, int merge, unsigned keybase,
-                                            const BinCtx& bc, int bin = 1, bool flush = false) {
-    if (FAST || K.interp < 2) {
-        const double fx = floor(m[0] + 0.5), fy = floor(m[1] + 0.5), fz = floor(m[2] + 0.5);
-        double ww = w;
-        if (FAST == 2 || (!FAST && K.interp == 1)) {   // weighted nearest neighbour
-            const double dx = m[0] - fx, dy = m[1] - fy, dz = m[2] - fz;
-            ww *= 1 - sqrt(dx * dx + dy * dy + dz * dz);
-        }
-        const int cx = wrap32((int)fx, K.N), cy = wrap32((int)fy, K.N), cz = wrap32((int)fz, K.nz);
-        emit<MG, FOM, MODE, FAST>(acc, K.stride, merge,
-                            make_emit<FOM>(keybase + rec_index32(cx, cy, cz, K.NT), kk,
-                                           inband && ww > 0, fr, fi, ww, bin),
-                            bc);
-    } else {
-        const double fx = floor(m[0]), fy = floor(m[1]), fz = floor(m[2]);
-        const double dx = m[0] - fx, dy = m[1] - fy, dz = m[2] - fz;
-        const int cx = (int)fx, cy = (int)fy, cz = (int)fz;
-#pragma unroll
-        for (int corner = 0; corner < 8; ++corner) {
-            const int xx = corner & 1, yy = (corner >> 1) & 1, zz = corner >> 2;
-            const int jx = wrap32(cx + xx, K.N), jy = wrap32(cy + yy, K.N), jz = wrap32(cz + zz, K.nz);
-            const double ww = (xx ? dx : 1 - dx) * (yy ? dy : 1 - dy) * (zz ? dz : 1 - dz) * w;
-            emit<MG, FOM, MODE, FAST>(acc, K.stride, merge,
-                                make_emit<FOM>(keybase + rec_index32(jx, jy, jz, K.NT), kk,
-                                               inband, fr, fi, ww, bin),
-                                bc);
-            // staged pair entries: at most one per thread and corner, so the
-            // list is flushed after every second corner (workgroup-uniform:
-            // only the sample's own emission, which every thread makes, asks)
-            if (MODE == MODE_FILL && flush && bc.st.on && (corner & 1)) stage_flush(bc);
-        }
-    }
-}
-
-__device__ __forceinline__ void coords(const ReconConst& K, const PartDev& P, double s0, double s1,
-                                       double sz, double m[3]) {
-    m[0] = (s0 * P.R[0] + s1 * P.R[1] + sz * P.R[2]) * K.mscale;
-    m[1] = (s0 * P.R[3] + s1 * P.R[4] + sz * P.R[5]) * K.mscale;
-    m[2] = (s0 * P.R[6] + s1 * P.R[7] + sz * P.R[8]) * K.mscz;
-}
-
-// One sample (h, k) with raw value F and the Friedel mate of its array
-// position, (-h, km) with value conj(F): fspace_pack_2D's loop body for both.
-// Away from the Nyquist row and without the Ewald offset the mate's
-// frequency is exactly -(h, k), so its coordinates are -m and its value the
-// conjugate: computed once, emitted twice. Every lane of a wavefront runs the
-// same emits (excluded samples carry incl = 0), so shuffles and ballots stay
-// uniform.
-//
-// With K.pairs (binned insertion; the Ewald offsets have their own branch)
-// a sample whose mate lands on exactly the opposite voxels (-v for v:
-// nearest neighbour all but exact .5 ties, trilinear always) is emitted
-// once, as pair entries at v that k_fold later also adds, conjugated, at
-// -v. Samples without such a mate (the x = 0 and x = FT/2
-// columns, the Nyquist row, ties) add to the volume directly, and the mate
-// of a tie is emitted on its own, as before.
-template <int MG, bool FOM, int MODE, int FAST = 0>
-__device__ __forceinline__ void insert_pair(float* __restrict__ acc, const ReconConst& K,
-                                            const PartDev& P, bool active, bool mirror, long h,
-                                            long k, long km, float2 F, int merge,
-                                            unsigned keybase, const BinCtx& bc, float2 ph) {
-    double s0, s1, s2, w;
-    float fr, fi;
-    const bool inband =
-        sample_value<MODE>(K, P, active, h, k, F, &s0, &s1, &s2, &w, &fr, &fi, &ph);
-    double m[3];
-    const double mz0 = FAST ? 0.0 : P.ew * s2;
-    if (FAST) {
-        // no Ewald offset: the z term of coords is a signed zero, which
-        // changes neither a non-zero sum nor the voxel that a zero rounds to
-        m[0] = (s0 * P.R[0] + s1 * P.R[1]) * K.mscale;
-        m[1] = (s0 * P.R[3] + s1 * P.R[4]) * K.mscale;
-        m[2] = (s0 * P.R[6] + s1 * P.R[7]) * K.mscz;
-    } else {
-        coords(K, P, s0, s1, mz0, m);
-    }
-    if (!FAST && K.ewald) {
-        // two emissions per frequency, at +mz0 (A) and -mz0 (B). Off the
-        // Nyquist row the mate's emissions at +mz0 and -mz0 lie at exactly
-        // -B and -A with the conjugate value, so with pair entries A stands
-        // for the mate's -mz0 emission and B for its +mz0 one (where the
-        // nearest voxels mirror too); the others are computed in full.
-        const bool pr = MODE == MODE_FILL && K.pairs;
-        double mb[3];
-        coords(K, P, s0, s1, -mz0, mb);
-        bool sa = pr && km == -k, sb = sa;
-        if (K.interp < 2) {
-#pragma unroll
-            for (int q = 0; q < 3; ++q) {
-                sa = sa && floor(-m[q] + 0.5) == -floor(m[q] + 0.5);
-                sb = sb && floor(-mb[q] + 0.5) == -floor(mb[q] + 0.5);
-            }
-        }
-        interp_emit<MG, FOM, MODE, FAST>(acc, K, m, inband, w, fr, fi, (int)k, merge, keybase, bc,
-                                         mirror && sa ? 1 : 0, pr);
-        interp_emit<MG, FOM, MODE, FAST>(acc, K, mb, inband, w, fr, fi, (int)k, merge, keybase, bc,
-                                         mirror && sb ? 1 : 0, pr);
-        // staged nearest-neighbour entries: at most two per thread here
-        if (MODE == MODE_FILL && pr && bc.st.on && K.interp < 2) stage_flush(bc);
-        double t0, t1, t2, tw;
-        float gr, gi;
-        const bool ib = sample_value<MODE>(K, P, mirror, -h, km, make_float2(F.x, -F.y), &t0,
-                                           &t1, &t2, &tw, &gr, &gi);
-        const bool needc = ib && !sb, needd = ib && !sa;   // C = -B, D = -A when paired
-        if (__ballot(needc || needd) == 0) return;   // wavefront-uniform
-        const double mz = P.ew * t2;
-        coords(K, P, t0, t1, mz, m);
-        interp_emit<MG, FOM, MODE, FAST>(acc, K, m, needc, tw, gr, gi, (int)km, merge, keybase, bc,
-                                         0);
-        coords(K, P, t0, t1, -mz, m);
-        interp_emit<MG, FOM, MODE, FAST>(acc, K, m, needd, tw, gr, gi, (int)km, merge, keybase, bc,
-                                         0);
-        return;
-    }
-    // the mate, per lane: -m and the conjugate away from the Nyquist row,
-    // else computed in full; emitted below by all lanes together
-    double mm[3];
-    double tw = w;
-    float gr = fr, gi = -fi;
-    bool ib = inband && mirror;
-    if (km == -k) {
-        mm[0] = -m[0];
-        mm[1] = -m[1];
-        mm[2] = -m[2];
-    } else if (FAST) {
-        // the Nyquist row (k = km = -FT/2): the mate's phase angle is
-        // -(h phx + k phy) - FT phy, so its factor follows from the sample's
-        double t0, t1, t2;
-        const float2 pm = make_float2(
-            (float)((double)ph.x * P.nyq[0] + (double)ph.y * P.nyq[1]),
-            (float)((double)ph.x * P.nyq[1] - (double)ph.y * P.nyq[0]));
-        ib = sample_value<MODE>(K, P, mirror, -h, km, make_float2(F.x, -F.y), &t0, &t1, &t2,
-                                &tw, &gr, &gi, &pm);
-        mm[0] = (t0 * P.R[0] + t1 * P.R[1]) * K.mscale;
-        mm[1] = (t0 * P.R[3] + t1 * P.R[4]) * K.mscale;
-        mm[2] = (t0 * P.R[6] + t1 * P.R[7]) * K.mscz;
-    } else {
-        double t0, t1, t2;
-        ib = sample_value<MODE>(K, P, mirror, -h, km, make_float2(F.x, -F.y), &t0, &t1, &t2,
-                                &tw, &gr, &gi);
-        coords(K, P, t0, t1, 0.0, mm);
-    }
-    if (FAST || (MODE == MODE_FILL && K.pairs)) {
-        // trilinear: the mate's corners are the sample's negated, with the
-        // same weights (floor(-m) = -floor(m) - 1 and 1 - dx; a coordinate
-        // that is an integer only swaps a zero-weight corner)
-        bool sym = km == -k;
-        if (FAST || K.interp < 2) {
-#pragma unroll
-            for (int q = 0; q < 3; ++q) sym = sym && floor(-m[q] + 0.5) == -floor(m[q] + 0.5);
-        }
-        const bool pair = mirror && sym;
-        interp_emit<MG, FOM, MODE, FAST>(acc, K, m, inband, w, fr, fi, (int)k, merge, keybase, bc,
-                                   pair ? 1 : 0, true);
-        const bool mate = ib && !sym;
-        if (__ballot(mate) == 0) return;   // wavefront-uniform
-        interp_emit<MG, FOM, MODE, FAST>(acc, K, mm, mate, tw, gr, gi, (int)km, merge, keybase, bc, 0);
-        return;
-    }
-    interp_emit<MG, FOM, MODE, FAST>(acc, K, m, inband, w, fr, fi, (int)k, merge, keybase, bc);
-    interp_emit<MG, FOM, MODE, FAST>(acc, K, mm, ib, tw, gr, gi, (int)km, merge, keybase, bc);
-}
-
-// Column tasks: task = (particle, x) with x in [0, FT/2]; G tasks per WG.
-// The nearest-neighbour specialisations (FAST 1: nearest, 2: weighted
-// nearest, both with pair entries and staging, no Ewald) are held to 5 waves
-// per SIMD (at most 96 VGPRs): their 31.7 KB of LDS allows 5 workgroups per
-// CU, and one register more would round the allocation up to 104 and allow
-// only 4 (the weighted one spills 12 B for it).
-template <int FT, bool FOM, int MODE, int FAST = 0>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FAST ? 5 : 1)))
-void k_cols(const float2* __restrict__ inter,
-                                              const float* __restrict__ bkg,
-                                              const PartDev* __restrict__ recs, int nb, int box,
-                                              ReconConst K, float* __restrict__ acc,
-                                              const float2* __restrict__ twg, BinCtx bc) {
-    constexpr int T = FftThreads<FT>::value;
-    constexpr int G = 256 / T;
-    constexpr int NT = G * T;
-    constexpr int HX = FT / 2 + 1;
-    constexpr int MG = T < 16 ? T : 16;   // run-merge group: lanes of one column
-    constexpr int LDSN = G * FT + FT;
-    constexpr int SCAP = MODE == MODE_FILL ? BSX_STAGE_CAP : 1;
-    constexpr int SHASH = MODE == MODE_FILL ? BSX_STAGE_HASH : 1;
-    __shared__ float2 lds[LDSN];
-    __shared__ float4 st_ent[SCAP];
-    __shared__ float2 st_ent2[FOM ? SCAP : 1];
-    __shared__ int4 st_hinfo[SHASH];
-    __shared__ int st_hkey[SHASH], st_hcnt[SHASH], st_nent;
-    const int tid = threadIdx.x;
-    const int g = tid / T, t = tid - g * T;
-    const long task = (long)blockIdx.x * G + g;
-    const int p = (int)(task / HX);
-    const int x = (int)(task - (long)p * HX);
-    const bool valid = p < nb;
-    float2* line = lds + g * FT;
-    {
-        float2* tw = lds + G * FT;
-        for (int i = tid; i < FT; i += NT) tw[i] = twg[i];
-        const float2* col = inter + ((size_t)p * HX + x) * box;
-        for (int i = t; i < FT; i += T) line[i] = (valid && i < box) ? col[i] : make_float2(0.f, 0.f);
-        __syncthreads();
-        FftLine<FT, -1, T>::run(line, tw, t);
-    }
-    // staging (pair entries: at most one binned emission per thread and
-    // round, so 2 rounds fit the list; the 512-entry list keeps the LDS of a
-    // workgroup under 32 KB, 5 workgroups per CU)
-    const bool staged = FAST || (MODE == MODE_FILL && K.pairs && NT == 256 &&
-                                 2 * NT <= BSX_STAGE_CAP);
-    bc.st = Stage{st_ent, &st_nent, st_hkey, st_hcnt, st_hinfo, staged ? 1 : 0,
-                  FOM ? st_ent2 : nullptr};
-    if (staged) {
-        if (tid < BSX_STAGE_HASH) {
-            st_hkey[tid] = -1;
-            st_hcnt[tid] = 0;
-        }
-        if (tid == 0) st_nent = 0;
-        __syncthreads();
-    }
-    // At FT 512 a wavefront is one column (T == 64), so its particle is
-    // uniform: the record is then read with scalar loads, kept in SGPRs.
-    const int prec = valid ? p : 0;
-    const PartDev& P = recs[T == 64 ? __builtin_amdgcn_readfirstlane(prec) : prec];
-    const unsigned keybase = (unsigned)P.half * (unsigned)(K.NT * K.NT * K.NT) * 4096u;
-    const float inv = 1.0f / FT;
-    const float b = valid ? bkg[p] : 0.f;
-    const long h = (x <= (FT - 1) / 2) ? x : x - FT;
-    const bool mirror = valid && x >= 1 && x <= FT / 2 - 1;
-    const int merge = K.merge;
-    // phase factor of this thread's sample, advanced by exact FP64 rotations
-    // (k grows by T per round and wraps by -FT after round 3, as y passes FT/2)
-    double er, ei;
-    {
-        float sn, cs;
-        sincos_red((double)h * P.phx + (double)t * P.phy, &sn, &cs);
-        er = cs;
-        ei = sn;
-    }
-#pragma unroll 1
-    for (int r = 0; r < 8; ++r) {
-        const int y = t + r * T;
-        float2 F = line[y];
-        F.x *= inv;
-        F.y *= inv;
-        if (x == 0 && y == 0) F.x += b * FT;
-        const long k = (y <= (FT - 1) / 2) ? y : y - FT;
-        // Friedel mate of the column: array position (FT-x, FT-y), value conj
-        const int ym = (FT - y) & (FT - 1);
-        const long km = (ym <= (FT - 1) / 2) ? ym : ym - FT;
-        insert_pair<MG, FOM, MODE, FAST>(acc, K, P, valid, mirror, h, k, km, F, merge, keybase, bc,
-                                   make_float2((float)er, (float)ei));
-        {
-            const double c = r == 3 ? P.rot[2] : P.rot[0], sd = r == 3 ? P.rot[3] : P.rot[1];
-            const double nr = er * c - ei * sd;
-            ei = er * sd + ei * c;
-            er = nr;
-        }
-        if (MODE == MODE_FILL && staged && (r & 1) == 1) stage_flush(bc);
-    }
-}
-
-// Bins are processed in pieces of at most `piece` entries (a whole number of
-// chunks, 8192 to 32768; 16384 by default, chosen by bsx_recon_autotune) so
-// that the few hot bins around the origin (every plane passes through the
-// low-frequency core) are spread over many workgroups.
-#define BSX_PIECE_DEFAULT 16384
-#define BSX_PIECE_MIN 8192
-#define BSX_PIECE_MAX 32768
-
 // Per-bin piece offsets (one workgroup): poff[b] = sum over bins below b of
 // ceil(binned / PIECE), poff[nbins] = all pieces, pbin[piece] = its bin (at
 // most maxpieces pieces are listed); `total` accumulates the entries binned
@@ -1108,6 +218,27 @@ __global__ void k_set32(unsigned* __restrict__ p, long long n, unsigned v, int v
     uint4* q = reinterpret_cast<uint4*>(p);
     for (long long i = t; i < n4; i += stride) q[i] = make_uint4(v, v, v, v);
     for (long long i = 4 * n4 + t; i < n; i += stride) p[i] = v;
+}
+
+// One launch for the clears of a reset: the volume records a (na words), and
+// where they are not clean already the binned accumulator x (nx words), the bin
+// counters f (nf) and the chunk table c (nc, to -1); pool: the free-chunk
+// counter and the fallback flags. a, x: 16-byte aligned.
+__global__ __launch_bounds__(256) void k_reset(unsigned* __restrict__ a, long long na,
+                                               unsigned* __restrict__ x, long long nx,
+                                               unsigned* __restrict__ f, long long nf,
+                                               unsigned* __restrict__ c, long long nc,
+                                               unsigned* __restrict__ pool) {
+    const long long stride = (long long)gridDim.x * 256, t = blockIdx.x * 256LL + threadIdx.x;
+    uint4* a4 = reinterpret_cast<uint4*>(a);
+    for (long long i = t; i < na / 4; i += stride) a4[i] = make_uint4(0, 0, 0, 0);
+    for (long long i = na / 4 * 4 + t; i < na; i += stride) a[i] = 0;
+    uint4* x4 = reinterpret_cast<uint4*>(x);
+    for (long long i = t; i < nx / 4; i += stride) x4[i] = make_uint4(0, 0, 0, 0);
+    for (long long i = nx / 4 * 4 + t; i < nx; i += stride) x[i] = 0;
+    for (long long i = t; i < nf; i += stride) f[i] = 0;
+    for (long long i = t; i < nc; i += stride) c[i] = 0xFFFFFFFFu;
+    if (t < 2 && pool) pool[t] = 0;
 }
 
 // Clears the bin counters and the used chunk-table entries for the next
@@ -1257,87 +388,153 @@ __global__ __launch_bounds__(512) void k_tile_accum(const int* __restrict__ fill
 }
 
 // ------------------------------------------------------------------- K4
+// FP64 values added over a workgroup of 16 wavefronts, then atomically to
+// dst[q] by one thread.
+template <int Q>
+__device__ __forceinline__ void block_add(double (&v)[Q], double* __restrict__ dst) {
+    __shared__ double sh[16][Q];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) v[q] += __shfl_xor(v[q], o, 64);
+        if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6][q] = v[q];
+    }
+    __syncthreads();
+    if (threadIdx.x < Q) {
+        double t = 0;
+        for (int w = 0; w < (int)blockDim.x / 64; ++w) t += sh[w][threadIdx.x];
+        atomicAdd(dst + threadIdx.x, t);
+    }
+}
+
 // Sum of half sets, weighing (fspace_reconstruction_weigh,
 // Bimage_reconstruct.cpp:486-515) in FP64, SNR FOM (:610-634), centre shift
-// (phase_shift_to_center: x (-1)^(h+k+l) for even N, computed exactly via the
-// phase for odd N), output complex volume.
-__global__ __launch_bounds__(256) void k_weigh(const float* __restrict__ acc, long long n3, int N,
-                                               int NT, long long nrec, int stride, int hmask,
-                                               int nhalves, int fom,
-                                               float2* __restrict__ out,
-                                               float* __restrict__ fom_out,
-                                               unsigned long long* __restrict__ cov,
-                                               double* __restrict__ wsum) {
-    long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    double wloc = 0;
-    int cloc = 0;
-    for (; i < n3; i += (long long)gridDim.x * blockDim.x) {
-        double fr = 0, fi = 0, W = 0, P = 0, W2 = 0;
-        const long long ri = rec_index(i % N, (i / N) % N, i / ((long long)N * N), NT);
+// (phase_shift_to_center: x (-1)^(h+k+l), N being even) and the Friedel
+// residual sums (Bimage::friedel_check, Bimage_fspace.cpp:2024-2074). With FOLD the binned accumulator X is first
+// brought into the records S and cleared, as k_fold does.
+//
+// One thread takes a voxel v and its Friedel mate u = -v: the fold needs both
+// X records, the residual both weighed values, so each record is read once and
+// nothing is read back. fin: coverage, sum w, and the residual's sums of w,
+// w dre^2, w dim^2 over the half space x < N / 2 (on the plane x = 0
+// both voxels of a pair count).
+// Bound by memory at large maps; at small ones by the workgroups' five
+// atomics, so at most 512 workgroups of 1024 threads run. The three separate
+// passes this replaces (fold, weigh, residual; 2,048 workgroups each, the fold
+// repeated for every map): 96 -> 8 us at 32^3, 603 -> 164 us for the three maps
+// of two 128^3 halves with FOM sums.
+template <bool FOM, bool FOLD>
+__global__ __launch_bounds__(1024) void k_weigh_pairs(float* __restrict__ S, float* __restrict__ X,
+                                                      int N, int nz, int NT, long long nrec, int hmask,
+                                                      int nhalves, float2* __restrict__ out,
+                                                      float* __restrict__ fom_out,
+                                                      double* __restrict__ fin) {
+    constexpr int RS = FOM ? 5 : 3;
+    const unsigned nxh = N / 2 + 1, total = nxh * (unsigned)N * (unsigned)nz;
+    double sums[5] = {0, 0, 0, 0, 0};
+    for (unsigned i = blockIdx.x * 1024u + threadIdx.x; i < total; i += gridDim.x * 1024u) {
+        const int x = (int)(i % nxh);
+        const unsigned yz = i / nxh;
+        const int y = (int)(yz % (unsigned)N), z = (int)(yz / (unsigned)N);
+        const int mx = x ? N - x : 0, my = y ? N - y : 0, mz = z ? nz - z : 0;
+        // planes that hold their own mates: the lower (y, z) takes the pair
+        if (mx == x && mz * N + my < z * N + y) continue;
+        const bool self = mx == x && my == y && mz == z;
+        const size_t rv = (size_t)rec_index(x, y, z, NT) * RS;
+        const size_t ru = (size_t)rec_index(mx, my, mz, NT) * RS;
+        double av[5] = {0, 0, 0, 0, 0}, au[5] = {0, 0, 0, 0, 0};
         for (int hh = 0; hh < nhalves; ++hh) {
-            if (!((hmask >> hh) & 1)) continue;
-            const float* r = acc + ((size_t)hh * nrec + ri) * stride;
-            fr += r[0];
-            fi += r[1];
-            W += r[2];
-            if (fom) { P += r[3]; W2 += r[4]; }
-        }
-        wloc += W;
-        float ofr = 0.f, ofi = 0.f, oP = 0.f;
-        if (W > 1e-30) {
-            ofr = (float)(fr / W);
-            ofi = (float)(fi / W);
-            if (fom) {
-                const double w2 = W - W2 / W;
-                if (w2 > 1) P /= w2;
-                else if (W > 1) P /= W;
-                if (P < 0) P = 0;
+            const bool want = (hmask >> hh) & 1;
+            if (!FOLD && !want) continue;
+            float* s = S + (size_t)hh * nrec * RS;
+            float sv[RS], su[RS];
+#pragma unroll
+            for (int c = 0; c < RS; ++c) {
+                sv[c] = s[rv + c];
+                su[c] = s[ru + c];
             }
-            ++cloc;
-        } else {
-            P = 0;
-            W = 1e-30;
+            if (FOLD) {
+                float* xa = X + (size_t)hh * nrec * RS;
+                float xv[RS], xu[RS];
+#pragma unroll
+                for (int c = 0; c < RS; ++c) {
+                    xv[c] = xa[rv + c];
+                    xu[c] = xa[ru + c];
+                }
+#pragma unroll
+                for (int c = 0; c < RS; ++c) {
+                    // a pair entry stands for its value at v and the conjugate
+                    // at -v; the weights and FOM sums are those of both
+                    const float m = c == 1 ? -xu[c] : xu[c];
+                    sv[c] += xv[c] + m;
+                    su[c] += c == 1 ? xu[c] - xv[c] : xu[c] + xv[c];
+                    s[rv + c] = sv[c];
+                    xa[rv + c] = 0.f;
+                    if (!self) {
+                        s[ru + c] = su[c];
+                        xa[ru + c] = 0.f;
+                    }
+                }
+            }
+            if (want)
+#pragma unroll
+                for (int c = 0; c < RS; ++c) {
+                    av[c] += sv[c];
+                    au[c] += su[c];
+                }
         }
-        if (fom_out) {
-            if (i == 0) P = 1;
-            const double signal = (double)ofr * ofr + (double)ofi * ofi;
-            double noise = P - signal;
-            if (noise < signal) noise = signal;
-            if (W > 1 && signal > 1e-30 && noise > 1e-30) oP = (float)((W * signal - P) / noise);
-            else oP = 0.f;
-            if (i == 0) oP = 1.f;
-            fom_out[i] = oP;
+        const bool odd = (x + y + z) & 1;
+        float2 val[2];
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+            if (m == 1 && self) {
+                val[1] = val[0];
+                continue;
+            }
+            const double* a = m ? au : av;
+            double W = a[2], P = FOM ? a[3] : 0;
+            sums[1] += W;
+            float ofr = 0.f, ofi = 0.f;
+            if (W > 1e-30) {
+                ofr = (float)(a[0] / W);
+                ofi = (float)(a[1] / W);
+                if (FOM) {
+                    const double w2 = W - a[4] / W;
+                    if (w2 > 1) P /= w2;
+                    else if (W > 1) P /= W;
+                    if (P < 0) P = 0;
+                }
+                sums[0] += 1;
+            } else {
+                P = 0;
+                W = 1e-30;
+            }
+            const size_t at = m ? ((size_t)mz * N + my) * N + mx : ((size_t)z * N + y) * N + x;
+            if (fom_out) {
+                if (at == 0) P = 1;
+                const double signal = (double)ofr * ofr + (double)ofi * ofi;
+                double noise = P - signal;
+                if (noise < signal) noise = signal;
+                float oP = 0.f;
+                if (W > 1 && signal > 1e-30 && noise > 1e-30) oP = (float)((W * signal - P) / noise);
+                if (at == 0) oP = 1.f;
+                fom_out[at] = oP;
+            }
+            val[m] = odd ? make_float2(-ofr, -ofi) : make_float2(ofr, ofi);
+            out[at] = val[m];
         }
-        const long long xx = i % N, yy = (i / N) % N, zz = i / ((long long)N * N);
-        const long h = xx > (N - 1) / 2 ? xx - N : xx;
-        const long k = yy > (N - 1) / 2 ? yy - N : yy;
-        const long l = zz > (N - 1) / 2 ? zz - N : zz;
-        if ((N & 1) == 0) {
-            if ((h + k + l) & 1) { ofr = -ofr; ofi = -ofi; }
-        } else {
-            const double t = -2 * M_PI * (double)(N / 2) / N;
-            double sn, cs;
-            sincos(h * t + k * t + l * t, &sn, &cs);
-            const double a = ofr, b = ofi;
-            ofr = (float)(a * cs - b * sn);
-            ofi = (float)(a * sn + b * cs);
+        if (x < N / 2) {
+            const float2 a = val[0], b = val[1];
+            const double n = (x == 0 && !self) ? 2 : 1;
+            const double w = n * ((double)a.x * a.x + (double)a.y * a.y + (double)b.x * b.x + (double)b.y * b.y) / 2;
+            double d = (double)a.x - b.x;
+            sums[3] += d * d * w;
+            d = (double)a.y + b.y;
+            sums[4] += d * d * w;
+            sums[2] += w;
         }
-        out[i] = make_float2(ofr, ofi);
     }
-    // block reductions of coverage and weight
-    __shared__ double sw[256];
-    __shared__ unsigned int sc[256];
-    sw[threadIdx.x] = wloc;
-    sc[threadIdx.x] = cloc;
-    __syncthreads();
-    for (int o = blockDim.x / 2; o > 0; o >>= 1) {
-        if (threadIdx.x < o) { sw[threadIdx.x] += sw[threadIdx.x + o]; sc[threadIdx.x] += sc[threadIdx.x + o]; }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        atomicAdd(cov, (unsigned long long)sc[0]);
-        atomicAdd(wsum, sw[0]);
-    }
+    block_add(sums, fin);
 }
 
 // Shell sums of fspace_reconstruction_stats (Bimage_reconstruct.cpp:526-599).
@@ -1444,39 +641,6 @@ __global__ void k_stats_sum(const double* __restrict__ part, int nblocks, int m,
     out[i] = s;
 }
 
-// Friedel residual sums (Bimage::friedel_check, Bimage_fspace.cpp:2024-2074).
-__global__ __launch_bounds__(256) void k_friedel(const float2* __restrict__ v, int N, int nz,
-                                                 double* __restrict__ sums) {
-    const long long nx2 = (N + 1) / 2;
-    const long long total = nx2 * N * nz;
-    double s = 0, rr = 0, ri = 0;
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < total;
-         i += (long long)gridDim.x * blockDim.x) {
-        const long long xx = i % nx2, yy = (i / nx2) % N, zz = i / (nx2 * N);
-        const long long xf = xx ? N - xx : 0, yf = yy ? N - yy : 0, zf = zz ? nz - zz : 0;
-        const float2 a = v[(zz * N + yy) * N + xx];
-        const float2 b = v[(zf * N + yf) * N + xf];
-        const double w = ((double)a.x * a.x + (double)a.y * a.y + (double)b.x * b.x + (double)b.y * b.y) / 2;
-        double d = (double)a.x - b.x;
-        rr += d * d * w;
-        d = (double)a.y + b.y;
-        ri += d * d * w;
-        s += w;
-    }
-    __shared__ double sh[3][256];
-    sh[0][threadIdx.x] = s;
-    sh[1][threadIdx.x] = rr;
-    sh[2][threadIdx.x] = ri;
-    __syncthreads();
-    for (int o = blockDim.x / 2; o > 0; o >>= 1) {
-        if (threadIdx.x < o)
-            for (int q = 0; q < 3; ++q) sh[q][threadIdx.x] += sh[q][threadIdx.x + o];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0)
-        for (int q = 0; q < 3; ++q) atomicAdd(sums + q, sh[q][0]);
-}
-
 // Folds the binned accumulator X into the volume records S (3 floats per
 // record, both in the tiled layout, `nrec` records per half) and clears X.
 // pairs = 0: X holds plain sums, S += X. pairs = 1: an X record at v stands
@@ -1552,75 +716,6 @@ __global__ void k_set_planes(float* __restrict__ acc, long long n3, int N, int N
 }
 
 // ================================================================== host side
-struct bsx_recon {
-    bsx_recon_params p;
-    ReconConst K;
-    double hi_res;
-    int dev;
-    bool binned = true;            // tile-binned insertion (else direct atomics)
-    float* acc = nullptr;
-    float* xacc = nullptr;         // binned accumulator, folded into acc by k_fold
-    size_t acc_elems = 0;
-    float2* inter = nullptr;
-    float* bkg = nullptr;
-    double2* resc = nullptr;       // per record (scale, shift) of -rescale (flags bit 1)
-    PartDev* recs = nullptr;
-    int* nonfinite = nullptr;
-    int64_t recs_cap = 0;
-    int* fill = nullptr;           // per (half, tile) bin: entries reserved
-    int* chunks = nullptr;         // per bin: pool chunk of each bin chunk
-    int* pool = nullptr;           // next free chunk, fallback flags
-    int npool = 0;
-    int maxc = 0;
-    int* poff = nullptr;           // piece offsets per bin
-    int* pbin = nullptr;           // bin of each piece
-    unsigned long long* entries = nullptr;   // bin entries of the current insert
-    float4* bins = nullptr;
-    float2* bins2 = nullptr;       // FOM sums of the pool entries (FOM only)
-    size_t bins_cap = 0;
-    int nbins = 0;
-    int batch = 0;
-    int batch_cap = 0;               // batch the buffers were sized for
-    int piece = BSX_PIECE_DEFAULT;   // tile-pass piece length (entries)
-    int64_t inserted[2] = {0, 0};
-    int fallback_flags = 0;        // atomic-fallback flags seen (1 table, 2 pool, 4 wait bound)
-    double ktime[7] = {0, 0, 0, 0, 0, 0, 0};   // background rows fallback scan fill tile direct
-    double last_entries = 0;
-    int64_t last_launches = 0;
-    std::vector<hipEvent_t> evs;
-    std::vector<int> evlab;
-    size_t nev = 0;
-    size_t bytes = 0;
-    PartDev* hrecs = nullptr;      // pinned staging of the records
-    int64_t hrecs_cap = 0;
-    hipEvent_t copied = nullptr;   // staging buffer reusable once this completes
-    bool timing = false;
-    // BSX_FLAG_GRAPH: the batch loop of an insert, captured on the second
-    // call with the same (images, record count, batch, run merge, piece) and
-    // replayed while that set is inserted again; up to 8 such sets (e.g. the
-    // chunks of a pipelined insert) are kept, the least recently used evicted
-    struct GraphEntry {
-        const float* imgs;
-        int64_t n;
-        int batch, merge, piece;   // kernel constants baked into the graph
-        int seen;                  // calls seen (capture on the second)
-        hipGraphExec_t exec;
-        uint64_t used;
-    };
-    std::vector<GraphEntry> graphs;
-    uint64_t graph_clock = 0;
-    int64_t graph_launches = 0;
-    hipStream_t cap_stream = nullptr;   // capture happens here (the caller's stream may be
-                                        // the legacy default stream, which cannot capture)
-    std::vector<int> sym_order;         // point-group operator orders (empty: C1)
-    std::vector<double> sym_axis;       // their unit axes, 3 per operator
-    // group runs (bsx_recon_group_run): weighed transform and the finish
-    // sums (coverage count, 4 FP64 sums), kept so that the finish needs no
-    // allocation inside a captured graph
-    float2* gvol = nullptr;
-    unsigned long long* gfin = nullptr;
-};
-
 // Drops every captured insert graph (their kernels hold the record buffers'
 // addresses and the record count).
 static void clear_graphs(bsx_recon* h) {
@@ -1628,9 +723,6 @@ static void clear_graphs(bsx_recon* h) {
         if (e.exec) (void)hipGraphExecDestroy(e.exec);
     h->graphs.clear();
 }
-
-// KT_FALLBACK holds the atomic-fallback flags of the insert, not a time
-enum { KT_BG = 0, KT_ROWS, KT_FALLBACK, KT_SCAN, KT_FILL, KT_TILE, KT_DIRECT, KT_END };
 
 // Timing marks: an event after each kernel, labelled with the kernel it closes.
 static int tmark(bsx_recon* h, hipStream_t s, int label) {
@@ -1984,90 +1076,39 @@ __global__ __launch_bounds__(256) void k_sym_op(const float* __restrict__ in,
     out[v] = acc;
 }
 
-template <int FT>
-static int launch_batch(bsx_recon* h, const float* imgs, int64_t p0, int nb, hipStream_t s) {
-    constexpr int T = FftThreads<FT>::value;
-    constexpr int G = 256 / T;
-    // one line per column group: 8 rows per workgroup at FT = 512 (20 KB of
-    // LDS, 8 workgroups per CU; 16 rows measured 12 % slower)
-    constexpr int LINES = G;
-    constexpr int NT = G * T;
-    const int box = h->p.box;
-    const float2* tw = twiddles(FT, s);
-    BSX_REQUIRE(tw, BSX_ERR_DEVICE, "twiddles(%d) failed", FT);
-    const int tiles = (box + 2 * LINES - 1) / (2 * LINES);
-    hipLaunchKernelGGL((k_rows<FT, LINES>), dim3(nb * tiles), dim3(NT), 0, s, imgs,
-                       h->recs + p0, h->bkg + p0, box, tiles, h->inter, tw,
-                       h->resc ? h->resc + p0 : nullptr);
-    BSX_HIP(hipGetLastError());
-    int r = tmark(h, s, KT_ROWS);
-    if (r) return r;
-    const long ntask = (long)nb * (FT / 2 + 1);
-    const dim3 grid((unsigned)((ntask + G - 1) / G));
-    const PartDev* rec = h->recs + p0;
-    const float* bk = h->bkg + p0;
-    if (h->binned) {
-        BinCtx bf{h->fill,  h->chunks, h->pool,  h->bins,       h->xacc,
-                  h->npool, h->maxc,   Stage{}, h->bins2,      h->K.stride};
-        // nearest-neighbour pair entries with LDS staging: the specialised
-        // kernel; with the FOM sums the generic kernel reserves per wavefront
-        if (h->K.fom)
-            hipLaunchKernelGGL((k_cols<FT, true, MODE_FILL>), grid, dim3(NT), 0, s, h->inter, bk,
-                               rec, nb, box, h->K, h->acc, tw, bf);
-        else if (h->K.pairs && h->K.interp == 0 && !h->K.ewald && NT == 256)
-            hipLaunchKernelGGL((k_cols<FT, false, MODE_FILL, 1>), grid, dim3(NT), 0, s, h->inter,
-                               bk, rec, nb, box, h->K, h->acc, tw, bf);
-        else if (h->K.pairs && h->K.interp == 1 && !h->K.ewald && NT == 256)
-            hipLaunchKernelGGL((k_cols<FT, false, MODE_FILL, 2>), grid, dim3(NT), 0, s, h->inter,
-                               bk, rec, nb, box, h->K, h->acc, tw, bf);
-        else
-            hipLaunchKernelGGL((k_cols<FT, false, MODE_FILL>), grid, dim3(NT), 0, s, h->inter, bk,
-                               rec, nb, box, h->K, h->acc, tw, bf);
-        BSX_HIP(hipGetLastError());
-        if ((r = tmark(h, s, KT_FILL))) return r;
-        const unsigned maxpieces = (unsigned)(h->nbins + (size_t)h->npool * BSX_CHUNK / h->piece + 1);
-        hipLaunchKernelGGL(k_piece_scan, dim3(1), dim3(1024), 0, s, h->fill, h->nbins, h->maxc,
-                           h->piece, h->poff, h->pbin, (int)maxpieces, h->entries);
-        BSX_HIP(hipGetLastError());
-        if ((r = tmark(h, s, KT_SCAN))) return r;
-        if (h->K.fom)
-            hipLaunchKernelGGL(k_tile_accum<true>, dim3(maxpieces), dim3(512), 0, s, h->fill,
-                               h->chunks, h->maxc, h->piece, h->poff, h->pbin, h->nbins, h->bins,
-                               h->bins2, h->xacc);
-        else
-            hipLaunchKernelGGL(k_tile_accum<false>, dim3(maxpieces), dim3(512), 0, s, h->fill,
-                               h->chunks, h->maxc, h->piece, h->poff, h->pbin, h->nbins, h->bins,
-                               nullptr, h->xacc);
-        BSX_HIP(hipGetLastError());
-        hipLaunchKernelGGL(k_bin_reset, dim3((h->nbins + 255) / 256), dim3(256), 0, s, h->fill,
-                           h->chunks, h->maxc, h->nbins, h->pool);
-        BSX_HIP(hipGetLastError());
-        if ((r = tmark(h, s, KT_TILE))) return r;
-    } else {
-        BinCtx bc{nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, Stage{}, nullptr, h->K.stride};
-        if (h->K.fom)
-            hipLaunchKernelGGL((k_cols<FT, true, MODE_DIRECT>), grid, dim3(NT), 0, s, h->inter,
-                               bk, rec, nb, box, h->K, h->acc, tw, bc);
-        else
-            hipLaunchKernelGGL((k_cols<FT, false, MODE_DIRECT>), grid, dim3(NT), 0, s, h->inter,
-                               bk, rec, nb, box, h->K, h->acc, tw, bc);
-        BSX_HIP(hipGetLastError());
-        if ((r = tmark(h, s, KT_DIRECT))) return r;
-    }
-    return BSX_OK;
-}
-
+// Insertion of one batch: rows and fill, then for binned entries the piece
+// table, the tile pass and the clearing of the bins.
 static int run_batch(bsx_recon* h, const float* imgs, int64_t p0, int nb, hipStream_t s) {
+    int r;
     switch (h->p.ft_size) {
-        case 32: return launch_batch<32>(h, imgs, p0, nb, s);
-        case 64: return launch_batch<64>(h, imgs, p0, nb, s);
-        case 128: return launch_batch<128>(h, imgs, p0, nb, s);
-        case 256: return launch_batch<256>(h, imgs, p0, nb, s);
-        case 512: return launch_batch<512>(h, imgs, p0, nb, s);
+        case 32: r = insert_batch<32>(h, imgs, p0, nb, s, tmark); break;
+        case 64: r = insert_batch<64>(h, imgs, p0, nb, s, tmark); break;
+        case 128: r = insert_batch<128>(h, imgs, p0, nb, s, tmark); break;
+        case 256: r = insert_batch<256>(h, imgs, p0, nb, s, tmark); break;
+        case 512: r = insert_batch<512>(h, imgs, p0, nb, s, tmark); break;
         default:
             set_error("ft_size %d not supported (32..512, power of 2)", h->p.ft_size);
             return BSX_ERR_ARG;
     }
+    if (r || !h->binned) return r;
+    const unsigned maxpieces = (unsigned)(h->nbins + (size_t)h->npool * BSX_CHUNK / h->piece + 1);
+    hipLaunchKernelGGL(k_piece_scan, dim3(1), dim3(1024), 0, s, h->fill, h->nbins, h->maxc,
+                       h->piece, h->poff, h->pbin, (int)maxpieces, h->entries);
+    BSX_HIP(hipGetLastError());
+    if ((r = tmark(h, s, KT_SCAN))) return r;
+    if (h->K.fom)
+        hipLaunchKernelGGL(k_tile_accum<true>, dim3(maxpieces), dim3(512), 0, s, h->fill,
+                           h->chunks, h->maxc, h->piece, h->poff, h->pbin, h->nbins, h->bins,
+                           h->bins2, h->xacc);
+    else
+        hipLaunchKernelGGL(k_tile_accum<false>, dim3(maxpieces), dim3(512), 0, s, h->fill,
+                           h->chunks, h->maxc, h->piece, h->poff, h->pbin, h->nbins, h->bins,
+                           nullptr, h->xacc);
+    BSX_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_bin_reset, dim3((h->nbins + 255) / 256), dim3(256), 0, s, h->fill,
+                       h->chunks, h->maxc, h->nbins, h->pool);
+    BSX_HIP(hipGetLastError());
+    return tmark(h, s, KT_TILE);
 }
 
 extern "C" {
@@ -2266,16 +1307,14 @@ int bsx_recon_destroy(bsx_recon* h) {
 
 int bsx_recon_reset(bsx_recon* h, void* stream) {
     BSX_REQUIRE(h, BSX_ERR_ARG, "null handle");
-    BSX_HIP(hipMemsetAsync(h->acc, 0, h->acc_elems * sizeof(float), (hipStream_t)stream));
-    if (h->binned) {
-        BSX_HIP(hipMemsetAsync(h->xacc, 0, h->acc_elems * sizeof(float), (hipStream_t)stream));
-        // bin state is cleared after every batch; cleared again here in case an
-        // earlier insert stopped between its fill and its reset
-        BSX_HIP(hipMemsetAsync(h->fill, 0, sizeof(int) * h->nbins, (hipStream_t)stream));
-        BSX_HIP(hipMemsetAsync(h->chunks, 0xFF, sizeof(int) * (size_t)h->nbins * h->maxc,
-                               (hipStream_t)stream));
-        BSX_HIP(hipMemsetAsync(h->pool, 0, sizeof(int) * 2, (hipStream_t)stream));
-    }
+    const long long n = (long long)h->acc_elems;
+    const bool x = h->binned && h->xdirty, b = h->binned && h->bins_dirty;
+    hipLaunchKernelGGL(k_reset, dim3((unsigned)std::min(2048LL, (n / 4 + 255) / 256)), dim3(256), 0,
+                       (hipStream_t)stream, (unsigned*)h->acc, n, (unsigned*)h->xacc, x ? n : 0,
+                       (unsigned*)h->fill, b ? (long long)h->nbins : 0, (unsigned*)h->chunks,
+                       b ? (long long)h->nbins * h->maxc : 0, (unsigned*)h->pool);
+    BSX_HIP(hipGetLastError());
+    h->xdirty = h->bins_dirty = false;
     h->inserted[0] = h->inserted[1] = 0;
     return BSX_OK;
 }
@@ -2483,6 +1522,7 @@ int bsx_recon_insert(bsx_recon* h, const float* imgs_dev, const bsx_particle* pa
         BSX_HIP(hipStreamSynchronize(s));
         BSX_REQUIRE(!bad, BSX_ERR_NONFINITE, "non-finite values in the particle images");
     }
+    h->xdirty = h->bins_dirty = h->binned;
     const int64_t nbatches = (n + h->batch - 1) / h->batch;
     auto batch_loop = [&](hipStream_t st) -> int {
         for (int64_t b = 0; b < nbatches; ++b) {
@@ -2541,6 +1581,7 @@ int bsx_recon_insert(bsx_recon* h, const float* imgs_dev, const bsx_particle* pa
                                                       nullptr, ++h->graph_clock});
         }
     }
+    h->bins_dirty = false;   // every batch cleared its bins
     h->inserted[0] += add[0];
     h->inserted[1] += add[1];
     h->last_launches = nbatches;
@@ -2944,14 +1985,15 @@ int bsx_recon_kernel_times(const bsx_recon* h, double* ms, int n) {
 }
 
 // Brings the binned accumulator into the volume records (stream-ordered after
-// the inserts); a no-op pass when nothing was binned since the last fold.
+// the inserts) where entries were binned since the last fold.
 static int fold(bsx_recon* h, hipStream_t s) {
-    if (!h->binned) return BSX_OK;
+    if (!h->binned || !h->xdirty) return BSX_OK;
     const long long n3 = (long long)h->K.N * h->K.N * h->K.N;
     const long long nrec = (long long)h->K.NT * h->K.NT * h->K.NT * 4096;
     hipLaunchKernelGGL(k_fold, dim3(2048), dim3(256), 0, s, h->acc, h->xacc, n3, h->K.N, h->K.NT,
                        nrec, h->p.nhalves, h->K.pairs, h->K.stride);
     BSX_HIP(hipGetLastError());
+    h->xdirty = false;
     return BSX_OK;
 }
 
@@ -3088,19 +2130,22 @@ int bsx_recon_stats(bsx_recon* h, int imap, int nmaps, double resolution, double
     return BSX_OK;
 }
 
-// Weighing of the summed halves in hmask into vol (and the FOM map) with the
-// coverage count and the FP64 weight and Friedel sums accumulated into fin
-// (a coverage counter followed by 4 doubles), which the caller has cleared.
-static int launch_weigh(bsx_recon* h, int hmask, float2* vol, float* fom_dev,
-                        unsigned long long* fin, hipStream_t s) {
+// Weighing of the summed halves in hmask into vol (and the FOM map), after
+// folding the binned accumulator where `fold` is set; the coverage count and the
+// weight and Friedel sums are added to fin (5 doubles), which the caller has
+// cleared.
+static int launch_weigh(bsx_recon* h, int hmask, bool fold, float2* vol, float* fom_dev, double* fin,
+                        hipStream_t s) {
     const int N = h->K.N, nz = h->K.nz;
-    const long long n3 = (long long)N * N * nz;
     const long long nrec = (long long)h->K.NT * h->K.NT * h->K.NT * 4096;
-    double* dsum = (double*)(fin + 1);
-    hipLaunchKernelGGL(k_weigh, dim3(2048), dim3(256), 0, s, h->acc, n3, N, h->K.NT, nrec,
-                       h->K.stride, hmask, h->p.nhalves, h->K.fom, vol, fom_dev, fin, dsum);
-    BSX_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_friedel, dim3(1024), dim3(256), 0, s, vol, N, nz, dsum + 1);
+    const long long pairs = (long long)(N / 2 + 1) * N * nz;
+    const dim3 grid((unsigned)std::min(512LL, (pairs + 1023) / 1024));
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(1024), 0, s, h->acc, h->xacc, N, nz, h->K.NT, nrec, hmask,
+                           h->p.nhalves, vol, fom_dev, fin);
+    };
+    if (h->K.fom) fold ? go(k_weigh_pairs<true, true>) : go(k_weigh_pairs<true, false>);
+    else fold ? go(k_weigh_pairs<false, true>) : go(k_weigh_pairs<false, false>);
     BSX_HIP(hipGetLastError());
     return BSX_OK;
 }
@@ -3120,12 +2165,11 @@ static int launch_inverse(bsx_recon* h, float2* work, float* map_dev, hipStream_
     return r;
 }
 
-// The stats of a finish from the coverage count and the sums of launch_weigh.
-static void fill_stats(const bsx_recon* h, int hmask, unsigned long long cov, const double* sum,
-                       bsx_stats* stats) {
-    stats->coverage = (int64_t)cov;
-    stats->weight_sum = sum[0];
-    double sw = sum[1], rr = sum[2], ri = sum[3];
+// The stats of a finish from the sums of launch_weigh.
+static void fill_stats(const bsx_recon* h, int hmask, const double* fin, bsx_stats* stats) {
+    stats->coverage = (int64_t)fin[0];
+    stats->weight_sum = fin[1];
+    double sw = fin[2], rr = fin[3], ri = fin[4];
     double fr = 0;
     if (sw > 0) {
         rr = sqrt(rr / sw);
@@ -3154,8 +2198,6 @@ int bsx_recon_finish(bsx_recon* h, int imap, int nmaps, float* map_dev, float* f
     }
     hipStream_t s = (hipStream_t)stream;
     BSX_HIP(hipSetDevice(h->dev));
-    const int rf = fold(h, s);
-    if (rf) return rf;
     const int N = h->K.N, nz = h->K.nz;
     const long long n3 = (long long)N * N * nz;   // a 2D map: one plane
     float2* vol = (float2*)ft_dev;
@@ -3164,19 +2206,16 @@ int bsx_recon_finish(bsx_recon* h, int imap, int nmaps, float* map_dev, float* f
         BSX_HIP(hipMalloc((void**)&tmp, sizeof(float2) * n3));
         vol = tmp;
     }
-    unsigned long long* dcov = nullptr;
-    double* dsum = nullptr;
-    BSX_HIP(hipMalloc((void**)&dcov, sizeof(unsigned long long) + 4 * sizeof(double)));
-    dsum = (double*)(dcov + 1);
-    BSX_HIP(hipMemsetAsync(dcov, 0, sizeof(unsigned long long) + 4 * sizeof(double), s));
+    double* dfin = nullptr;
+    BSX_HIP(hipMalloc((void**)&dfin, 5 * sizeof(double)));
+    BSX_HIP(hipMemsetAsync(dfin, 0, 5 * sizeof(double), s));
     {
-        const int rw = launch_weigh(h, hmask, vol, fom_dev, dcov, s);
+        const int rw = launch_weigh(h, hmask, h->binned && h->xdirty, vol, fom_dev, dfin, s);
         if (rw) return rw;
+        h->xdirty = false;
     }
-    unsigned long long hcov = 0;
-    double hsum[4] = {0, 0, 0, 0};
-    BSX_HIP(hipMemcpyAsync(&hcov, dcov, sizeof(hcov), hipMemcpyDeviceToHost, s));
-    BSX_HIP(hipMemcpyAsync(hsum, dsum, 4 * sizeof(double), hipMemcpyDeviceToHost, s));
+    double fin[5] = {0, 0, 0, 0, 0};
+    BSX_HIP(hipMemcpyAsync(fin, dfin, sizeof(fin), hipMemcpyDeviceToHost, s));
     // atomic-fallback flags of the inserts since the last read (graph
     // replays included); cleared for the next inserts
     int hflags = 0;
@@ -3201,9 +2240,9 @@ int bsx_recon_finish(bsx_recon* h, int imap, int nmaps, float* map_dev, float* f
     BSX_HIP(hipStreamSynchronize(s));
     h->fallback_flags |= hflags;
     if (tmp) BSX_HIP(hipFree(tmp));
-    BSX_HIP(hipFree(dcov));
+    BSX_HIP(hipFree(dfin));
     if (r != BSX_OK) return r;
-    if (stats) fill_stats(h, hmask, hcov, hsum, stats);
+    if (stats) fill_stats(h, hmask, fin, stats);
     return BSX_OK;
 }
 
@@ -3239,9 +2278,8 @@ static int group_member_launch(bsx_recon* h, const float* imgs, int64_t n, float
         const int rr = run_batch(h, imgs, p0, (int)std::min<int64_t>(h->batch, n - p0), s);
         if (rr) return rr;
     }
-    int r = fold(h, s);
+    const int r = launch_weigh(h, h->p.nhalves > 1 ? 3 : 1, h->binned, h->gvol, nullptr, h->gfin, s);
     if (r) return r;
-    if ((r = launch_weigh(h, h->p.nhalves > 1 ? 3 : 1, h->gvol, nullptr, h->gfin, s))) return r;
     return launch_inverse(h, h->gvol, map_dev, s);
 }
 
@@ -3311,6 +2349,8 @@ int bsx_recon_group_run(bsx_recon_group* g, const float* const* imgs_dev,
         if (!h->gvol) BSX_HIP(hipMalloc((void**)&h->gvol, sizeof(float2) * n3));
         if (!h->gfin) BSX_HIP(hipMalloc((void**)&h->gfin, 64));
     }
+    // a run that stops half-way leaves its members to be cleared
+    for (bsx_recon* h : g->hs) h->xdirty = h->bins_dirty = h->binned;
     // host side of every member's insert: records uploaded on s
     std::vector<int64_t> nrec(m), add(2 * m);
     for (int i = 0; i < m; ++i) {
@@ -3379,11 +2419,11 @@ int bsx_recon_group_run(bsx_recon_group* g, const float* const* imgs_dev,
     }
     if (same) g->seen++;
     // finish sums and capacity-fallback flags of every member
-    std::vector<unsigned long long> fin(5 * m);
+    std::vector<double> fin(5 * m);
     std::vector<int> flags(m, 0);
     for (int i = 0; i < m; ++i) {
         bsx_recon* h = g->hs[i];
-        BSX_HIP(hipMemcpyAsync(&fin[5 * i], h->gfin, 5 * sizeof(unsigned long long),
+        BSX_HIP(hipMemcpyAsync(&fin[5 * i], h->gfin, 5 * sizeof(double),
                                hipMemcpyDeviceToHost, s));
         if (h->binned)
             BSX_HIP(hipMemcpyAsync(&flags[i], h->pool + 1, sizeof(int), hipMemcpyDeviceToHost, s));
@@ -3395,11 +2435,8 @@ int bsx_recon_group_run(bsx_recon_group* g, const float* const* imgs_dev,
         h->inserted[1] = add[2 * i + 1];
         h->fallback_flags |= flags[i];
         h->last_launches = (nrec[i] + h->batch - 1) / h->batch;
-        if (stats) {
-            double sum[4];
-            memcpy(sum, &fin[5 * i + 1], sizeof(sum));
-            fill_stats(h, h->p.nhalves > 1 ? 3 : 1, fin[5 * i], sum, &stats[i]);
-        }
+        h->xdirty = h->bins_dirty = false;   // cleared, inserted and folded above
+        if (stats) fill_stats(h, h->p.nhalves > 1 ? 3 : 1, &fin[5 * i], &stats[i]);
     }
     return BSX_OK;
 }
