@@ -7,6 +7,7 @@
 //        FSI_Kernel, include/FSI_Kernel.h:28-68), centre shift as project()
 //   k_fsc            : FP64 shell sums of Bimage::fsc (Bimage_resolution.cpp:330-406)
 //   k_frc_pairs      : img_recip_space_fom, fom_type 0 (src/mg/mg_refine.cpp:660-781)
+#include <climits>
 #include <cmath>
 #include <mutex>
 #include <vector>
@@ -46,35 +47,198 @@ __global__ void k_phase_origin(float2* __restrict__ v, int N, double sx, double 
 }
 
 // ------------------------------------------------------------- extraction
-// One thread per section pixel; blockIdx.y = view. Kernel table in LDS.
+// 8 x 8 pixel tiles of a section, WPT wavefronts each. The tile samples a patch of
+// a plane, so the taps of its 64 samples lie in a small box of the transform. A
+// lane's taps are scattered over many cache lines, and a load instruction costs
+// the texture path about a cycle per line it touches; with W^3 = 512 taps a
+// sample, each voxel of the box is used about 10 times.
+// WPT > 0: the box is loaded into LDS once (rows of 16 or 32 lanes), the taps are
+// read from there in the order and precision of fsi_sample, and the wavefronts
+// share the tap planes, whose sums are added in order. A box beyond `cap` voxels
+// (matrices that are no rotations) is sampled from memory.
+// WPT 0: narrow kernels (at W = 4 a voxel is used about twice) take the taps from
+// memory, four tiles a workgroup with the kernel table in LDS.
+// Whole calls with the map transform, 200 sections of 128^2, before (one thread a
+// pixel of a row, taps from memory) and now: W = 3 341 / 336 us, 4 525 / 465,
+// 5 802 / 493, 6 999 / 616, 8 1,936 / 987; 50 sections of 256^2: 604 / 535,
+// 847 / 669, 1,181 / 635, 1,432 / 752, 2,715 / 1,104. LDS reads bound it at W = 8
+// (busy 55 %, 60 % of that bank conflicts: the lanes' boxes start anywhere); one
+// and two wavefronts a tile at W = 8: 1,100 and 1,025 us, four at W = 6: 651.
+struct __attribute__((packed, aligned(4))) Float4u {
+    float v[4];
+};
+
+// Row of the kernel table for a fraction, in 16-byte loads (each lane has a row of
+// its own, so a load instruction costs one cache line per lane whatever its
+// width).
 template <int WD>
-__global__ __launch_bounds__(256) void k_extract(const float2* __restrict__ ft, int N,
-                                                 const double* __restrict__ mats, double inv,
-                                                 double rs, double maxs2, int center,
-                                                 const float* __restrict__ ktab,
-                                                 float2* __restrict__ out) {
-    __shared__ float K[(FSI_NDIV + 1) * WD];
-    for (int i = threadIdx.x; i < (FSI_NDIV + 1) * WD; i += blockDim.x) K[i] = ktab[i];
-    __syncthreads();
-    const int v = blockIdx.y;
-    const long long npix = (long long)N * N;
-    const long long pix = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (pix >= npix) return;
+__device__ __forceinline__ void table_row(const float* __restrict__ ktab, double frac, float (&w)[WD]) {
+    const float* r = ktab + ((int)(frac * FSI_NDIV + 0.5)) * WD;
+#pragma unroll
+    for (int q = 0; q + 4 <= WD; q += 4) {
+        const Float4u f = *(const Float4u*)(r + q);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w[q + e] = f.v[e];
+    }
+#pragma unroll
+    for (int q = WD / 4 * 4; q < WD; ++q) w[q] = r[q];
+}
+
+template <int WD, int WPT>
+__global__ __launch_bounds__(WPT ? 64 * WPT : 256) __attribute__((amdgpu_waves_per_eu(WPT ? 4 : 1))) void k_extract(const float2* __restrict__ ft, int N,
+                                                const double* __restrict__ mats, double inv,
+                                                double rs, double maxs2, int center, int tiles,
+                                                int nviews, int nblk, int cap, const float* __restrict__ ktab,
+                                                float2* __restrict__ out) {
+    constexpr int HW = (WD - 1) / 2;
+    constexpr bool LDSBOX = WPT > 0;
+    constexpr int PW = WPT ? (WD + WPT - 1) / WPT : WD;   // tap planes per wavefront
+    extern __shared__ float2 box[];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    // hardware block b runs on XCD b % 8: each XCD takes a contiguous range of
+    // (view, tile), so that the tiles of a section meet in one L2
+    const int per_xcd = (nblk + 7) / 8;
+    const int blk = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
+    if (blk >= nblk) return;
+    // without LDS boxes a workgroup takes four tiles and holds the kernel table
+    const float* K = ktab;
+    if (!LDSBOX) {
+        float* t = (float*)box;
+        for (int i = threadIdx.x; i < (FSI_NDIV + 1) * WD; i += 256) t[i] = ktab[i];
+        __syncthreads();
+        K = t;
+    }
+    const int task = LDSBOX ? blk : blk * 4 + wave;
+    const int v = task / (tiles * tiles), tile = task - v * tiles * tiles;
+    if (v >= nviews) return;
+    // tiles of the centred frequency plane (from -N/2 on), so that the 64
+    // samples of a tile are one patch of the plane
+    const int h = tile % tiles * 8 + (lane & 7) - N / 2;
+    const int k = tile / tiles * 8 + (lane >> 3) - N / 2;
+    const bool inside = h <= (N - 1) / 2 && k <= (N - 1) / 2;
     const double* M = mats + 9 * v;
-    const int xx = (int)(pix % N), yy = (int)(pix / N);
-    const int hx = (N - 1) / 2;
-    const double ivy = (double)(yy > hx ? yy - N : yy) * inv;
-    const double ivx = (double)(xx > hx ? xx - N : xx) * inv;
+    const double ivy = (double)k * inv, ivx = (double)h * inv;
     const double s2 = ivx * ivx + ivy * ivy;
+    const bool band = inside && s2 <= maxs2;
+    double m[3] = {0, 0, 0};
+    for (int c = 0; c < 3; ++c) m[c] = (ivx * M[3 * c] + ivy * M[3 * c + 1] + 0.0 * M[3 * c + 2]) * rs;
     double vr = 0, vi = 0;
-    if (s2 <= maxs2) {
-        double m[3];
-        for (int k = 0; k < 3; ++k) m[k] = (ivx * M[3 * k] + ivy * M[3 * k + 1] + 0.0 * M[3 * k + 2]) * rs;
+    if (LDSBOX) {
+        if (__ballot(band)) {   // wavefront-uniform
+            const double fl[3] = {floor(m[0]), floor(m[1]), floor(m[2])};
+            // the coordinates are monotone in h and in k, so the tile's corners
+            // (lanes 0, 7, 56, 63) bound the box; uniform values
+            int lo[3], n[3];
+            bool fits = true;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                const int f = (int)fl[c] - HW;
+                const int c0 = __builtin_amdgcn_readlane(f, 0), c1 = __builtin_amdgcn_readlane(f, 7);
+                const int c2 = __builtin_amdgcn_readlane(f, 56), c3 = __builtin_amdgcn_readlane(f, 63);
+                lo[c] = min(min(c0, c1), min(c2, c3));
+                n[c] = max(max(c0, c1), max(c2, c3)) + WD - lo[c];
+                fits = fits && n[c] <= 32 && lo[c] >= -N && lo[c] + n[c] <= N;   // one periodic wrap
+            }
+            const int sx = n[0] | 1;   // odd row stride: rows start in different banks
+            fits = fits && sx * n[1] * n[2] <= cap;
+            if (fits) {
+                // this lane's kernel weights, in flight together with the box
+                float wx[WD], wy[WD], wz[PW];
+                table_row<WD>(ktab, m[0] - fl[0], wx);
+                table_row<WD>(ktab, m[1] - fl[1], wy);
+                const float* kz = ktab + ((int)((m[2] - fl[2]) * FSI_NDIV + 0.5)) * WD;
+#pragma unroll
+                for (int q = 0; q < PW; ++q) wz[q] = kz[min(wave * PW + q, WD - 1)];
+                // lanes per row and rows per step; a lane keeps its RY row offsets
+                // of a plane, the planes are uniform; two planes of loads in flight
+                const int rl = n[0] <= 16 ? 16 : 32, per = 64 * WPT / rl;
+                const int lx = threadIdx.x & (rl - 1), ly = threadIdx.x / rl;
+                const bool on = lx < n[0];
+                int jx = lo[0] + min(lx, n[0] - 1);
+                jx += jx < 0 ? N : 0;
+                constexpr int RY = WPT >= 4 ? 3 : 5;
+                for (int y0 = 0; y0 < n[1]; y0 += RY * per) {
+                    int off[RY];
+#pragma unroll
+                    for (int u = 0; u < RY; ++u) {
+                        int jy = lo[1] + min(y0 + u * per + ly, n[1] - 1);   // past the end: reread
+                        jy += jy < 0 ? N : 0;
+                        off[u] = jy * N + jx;
+                    }
+                    for (int z = 0; z < n[2]; z += 2) {
+                        int ja = lo[2] + z, jb = lo[2] + min(z + 1, n[2] - 1);
+                        ja += ja < 0 ? N : 0;
+                        jb += jb < 0 ? N : 0;
+                        const float2* pa = ft + (size_t)ja * N * N;
+                        const float2* pb = ft + (size_t)jb * N * N;
+                        float2 va[RY], vb[RY];
+#pragma unroll
+                        for (int u = 0; u < RY; ++u) {
+                            va[u] = pa[off[u]];
+                            vb[u] = pb[off[u]];
+                        }
+                        float2* d = box + (z * n[1] + y0 + ly) * sx + lx;
+#pragma unroll
+                        for (int u = 0; u < RY; ++u)
+                            if (on && y0 + u * per + ly < n[1]) {
+                                d[u * per * sx] = va[u];
+                                if (z + 1 < n[2]) d[(n[1] + u * per) * sx] = vb[u];
+                            }
+                    }
+                }
+                __syncthreads();
+                float pr[PW], pi[PW];
+#pragma unroll
+                for (int q = 0; q < PW; ++q) pr[q] = pi[q] = 0.f;
+                if (band) {
+                    const float2* t = box + (((int)fl[2] - HW - lo[2] + wave * PW) * n[1] + (int)fl[1] - HW - lo[1]) * sx +
+                                      (int)fl[0] - HW - lo[0];
+#pragma unroll
+                    for (int q = 0; q < PW; ++q, t += n[1] * sx) {
+                        if (wave * PW + q >= WD) break;
+                        const float kzz = wz[q];
+#pragma unroll
+                        for (int y2 = 0; y2 < WD; ++y2) {
+                            const float w = wy[y2] * kzz;
+                            const float2* row = t + y2 * sx;
+#pragma unroll
+                            for (int e = 0; e < WD; ++e) {
+                                const float kw = wx[e] * w;
+                                const float2 a = row[e];
+                                pr[q] = fmaf(a.x, kw, pr[q]);
+                                pi[q] = fmaf(a.y, kw, pi[q]);
+                            }
+                        }
+                    }
+                }
+                // plane sums of every wavefront, added in the order of the planes
+                __syncthreads();
+                if (wave)
+#pragma unroll
+                    for (int q = 0; q < PW; ++q) box[((wave - 1) * PW + q) * 64 + lane] = make_float2(pr[q], pi[q]);
+                __syncthreads();
+                if (wave) return;
+#pragma unroll
+                for (int q = 0; q < PW; ++q) {
+                    vr += pr[q];
+                    vi += pi[q];
+                }
+                for (int q = 0; q < WD - PW; ++q) {
+                    const float2 p = box[q * 64 + lane];
+                    vr += p.x;
+                    vi += p.y;
+                }
+            } else if (band && wave == 0) {
+                fsi_sample<WD>(ft, N, m, ktab, vr, vi);
+            }
+        }
+        if (wave) return;
+    } else if (band) {
         fsi_sample<WD>(ft, N, m, K, vr, vi);
     }
+    if (!inside) return;
     if (center) {
         // phase_shift_to_center of a 2D section: x (-1)^(h+k) for even N
-        const long h = xx > hx ? xx - N : xx, k = yy > hx ? yy - N : yy;
         if ((N & 1) == 0) {
             if ((h + k) & 1) { vr = -vr; vi = -vi; }
         } else {
@@ -86,7 +250,7 @@ __global__ __launch_bounds__(256) void k_extract(const float2* __restrict__ ft, 
             vi = a * sn + b * cs;
         }
     }
-    out[(long long)v * npix + pix] = make_float2((float)vr, (float)vi);
+    out[((long long)v * N + (k < 0 ? k + N : k)) * N + (h < 0 ? h + N : h)] = make_float2((float)vr, (float)vi);
 }
 
 // -------------------------------------------------------------------- FSC
@@ -281,11 +445,23 @@ static int extract_launch(const float* ft_dev, int n, double sampling, const dou
                           const float* dtab, float* out_dev, hipStream_t s) {
     const double inv = 1.0 / (n * sampling), rs = n * sampling;
     const double maxs2 = 1.0 / (resolution * resolution);
-    dim3 grid((unsigned)(((long long)n * n + 255) / 256), (unsigned)nviews);
+    const int tiles = (n + 7) / 8;
+    BSX_REQUIRE((long long)tiles * tiles * nviews < (1ll << 31) - 8, BSX_ERR_ARG,
+                "section extraction: %lld views of %d x %d are too many", (long long)nviews, n, n);
+    const int ntile = (int)(tiles * tiles * nviews);
     const float2* ft = (const float2*)ft_dev;
     float2* out = (float2*)out_dev;
     switch (kernel_width) {
-#define BSX_EXT(W) case W: hipLaunchKernelGGL((k_extract<W>), grid, dim3(256), 0, s, ft, n, dmats, inv, rs, maxs2, center, dtab, out); break;
+// LDS boxes from width 5 on (see k_extract); cap holds the largest box of an 8 x 8
+// patch over random rotations (37 KB at W = 8, four workgroups per CU)
+#define BSX_EXT(W) case W: { \
+        constexpr int WPT = W >= 8 ? 4 : W >= 5 ? 2 : 0; \
+        constexpr int cap = WPT ? (W + 10) * (W + 9) * (W + 7) + 64 : 0; \
+        constexpr size_t lds = WPT ? sizeof(float2) * cap : sizeof(float) * (FSI_NDIV + 1) * W; \
+        const int nblk = WPT ? ntile : (ntile + 3) / 4; \
+        hipLaunchKernelGGL((k_extract<W, WPT>), dim3((unsigned)((nblk + 7) / 8 * 8)), dim3(WPT ? 64 * WPT : 256), \
+                           lds, s, ft, n, dmats, inv, rs, maxs2, center, tiles, (int)nviews, nblk, cap, dtab, out); \
+        break; }
         BSX_EXT(1) BSX_EXT(2) BSX_EXT(3) BSX_EXT(4) BSX_EXT(5)
         BSX_EXT(6) BSX_EXT(7) BSX_EXT(8) BSX_EXT(9) BSX_EXT(10)
 #undef BSX_EXT

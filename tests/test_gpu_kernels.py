@@ -92,3 +92,21 @@ def test_frc_score_vs_oracle(gpu):
     with pytest.raises(Exception):
         recon.img_recip_space_fom(torch.from_numpy(P).cuda(), torch.from_numpy(R).cuda(),
                                   np.array([[0, 5]], np.int32), 1.5, 4.0)
+
+
+@pytest.mark.parametrize("n,width", [(24, 3), (24, 8), (32, 5), (48, 4), (48, 9), (96, 10), (64, 7), (20, 6), (21, 8)])
+def test_sections_of_every_tile_path(n, width):
+    """Central sections against the FP64 oracle for kernel widths on both sides
+    of the LDS box rule, edges that are no multiple of the 8 x 8 tile, views
+    along the axes, and a matrix that shrinks the plane (its box has repeated
+    taps); FP32 rounding: 1e-5 of the maximum."""
+    rng = np.random.default_rng(n + width)
+    ft = (rng.normal(size=(n, n, n)) + 1j * rng.normal(size=(n, n, n))).astype(np.complex64)
+    mats = np.concatenate([np.eye(3)[None], synth.view_to_matrix([[1, 0, 0, 0.3], [0, 0, -1, 1.0]]),
+                           synth.view_to_matrix(synth.uniform_views(4, rng)), 0.3 * np.eye(3)[None]])
+    say(f"sections n={n} width={width} views={len(mats)}")
+    out = recon.central_sections(torch.as_tensor(ft).cuda(), mats, 1.5, 1.5, width, 2, True).cpu().numpy()
+    o = Oracle(64)
+    for i, m in enumerate(mats):
+        ref = o.central_section(ft, 1.5, m, 1.5, width, 2, 1)
+        assert np.abs(out[i] - ref).max() <= 1e-5 * np.abs(ref).max()
