@@ -1,5 +1,5 @@
 // bsx_extract.hip — the mirror of insertion and the quality measures:
-//   k_real_to_complex + 3 axis FFTs + k_phase_origin : map transform
+//   3 axis FFTs (real input, phase shift with the last) : map transform
 //       (Bimage::project prologue, src/img/Bimage_project.cpp:373-375)
 //   k_extract        : central sections by FSI-kernel gather interpolation
 //       (Bimage::central_section, Bimage_project.cpp:288-338;
@@ -14,37 +14,7 @@
 
 #include "bsx_common.h"
 
-namespace bsx {
-int fft_axis_ex(float2* data, float* real_out, int nx, int ny, int nz, int64_t batch, int axis,
-                int sign, float scale, hipStream_t s);
-}
 using namespace bsx;
-
-// ------------------------------------------------------------ map transform
-__global__ void k_real_to_complex(const float* __restrict__ in, float2* __restrict__ out,
-                                  long long n) {
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (long long)gridDim.x * blockDim.x)
-        out[i] = make_float2(in[i], 0.f);
-}
-
-// phase_shift_to_origin (Bimage_complex.cpp:490-543): x e^{i phi},
-// phi = h*sx + (l*sz + k*sy), s = origin/size * 2 pi.
-__global__ void k_phase_origin(float2* __restrict__ v, int N, double sx, double sy, double sz) {
-    const long long n3 = (long long)N * N * N;
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n3;
-         i += (long long)gridDim.x * blockDim.x) {
-        const long long xx = i % N, yy = (i / N) % N, zz = i / ((long long)N * N);
-        const long h = xx > (N - 1) / 2 ? xx - N : xx;
-        const long k = yy > (N - 1) / 2 ? yy - N : yy;
-        const long l = zz > (N - 1) / 2 ? zz - N : zz;
-        const double phi = h * sx + (l * sz + k * sy);
-        double sn, cs;
-        sincos(phi, &sn, &cs);
-        const float2 a = v[i];
-        v[i] = make_float2((float)(a.x * cs - a.y * sn), (float)(a.x * sn + a.y * cs));
-    }
-}
 
 // ------------------------------------------------------------- extraction
 // 8 x 8 pixel tiles of a section, WPT wavefronts each. The tile samples a patch of
@@ -292,46 +262,52 @@ __global__ __launch_bounds__(256) void k_fsc(const float2* __restrict__ a,
 
 // FP64 shell sums of Bimage::fsc_dpr (Bimage_resolution.cpp:93-181) for two
 // real maps transformed separately (the same F1, F2 as unpacking the packed
-// transform): over x < N/2, linear interpolation between shells i and i+1
-// (both must exist), sums[c * maxrad + i] for c = |F1|^2, |F2|^2,
-// Re F1 conj F2, |F1|^2 + |F2|^2, (|F1|^2 + |F2|^2) dphi^2.
+// transform): over x < N/2 (all that a and b hold), linear interpolation between
+// shells i and i+1 (both must exist), sums[c * maxrad + i] for c = |F1|^2,
+// |F2|^2, Re F1 conj F2, (|F1|^2 + |F2|^2) dphi^2 (the sum of the first two
+// weighs the last). The phase difference is the angle of F2 conj F1; where one
+// value is zero, that of the other. The LDS adds bound it (neighbouring lanes
+// share shells): 103 us at 256^3 (131 us with five sums, two phase angles and
+// whole transforms).
 __global__ __launch_bounds__(256) void k_fsc_dpr(const float2* __restrict__ a,
                                                  const float2* __restrict__ b, int N, int nz,
-                                                 double inv_ratio, long maxrad,
+                                                 double inv_ratio, int maxrad,
                                                  double* __restrict__ sums) {
-    extern __shared__ double sh[];   // 5 * maxrad
-    for (long i = threadIdx.x; i < 5 * maxrad; i += blockDim.x) sh[i] = 0;
+    extern __shared__ double sh[];   // 4 * maxrad
+    for (int i = threadIdx.x; i < 4 * maxrad; i += blockDim.x) sh[i] = 0;
     __syncthreads();
-    const int hx = N / 2;
+    const unsigned hx = N / 2;
     const long long nv = (long long)hx * N * nz;   // nz = 1: a 2D image
     for (long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x; t < nv;
          t += (long long)gridDim.x * blockDim.x) {
-        const long long xx = t % hx, yz = t / hx, yy = yz % N, zz = yz / N;
-        const double h = xx > (N - 1) / 2 ? (double)(xx - N) : (double)xx;
+        const unsigned yz = (unsigned)(t / hx);
+        const int xx = (int)(t - (long long)yz * hx), yy = (int)(yz % (unsigned)N), zz = (int)(yz / (unsigned)N);
+        const double h = xx;
         const double k = yy > (N - 1) / 2 ? (double)(yy - N) : (double)yy;
         const double l = zz > (nz - 1) / 2 ? (double)(zz - nz) : (double)zz;
         const double radius = inv_ratio * sqrt(h * h + k * k + l * l);
-        const long ir = (long)radius;
-        if (ir + 1 >= maxrad) continue;
+        if (!(radius < maxrad - 1)) continue;
+        const int ir = (int)radius;
         const double f = radius - ir, f1 = 1 - f;
-        const long long i = (zz * N + yy) * N + xx;
-        const float2 u = a[i], v = b[i];
+        const float2 u = a[t], v = b[t];
         const double I1 = (double)u.x * u.x + (double)u.y * u.y;
         const double I2 = (double)v.x * v.x + (double)v.y * v.y;
-        double dphi = atan2((double)u.y, (double)u.x) - atan2((double)v.y, (double)v.x);
-        dphi = remainder(dphi, 2 * M_PI);
-        dphi *= dphi;
         const double re = (double)u.x * v.x + (double)u.y * v.y;
-        const double is = I1 + I2;
-        const double val[5] = {I1, I2, re, is, is * dphi};
+        double dphi;
+        if (I1 > 0 && I2 > 0) {
+            dphi = atan2((double)u.y * v.x - (double)u.x * v.y, re);
+        } else {
+            dphi = atan2((double)u.y, (double)u.x) - atan2((double)v.y, (double)v.x);
+        }
+        const double val[4] = {I1, I2, re, (I1 + I2) * (dphi * dphi)};
 #pragma unroll
-        for (int c = 0; c < 5; ++c) {
+        for (int c = 0; c < 4; ++c) {
             atomicAdd(&sh[c * maxrad + ir], f1 * val[c]);
             atomicAdd(&sh[c * maxrad + ir + 1], f * val[c]);
         }
     }
     __syncthreads();
-    for (long i = threadIdx.x; i < 5 * maxrad; i += blockDim.x)
+    for (int i = threadIdx.x; i < 4 * maxrad; i += blockDim.x)
         if (sh[i] != 0) atomicAdd(&sums[i], sh[i]);
 }
 
@@ -405,18 +381,11 @@ int bsx_map_transform(const float* map_dev, int n, const double origin[3], float
     hipStream_t s = (hipStream_t)stream;
     const long long n3 = (long long)n * n * n;
     float2* v = (float2*)ft_dev;
-    hipLaunchKernelGGL(k_real_to_complex, dim3(2048), dim3(256), 0, s, map_dev, v, n3);
-    BSX_HIP(hipGetLastError());
     const float sc = (float)(1.0 / sqrt((double)n3));
-    int r = fft_axis_ex(v, nullptr, n, n, n, 1, 0, -1, 1.0f, s);
+    int r = fft_real_x(map_dev, v, n, (long long)n * n, n, s);
     if (r == BSX_OK) r = fft_axis_ex(v, nullptr, n, n, n, 1, 1, -1, 1.0f, s);
-    if (r == BSX_OK) r = fft_axis_ex(v, nullptr, n, n, n, 1, 2, -1, sc, s);
-    if (r != BSX_OK) return r;
-    const double sx = origin[0] / n * 2 * M_PI, sy = origin[1] / n * 2 * M_PI,
-                 sz = origin[2] / n * 2 * M_PI;
-    hipLaunchKernelGGL(k_phase_origin, dim3(2048), dim3(256), 0, s, v, n, sx, sy, sz);
-    BSX_HIP(hipGetLastError());
-    return BSX_OK;
+    if (r == BSX_OK) r = fft_z_to_origin(v, n, sc, origin, s);
+    return r;
 }
 
 // Argument checks shared by bsx_extract and bsx_extract_noalloc; normalises
@@ -597,31 +566,31 @@ static int fsc_dpr_impl(const float* map1_dev, const float* map2_dev, int n, int
     const long maxrad = (long)(2 + rad_scale / hi_res);
     BSX_REQUIRE(maxrad <= *nrows, BSX_ERR_ARG, "bsx_fsc_dpr: %ld rows exceed capacity %d", maxrad,
                 *nrows);
-    const long long n3 = (long long)n * n * nz;
+    const long long n3 = (long long)(n / 2) * n * nz;   // a transform's kept half
     float2* v = nullptr;
     double* d = nullptr;
     BSX_HIP(hipMalloc(&v, sizeof(float2) * 2 * n3));
-    if (hipMalloc(&d, sizeof(double) * 5 * maxrad) != hipSuccess) {
+    if (hipMalloc(&d, sizeof(double) * 4 * maxrad) != hipSuccess) {
         (void)hipFree(v);
         set_error("bsx_fsc_dpr: allocation failed");
         return BSX_ERR_NOMEM;
     }
     int r = BSX_OK;
-    for (int m = 0; m < 2 && r == BSX_OK; ++m) {
-        hipLaunchKernelGGL(k_real_to_complex, dim3(2048), dim3(256), 0, s, m ? map2_dev : map1_dev,
-                           v + m * n3, n3);
-        for (int axis = 0; axis < (nz > 1 ? 3 : 2) && r == BSX_OK; ++axis)
-            r = fft_axis_ex(v + m * n3, nullptr, n, n, nz, 1, axis, -1, 1.0f, s);
-    }
+    // the sums read x < n / 2 only: the x pass keeps that half, the other passes
+    // transform both halves' columns in one launch each
+    for (int m = 0; m < 2 && r == BSX_OK; ++m)
+        r = fft_real_x(m ? map2_dev : map1_dev, v + m * n3, n, (long long)n * nz, n / 2, s);
+    for (int axis = 1; axis < (nz > 1 ? 3 : 2) && r == BSX_OK; ++axis)
+        r = fft_axis_ex(v, nullptr, n / 2, n, nz, 2, axis, -1, 1.0f, s);
     if (r == BSX_OK) {
-        (void)hipMemsetAsync(d, 0, sizeof(double) * 5 * maxrad, s);
-        hipLaunchKernelGGL(k_fsc_dpr, dim3(1024), dim3(256), sizeof(double) * 5 * maxrad, s, v,
-                           v + n3, n, nz, 1.0 / sampling_ratio, maxrad, d);
+        (void)hipMemsetAsync(d, 0, sizeof(double) * 4 * maxrad, s);
+        hipLaunchKernelGGL(k_fsc_dpr, dim3(1024), dim3(256), sizeof(double) * 4 * maxrad, s, v,
+                           v + n3, n, nz, 1.0 / sampling_ratio, (int)maxrad, d);
         if (hipGetLastError() != hipSuccess) r = BSX_ERR_DEVICE;
     }
-    std::vector<double> h(5 * maxrad);
+    std::vector<double> h(4 * maxrad);
     if (r == BSX_OK &&
-        (hipMemcpyAsync(h.data(), d, sizeof(double) * 5 * maxrad, hipMemcpyDeviceToHost, s) !=
+        (hipMemcpyAsync(h.data(), d, sizeof(double) * 4 * maxrad, hipMemcpyDeviceToHost, s) !=
              hipSuccess ||
          hipStreamSynchronize(s) != hipSuccess))
         r = BSX_ERR_DEVICE;
@@ -640,8 +609,8 @@ static int fsc_dpr_impl(const float* map1_dev, const float* map2_dev, int n, int
             const double f12 = h[i] * h[maxrad + i];
             if (f12 > 1e-30) fsc /= sqrt(f12);
             fsc = std::min(1.0, std::max(-1.0, fsc));
-            const double fs = h[3 * maxrad + i];
-            dpr = fs > 1e-30 ? sqrt(h[4 * maxrad + i] / fs) * 180.0 / M_PI : 0;
+            const double fs = h[i] + h[maxrad + i];
+            dpr = fs > 1e-30 ? sqrt(h[3 * maxrad + i] / fs) * 180.0 / M_PI : 0;
         }
         curves[3 * i] = i / rad_scale;
         curves[3 * i + 1] = fsc;

@@ -61,137 +61,200 @@ bool fft_length_supported(int n) {
     }
 }
 
-// ------------------------------------------------------------- axis kernel
-// Lines: line index -> base = (line / inner) * outer + (line % inner);
-// element i of a line at base + i * stride. B lines per workgroup, processed
-// G = 256/T at a time. If real_out is set, the real part (x scale) is written
-// to real_out at the same element index instead of updating `data`.
-template <int L, int S, int B>
-__global__ __launch_bounds__(256) void k_fft_axis(float2* __restrict__ data,
-                                                  float* __restrict__ real_out, long long nlines,
-                                                  long long inner, long long outer,
-                                                  long long stride, float scale,
-                                                  const float2* __restrict__ twg) {
-    constexpr int T = FftThreads<L>::value;
-    constexpr int G = 256 / T;
-    constexpr int NT = G * T;
-    static_assert(B % G == 0, "bundle must be a multiple of the line groups");
-    __shared__ float2 lds[B * L + L];
-    float2* tw = lds + B * L;
+// ------------------------------------------------------------ axis kernels
+// Both kernels hold B lines in padded LDS lines, one value further apart than
+// their size, so that neither the passes nor the transposed accesses of the
+// strided axes meet in one bank. They are bound by memory: a 256^3 pass takes
+// 45 us (x) and 43 us (y, z), 6 TB/s; with plain lines and a 64-bit division per
+// element it took 56 and 78 us.
+template <int L> constexpr int fft_pitch = line_size<L> + 1;
+
+// x axis: a workgroup's lines are contiguous in memory. RIN: the input is real
+// (`real_in`, the same lines); the first `keep` values of a line (L: all) go to
+// `data`, lines `keep` apart (in place unless RIN or keep < L).
+template <int L, int S, int B, bool RIN>
+__global__ __launch_bounds__(256) void k_fft_x(const float* __restrict__ real_in, float2* data,
+                                               float* __restrict__ real_out, long long nlines, int keep,
+                                               float scale, const float2* __restrict__ twg) {
+    constexpr int T = FftThreads<L>::value, G = 256 / T, NT = G * T, LP = fft_pitch<L>;
+    constexpr int E = B * L / NT;   // values per thread
+    static_assert(B % G == 0 && E * NT == B * L, "whole lines per group, whole values per thread");
+    __shared__ float2 lds[B * LP + L];
+    float2* tw = lds + B * LP;
     const int tid = threadIdx.x;
-    if (tid >= NT) return;   // uniform per wavefront only when NT % 64 == 0; see launch
     for (int i = tid; i < L; i += NT) tw[i] = twg[i];
-    const long long line0 = (long long)blockIdx.x * B;
-    if (stride == 1) {
-        for (int idx = tid; idx < B * L; idx += NT) {
-            const int l = idx / L, i = idx % L;
-            const long long line = line0 + l;
-            if (line < nlines) {
-                const long long base = (line / inner) * outer + (line % inner);
-                lds[l * L + i] = data[base + i];
-            }
+    const long long line0 = (long long)blockIdx.x * B, left = (nlines - line0) * L;
+    float2 v[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const int idx = tid + e * NT;
+        v[e] = make_float2(0.f, 0.f);
+        if (idx < left) {
+            if (RIN) v[e].x = real_in[line0 * L + idx];
+            else v[e] = data[line0 * L + idx];
         }
-    } else {
-        for (int idx = tid; idx < B * L; idx += NT) {
-            const int l = idx % B, i = idx / B;
-            const long long line = line0 + l;
-            if (line < nlines) {
-                const long long base = (line / inner) * outer + (line % inner);
-                lds[l * L + i] = data[base + (long long)i * stride];
-            }
-        }
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const int idx = tid + e * NT, l = idx / L, i = idx - l * L;
+        lds[l * LP + line_at<true>(i)] = v[e];
     }
     __syncthreads();
     const int g = tid / T, t = tid % T;
 #pragma unroll 1
-    for (int r0 = 0; r0 < B; r0 += G) FftLine<L, S, T>::run(lds + (r0 + g) * L, tw, t);
-    if (stride == 1) {
-        for (int idx = tid; idx < B * L; idx += NT) {
-            const int l = idx / L, i = idx % L;
-            const long long line = line0 + l;
-            if (line < nlines) {
-                const long long base = (line / inner) * outer + (line % inner);
-                float2 v = lds[l * L + i];
-                if (real_out) real_out[base + i] = v.x * scale;
-                else data[base + i] = make_float2(v.x * scale, v.y * scale);
-            }
-        }
-    } else {
-        for (int idx = tid; idx < B * L; idx += NT) {
-            const int l = idx % B, i = idx / B;
-            const long long line = line0 + l;
-            if (line < nlines) {
-                const long long base = (line / inner) * outer + (line % inner);
-                float2 v = lds[l * L + i];
-                const long long e = base + (long long)i * stride;
-                if (real_out) real_out[e] = v.x * scale;
-                else data[e] = make_float2(v.x * scale, v.y * scale);
-            }
-        }
+    for (int r0 = 0; r0 < B; r0 += G) FftLine<L, S, T, true>::run(lds + (r0 + g) * LP, tw, t);
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const int idx = tid + e * NT, l = idx / L, i = idx - l * L;
+        if (idx >= left || i >= keep) continue;
+        const float2 z = lds[l * LP + line_at<true>(i)];
+        const long long at = (line0 + l) * keep + i;
+        if (real_out) real_out[at] = z.x * scale;
+        else data[at] = make_float2(z.x * scale, z.y * scale);
     }
 }
 
-// Workgroup sizes: NT = (256/T)*T threads. For lengths where NT is not a
-// multiple of 64 the early return above is never taken because the launch
-// uses exactly NT threads.
+// phase_shift_to_origin (Bimage_complex.cpp:490-543) of a cubic map's
+// transform: x e^{i phi}, phi = h sx + (l sz + k sy), s = origin / size 2 pi.
+struct FftPhase {
+    double sx, sy, sz;
+};
+
+// y or z axis: element i of line q at (q / inner) outer + q % inner + i stride;
+// consecutive lanes take consecutive lines. If real_out is set, the real part
+// goes there instead of updating `data`. PH (z axis of a cube): the phase shift.
+template <int L, int S, int B, bool PH>
+__global__ __launch_bounds__(256) void k_fft_s(float2* __restrict__ data, float* __restrict__ real_out,
+                                               long long nlines, long long inner, long long outer,
+                                               long long stride, float scale,
+                                               const float2* __restrict__ twg, FftPhase ph) {
+    constexpr int T = FftThreads<L>::value, G = 256 / T, NT = G * T, LP = fft_pitch<L>;
+    static_assert(B % G == 0 && NT % B == 0, "whole lines per group, one line per thread");
+    constexpr int D = NT / B, E = L / D;   // elements a step, values per thread
+    static_assert(E * D == L, "whole values per thread");
+    __shared__ float2 lds[B * LP + L];
+    float2* tw = lds + B * LP;
+    const int tid = threadIdx.x;
+    for (int i = tid; i < L; i += NT) tw[i] = twg[i];
+    const int l = tid % B, i0 = tid / B;
+    const long long line = (long long)blockIdx.x * B + l;
+    const bool ok = line < nlines;
+    const long long hi = ok ? line / inner : 0, lo = ok ? line - hi * inner : 0;
+    float2* src = data + hi * outer + lo;
+    float2 v[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) v[e] = ok ? src[(i0 + e * D) * stride] : make_float2(0.f, 0.f);
+#pragma unroll
+    for (int e = 0; e < E; ++e) lds[l * LP + line_at<true>(i0 + e * D)] = v[e];
+    __syncthreads();
+    const int g = tid / T, t = tid % T;
+#pragma unroll 1
+    for (int r0 = 0; r0 < B; r0 += G) FftLine<L, S, T, true>::run(lds + (r0 + g) * LP, tw, t);
+    if (!ok) return;
+    double pxy = 0, ky = 0;
+    if (PH) {
+        const int x = (int)(lo % L), y = (int)(lo / L);
+        pxy = (x > (L - 1) / 2 ? x - L : x) * ph.sx;
+        ky = (y > (L - 1) / 2 ? y - L : y) * ph.sy;
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const int i = i0 + e * D;
+        float2 z = lds[l * LP + line_at<true>(i)];
+        z.x *= scale;
+        z.y *= scale;
+        if (PH) {
+            const double phi = pxy + ((i > (L - 1) / 2 ? i - L : i) * ph.sz + ky);
+            double sn, cs;
+            sincos(phi, &sn, &cs);
+            z = make_float2((float)(z.x * cs - z.y * sn), (float)(z.x * sn + z.y * cs));
+        }
+        if (real_out) real_out[hi * outer + lo + i * stride] = z.x;
+        else src[i * stride] = z;
+    }
+}
+
+// Lines per workgroup of a strided axis: a multiple of the line groups that
+// divides the threads, at least 16 (128-byte runs).
+template <int L> constexpr int strided_lines() {
+    constexpr int G = 256 / FftThreads<L>::value, NT = G * FftThreads<L>::value;
+    int b = G;
+    while (b < 16 || NT % b) b += G;
+    return b;
+}
+
 template <int L, int S>
-static int launch_axis(float2* data, float* real_out, long long nlines, long long inner,
-                       long long outer, long long stride, float scale, hipStream_t s) {
+static int launch_axis(const float* real_in, float2* data, float* real_out, long long nlines,
+                       long long inner, long long outer, long long stride, int keep, float scale,
+                       const FftPhase* ph, hipStream_t s) {
     constexpr int T = FftThreads<L>::value;
     constexpr int G = 256 / T;
     constexpr int NT = G * T;
     const float2* tw = twiddles(L, s);
     BSX_REQUIRE(tw != nullptr, BSX_ERR_DEVICE, "twiddle table allocation failed for L=%d", L);
-    if (stride == 1) {
-        constexpr int B = G;
-        long long nb = (nlines + B - 1) / B;
-        hipLaunchKernelGGL((k_fft_axis<L, S, B>), dim3((unsigned)nb), dim3(NT), 0, s, data,
-                           real_out, nlines, inner, outer, stride, scale, tw);
-    } else {
-        // bundle of >= 16 adjacent lines so each load touches >= 128 B runs
-        constexpr int B0 = G >= 16 ? G : ((16 + G - 1) / G) * G;
-        constexpr int B = (B0 * L * 8 + L * 8 > 64 * 1024) ? G * ((64 * 1024 / (L * 8) - 1) / G) : B0;
-        static_assert(B >= G, "bundle");
-        long long nb = (nlines + B - 1) / B;
-        hipLaunchKernelGGL((k_fft_axis<L, S, B>), dim3((unsigned)nb), dim3(NT), 0, s, data,
-                           real_out, nlines, inner, outer, stride, scale, tw);
-    }
+    constexpr int B = strided_lines<L>();
+    const dim3 gx((unsigned)((nlines + G - 1) / G)), gs((unsigned)((nlines + B - 1) / B));
+    if (stride == 1 && real_in)
+        hipLaunchKernelGGL((k_fft_x<L, S, G, true>), gx, dim3(NT), 0, s, real_in, data, real_out, nlines,
+                           keep, scale, tw);
+    else if (stride == 1)
+        hipLaunchKernelGGL((k_fft_x<L, S, G, false>), gx, dim3(NT), 0, s, (const float*)nullptr, data,
+                           real_out, nlines, L, scale, tw);
+    else if (ph)
+        hipLaunchKernelGGL((k_fft_s<L, S, B, true>), gs, dim3(NT), 0, s, data, real_out, nlines, inner,
+                           outer, stride, scale, tw, *ph);
+    else
+        hipLaunchKernelGGL((k_fft_s<L, S, B, false>), gs, dim3(NT), 0, s, data, real_out, nlines, inner,
+                           outer, stride, scale, tw, FftPhase{0, 0, 0});
     BSX_HIP(hipGetLastError());
     return BSX_OK;
 }
 
 template <int S>
-static int dispatch_axis(int L, float2* data, float* real_out, long long nlines, long long inner,
-                         long long outer, long long stride, float scale, hipStream_t s) {
+static int dispatch_axis(int L, const float* real_in, float2* data, float* real_out, long long nlines,
+                         long long inner, long long outer, long long stride, int keep, float scale,
+                         const FftPhase* ph, hipStream_t s) {
     switch (L) {
-        case 16: return launch_axis<16, S>(data, real_out, nlines, inner, outer, stride, scale, s);
-        case 32: return launch_axis<32, S>(data, real_out, nlines, inner, outer, stride, scale, s);
-        case 64: return launch_axis<64, S>(data, real_out, nlines, inner, outer, stride, scale, s);
-        case 128: return launch_axis<128, S>(data, real_out, nlines, inner, outer, stride, scale, s);
-        case 256: return launch_axis<256, S>(data, real_out, nlines, inner, outer, stride, scale, s);
-        case 512: return launch_axis<512, S>(data, real_out, nlines, inner, outer, stride, scale, s);
-        case 24: return launch_axis<24, S>(data, real_out, nlines, inner, outer, stride, scale, s);
-        case 48: return launch_axis<48, S>(data, real_out, nlines, inner, outer, stride, scale, s);
-        case 96: return launch_axis<96, S>(data, real_out, nlines, inner, outer, stride, scale, s);
-        case 192: return launch_axis<192, S>(data, real_out, nlines, inner, outer, stride, scale, s);
-        case 384: return launch_axis<384, S>(data, real_out, nlines, inner, outer, stride, scale, s);
+#define BSX_AXIS(LEN) case LEN: return launch_axis<LEN, S>(real_in, data, real_out, nlines, inner, outer, \
+                                                           stride, keep, scale, ph, s);
+        BSX_AXIS(16) BSX_AXIS(32) BSX_AXIS(64) BSX_AXIS(128) BSX_AXIS(256) BSX_AXIS(512)
+        BSX_AXIS(24) BSX_AXIS(48) BSX_AXIS(96) BSX_AXIS(192) BSX_AXIS(384)
+#undef BSX_AXIS
         default:
             set_error("FFT length %d not supported (16..512 powers of 2, 3*2^k to 384)", L);
             return BSX_ERR_ARG;
     }
 }
 
-// Public launcher used by the finish and map-transform paths.
-int fft_axis_ex(float2* data, float* real_out, int nx, int ny, int nz, int64_t batch, int axis,
-                int sign, float scale, hipStream_t s) {
+static int axis_any(float2* data, float* real_out, int nx, int ny, int nz, int64_t batch, int axis,
+                    int sign, float scale, const FftPhase* ph, hipStream_t s) {
     long long nxy = (long long)nx * ny, n3 = nxy * nz;
     long long L, nlines, inner, outer, stride;
     if (axis == 0) { L = nx; nlines = n3 / nx * batch; inner = 1; outer = nx; stride = 1; }
     else if (axis == 1) { L = ny; nlines = (long long)nx * nz * batch; inner = nx; outer = nxy; stride = nx; }
     else { L = nz; nlines = nxy * batch; inner = nxy; outer = n3; stride = nxy; }
     if (L == 1) return BSX_OK;
-    return sign < 0 ? dispatch_axis<-1>((int)L, data, real_out, nlines, inner, outer, stride, scale, s)
-                    : dispatch_axis<+1>((int)L, data, real_out, nlines, inner, outer, stride, scale, s);
+    // a strided axis of a one-wide array is contiguous
+    auto go = sign < 0 ? dispatch_axis<-1> : dispatch_axis<+1>;
+    return go((int)L, nullptr, data, real_out, nlines, inner, outer, stride, (int)L, scale, ph, s);
+}
+
+// Public launcher used by the finish and map-transform paths.
+int fft_axis_ex(float2* data, float* real_out, int nx, int ny, int nz, int64_t batch, int axis,
+                int sign, float scale, hipStream_t s) {
+    return axis_any(data, real_out, nx, ny, nz, batch, axis, sign, scale, nullptr, s);
+}
+
+// Forward transform of the `nlines` real lines of nx values at `in`; the first
+// `keep` frequencies of each go to `out`, lines `keep` apart.
+int fft_real_x(const float* in, float2* out, int nx, long long nlines, int keep, hipStream_t s) {
+    return dispatch_axis<-1>(nx, in, out, nullptr, nlines, 1, nx, 1, keep, 1.0f, nullptr, s);
+}
+
+// Forward transform of an n^3 map along z, x scale, moved to `origin` (voxels).
+int fft_z_to_origin(float2* data, int n, float scale, const double origin[3], hipStream_t s) {
+    const FftPhase ph{origin[0] / n * 2 * M_PI, origin[1] / n * 2 * M_PI, origin[2] / n * 2 * M_PI};
+    return axis_any(data, nullptr, n, n, n, 1, 2, -1, scale, &ph, s);
 }
 
 int fft_axis(float2* data, int nx, int ny, int nz, int64_t batch, int axis, int sign, float scale,

@@ -37,6 +37,10 @@ const char* last_error();
 // sign -1 forward, +1 backward. scale multiplies every output.
 int fft_axis(float2* data, int nx, int ny, int nz, int64_t batch, int axis, int sign,
              float scale, hipStream_t s);
+int fft_axis_ex(float2* data, float* real_out, int nx, int ny, int nz, int64_t batch, int axis,
+                int sign, float scale, hipStream_t s);
+int fft_real_x(const float* in, float2* out, int nx, long long nlines, int keep, hipStream_t s);
+int fft_z_to_origin(float2* data, int n, float scale, const double origin[3], hipStream_t s);
 bool fft_length_supported(int n);
 
 // Per-particle transform stages (bsx_recon.hip).

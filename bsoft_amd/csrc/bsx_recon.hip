@@ -28,11 +28,6 @@
 
 #include "bsx_insert.h"
 
-namespace bsx {
-int fft_axis_ex(float2* data, float* real_out, int nx, int ny, int nz, int64_t batch, int axis,
-                int sign, float scale, hipStream_t s);
-}
-
 // ------------------------------------------------------------------- K1
 // Block-wide sums of 256 threads (FP64 and int).
 __device__ __forceinline__ void block_sum256(double& a, double& b, int& c, int& d) {

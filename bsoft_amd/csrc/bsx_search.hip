@@ -37,10 +37,6 @@
 #include "bsx_common.h"
 #include "bsx_fft_dev.h"
 
-namespace bsx {
-int fft_axis_ex(float2* data, float* real_out, int nx, int ny, int nz, int64_t batch, int axis,
-                int sign, float scale, hipStream_t s);
-}
 using namespace bsx;
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
@@ -1346,13 +1342,6 @@ __global__ __launch_bounds__(256) void k_cnn_norm(const float2* __restrict__ gri
     for (int i = threadIdx.x; i < S2; i += blockDim.x) O[i] = (float)(G[i].x - mean) * inv;
 }
 
-__global__ void k_real_to_complex_b(const float* __restrict__ in, float2* __restrict__ out,
-                                    long long n) {
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (long long)gridDim.x * blockDim.x)
-        out[i] = make_float2(in[i], 0.f);
-}
-
 }  // namespace
 
 // ================================================================ host side
@@ -1692,10 +1681,7 @@ int bsx_search_stage(bsx_search* h, const float* imgs_dev, const bsx_particle* p
     BSX_HIP(hipMemcpyAsync(h->d_sp, sp.data(), sizeof(SPart) * n, hipMemcpyHostToDevice, s));
     for (int64_t p0 = 0; p0 < n; p0 += chunk) {
         const int64_t nb = std::min(chunk, n - p0);
-        hipLaunchKernelGGL(k_real_to_complex_b, dim3(2048), dim3(256), 0, s, imgs_dev + p0 * per,
-                           h->d_spec, (long long)(nb * per));
-        BSX_HIP(hipGetLastError());
-        rc = fft_axis_ex(h->d_spec, nullptr, N, N, 1, nb, 0, -1, 1.0f, s);
+        rc = fft_real_x(imgs_dev + p0 * per, h->d_spec, N, (long long)nb * N, N, s);
         if (!rc) rc = fft_axis_ex(h->d_spec, nullptr, N, N, 1, nb, 1, -1, 1.0f / N, s);
         if (rc) return rc;
         hipLaunchKernelGGL(k_part_stage, dim3((unsigned)nb), dim3(256), sizeof(float2) * Nd, s,

@@ -7,7 +7,8 @@ import numpy as np
 import pytest
 import torch
 
-from bsoft_amd import recon, synth
+from bsoft_amd import bresolve, recon, synth
+from oracle import resolution_ref
 from oracle.oracle import Oracle
 
 pytestmark = pytest.mark.gpu
@@ -92,6 +93,51 @@ def test_frc_score_vs_oracle(gpu):
     with pytest.raises(Exception):
         recon.img_recip_space_fom(torch.from_numpy(P).cuda(), torch.from_numpy(R).cuda(),
                                   np.array([[0, 5]], np.int32), 1.5, 4.0)
+
+
+@pytest.mark.parametrize("shape,dims", [((3, 24, 96), 2), ((5, 48, 24), 2), ((1, 384, 16), 2), ((24, 48, 96), 3),
+                                        ((16, 16, 16), 3), ((2, 192, 24, 16), 3), ((512, 16, 16), 3)])
+def test_fft_ragged_line_bundles(shape, dims):
+    """Axis transforms whose numbers of lines are no multiple of a workgroup's
+    bundle, against numpy's FP64 transform (2e-6 of the maximum, FP32 rounding
+    over at most 27 butterfly stages)."""
+    rng = np.random.default_rng(sum(shape))
+    x = (rng.normal(size=shape) + 1j * rng.normal(size=shape)).astype(np.complex64)
+    say(f"fft shape={shape} dims={dims}")
+    axes = tuple(range(len(shape) - dims, len(shape)))
+    ref = np.fft.fftn(x.astype(np.complex128), axes=axes, norm="ortho")
+    got = recon.fft(torch.as_tensor(x).cuda(), dims, -1, 1).cpu().numpy()
+    assert np.abs(got - ref).max() <= 2e-6 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("n,origin", [(16, (8, 8, 8)), (24, (11.5, 12, 3.25)), (48, (0, 24, 47)), (96, (48, 48, 48))])
+def test_map_transform_origin(n, origin):
+    """Map transform of a real map moved to an origin that is no grid centre,
+    against numpy (1e-6 of the maximum)."""
+    rng = np.random.default_rng(n)
+    v = rng.normal(size=(n, n, n)).astype(np.float32)
+    say(f"map transform n={n} origin={origin}")
+    f = np.fft.fftfreq(n, 1 / n)
+    ph = 2j * np.pi / n * (f[None, None, :] * origin[0] + f[None, :, None] * origin[1] + f[:, None, None] * origin[2])
+    ref = np.fft.fftn(v.astype(np.float64), norm="ortho") * np.exp(ph)
+    got = recon.map_transform(torch.as_tensor(v).cuda(), origin).cpu().numpy()
+    assert np.abs(got - ref).max() <= 1e-6 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("shape", [(16, 16, 16), (24, 24, 24), (96, 96), (1, 48, 48)])
+def test_fsc_dpr_with_empty_transforms(shape):
+    """FSC and DPR where one map has no power, or both have none: the shells'
+    phase difference is then the other value's angle, weighed with its power."""
+    rng = np.random.default_rng(len(shape))
+    v = torch.as_tensor(rng.normal(size=shape).astype(np.float32)).cuda()
+    z = torch.zeros_like(v)
+    say(f"fsc_dpr shape={shape}")
+    s, fsc, dpr = bresolve.fsc_dpr(z, z, 1.5)
+    assert np.all(fsc[1:] == 0) and np.all(dpr == 0)
+    s, fsc, dpr = bresolve.fsc_dpr(v, z, 1.5)
+    ref = resolution_ref.fsc_dpr(v.cpu().numpy().astype(np.float64), np.zeros(shape), 1.5)
+    np.testing.assert_allclose(fsc, ref[1], atol=1e-6)
+    np.testing.assert_allclose(dpr, ref[2], rtol=1e-4, atol=1e-4)
 
 
 @pytest.mark.parametrize("n,width", [(24, 3), (24, 8), (32, 5), (48, 4), (48, 9), (96, 10), (64, 7), (20, 6), (21, 8)])
