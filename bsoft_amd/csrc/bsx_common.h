@@ -4,6 +4,9 @@
 #pragma once
 
 #include <cmath>
+#include <map>
+#include <mutex>
+#include <system_error>
 #include <vector>
 #include <thread>
 #include <algorithm>
@@ -24,22 +27,29 @@ inline double lambda_of(double av) {
 }
 
 // Host loop over [0, n) split into contiguous ranges on up to 16 threads
-// (f(begin, end, thread)); runs inline below `grain` items. Used for the
-// per-particle record preparation, which is independent per item.
+// (f(begin, end, thread)), `share` items or more each; runs inline below `grain`
+// items. Used for the per-particle record preparation, which is independent per
+// item.
 template <class F>
-inline void host_parallel(int64_t n, int64_t grain, F f) {
+inline void host_parallel(int64_t n, int64_t grain, F f, int64_t share = 0) {
     unsigned nt = std::thread::hardware_concurrency();
     nt = std::max(1u, std::min(nt, 16u));
     if (n < grain || nt == 1) {
         f((int64_t)0, n, 0u);
         return;
     }
-    nt = (unsigned)std::min<int64_t>(nt, (n + grain - 1) / grain);
+    if (share <= 0) share = grain;
+    nt = (unsigned)std::min<int64_t>(nt, (n + share - 1) / share);
     std::vector<std::thread> pool;
     const int64_t per = (n + nt - 1) / nt;
     for (unsigned t = 1; t < nt; ++t) {
         const int64_t b = t * per, e = std::min(n, b + per);
-        if (b < e) pool.emplace_back(f, b, e, t);
+        if (b >= e) break;
+        try {
+            pool.emplace_back(f, b, e, t);
+        } catch (const std::system_error&) {   // no thread to be had: the range runs here
+            f(b, e, t);
+        }
     }
     f((int64_t)0, std::min(n, per), 0u);
     for (auto& th : pool) th.join();
@@ -288,6 +298,21 @@ inline std::vector<float> fsi_table(int wd, int power) {
     std::vector<float> t((size_t)(FSI_NDIV + 1) * (power < 0 ? 1 : wd));
     fsi_table_into(t.data(), wd, power);
     return t;
+}
+
+// The same, kept for the next call (4,000 sines, cosines and powers take longer
+// than a small extraction). Entries are never changed or dropped; at most 32
+// (width, power) pairs are kept, further ones are recomputed per thread.
+inline const std::vector<float>& fsi_table_kept(int wd, int power) {
+    static std::mutex mu;
+    static std::map<std::pair<int, int>, std::vector<float>> tabs;
+    static thread_local std::vector<float> other;
+    const auto key = std::make_pair(power < 0 ? 1 : wd, std::max(power, -1));
+    std::lock_guard<std::mutex> g(mu);
+    auto it = tabs.find(key);
+    if (it != tabs.end()) return it->second;
+    if (tabs.size() >= 32) return other = fsi_table(wd, power);
+    return tabs[key] = fsi_table(wd, power);
 }
 
 // Periodic index in [0, N): one compare in the usual in-range case, a

@@ -9,6 +9,7 @@
 //   k_frc_pairs      : img_recip_space_fom, fom_type 0 (src/mg/mg_refine.cpp:660-781)
 #include <climits>
 #include <cmath>
+#include <cstring>
 #include <mutex>
 #include <vector>
 
@@ -446,21 +447,21 @@ int bsx_extract(const float* ft_dev, int n, double sampling, const double* mats,
                          kernel_power, out_dev, "bsx_extract");
     if (r != BSX_OK || nviews == 0) return r;
     hipStream_t s = (hipStream_t)stream;
-    std::vector<float> tab = fsi_table(kernel_width, kernel_power);
-    float* dtab = nullptr;
-    double* dmats = nullptr;
-    BSX_HIP(hipMalloc(&dtab, sizeof(float) * tab.size()));
-    BSX_HIP(hipMalloc(&dmats, sizeof(double) * 9 * nviews));
-    BSX_HIP(hipMemcpyAsync(dtab, tab.data(), sizeof(float) * tab.size(), hipMemcpyHostToDevice, s));
-    BSX_HIP(hipMemcpyAsync(dmats, mats, sizeof(double) * 9 * nviews, hipMemcpyHostToDevice, s));
-    r = extract_launch(ft_dev, n, sampling, dmats, nviews, resolution, kernel_width, center, dtab,
-                       out_dev, s);
-    hipError_t se = hipStreamSynchronize(s);
-    (void)hipFree(dtab);
-    (void)hipFree(dmats);
-    if (r != BSX_OK) return r;
-    BSX_HIP(se);
-    return BSX_OK;
+    const std::vector<float>& tab = fsi_table_kept(kernel_width, kernel_power);
+    // matrices, then the kernel table: one copy from pinned memory
+    const size_t nm = sizeof(double) * 9 * nviews, nt = sizeof(float) * tab.size();
+    Scratch dev, pin(true);
+    BSX_HIP(dev.get(nm + nt));
+    BSX_HIP(pin.get(nm + nt));
+    memcpy(pin.as<char>(), mats, nm);
+    memcpy(pin.as<char>() + nm, tab.data(), nt);
+    BSX_HIP(hipMemcpyAsync(dev.as<char>(), pin.as<char>(), nm + nt, hipMemcpyHostToDevice, s));
+    r = extract_launch(ft_dev, n, sampling, dev.as<double>(), nviews, resolution, kernel_width, center,
+                       (const float*)(dev.as<char>() + nm), out_dev, s);
+    BSX_HIP(hipStreamSynchronize(s));
+    dev.release();
+    pin.release();
+    return r;
 }
 
 // ---------------------------------------------- allocation-free extraction
@@ -532,8 +533,9 @@ int bsx_fsc(const float* a_dev, const float* b_dev, int n, double sampling, doub
     long maxrad = (long)(n * sampling / hi_res);
     BSX_REQUIRE(maxrad <= *nshell, BSX_ERR_ARG, "bsx_fsc: %ld shells exceed capacity %d", maxrad,
                 *nshell);
-    double* d = nullptr;
-    BSX_HIP(hipMalloc(&d, sizeof(double) * 3 * (maxrad + 1)));
+    Scratch buf;
+    BSX_HIP(buf.get(sizeof(double) * 3 * (maxrad + 1)));
+    double* d = buf.as<double>();
     BSX_HIP(hipMemsetAsync(d, 0, sizeof(double) * 3 * (maxrad + 1), s));
     hipLaunchKernelGGL(k_fsc, dim3(1024), dim3(256), sizeof(double) * 3 * maxrad, s,
                        (const float2*)a_dev, (const float2*)b_dev, n, maxrad, d);
@@ -542,7 +544,7 @@ int bsx_fsc(const float* a_dev, const float* b_dev, int n, double sampling, doub
     if (maxrad > 0)
         BSX_HIP(hipMemcpyAsync(h.data(), d, sizeof(double) * 3 * maxrad, hipMemcpyDeviceToHost, s));
     BSX_HIP(hipStreamSynchronize(s));
-    (void)hipFree(d);
+    buf.release();
     BSX_HIP(le);
     for (long i = 0; i < maxrad; ++i) {
         double den = h[i] * h[maxrad + i];
@@ -567,14 +569,13 @@ static int fsc_dpr_impl(const float* map1_dev, const float* map2_dev, int n, int
     BSX_REQUIRE(maxrad <= *nrows, BSX_ERR_ARG, "bsx_fsc_dpr: %ld rows exceed capacity %d", maxrad,
                 *nrows);
     const long long n3 = (long long)(n / 2) * n * nz;   // a transform's kept half
-    float2* v = nullptr;
-    double* d = nullptr;
-    BSX_HIP(hipMalloc(&v, sizeof(float2) * 2 * n3));
-    if (hipMalloc(&d, sizeof(double) * 4 * maxrad) != hipSuccess) {
-        (void)hipFree(v);
+    Scratch vols, sums;
+    if (vols.get(sizeof(float2) * 2 * n3) != hipSuccess || sums.get(sizeof(double) * 4 * maxrad) != hipSuccess) {
         set_error("bsx_fsc_dpr: allocation failed");
         return BSX_ERR_NOMEM;
     }
+    float2* v = vols.as<float2>();
+    double* d = sums.as<double>();
     int r = BSX_OK;
     // the sums read x < n / 2 only: the x pass keeps that half, the other passes
     // transform both halves' columns in one launch each
@@ -594,12 +595,12 @@ static int fsc_dpr_impl(const float* map1_dev, const float* map2_dev, int n, int
              hipSuccess ||
          hipStreamSynchronize(s) != hipSuccess))
         r = BSX_ERR_DEVICE;
-    (void)hipFree(v);
-    (void)hipFree(d);
     if (r) {
         set_error("bsx_fsc_dpr: device error");
         return r;
     }
+    vols.release();
+    sums.release();
     // curves: (s, FSC, DPR in degrees) per row (Bimage_resolution.cpp:225-239)
     for (long i = 0; i < maxrad; ++i) {
         double fsc = h[2 * maxrad + i], dpr = 0;
@@ -652,10 +653,11 @@ int bsx_score_frc(const float* part_dev, int64_t nparts, const float* ref_dev, i
     if (max_rad_cv <= max_rad) max_rad_cv = max_rad + 1;
     double min_rad_sq = 0;
     if (lo_res > 0) { min_rad_sq = n * sampling / lo_res; min_rad_sq *= min_rad_sq; }
-    int* dp = nullptr;
-    double* dout = nullptr;
-    BSX_HIP(hipMalloc(&dp, sizeof(int) * 2 * npairs));
-    BSX_HIP(hipMalloc(&dout, sizeof(double) * npairs));
+    Scratch bp, bo;
+    BSX_HIP(bp.get(sizeof(int) * 2 * npairs));
+    BSX_HIP(bo.get(sizeof(double) * npairs));
+    int* dp = bp.as<int>();
+    double* dout = bo.as<double>();
     BSX_HIP(hipMemcpyAsync(dp, pairs, sizeof(int) * 2 * npairs, hipMemcpyHostToDevice, s));
     hipLaunchKernelGGL(k_frc_pairs, dim3((unsigned)npairs), dim3(256), sizeof(double) * 3 * n, s,
                        (const float2*)part_dev, (const float2*)ref_dev, n, dp, min_rad_sq,
@@ -663,8 +665,8 @@ int bsx_score_frc(const float* part_dev, int64_t nparts, const float* ref_dev, i
     hipError_t le = hipGetLastError();
     BSX_HIP(hipMemcpyAsync(out, dout, sizeof(double) * npairs, hipMemcpyDeviceToHost, s));
     BSX_HIP(hipStreamSynchronize(s));
-    (void)hipFree(dp);
-    (void)hipFree(dout);
+    bp.release();
+    bo.release();
     BSX_HIP(le);
     return BSX_OK;
 }

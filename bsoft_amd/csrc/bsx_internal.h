@@ -2,6 +2,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <stddef.h>
 #include <stdint.h>
 #include <string>
 
@@ -30,6 +31,32 @@ const char* last_error();
             return (code);                                                              \
         }                                                                               \
     } while (0)
+
+// ---- workspaces of calls without a handle (bsx_fft.hip) ----
+// A device (or pinned host) buffer for one call. Allocating and freeing on every
+// call cost more than the kernels of small calls and stalled large ones for
+// milliseconds, so a buffer that its call has finished with is kept for the next
+// one: at most 16 buffers and 512 MB of each kind, the least recently used going
+// first, all of them given back when an allocation fails. release() says that the
+// call's stream has been waited for, i.e. that nothing uses the buffer any more, so
+// any thread may take it for any stream; a buffer that is destroyed without it
+// (an error return) is freed, which waits for the device.
+class Scratch {
+public:
+    explicit Scratch(bool pinned = false) : pinned_(pinned) {}
+    Scratch(const Scratch&) = delete;
+    Scratch& operator=(const Scratch&) = delete;
+    ~Scratch();
+    hipError_t get(size_t bytes);
+    void release();
+    template <class T> T* as() const { return static_cast<T*>(p_); }
+
+private:
+    void* p_ = nullptr;
+    size_t bytes_ = 0;
+    int dev_ = 0;
+    bool pinned_;
+};
 
 // ---- FFT launchers (bsx_fft.hip) ----
 // Batched in-place C2C transform along one axis of a (nz, ny, nx) complex

@@ -423,7 +423,7 @@ __global__ __launch_bounds__(1024) void k_weigh_pairs(float* __restrict__ S, flo
                                                       int N, int nz, int NT, long long nrec, int hmask,
                                                       int nhalves, float2* __restrict__ out,
                                                       float* __restrict__ fom_out,
-                                                      double* __restrict__ fin) {
+                                                      double* __restrict__ fin, int* __restrict__ flags) {
     constexpr int RS = FOM ? 5 : 3;
     const unsigned nxh = N / 2 + 1, total = nxh * (unsigned)N * (unsigned)nz;
     double sums[5] = {0, 0, 0, 0, 0};
@@ -530,6 +530,10 @@ __global__ __launch_bounds__(1024) void k_weigh_pairs(float* __restrict__ S, flo
         }
     }
     block_add(sums, fin);
+    if (flags && blockIdx.x == 0 && threadIdx.x == 0) {
+        *(int*)(fin + 5) = *flags;
+        *flags = 0;
+    }
 }
 
 // Shell sums of fspace_reconstruction_stats (Bimage_reconstruct.cpp:526-599).
@@ -1262,6 +1266,7 @@ int bsx_recon_create(bsx_recon** out, const bsx_recon_params* p) {
         BSX_HIP(hipMemset(h->fill, 0, sizeof(int) * h->nbins));
         BSX_HIP(hipMemset(h->chunks, 0xFF, sizeof(int) * (size_t)h->nbins * h->maxc));
         BSX_HIP(hipMemset(h->pool, 0, sizeof(int) * 2));
+        BSX_HIP(hipMemset(h->entries, 0, sizeof(unsigned long long)));
     }
     BSX_HIP(hipMemset(h->acc, 0, h->acc_elems * sizeof(float)));
     BSX_HIP(hipDeviceSynchronize());
@@ -1446,6 +1451,10 @@ static int insert_prepare(bsx_recon* h, const bsx_particle* parts, int64_t n, hi
     {
         std::vector<double> tmax(16, 0.0);
         std::vector<int> trun(16, 0);
+        // a record takes 0.13 us and a thread some 15 us to start, or milliseconds
+        // when other threads of the process have used up the CPU share, so that
+        // smaller sets stay on this thread (3,001 records: 390 us, 160 us on 8
+        // threads, at times 3 ms); 10,000 records 700 us on 2 threads, 350 us on 16
         host_parallel(n, 8192, [&](int64_t b, int64_t e, unsigned t) {
             double m = 0;
             int run = 0;
@@ -1464,7 +1473,7 @@ static int insert_prepare(bsx_recon* h, const bsx_particle* parts, int64_t n, hi
             }
             tmax[t] = m;
             trun[t] = run;
-        });
+        }, 640);
         for (double m : tmax) max_step = std::max(max_step, m);
         for (int r : trun) max_run = std::max(max_run, r);
     }
@@ -1503,7 +1512,8 @@ int bsx_recon_insert(bsx_recon* h, const float* imgs_dev, const bsx_particle* pa
     if (check_nan) BSX_HIP(hipMemsetAsync(h->nonfinite, 0, sizeof(int), s));
     h->timing = h->p.flags & BSX_FLAG_TIMING;
     h->nev = 0;
-    if (h->binned) BSX_HIP(hipMemsetAsync(h->entries, 0, sizeof(unsigned long long), s));
+    // (the entry count is read with the timing only)
+    if (h->binned && h->timing) BSX_HIP(hipMemsetAsync(h->entries, 0, sizeof(unsigned long long), s));
     int r = tmark(h, s, -1);
     if (r) return r;
     hipLaunchKernelGGL(k_background, dim3((unsigned)n), dim3(256), 0, s, imgs_dev, h->recs,
@@ -1916,8 +1926,9 @@ int bsx_rescale_to_avg_std(float* data_dev, int64_t n, double avg, double std, v
                 "bsx_rescale_to_avg_std: cannot use a negative standard deviation (%g)", std);
     hipStream_t s = (hipStream_t)stream;
     const int nblk = (int)std::min<int64_t>(1024, (n + 255) / 256);
-    double2* part = nullptr;
-    BSX_HIP(hipMalloc((void**)&part, sizeof(double2) * (nblk + 1)));
+    Scratch buf;
+    BSX_HIP(buf.get(sizeof(double2) * (nblk + 1)));
+    double2* part = buf.as<double2>();
     hipLaunchKernelGGL(k_moments, dim3(nblk), dim3(256), 0, s, data_dev, (long long)n, part);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) {
@@ -1931,8 +1942,8 @@ int bsx_rescale_to_avg_std(float* data_dev, int64_t n, double avg, double std, v
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipStreamSynchronize(s);
-    (void)hipFree(part);
     BSX_HIP(e);
+    buf.release();
     return BSX_OK;
 }
 
@@ -2128,16 +2139,16 @@ int bsx_recon_stats(bsx_recon* h, int imap, int nmaps, double resolution, double
 // Weighing of the summed halves in hmask into vol (and the FOM map), after
 // folding the binned accumulator where `fold` is set; the coverage count and the
 // weight and Friedel sums are added to fin (5 doubles), which the caller has
-// cleared.
+// cleared; with `flags` the fallback flags move from there to fin's sixth place.
 static int launch_weigh(bsx_recon* h, int hmask, bool fold, float2* vol, float* fom_dev, double* fin,
-                        hipStream_t s) {
+                        int* flags, hipStream_t s) {
     const int N = h->K.N, nz = h->K.nz;
     const long long nrec = (long long)h->K.NT * h->K.NT * h->K.NT * 4096;
     const long long pairs = (long long)(N / 2 + 1) * N * nz;
     const dim3 grid((unsigned)std::min(512LL, (pairs + 1023) / 1024));
     auto go = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, grid, dim3(1024), 0, s, h->acc, h->xacc, N, nz, h->K.NT, nrec, hmask,
-                           h->p.nhalves, vol, fom_dev, fin);
+                           h->p.nhalves, vol, fom_dev, fin, flags);
     };
     if (h->K.fom) fold ? go(k_weigh_pairs<true, true>) : go(k_weigh_pairs<true, false>);
     else fold ? go(k_weigh_pairs<false, true>) : go(k_weigh_pairs<false, false>);
@@ -2196,49 +2207,44 @@ int bsx_recon_finish(bsx_recon* h, int imap, int nmaps, float* map_dev, float* f
     const int N = h->K.N, nz = h->K.nz;
     const long long n3 = (long long)N * N * nz;   // a 2D map: one plane
     float2* vol = (float2*)ft_dev;
-    float2* tmp = nullptr;
+    Scratch tmp, wtmp, fin, pin(true);
     if (!vol) {
-        BSX_HIP(hipMalloc((void**)&tmp, sizeof(float2) * n3));
-        vol = tmp;
+        BSX_HIP(tmp.get(sizeof(float2) * n3));
+        vol = tmp.as<float2>();
     }
-    double* dfin = nullptr;
-    BSX_HIP(hipMalloc((void**)&dfin, 5 * sizeof(double)));
-    BSX_HIP(hipMemsetAsync(dfin, 0, 5 * sizeof(double), s));
+    // the finish sums and, after them, the atomic-fallback flags of the inserts
+    // since the last read (graph replays included; cleared for the next inserts)
+    BSX_HIP(fin.get(6 * sizeof(double)));
+    BSX_HIP(pin.get(6 * sizeof(double)));
+    BSX_HIP(hipMemsetAsync(fin.as<double>(), 0, 6 * sizeof(double), s));
     {
-        const int rw = launch_weigh(h, hmask, h->binned && h->xdirty, vol, fom_dev, dfin, s);
+        const int rw = launch_weigh(h, hmask, h->binned && h->xdirty, vol, fom_dev, fin.as<double>(),
+                                    h->binned ? h->pool + 1 : nullptr, s);
         if (rw) return rw;
         h->xdirty = false;
     }
-    double fin[5] = {0, 0, 0, 0, 0};
-    BSX_HIP(hipMemcpyAsync(fin, dfin, sizeof(fin), hipMemcpyDeviceToHost, s));
-    // atomic-fallback flags of the inserts since the last read (graph
-    // replays included); cleared for the next inserts
-    int hflags = 0;
-    if (h->binned) {
-        BSX_HIP(hipMemcpyAsync(&hflags, h->pool + 1, sizeof(int), hipMemcpyDeviceToHost, s));
-        BSX_HIP(hipMemsetAsync(h->pool + 1, 0, sizeof(int), s));
-    }
+    BSX_HIP(hipMemcpyAsync(pin.as<double>(), fin.as<double>(), 6 * sizeof(double), hipMemcpyDeviceToHost, s));
     int r = BSX_OK;
     if (map_dev) {
         // inverse transform: work on a copy when the caller wants the transform back
         float2* work = vol;
-        float2* wtmp = nullptr;
         if (ft_dev) {
-            BSX_HIP(hipMalloc((void**)&wtmp, sizeof(float2) * n3));
-            BSX_HIP(hipMemcpyAsync(wtmp, vol, sizeof(float2) * n3, hipMemcpyDeviceToDevice, s));
-            work = wtmp;
+            BSX_HIP(wtmp.get(sizeof(float2) * n3));
+            work = wtmp.as<float2>();
+            BSX_HIP(hipMemcpyAsync(work, vol, sizeof(float2) * n3, hipMemcpyDeviceToDevice, s));
         }
         r = launch_inverse(h, work, map_dev, s);
-        BSX_HIP(hipStreamSynchronize(s));
-        if (wtmp) BSX_HIP(hipFree(wtmp));
     }
     BSX_HIP(hipStreamSynchronize(s));
-    h->fallback_flags |= hflags;
-    if (tmp) BSX_HIP(hipFree(tmp));
-    BSX_HIP(hipFree(dfin));
-    if (r != BSX_OK) return r;
-    if (stats) fill_stats(h, hmask, fin, stats);
-    return BSX_OK;
+    int flags = 0;
+    memcpy(&flags, pin.as<double>() + 5, sizeof(flags));
+    h->fallback_flags |= flags;
+    if (r == BSX_OK && stats) fill_stats(h, hmask, pin.as<double>(), stats);
+    tmp.release();
+    wtmp.release();
+    fin.release();
+    pin.release();
+    return r;
 }
 
 
@@ -2273,7 +2279,7 @@ static int group_member_launch(bsx_recon* h, const float* imgs, int64_t n, float
         const int rr = run_batch(h, imgs, p0, (int)std::min<int64_t>(h->batch, n - p0), s);
         if (rr) return rr;
     }
-    const int r = launch_weigh(h, h->p.nhalves > 1 ? 3 : 1, h->binned, h->gvol, nullptr, h->gfin, s);
+    const int r = launch_weigh(h, h->p.nhalves > 1 ? 3 : 1, h->binned, h->gvol, nullptr, h->gfin, nullptr, s);
     if (r) return r;
     return launch_inverse(h, h->gvol, map_dev, s);
 }

@@ -1525,7 +1525,7 @@ int bsx_search_create(bsx_search** out, const bsx_search_params* prm) {
     int64_t c1 = 0, c2 = 0, c3 = 0;
     rc = grow(h, &h->d_hk, &c1, h->Nd, "disk table");
     if (rc == BSX_OK) rc = grow(h, &h->d_ring, &c2, R + 1, "ring table");
-    std::vector<float> tab = fsi_table(h->p.kernel_width, h->p.kernel_power);
+    const std::vector<float>& tab = fsi_table_kept(h->p.kernel_width, h->p.kernel_power);
     if (rc == BSX_OK) rc = grow(h, &h->d_ktab, &c3, (int64_t)tab.size(), "kernel table");
     if (rc == BSX_OK &&
         (hipMemcpy(h->d_hk, h->hk.data(), sizeof(int2) * h->Nd, hipMemcpyHostToDevice) != hipSuccess ||
@@ -1630,7 +1630,9 @@ int bsx_search_stage(bsx_search* h, const float* imgs_dev, const bsx_particle* p
                     BSX_ERR_ARG, "bsx_search_stage: particle %lld has invalid parameters", (long long)i);
     }
     // records (CTF coefficients, wavelength) built on host threads
-    std::vector<SPart> sp((size_t)n);
+    Scratch pin(true);
+    BSX_HIP(pin.get(sizeof(SPart) * std::max<int64_t>(n, 1)));
+    SPart* sp = pin.as<SPart>();
     const bool ctf_flag = (h->p.flags & BSX_SEARCH_CTF) != 0;
     host_parallel(n, 4096, [&](int64_t b, int64_t e, unsigned) {
         for (int64_t i = b; i < e; ++i) {
@@ -1656,20 +1658,24 @@ int bsx_search_stage(bsx_search* h, const float* imgs_dev, const bsx_particle* p
     if (rc) return rc;
     BSX_HIP(hipMemsetAsync(h->d_pbf, 0, sizeof(uint16_t) * ppad * Kp, s));
     h->nparts = n;
-    if (n == 0) return BSX_OK;
+    if (n == 0) {
+        pin.release();   // nothing was copied from it
+        return BSX_OK;
+    }
     const int64_t per = (int64_t)N * N;
     // fused path: one kernel reads each image once
     const size_t fused_lds = fused_stage_lds(N, h->R, Nd);
     if (fused_lds) {
         rc = grow(h, &h->d_sp, &h->sp_cap, n, "particle records");
         if (rc) return rc;
-        BSX_HIP(hipMemcpyAsync(h->d_sp, sp.data(), sizeof(SPart) * n, hipMemcpyHostToDevice, s));
+        BSX_HIP(hipMemcpyAsync(h->d_sp, sp, sizeof(SPart) * n, hipMemcpyHostToDevice, s));
         const float2* tw = twiddles(N, s);
         BSX_REQUIRE(tw, BSX_ERR_DEVICE, "twiddles(%d) failed", N);
         rc = launch_stage_fused(N, (unsigned)n, fused_lds, s, imgs_dev, tw, h->d_sp, h->d_hk,
                                 h->d_ring, h->R, Nd, Kp, h->d_fp, h->d_ctf, h->d_pbf);
         if (rc) return rc;
         BSX_HIP(hipStreamSynchronize(s));   // the host records are released on return
+        pin.release();
         return BSX_OK;
     }
     // otherwise: full spectra, in chunks of at most 256 MB
@@ -1678,7 +1684,7 @@ int bsx_search_stage(bsx_search* h, const float* imgs_dev, const bsx_particle* p
     if (!rc) rc = grow(h, &h->d_sp, &h->sp_cap, n, "particle records");
     if (rc) return rc;
     // all records stay on the device: the origin/defocus fit reads them later
-    BSX_HIP(hipMemcpyAsync(h->d_sp, sp.data(), sizeof(SPart) * n, hipMemcpyHostToDevice, s));
+    BSX_HIP(hipMemcpyAsync(h->d_sp, sp, sizeof(SPart) * n, hipMemcpyHostToDevice, s));
     for (int64_t p0 = 0; p0 < n; p0 += chunk) {
         const int64_t nb = std::min(chunk, n - p0);
         rc = fft_real_x(imgs_dev + p0 * per, h->d_spec, N, (long long)nb * N, N, s);
@@ -1690,6 +1696,7 @@ int bsx_search_stage(bsx_search* h, const float* imgs_dev, const bsx_particle* p
         BSX_HIP(hipGetLastError());
         BSX_HIP(hipStreamSynchronize(s));   // records and spectra are reused
     }
+    pin.release();
     return BSX_OK;
 }
 
@@ -2137,13 +2144,12 @@ int bsx_search_cnn_input(bsx_search* h, int32_t S, float* out_dev, void* stream)
         if (i > 0) gidx[(size_t)((-kk + S) % S) * S + (-hh + S) % S] = -i - 1;
     }
     hipStream_t s = (hipStream_t)stream;
-    int* dg = nullptr;
-    int64_t gcap = 0;
-    int rc = grow(h, &dg, &gcap, (int64_t)S * S, "network input table");
-    if (rc) return rc;
+    Scratch tab;
+    BSX_HIP(tab.get(sizeof(int) * S * S));
+    int* dg = tab.as<int>();
     const int64_t S2 = (int64_t)S * S;
     const int64_t chunk = std::max<int64_t>(1, std::min<int64_t>(n, (256ll << 20) / (8 * S2)));
-    rc = grow(h, &h->d_spec, &h->spec_cap, chunk * S2, "network input grids");
+    int rc = grow(h, &h->d_spec, &h->spec_cap, chunk * S2, "network input grids");
     if (rc == BSX_OK &&
         hipMemcpyAsync(dg, gidx.data(), sizeof(int) * S2, hipMemcpyHostToDevice, s) != hipSuccess) {
         set_error("bsx_search_cnn_input: table upload failed");
@@ -2160,9 +2166,8 @@ int bsx_search_cnn_input(bsx_search* h, int32_t S, float* out_dev, void* stream)
         hipLaunchKernelGGL(k_cnn_norm, dim3((unsigned)nb), dim3(256), 0, s, h->d_spec, S, p0, out_dev);
         if (hipGetLastError() != hipSuccess) { set_error("bsx_search_cnn_input: launch failed"); rc = BSX_ERR_DEVICE; break; }
     }
-    (void)hipStreamSynchronize(s);   // the table and the grids are released / reused
-    h->bytes -= sizeof(int) * gcap;
-    (void)hipFree(dg);
+    BSX_HIP(hipStreamSynchronize(s));   // the table and the grids are released / reused
+    tab.release();
     return rc;
 }
 

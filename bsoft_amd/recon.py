@@ -409,8 +409,11 @@ def central_sections(ft: torch.Tensor, mats: np.ndarray, sampling: float, resolu
 def project(ft: torch.Tensor, views: np.ndarray, sampling: float, resolution: float,
             kernel_width: int = 8, kernel_power: int = 2) -> torch.Tensor:
     """Bimage::project over a list of views (x, y, z, angle)."""
-    return central_sections(ft, view_to_matrix(views), sampling, resolution, kernel_width,
-                            kernel_power, True)
+    v = np.ascontiguousarray(views, dtype=np.float64).reshape(-1, 4)
+    mats = np.empty((len(v), 9))
+    call("bsx_view_matrices", v.ctypes.data_as(C.POINTER(C.c_double)), len(v),
+         mats.ctypes.data_as(C.POINTER(C.c_double)))
+    return central_sections(ft, mats, sampling, resolution, kernel_width, kernel_power, True)
 
 
 def fsc(a: torch.Tensor, b: torch.Tensor, sampling: float, hi_res: float) -> np.ndarray:

@@ -156,3 +156,41 @@ def test_sections_of_every_tile_path(n, width):
     for i, m in enumerate(mats):
         ref = o.central_section(ft, 1.5, m, 1.5, width, 2, 1)
         assert np.abs(out[i] - ref).max() <= 1e-5 * np.abs(ref).max()
+
+
+def test_workspaces_shared_by_threads_and_streams():
+    """Calls without a handle keep their workspaces between calls: four threads,
+    each on a stream of its own and with sizes of its own, get the results of
+    the same calls made one after the other."""
+    import threading
+    rng = np.random.default_rng(8)
+    work = []
+    for n in (32, 48, 64, 32):
+        a = torch.as_tensor(rng.normal(size=(n, n, n)).astype(np.float32)).cuda()
+        b = torch.as_tensor(rng.normal(size=(n, n, n)).astype(np.float32)).cuda()
+        work.append((a, b, synth.uniform_views(5, rng)))
+
+    def one(a, b, views):
+        s, fsc, dpr = bresolve.fsc_dpr(a, b, 1.5)
+        ft = recon.map_transform(a)
+        return fsc, dpr, recon.project(ft, views, 1.5, 3.0, 5).cpu().numpy()
+
+    want = [one(*w) for w in work]
+    torch.cuda.synchronize()
+    bad = []
+
+    def loop(i):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(10):
+                got = one(*work[i])
+                for g, w in zip(got, want[i]):
+                    if not np.allclose(g, w, rtol=1e-9, atol=1e-12):
+                        bad.append(i)
+
+    say("workspaces: 4 threads x 10 rounds")
+    ts = [threading.Thread(target=loop, args=(i,)) for i in range(4)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not bad
