@@ -44,13 +44,8 @@ typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16;
 
 namespace {
 
-constexpr int GM = 128;          // GEMM tile rows (particles)
-constexpr int GN = 128;          // GEMM tile columns (library views)
 constexpr int GK = 64;           // K step staged in LDS
 constexpr int LROW = GK * 2 + 16;  // bytes per staged row (16-byte pad: conflict-free b128 reads)
-constexpr int CROW = GN + 1;     // floats per epilogue row
-constexpr int GEMM_LDS = 2 * (GM + GN) * LROW;   // 73,728 B, aliased by the 66,048-B epilogue tile
-static_assert(GM * CROW * 4 <= GEMM_LDS, "epilogue tile must fit the staging buffers");
 
 __device__ inline uint16_t to_bf16(float f) {
     uint32_t u = __float_as_uint(f);
@@ -435,7 +430,7 @@ __global__ __launch_bounds__(512) void k_gemm_topk4(const uint16_t* __restrict__
 // ------------------------------------------------- proposal-restricted GEMM
 // Routing of (particle, proposal slot) pairs to their proposed class, so
 // that one class's member views are scored against all particles that
-// proposed it with one MFMA tile (a grouped GEMM).
+// proposed it with one MFMA tile (a grouped GEMM). All on the device.
 __global__ void k_route_count(const int* __restrict__ cls, int64_t n, int k, int nclass,
                               int* __restrict__ counts) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -444,198 +439,200 @@ __global__ void k_route_count(const int* __restrict__ cls, int64_t n, int k, int
     if (c >= 0 && c < nclass) atomicAdd(counts + c, 1);
 }
 
-__global__ void k_route_fill(const int* __restrict__ cls, int64_t n, int k, int nclass,
-                             int* __restrict__ cursors, int* __restrict__ pairs) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n * k) return;
-    const int c = cls[t];
-    if (c >= 0 && c < nclass) pairs[atomicAdd(cursors + c, 1)] = (int)t;   // t = particle * k + slot
-}
-
-// Unrouted slots (no valid class) still need empty lists for the merge.
-__global__ void k_route_empty(const int* __restrict__ cls, int64_t n, int k, int nclass, int T,
-                              float* __restrict__ pscore, int* __restrict__ pidx) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n * k) return;
-    const int c = cls[t];
-    if (c >= 0 && c < nclass) return;
-    for (int q = 0; q < T; ++q) { pscore[t * T + q] = -INFINITY; pidx[t * T + q] = -1; }
-}
-
 struct GroupItem {
     int cls, p0, np, pad_;
 };
+constexpr int RM = 64, RN = 64;   // routed pairs x member views of a grouped GEMM tile
 
-// One workgroup per work item: up to 128 routed pairs of one class against
-// the class's member views (128 per column tile). Rows are gathered by
-// index (zero row for padding); the per-pair top-T over the members goes to
-// pscore/pidx[(particle * k + slot) * T + q].
+// Exclusive sums of the class counts (the fill's cursors) and the list of work
+// items, up to RM routed pairs of one class each: one workgroup, so that the
+// host need not see the counts. nitems: the number of items.
+__global__ __launch_bounds__(1024) void k_route_scan(const int* __restrict__ counts, int nclass,
+                                                     int* __restrict__ cursors,
+                                                     GroupItem* __restrict__ items,
+                                                     int* __restrict__ nitems) {
+    __shared__ int sp[1024], si[1024];
+    const int tid = threadIdx.x;
+    const int per = (nclass + 1023) / 1024;
+    const int c0 = min(nclass, tid * per), c1 = min(nclass, c0 + per);
+    int np = 0, ni = 0;
+    for (int c = c0; c < c1; ++c) {
+        np += counts[c];
+        ni += (counts[c] + RM - 1) / RM;
+    }
+    sp[tid] = np;
+    si[tid] = ni;
+    __syncthreads();
+    for (int o = 1; o < 1024; o <<= 1) {
+        const int a = tid >= o ? sp[tid - o] : 0, b = tid >= o ? si[tid - o] : 0;
+        __syncthreads();
+        sp[tid] += a;
+        si[tid] += b;
+        __syncthreads();
+    }
+    int p = sp[tid] - np, i = si[tid] - ni;
+    for (int c = c0; c < c1; ++c) {
+        const int n = counts[c];
+        cursors[c] = p;
+        for (int q = 0; q < n; q += RM) items[i++] = GroupItem{c, p + q, min(RM, n - q), 0};
+        p += n;
+    }
+    if (tid == 1023) *nitems = si[1023];
+}
+
+// Places every (particle, slot) pair in its class's range; slots without a valid
+// class still need empty lists for the merge.
+__global__ void k_route_fill(const int* __restrict__ cls, int64_t n, int k, int nclass, int T,
+                             int* __restrict__ cursors, int* __restrict__ pairs,
+                             float* __restrict__ pscore, int* __restrict__ pidx) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= n * k) return;
+    const int c = cls[t];
+    if (c >= 0 && c < nclass) {
+        pairs[atomicAdd(cursors + c, 1)] = (int)t;   // t = particle * k + slot
+        return;
+    }
+    for (int q = 0; q < T; ++q) { pscore[t * T + q] = -INFINITY; pidx[t * T + q] = -1; }
+}
+
+// One workgroup (4 waves of 32 x 32) per work item: up to 64 routed pairs of one
+// class against the class's member views, 64 a tile. At 4-degree views in
+// 15-degree classes a class has some 53 members and, for 8,000 particles x 16
+// proposals, some 29 pairs, and every view's row is read about once: reading the
+// rows bounds it (1.3 GB there), so that tiles are small (four workgroups a CU
+// keep loads in flight) and rows beyond the pairs or members are not read.
+// 128 x 128 tiles took 417 us, these 226 us (3.7 TB/s of lines). The per-pair top T over the
+// members goes to pscore/pidx[(particle * k + slot) * T + q].
 template <int T>
 __global__ __launch_bounds__(256) void k_gemm_grouped(
-    const uint16_t* __restrict__ A, const uint16_t* __restrict__ B, const uint16_t* __restrict__ zrow,
-    int Kp, const GroupItem* __restrict__ items, const int* __restrict__ pairs, int k,
-    const int* __restrict__ members, const int* __restrict__ mcount, int maxm,
+    const uint16_t* __restrict__ A, const uint16_t* __restrict__ B, int Kp,
+    const GroupItem* __restrict__ items, const int* __restrict__ nitems, const int* __restrict__ pairs,
+    int k, const int* __restrict__ members, const int* __restrict__ mcount, int maxm,
     float* __restrict__ pscore, int* __restrict__ pidx) {
-    __shared__ __attribute__((aligned(16))) char lds[GEMM_LDS];
-    __shared__ int srow[GM];
-    __shared__ int scol[GN];
+    constexpr int CR = RN + 1;   // floats per epilogue row
+    constexpr int STAGE = (RM + RN) * LROW;
+    static_assert(RM * CR * 4 <= 2 * STAGE && RM * 4 * T * 8 <= 2 * STAGE, "epilogue fits the staging buffers");
+    __shared__ __attribute__((aligned(16))) char lds[2 * STAGE];
+    __shared__ int scol[RN];
+    if ((int)blockIdx.x >= *nitems) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
     const GroupItem it = items[blockIdx.x];
-    const int my_row = tid & (GM - 1), my_half = tid >> 7;
-    const int ncls_members = mcount[it.cls];
-    if (tid < GM) srow[tid] = tid < it.np ? pairs[it.p0 + tid] : -1;
+    const int nm = mcount[it.cls];
+    const int my_row = tid & (RM - 1), my_q = tid >> 6;   // epilogue: row, column quarter
     float best[T];
     int bidx[T];
 #pragma unroll
     for (int q = 0; q < T; ++q) { best[q] = -INFINITY; bidx[q] = -1; }
     const int nk = Kp / GK;
-    int ld_row[4], ld_part[4];
+    // staging: 64 rows of 8 16-byte chunks, A and B, two rows per thread each
+    const int ld_row = tid >> 3, ld_part = tid & 7;
+    const uint16_t* pa[2];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const int c = tid + 256 * q;
-        ld_row[q] = c >> 3;
-        ld_part[q] = c & 7;
+    for (int q = 0; q < 2; ++q) {
+        const int r = ld_row + 32 * q;
+        pa[q] = r < it.np ? A + (size_t)(pairs[it.p0 + r] / k) * Kp + ld_part * 8 : nullptr;
     }
-    const int ntile = (ncls_members + GN - 1) / GN;
-    for (int t = 0; t < ntile; ++t) {
+    const int own = my_row < it.np ? pairs[it.p0 + my_row] : -1;
+    const bool mine_a = wm * 32 < it.np;
+    for (int t0 = 0; t0 < nm; t0 += RN) {
+        __syncthreads();   // the epilogue before has been read
+        if (tid < RN) scol[tid] = t0 + tid < nm ? members[(size_t)it.cls * maxm + t0 + tid] : -1;
         __syncthreads();
-        if (tid < GN) {
-            const int j = t * GN + tid;
-            scol[tid] = j < ncls_members ? members[(size_t)it.cls * maxm + j] : -1;
+        const uint16_t* pb[2];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const int v = scol[ld_row + 32 * q];
+            pb[q] = v >= 0 ? B + (size_t)v * Kp + ld_part * 8 : nullptr;
         }
-        __syncthreads();
-        const uint16_t* pa[4];
-        const uint16_t* pb[4];
+        const bool mine = mine_a && t0 + wn * 32 < nm;   // this wave's block holds something
+        f32x16 acc;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int pr = srow[ld_row[q]];
-            pa[q] = pr >= 0 ? A + (size_t)(pr / k) * Kp : zrow;
-            const int vc = scol[ld_row[q]];
-            pb[q] = vc >= 0 ? B + (size_t)vc * Kp : zrow;
-        }
-        f32x16 acc[2][2];
+        for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+        uint4 ra[2], rb[2];
+        auto load = [&](int k0) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+            for (int q = 0; q < 2; ++q) {
+                ra[q] = pa[q] ? *(const uint4*)(pa[q] + k0) : make_uint4(0, 0, 0, 0);
+                rb[q] = pb[q] ? *(const uint4*)(pb[q] + k0) : make_uint4(0, 0, 0, 0);
+            }
+        };
+        auto store = [&](int buf) {
+            char* d = lds + buf * STAGE + ld_row * LROW + ld_part * 16;
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-        uint4 ra0, ra1, ra2, ra3, rb0, rb1, rb2, rb3;
-#define BSX_GGLOAD(K0)                                               \
-    ra0 = *(const uint4*)(pa[0] + (K0) + ld_part[0] * 8);            \
-    ra1 = *(const uint4*)(pa[1] + (K0) + ld_part[1] * 8);            \
-    ra2 = *(const uint4*)(pa[2] + (K0) + ld_part[2] * 8);            \
-    ra3 = *(const uint4*)(pa[3] + (K0) + ld_part[3] * 8);            \
-    rb0 = *(const uint4*)(pb[0] + (K0) + ld_part[0] * 8);            \
-    rb1 = *(const uint4*)(pb[1] + (K0) + ld_part[1] * 8);            \
-    rb2 = *(const uint4*)(pb[2] + (K0) + ld_part[2] * 8);            \
-    rb3 = *(const uint4*)(pb[3] + (K0) + ld_part[3] * 8);
-#define BSX_GLSTORE(BUF)                                                            \
-    *(uint4*)((BUF) + ld_row[0] * LROW + ld_part[0] * 16) = ra0;                    \
-    *(uint4*)((BUF) + ld_row[1] * LROW + ld_part[1] * 16) = ra1;                    \
-    *(uint4*)((BUF) + ld_row[2] * LROW + ld_part[2] * 16) = ra2;                    \
-    *(uint4*)((BUF) + ld_row[3] * LROW + ld_part[3] * 16) = ra3;                    \
-    *(uint4*)((BUF) + (GM + ld_row[0]) * LROW + ld_part[0] * 16) = rb0;             \
-    *(uint4*)((BUF) + (GM + ld_row[1]) * LROW + ld_part[1] * 16) = rb1;             \
-    *(uint4*)((BUF) + (GM + ld_row[2]) * LROW + ld_part[2] * 16) = rb2;             \
-    *(uint4*)((BUF) + (GM + ld_row[3]) * LROW + ld_part[3] * 16) = rb3;
-        BSX_GGLOAD(0)
-        BSX_GLSTORE(lds)
+            for (int q = 0; q < 2; ++q) {
+                *(uint4*)(d + 32 * q * LROW) = ra[q];
+                *(uint4*)(d + (RM + 32 * q) * LROW) = rb[q];
+            }
+        };
+        load(0);
+        store(0);
         __syncthreads();
         for (int kt = 0; kt < nk; ++kt) {
-            const bool more = kt + 1 < nk;
-            if (more) {
-                const size_t k0 = (size_t)(kt + 1) * GK;
-                BSX_GGLOAD(k0)
+            if (kt + 1 < nk) load((kt + 1) * GK);
+            if (mine) {
+                const char* fa = lds + (kt & 1) * STAGE + (wm * 32 + (lane & 31)) * LROW + (lane >> 5) * 16;
+                const char* fb = lds + (kt & 1) * STAGE + (RM + wn * 32 + (lane & 31)) * LROW + (lane >> 5) * 16;
+#pragma unroll
+                for (int ks = 0; ks < GK / 16; ++ks)
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)(fa + ks * 32),
+                                                                  *(const bf16x8*)(fb + ks * 32), acc, 0, 0, 0);
             }
-            const char* buf = lds + (kt & 1) * (GM + GN) * LROW;
-#pragma unroll
-            for (int ks = 0; ks < GK / 16; ++ks) {
-                bf16x8 fa[2], fb[2];
-                const int off = ks * 32 + (lane >> 5) * 16;
-#pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    fa[i] = *(const bf16x8*)(buf + (wm * 64 + i * 32 + (lane & 31)) * LROW + off);
-                    fb[i] = *(const bf16x8*)(buf + (GM + wn * 64 + i * 32 + (lane & 31)) * LROW + off);
-                }
-#pragma unroll
-                for (int i = 0; i < 2; ++i)
-#pragma unroll
-                    for (int j = 0; j < 2; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
-            }
-            if (more) {
-                char* nb = lds + ((kt + 1) & 1) * (GM + GN) * LROW;
-                BSX_GLSTORE(nb)
-            }
+            if (kt + 1 < nk) store((kt + 1) & 1);
             __syncthreads();
         }
-#undef BSX_GGLOAD
-#undef BSX_GLSTORE
         float* C = (float*)lds;
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int row = wm * 64 + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                    const int col = wn * 64 + j * 32 + (lane & 31);
-                    C[row * CROW + col] = acc[i][j][r];
-                }
+        for (int r = 0; r < 16; ++r)
+            C[(wm * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * CR + wn * 32 + (lane & 31)] = acc[r];
         __syncthreads();
-        const float* cr = C + my_row * CROW + my_half * 64;
-        for (int j = 0; j < 64; ++j) {
-            const int vc = scol[my_half * 64 + j];
-            if (vc < 0) continue;
-            const float v = cr[j];
-            if (v > best[T - 1]) {
-                best[T - 1] = v;
-                bidx[T - 1] = vc;
+        if (own >= 0)
+            for (int j = my_q * (RN / 4); j < min((my_q + 1) * (RN / 4), nm - t0); ++j) {
+                const float v = C[my_row * CR + j];
+                if (v > best[T - 1]) {
+                    best[T - 1] = v;
+                    bidx[T - 1] = scol[j];
 #pragma unroll
-                for (int q = T - 1; q > 0; --q) {
-                    if (best[q] > best[q - 1]) {
-                        const float tv = best[q]; best[q] = best[q - 1]; best[q - 1] = tv;
-                        const int ti = bidx[q]; bidx[q] = bidx[q - 1]; bidx[q - 1] = ti;
+                    for (int q = T - 1; q > 0; --q) {
+                        if (best[q] > best[q - 1]) {
+                            const float tv = best[q]; best[q] = best[q - 1]; best[q - 1] = tv;
+                            const int ti = bidx[q]; bidx[q] = bidx[q - 1]; bidx[q - 1] = ti;
+                        }
                     }
                 }
             }
-        }
     }
-    // combine the two column halves of each row into the row's list
+    // combine the four column quarters of each row into the row's list
     __syncthreads();
     float* xs = (float*)lds;
-    int* xi = (int*)(lds + GM * 2 * T * sizeof(float));
+    int* xi = (int*)(lds + RM * 4 * T * sizeof(float));
 #pragma unroll
     for (int q = 0; q < T; ++q) {
-        xs[(my_row * 2 + my_half) * T + q] = best[q];
-        xi[(my_row * 2 + my_half) * T + q] = bidx[q];
+        xs[(my_q * T + q) * RM + my_row] = best[q];
+        xi[(my_q * T + q) * RM + my_row] = bidx[q];
     }
     __syncthreads();
-    if (my_half == 0 && my_row < it.np) {
+    if (my_q != 0 || own < 0) return;
+    for (int e = T; e < 4 * T; ++e) {
+        const float v = xs[e * RM + my_row];
+        const int id = xi[e * RM + my_row];
+        if (id >= 0 && v > best[T - 1]) {
+            best[T - 1] = v;
+            bidx[T - 1] = id;
 #pragma unroll
-        for (int q = 0; q < T; ++q) {
-            const float v = xs[(my_row * 2 + 1) * T + q];
-            const int id = xi[(my_row * 2 + 1) * T + q];
-            if (id >= 0 && v > best[T - 1]) {
-                best[T - 1] = v;
-                bidx[T - 1] = id;
-#pragma unroll
-                for (int z = T - 1; z > 0; --z) {
-                    if (best[z] > best[z - 1]) {
-                        const float tv = best[z]; best[z] = best[z - 1]; best[z - 1] = tv;
-                        const int ti = bidx[z]; bidx[z] = bidx[z - 1]; bidx[z - 1] = ti;
-                    }
+            for (int z = T - 1; z > 0; --z) {
+                if (best[z] > best[z - 1]) {
+                    const float tv = best[z]; best[z] = best[z - 1]; best[z - 1] = tv;
+                    const int ti = bidx[z]; bidx[z] = bidx[z - 1]; bidx[z - 1] = ti;
                 }
             }
         }
-        const size_t o = (size_t)srow[my_row] * T;
+    }
+    const size_t o = (size_t)own * T;
 #pragma unroll
-        for (int q = 0; q < T; ++q) {
-            pscore[o + q] = best[q];
-            pidx[o + q] = bidx[q];
-        }
+    for (int q = 0; q < T; ++q) {
+        pscore[o + q] = best[q];
+        pidx[o + q] = bidx[q];
     }
 }
 
@@ -706,32 +703,77 @@ __global__ __launch_bounds__(256) void k_topk_merge(const float* __restrict__ ps
 // Ring correlation of img_recip_space_fom (fom_type 0, unit ring weights,
 // CTF on the section) over rings 0..R-1, one wavefront per comparison; ring
 // sums reduced across the wavefront in a fixed order.
-__device__ inline float wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+//
+// Sum over the 64 lanes by halving (lanes 32, 16, 8, 4, 2, 1 apart), in every
+// lane: permlane swaps for the first two steps, DPP row rotations and quad
+// permutations for the others, whose operands are equal to those of the xor
+// distance since the steps before left the halves alike. VALU only: the same
+// sums through ds_bpermute (six LDS round trips each, three sums a ring) took
+// most of k_rescore's time (8,000 particles x 8 candidates of 895 points: 332 us;
+// now, with four rings of loads in flight and one root per lane, 189 us).
+template <int CTRL>
+__device__ __forceinline__ float dpp_f(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+__device__ __forceinline__ float wave_sum(float v) {
+    const unsigned u = __float_as_uint(v);
+    const auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    const unsigned w = __float_as_uint(v);
+    const auto b = __builtin_amdgcn_permlane16_swap(w, w, false, false);
+    v = __uint_as_float(b[0]) + __uint_as_float(b[1]);
+    v += dpp_f<0x128>(v);   // row_ror:8
+    v += dpp_f<0x124>(v);   // row_ror:4
+    v += dpp_f<0x4E>(v);    // quad_perm [2,3,0,1]
+    v += dpp_f<0xB1>(v);    // quad_perm [1,0,3,2]
     return v;
 }
 
 __device__ inline float frc_wave(const float2* __restrict__ P, const float* __restrict__ Cf,
                                  const float2* __restrict__ S, const int* __restrict__ ring_start,
                                  int R, int lane) {
-    float f = 0.f;
-    for (int j = 0; j < R; ++j) {
-        float num = 0.f, dp = 0.f, dr = 0.f;
-        for (int i = ring_start[j] + lane; i < ring_start[j + 1]; i += 64) {
-            const float2 a = P[i];
-            const float c = Cf[i];
-            const float2 r = make_float2(S[i].x * c, S[i].y * c);
-            num += a.x * r.x + a.y * r.y;
-            dp += a.x * a.x + a.y * a.y;
-            dr += r.x * r.x + r.y * r.y;
+    constexpr int U = 4;   // rings whose first 64 points are loaded together
+    // lane j keeps the sums of ring j (R <= 64), so that the root and the division
+    // are done once for all rings; the terms are then added in the rings' order
+    float rn = 0.f, rp = 0.f, rr = 0.f;
+    for (int j0 = 0; j0 < R; j0 += U) {
+        float2 a[U], t[U];
+        float c[U];
+        int at[U], end[U];
+#pragma unroll
+        for (int q = 0; q < U; ++q) {
+            end[q] = j0 + q < R ? ring_start[j0 + q + 1] : 0;
+            at[q] = (j0 + q < R ? ring_start[j0 + q] : 0) + lane;
+            const int i = at[q] < end[q] ? at[q] : 0;   // idle lanes read the centre
+            a[q] = P[i];
+            t[q] = S[i];
+            c[q] = Cf[i];
         }
-        num = wave_sum(num);
-        dp = wave_sum(dp);
-        dr = wave_sum(dr);
-        const float den = dp * dr;
-        if (den > 0.f) f += num / sqrtf(den);
+#pragma unroll
+        for (int q = 0; q < U; ++q) {
+            if (j0 + q >= R) break;
+            float num = 0.f, dp = 0.f, dr = 0.f;
+            auto add = [&](float2 v, float2 w, float k) {
+                const float2 r = make_float2(w.x * k, w.y * k);
+                num += v.x * r.x + v.y * r.y;
+                dp += v.x * v.x + v.y * v.y;
+                dr += r.x * r.x + r.y * r.y;
+            };
+            if (at[q] < end[q]) add(a[q], t[q], c[q]);
+            for (int i = at[q] + 64; i < end[q]; i += 64) add(P[i], S[i], Cf[i]);
+            num = wave_sum(num);
+            dp = wave_sum(dp);
+            dr = wave_sum(dr);
+            const bool own = lane == j0 + q;
+            rn = own ? num : rn;
+            rp = own ? dp : rp;
+            rr = own ? dr : rr;
+        }
     }
+    const float den = rp * rr;
+    const int term = __float_as_int(den > 0.f ? rn / sqrtf(den) : 0.f);
+    float f = 0.f;
+    for (int j = 0; j < R; ++j) f += __int_as_float(__builtin_amdgcn_readlane(term, j));
     return f / (float)R;
 }
 
@@ -1395,8 +1437,6 @@ struct bsx_search {
     int64_t pairs_cap = 0;
     GroupItem* d_items = nullptr;
     int64_t items_cap = 0;
-    uint16_t* d_zrow = nullptr;
-    int64_t zrow_cap = 0;
     float* d_ktab = nullptr;
     float* d_pscore = nullptr;
     int* d_pidx = nullptr;
@@ -1548,7 +1588,7 @@ int bsx_search_destroy(bsx_search* h) {
                     h->d_ctf,  h->d_pbf,     h->d_spec,   h->d_sp,
                     h->d_ktab, h->d_pscore,  h->d_pidx,   h->d_libmats, h->d_lmats,
                     h->d_lfrc, h->d_sub,     h->d_members, h->d_mcount, h->d_counts,
-                    h->d_cursors, h->d_pairs, h->d_items, h->d_zrow, h->d_cube,
+                    h->d_cursors, h->d_pairs, h->d_items, h->d_cube,
                     h->d_rv,   h->d_rvi};
     for (void* q : ptrs)
         if (q) (void)hipFree(q);
@@ -1579,7 +1619,7 @@ int bsx_search_set_reference(bsx_search* h, const float* ft_dev, const double* m
                              int64_t nviews, void* stream) {
     BSX_REQUIRE(h && ft_dev && (mats || nviews == 0), BSX_ERR_ARG,
                 "bsx_search_set_reference: null argument");
-    BSX_REQUIRE(nviews >= 0 && nviews < (1ll << 31) - GN, BSX_ERR_ARG,
+    BSX_REQUIRE(nviews >= 0 && nviews < (1ll << 31) - 128, BSX_ERR_ARG,
                 "bsx_search_set_reference: nviews %lld out of range", (long long)nviews);
     for (int64_t i = 0; i < 9 * nviews; ++i)
         BSX_REQUIRE(std::isfinite(mats[i]) && fabs(mats[i]) <= 1.0 + 1e-9, BSX_ERR_ARG,
@@ -1619,7 +1659,7 @@ int bsx_search_set_reference(bsx_search* h, const float* ft_dev, const double* m
 int bsx_search_stage(bsx_search* h, const float* imgs_dev, const bsx_particle* parts, int64_t n,
                      void* stream) {
     BSX_REQUIRE(h && (n == 0 || (imgs_dev && parts)), BSX_ERR_ARG, "bsx_search_stage: null argument");
-    BSX_REQUIRE(n >= 0 && n < (1ll << 31) - GM, BSX_ERR_ARG, "bsx_search_stage: n %lld out of range",
+    BSX_REQUIRE(n >= 0 && n < (1ll << 31) - 128, BSX_ERR_ARG, "bsx_search_stage: n %lld out of range",
                 (long long)n);
     const int N = h->p.box, Nd = h->Nd, Kp = h->Kp;
     for (int64_t i = 0; i < n; ++i) {
@@ -1800,11 +1840,9 @@ int bsx_search_set_classes(bsx_search* h, const int32_t* members, int32_t nclass
     }
     int rc = grow(h, &h->d_members, &h->members_cap, (int64_t)nclasses * maxm, "class members");
     if (!rc) rc = grow(h, &h->d_mcount, &h->mcount_cap, nclasses, "class sizes");
-    if (!rc) rc = grow(h, &h->d_zrow, &h->zrow_cap, h->Kp, "zero row");
     if (rc) return rc;
     BSX_HIP(hipMemcpy(h->d_members, members, sizeof(int) * nclasses * maxm, hipMemcpyHostToDevice));
     BSX_HIP(hipMemcpy(h->d_mcount, cnt.data(), sizeof(int) * nclasses, hipMemcpyHostToDevice));
-    BSX_HIP(hipMemset(h->d_zrow, 0, sizeof(uint16_t) * h->Kp));
     h->nclass = nclasses;
     h->maxm = maxm;
     return BSX_OK;
@@ -1828,43 +1866,28 @@ int bsx_search_proposed(bsx_search* h, const int32_t* cls_dev, int32_t k, int32_
     if (!rc) rc = grow(h, &h->d_pidx, &h->pidx_cap, n * k * T, "proposal partials");
     if (rc) return rc;
     const unsigned g = (unsigned)((n * k + 255) / 256);
+    const int64_t most = h->nclass + n * k / RM;   // items: sum over classes of ceil(pairs / RM)
+    rc = grow(h, &h->d_items, &h->items_cap, most + 1, "work items");
+    if (rc) return rc;
+    int* nitems = (int*)(h->d_items + most);
     BSX_HIP(hipMemsetAsync(h->d_counts, 0, sizeof(int) * h->nclass, s));
     hipLaunchKernelGGL(k_route_count, dim3(g), dim3(256), 0, s, cls_dev, n, k, h->nclass, h->d_counts);
     BSX_HIP(hipGetLastError());
-    std::vector<int> cnt(h->nclass), off(h->nclass);
-    BSX_HIP(hipMemcpyAsync(cnt.data(), h->d_counts, sizeof(int) * h->nclass, hipMemcpyDeviceToHost, s));
-    BSX_HIP(hipStreamSynchronize(s));
-    std::vector<GroupItem> items;
-    int acc = 0;
-    for (int c = 0; c < h->nclass; ++c) {
-        off[c] = acc;
-        for (int p0 = 0; p0 < cnt[c]; p0 += GM)
-            items.push_back(GroupItem{c, acc + p0, std::min(GM, cnt[c] - p0), 0});
-        acc += cnt[c];
-    }
-    rc = grow(h, &h->d_items, &h->items_cap, std::max<int64_t>(1, (int64_t)items.size()), "work items");
-    if (rc) return rc;
-    BSX_HIP(hipMemcpyAsync(h->d_cursors, off.data(), sizeof(int) * h->nclass, hipMemcpyHostToDevice, s));
-    if (!items.empty())
-        BSX_HIP(hipMemcpyAsync(h->d_items, items.data(), sizeof(GroupItem) * items.size(),
-                               hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(k_route_fill, dim3(g), dim3(256), 0, s, cls_dev, n, k, h->nclass, h->d_cursors,
-                       h->d_pairs);
+    hipLaunchKernelGGL(k_route_scan, dim3(1), dim3(1024), 0, s, h->d_counts, h->nclass, h->d_cursors,
+                       h->d_items, nitems);
     BSX_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_route_empty, dim3(g), dim3(256), 0, s, cls_dev, n, k, h->nclass, T,
-                       h->d_pscore, h->d_pidx);
+    hipLaunchKernelGGL(k_route_fill, dim3(g), dim3(256), 0, s, cls_dev, n, k, h->nclass, T, h->d_cursors,
+                       h->d_pairs, h->d_pscore, h->d_pidx);
     BSX_HIP(hipGetLastError());
-    if (!items.empty()) {
-        if (T == 8)
-            hipLaunchKernelGGL((k_gemm_grouped<8>), dim3((unsigned)items.size()), dim3(256), 0, s,
-                               h->d_pbf, h->d_lbf, h->d_zrow, h->Kp, h->d_items, h->d_pairs, k,
-                               h->d_members, h->d_mcount, h->maxm, h->d_pscore, h->d_pidx);
-        else
-            hipLaunchKernelGGL((k_gemm_grouped<16>), dim3((unsigned)items.size()), dim3(256), 0, s,
-                               h->d_pbf, h->d_lbf, h->d_zrow, h->Kp, h->d_items, h->d_pairs, k,
-                               h->d_members, h->d_mcount, h->maxm, h->d_pscore, h->d_pidx);
-        BSX_HIP(hipGetLastError());
-    }
+    if (T == 8)
+        hipLaunchKernelGGL((k_gemm_grouped<8>), dim3((unsigned)most), dim3(256), 0, s, h->d_pbf, h->d_lbf,
+                           h->Kp, h->d_items, nitems, h->d_pairs, k, h->d_members, h->d_mcount, h->maxm,
+                           h->d_pscore, h->d_pidx);
+    else
+        hipLaunchKernelGGL((k_gemm_grouped<16>), dim3((unsigned)most), dim3(256), 0, s, h->d_pbf, h->d_lbf,
+                           h->Kp, h->d_items, nitems, h->d_pairs, k, h->d_members, h->d_mcount, h->maxm,
+                           h->d_pscore, h->d_pidx);
+    BSX_HIP(hipGetLastError());
     const unsigned mg = (unsigned)((n + 3) / 4);
     if (T == 8)
         hipLaunchKernelGGL((k_topk_merge<8>), dim3(mg), dim3(256), 0, s, h->d_pscore, h->d_pidx, k,
@@ -1873,7 +1896,7 @@ int bsx_search_proposed(bsx_search* h, const int32_t* cls_dev, int32_t k, int32_
         hipLaunchKernelGGL((k_topk_merge<16>), dim3(mg), dim3(256), 0, s, h->d_pscore, h->d_pidx, k,
                            n, h->p.topk, cand_dev, score_dev);
     BSX_HIP(hipGetLastError());
-    // the host work-item list is released on return
+    // complete on return: the partial lists are shared with calls on other streams
     BSX_HIP(hipStreamSynchronize(s));
     return BSX_OK;
 }
