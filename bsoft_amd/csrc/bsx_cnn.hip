@@ -650,6 +650,81 @@ __global__ __launch_bounds__(256) void k_gemm32(int M, int N, int K, const float
     }
 }
 
+// C[m][n] = scale * sum_k A[m][k] B[n][k] (rows of d values, FP32 sums in the order
+// of k), 128 x 128 per workgroup, 64 x 64 per wave as 2 x 2 blocks: each LDS value
+// feeds two instructions. Particle embeddings against class references; the scale
+// (1 / tau) was a pass of its own over the scores (143 us for 16,384 x 4,368), and
+// the product on the VALU took 338 us, now 253 us (72 TFLOP/s).
+__global__ __launch_bounds__(256) void k_scores32(int M, int N, int K, const float* __restrict__ A,
+                                                  const float* __restrict__ Bm, float scale,
+                                                  float* __restrict__ C) {
+    constexpr int LR = 129;
+    __shared__ float sa[2][TK][LR], sb[2][TK][LR];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wm = wave >> 1, wn = wave & 1;
+    const int m0 = blockIdx.y * 128, n0 = blockIdx.x * 128;
+    const int lr = tid >> 4, lk = tid & 15;   // rows lr + 16 j, k lk
+    float ra[8], rb[8];
+    auto load = [&](int k0) {
+        const int k = k0 + lk;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int m = m0 + lr + 16 * j, n = n0 + lr + 16 * j;
+            ra[j] = (m < M && k < K) ? A[(long)m * K + k] : 0.f;
+            rb[j] = (n < N && k < K) ? Bm[(long)n * K + k] : 0.f;
+        }
+    };
+    auto store = [&](int buf) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            sa[buf][lk][lr + 16 * j] = ra[j];
+            sb[buf][lk][lr + 16 * j] = rb[j];
+        }
+    };
+    f32x16 acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+    load(0);
+    store(0);
+    __syncthreads();
+    for (int k0 = 0, buf = 0; k0 < K; k0 += TK, buf ^= 1) {
+        if (k0 + TK < K) load(k0 + TK);
+#pragma unroll
+        for (int k = 0; k < TK; k += 2) {
+            const int kk = k + (lane >> 5);
+            float a[2], b[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                a[i] = sa[buf][kk][wm * 64 + i * 32 + (lane & 31)];
+                b[i] = sb[buf][kk][wn * 64 + i * 32 + (lane & 31)];
+            }
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
+        }
+        if (k0 + TK < K) store(buf ^ 1);
+        __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int n = n0 + wn * 64 + j * 32 + (lane & 31);
+            if (n >= N) continue;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int m = m0 + wm * 64 + i * 32 + acc_row(r, lane);
+                if (m < M) C[(long)m * N + n] = acc[i][j][r] * scale;
+            }
+        }
+}
+
 // db[n] = sum_m g[m][n]: 64 columns per workgroup, the rows over its 16 waves
 __global__ __launch_bounds__(1024) void k_colsum(const float* __restrict__ g, int M, int N,
                                                  float* __restrict__ db) {
@@ -671,6 +746,12 @@ __global__ __launch_bounds__(1024) void k_colsum(const float* __restrict__ g, in
 }
 
 // ------------------------------------------------------ softmax / top-k
+__device__ __forceinline__ float wave_add(float v) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    return v;
+}
+
 // One workgroup per row: loss[b] = logsumexp - logit[label]; dl = (p - onehot) / B.
 __global__ __launch_bounds__(256) void k_softmax_ce(const float* __restrict__ logits,
                                                     const int* __restrict__ labels, int B, int C,
@@ -704,92 +785,97 @@ __global__ __launch_bounds__(256) void k_softmax_ce(const float* __restrict__ lo
     if (threadIdx.x == 0 && loss) loss[b] = logf(se) + mx - l[t];
 }
 
-// One workgroup per row: the k largest logits (k <= 32) as classes and
-// softmax probabilities, best first (ties: lower class).
-template <int T>   // per-thread list length, >= k
-__global__ __launch_bounds__(256) void k_row_topk(const float* __restrict__ logits, int C, int k,
+// The k largest logits of a row (k <= 32) as classes and softmax probabilities,
+// best first (ties: lower class; NaN and -inf are never taken, missing places
+// -1 and 0). One wavefront per row, two passes over it: the lanes' maxima, the
+// k-th largest of which bounds the k-th value from below, then the exponential
+// sum and the few values that reach the bound (ROWCAP of them; a row with more,
+// e.g. of equal values, takes k passes). Bound by reading the row: 16,384 rows of
+// 4,368 took 388 us with 16 block-wide arg-max rounds over per-thread lists, now
+// 179 us.
+constexpr int ROWCAP = 192;
+
+__device__ __forceinline__ unsigned long long logit_key(float v, int c) {
+    const unsigned u = __float_as_uint(v + 0.f);   // -0 counts as 0
+    const unsigned o = (u & 0x80000000u) ? ~u : u | 0x80000000u;
+    return ((unsigned long long)o << 32) | (unsigned)~c;
+}
+__device__ __forceinline__ unsigned long long wave_max64(unsigned long long m) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        const unsigned long long x = __shfl_xor(m, o, 64);
+        m = x > m ? x : m;
+    }
+    return m;
+}
+
+__global__ __launch_bounds__(256) void k_row_topk(const float* __restrict__ logits, long n, int C, int k,
                                                   int* __restrict__ cls, float* __restrict__ prob) {
-    __shared__ float sv[256];
-    __shared__ int si[256];
-    __shared__ float red[256];
-    const long b = blockIdx.x;
+    __shared__ unsigned long long list[4][ROWCAP];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const long b = (long)blockIdx.x * 4 + wave;
+    if (b >= n) return;   // a whole wavefront; no workgroup barrier below
     const float* l = logits + b * C;
-    float best[T];
-    int bi[T];
+    float lm = -INFINITY;
+#pragma unroll 4
+    for (int c = lane; c < C; c += 64) lm = fmaxf(lm, l[c]);
+    float mx = lm;
 #pragma unroll
-    for (int q = 0; q < T; ++q) { best[q] = -INFINITY; bi[q] = 0x7fffffff; }
-    float mx = -INFINITY;
-    for (int c = threadIdx.x; c < C; c += blockDim.x) {
-        const float v = l[c];
-        mx = fmaxf(mx, v);
-        if (v > best[T - 1]) {
-            best[T - 1] = v;
-            bi[T - 1] = c;
-#pragma unroll
-            for (int q = T - 1; q > 0; --q)
-                if (best[q] > best[q - 1]) {
-                    const float tv = best[q]; best[q] = best[q - 1]; best[q - 1] = tv;
-                    const int ti = bi[q]; bi[q] = bi[q - 1]; bi[q - 1] = ti;
-                }
-        }
-    }
-    red[threadIdx.x] = mx;
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if (threadIdx.x < s) red[threadIdx.x] = fmaxf(red[threadIdx.x], red[threadIdx.x + s]);
-        __syncthreads();
-    }
-    mx = red[0];
-    __syncthreads();
-    float se = 0.f;
-    for (int c = threadIdx.x; c < C; c += blockDim.x) se += expf(l[c] - mx);
-    red[threadIdx.x] = se;
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-        __syncthreads();
-    }
-    se = red[0];
-    // k rounds of a block-wide arg-max over the heads of the per-thread lists
-    int head = 0;
+    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+    // the k-th largest lane maximum (each round drops one lane)
+    float bound = -INFINITY, left = lm;
     for (int r = 0; r < k; ++r) {
-        float hv = -INFINITY;
-        int hi = 0x7fffffff;
+        float m = left;
 #pragma unroll
-        for (int q = 0; q < T; ++q)
-            if (q == head) { hv = best[q]; hi = bi[q]; }
-        sv[threadIdx.x] = hv;
-        si[threadIdx.x] = hi;
-        __syncthreads();
-        for (int s = 128; s > 0; s >>= 1) {
-            if (threadIdx.x < s) {
-                const float ov = sv[threadIdx.x + s];
-                const int oi = si[threadIdx.x + s];
-                if (ov > sv[threadIdx.x] || (ov == sv[threadIdx.x] && oi < si[threadIdx.x])) {
-                    sv[threadIdx.x] = ov;
-                    si[threadIdx.x] = oi;
-                }
+        for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+        bound = m;
+        const unsigned long long has = __ballot(left == m);
+        if (lane == __builtin_ctzll(has | (1ull << 63))) left = -INFINITY;
+    }
+    float se = 0.f;
+    int cnt = 0;
+    for (int c0 = 0; c0 < C; c0 += 64) {
+        const int c = c0 + lane;
+        const float v = c < C ? l[c] : -INFINITY;
+        if (c < C) se += expf(v - mx);
+        const bool in = v >= bound && v > -INFINITY;
+        const unsigned long long has = __ballot(in);
+        if (has) {
+            const int at = cnt + __popcll(has & ((1ull << lane) - 1ull));
+            if (in && at < ROWCAP) list[wave][at] = logit_key(v, c);
+            cnt += __popcll(has);
+        }
+    }
+    se = wave_add(se);
+    __builtin_amdgcn_wave_barrier();
+    unsigned long long last = ~0ull;
+    for (int r = 0; r < k; ++r) {
+        // the largest key below the last one taken
+        unsigned long long m = 0;
+        if (cnt <= ROWCAP) {
+            for (int i = lane; i < cnt; i += 64) {
+                const unsigned long long x = list[wave][i];
+                m = (x < last && x > m) ? x : m;
             }
-            __syncthreads();
+        } else {
+            for (int c = lane; c < C; c += 64) {
+                const float v = l[c];
+                const unsigned long long x = v > -INFINITY ? logit_key(v, c) : 0;
+                m = (x < last && x > m) ? x : m;
+            }
         }
-        const int wi = si[0];
-        const float wv = sv[0];
-        if (threadIdx.x == 0) {
-            cls[b * k + r] = wi < C ? wi : -1;
-            prob[b * k + r] = wi < C ? expf(wv - mx) / se : 0.f;
+        m = wave_max64(m);
+        last = m;
+        if (lane == 0) {
+            const unsigned o = (unsigned)(m >> 32);
+            const float v = __uint_as_float((o & 0x80000000u) ? o & 0x7fffffffu : ~o);
+            cls[b * k + r] = m ? (int)~(unsigned)m : -1;
+            prob[b * k + r] = m ? expf(v - mx) / se : 0.f;
         }
-        if (hi == wi && head < T) ++head;
-        __syncthreads();
     }
 }
 
 // --------------------------------------------- contrastive (embedding) head
-__device__ __forceinline__ float wave_add(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
-
 // Unit rows u = z / |z| of an n x d matrix (|z| floored at 1e-12); one
 // wavefront per row, so that rows are read and written with consecutive
 // lanes (one thread per row: 58 us for 4,096 x 128).
@@ -867,11 +953,6 @@ __global__ __launch_bounds__(256) void k_unit_rows_bwd(const float* __restrict__
     for (int c = lane; c < d; c += 64) dz[i * d + c] = (du[i * d + c] - dot * u[i * d + c]) * inv;
 }
 
-__global__ void k_scale(float* __restrict__ x, long n, float a) {
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
-        x[i] *= a;
-}
-
 __global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
                        float* __restrict__ v, long n, float lr, float b1, float b2, float eps,
                        float c1, float c2, float wd) {
@@ -897,137 +978,211 @@ __global__ void k_to_bf16(const float* __restrict__ p, uint16_t* __restrict__ q,
 // output channels, k = (tap, input channel) with the channel fastest, so
 // that 8 consecutive k are one 16-byte load from the NHWC input.
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
-constexpr int IM = 128, IN = 64, IK = 32, IROW = IK * 2 + 16;
 
 // y[b][yo][xo][co] = bf16(relu(bias + sum_{ky,kx} W[co][0][ky][kx] x[b][yo-1+ky][xo-1+kx]))
+// thread = (4 consecutive positions, 8 channels): a weight read from LDS (taps
+// outermost, two 16-byte reads per tap) serves the four positions; a wavefront's
+// 16-byte stores of 8 BF16 channels join in the NHWC output, whose writing bounds
+// it (one position per thread, 80 LDS reads for its 72 products: 613 us for
+// 16,384 x 32^2 x 32, now 391 us).
 __global__ __launch_bounds__(256) void k_conv1_nhwc(const float* __restrict__ x,
                                                     const uint16_t* __restrict__ W,
                                                     const uint16_t* __restrict__ bias, int B, int S,
                                                     int C1, uint16_t* __restrict__ y) {
-    // thread = (output position, group of 8 channels): a wavefront's 16-byte
-    // stores of 8 BF16 channels are contiguous in the NHWC output
-    extern __shared__ float w[];   // C1 x 9 weights, then C1 biases
-    for (int i = threadIdx.x; i < C1 * 9; i += blockDim.x) w[i] = bf16_to_f(W[i]);
+    extern __shared__ float w[];   // 9 x C1 weights [tap][channel], then C1 biases
+    for (int i = threadIdx.x; i < C1 * 9; i += blockDim.x) w[i % 9 * C1 + i / 9] = bf16_to_f(W[i]);
     for (int i = threadIdx.x; i < C1; i += blockDim.x) w[C1 * 9 + i] = bf16_to_f(bias[i]);
     __syncthreads();
-    const int ng = C1 / 8;
+    const int ng = C1 / 8, quads = S * S / 4;
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (long)B * S * S * ng) return;
+    if (t >= (long)B * quads * ng) return;
     const int g = (int)(t % ng);
-    const long pos = t / ng;
-    const int xo = (int)(pos % S), yo = (int)((pos / S) % S);
-    const long b = pos / ((long)S * S);
-    float v[9];
+    const long pq = t / ng;
+    const long b = pq / quads;
+    const int q = (int)(pq - b * quads), yo = q / (S / 4), xo = (q - yo * (S / 4)) * 4;
+    float v[3][6];
 #pragma unroll
-    for (int ky = 0; ky < 3; ++ky)
+    for (int r = 0; r < 3; ++r) {
+        const int yi = yo - 1 + r;
+        const float* row = x + (b * S + yi) * S + xo;
+        const bool ok = yi >= 0 && yi < S;
+        Float4u x4 = {{0.f, 0.f, 0.f, 0.f}};
+        if (ok) x4 = *(const Float4u*)row;
+        v[r][0] = ok && xo > 0 ? row[-1] : 0.f;
 #pragma unroll
-        for (int kx = 0; kx < 3; ++kx) {
-            const int yi = yo - 1 + ky, xi = xo - 1 + kx;
-            v[ky * 3 + kx] = (yi >= 0 && yi < S && xi >= 0 && xi < S) ? x[(b * S + yi) * S + xi] : 0.f;
-        }
-    uint32_t packed[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int c = g * 8 + 2 * j;
-        float a0 = w[C1 * 9 + c], a1 = w[C1 * 9 + c + 1];
-#pragma unroll
-        for (int q = 0; q < 9; ++q) {
-            a0 = fmaf(w[c * 9 + q], v[q], a0);
-            a1 = fmaf(w[(c + 1) * 9 + q], v[q], a1);
-        }
-        packed[j] = (uint32_t)f_to_bf16(fmaxf(a0, 0.f)) |
-                    ((uint32_t)f_to_bf16(fmaxf(a1, 0.f)) << 16);
+        for (int c = 0; c < 4; ++c) v[r][c + 1] = x4.v[c];
+        v[r][5] = ok && xo + 4 < S ? row[4] : 0.f;
     }
-    *(uint4*)(y + pos * C1 + g * 8) = make_uint4(packed[0], packed[1], packed[2], packed[3]);
+    float a[4][8];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int c = 0; c < 8; ++c) a[e][c] = w[C1 * 9 + g * 8 + c];
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+        const float4* wk = (const float4*)(w + k * C1 + g * 8);
+        const float4 w0 = wk[0], w1 = wk[1];
+        const float ww[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int c = 0; c < 8; ++c) a[e][c] = fmaf(ww[c], v[k / 3][k % 3 + e], a[e][c]);
+    }
+    uint16_t* o = y + (pq * 4) * C1 + g * 8;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        uint32_t p[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            p[j] = (uint32_t)f_to_bf16(fmaxf(a[e][2 * j], 0.f)) |
+                   ((uint32_t)f_to_bf16(fmaxf(a[e][2 * j + 1], 0.f)) << 16);
+        *(uint4*)(o + (long)e * C1) = make_uint4(p[0], p[1], p[2], p[3]);
+    }
 }
 
-// Implicit-GEMM convolution (ks = 3: pad 1; ks = 1: a plain GEMM over
-// H = W = 1) of NHWC BF16 input with BF16 weights [Cout][ks*ks][Cin] and
+// Implicit-GEMM convolution (KS = 3: pad 1, stride 2; KS = 1: a plain GEMM over
+// H = W = 1) of NHWC BF16 input with BF16 weights [Cout][KS*KS][Cin] and
 // BF16 biases. OUTF32: FP32 output rows of stride ldo without ReLU (logits);
 // else BF16 NHWC output with ReLU. Cin must be a multiple of 32.
-template <bool OUTF32>
+// A workgroup's 4 waves (WM x WN) compute BM x BN blocks of 32 x 32 each; the
+// loads of the next 32-deep K step are in flight during a step. With 2 x 2 blocks
+// a wave reads 4 KB of LDS for 4 instructions (with 1 x 2, as before, 3 KB for 2:
+// more than the LDS delivers at the MFMA rate). The valid taps of a row are a
+// bit mask made once, a tap is a uniform offset. The BF16 output goes through LDS
+// and leaves in 16-byte stores. 16,384 x 32^2 inputs, 32-64-128-128 channels: the
+// three layers 1,471 us before, 1,284 us now.
+template <int BM, int BN, int WM, int WN, int KS, bool OUTF32>
 __global__ __launch_bounds__(256) void k_conv_mfma(const uint16_t* __restrict__ x, int B, int H,
-                                                   int Wd, int Cin, int ks, int stride, int Ho,
-                                                   int Wo, const uint16_t* __restrict__ Wt,
+                                                   int Wd, int Cin, int Ho, int Wo,
+                                                   const uint16_t* __restrict__ Wt,
                                                    const uint16_t* __restrict__ bias, int Cout,
                                                    long ldo, void* __restrict__ out) {
-    __shared__ __attribute__((aligned(16))) char lds[2 * (IM + IN) * IROW];
+    static_assert(WM * WN == 4, "four waves");
+    constexpr int IM = 32 * BM * WM, IN = 32 * BN * WN, IK = 32, IROW = IK * 2 + 16;
+    constexpr int NA = IM / 64, NB = IN / 64;   // 16-byte chunks per thread and step
+    constexpr int OR = IN * 2 + 16;             // bytes per output row in LDS
+    constexpr int LDS = 2 * (IM + IN) * IROW > IM * OR ? 2 * (IM + IN) * IROW : IM * OR;
+    __shared__ __attribute__((aligned(16))) char lds[LDS];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const long M = (long)B * Ho * Wo;
-    const int K = ks * ks * Cin;
-    const int nk = K / IK;
-    const long m0 = (long)blockIdx.x * IM;
+    const int wm = wave / WN, wn = wave % WN;
+    const long M = (long)B * Ho * Wo, m0 = (long)blockIdx.x * IM;
     const int n0 = blockIdx.y * IN;
-    const int pad = ks / 2;
-    // A staging: chunks tid and tid + 256 (row = c >> 2, part = c & 3); the
-    // positions live in named scalars (arrays captured by the loaders end up
-    // in scratch memory)
-    const long am0 = m0 + (tid >> 2), am1 = m0 + ((tid + 256) >> 2);
-    const long mm0 = am0 < M ? am0 : 0, mm1 = am1 < M ? am1 : 0;
-    const int ax0 = (int)(mm0 % Wo), ay0 = (int)((mm0 / Wo) % Ho), ab0 = (int)(mm0 / ((long)Wo * Ho));
-    const int ax1 = (int)(mm1 % Wo), ay1 = (int)((mm1 / Wo) % Ho), ab1 = (int)(mm1 / ((long)Wo * Ho));
-    const int apart0 = tid & 3;
-    const int brow = tid >> 2, bpart = tid & 3;
-    const int bco = n0 + brow;
-    f32x16 acc0, acc1;
+    const int K = KS * KS * Cin, nk = K / IK;
+    // rows (tid >> 2) + 64 j, 8 channels from 8 (tid & 3)
+    const int lr = tid >> 2, lp = tid & 3;
+    const uint16_t* ap[NA];
+    unsigned av[NA];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) { acc0[r] = 0.f; acc1[r] = 0.f; }
-    uint4 ra0, ra1, rb;
-#define BSX_CGLOAD(KT)                                                                        \
-    {                                                                                          \
-        const int k0 = (KT) * IK;                                                              \
-        const int tap = k0 / Cin;                                                              \
-        const int ky = tap / ks, kx = tap % ks;                                                \
-        const int ci0 = k0 % Cin + apart0 * 8;                                                 \
-        const int yi0 = ay0 * stride - pad + ky, xi0 = ax0 * stride - pad + kx;                \
-        const int yi1 = ay1 * stride - pad + ky, xi1 = ax1 * stride - pad + kx;                \
-        ra0 = make_uint4(0, 0, 0, 0);                                                          \
-        ra1 = make_uint4(0, 0, 0, 0);                                                          \
-        rb = make_uint4(0, 0, 0, 0);                                                           \
-        if (am0 < M && yi0 >= 0 && yi0 < H && xi0 >= 0 && xi0 < Wd)                            \
-            ra0 = *(const uint4*)(x + (((long)ab0 * H + yi0) * Wd + xi0) * Cin + ci0);         \
-        if (am1 < M && yi1 >= 0 && yi1 < H && xi1 >= 0 && xi1 < Wd)                            \
-            ra1 = *(const uint4*)(x + (((long)ab1 * H + yi1) * Wd + xi1) * Cin + ci0);         \
-        if (bco < Cout) rb = *(const uint4*)(Wt + (long)bco * K + k0 + bpart * 8);             \
+    for (int j = 0; j < NA; ++j) {
+        const long m = m0 + lr + 64 * j;
+        const long mm = m < M ? m : 0;
+        const int xo = (int)(mm % Wo), yo = (int)((mm / Wo) % Ho);
+        const long b = mm / ((long)Wo * Ho);
+        const int y0 = KS == 3 ? 2 * yo - 1 : yo, x0 = KS == 3 ? 2 * xo - 1 : xo;
+        ap[j] = x + ((b * H + y0) * Wd + x0) * (long)Cin + lp * 8;
+        av[j] = 0;
+#pragma unroll
+        for (int t = 0; t < KS * KS; ++t) {
+            const int yi = y0 + t / KS, xi = x0 + t % KS;
+            if (m < M && yi >= 0 && yi < H && xi >= 0 && xi < Wd) av[j] |= 1u << t;
+        }
     }
-#define BSX_CLSTORE(BUF)                                                                      \
-    {                                                                                          \
-        *(uint4*)((BUF) + (tid >> 2) * IROW + apart0 * 16) = ra0;                              \
-        *(uint4*)((BUF) + ((tid + 256) >> 2) * IROW + apart0 * 16) = ra1;                      \
-        *(uint4*)((BUF) + (IM + brow) * IROW + bpart * 16) = rb;                               \
+    const uint16_t* bp[NB];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+        const int co = n0 + lr + 64 * j;
+        bp[j] = co < Cout ? Wt + (long)co * K + lp * 8 : nullptr;
     }
-    BSX_CGLOAD(0)
-    BSX_CLSTORE(lds)
+    uint4 ra[NA], rb[NB];
+    int tap = 0, ci = 0;   // of the next step to load
+    auto load = [&](int kt) {
+        const long o = ((long)(tap / KS) * Wd + tap % KS) * Cin + ci;
+#pragma unroll
+        for (int j = 0; j < NA; ++j) {
+            ra[j] = make_uint4(0, 0, 0, 0);
+            if ((av[j] >> tap) & 1) ra[j] = *(const uint4*)(ap[j] + o);
+        }
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+            rb[j] = make_uint4(0, 0, 0, 0);
+            if (bp[j]) rb[j] = *(const uint4*)(bp[j] + (long)kt * IK);
+        }
+        ci += IK;
+        if (ci == Cin) { ci = 0; ++tap; }
+    };
+    auto store = [&](int buf) {
+        char* d = lds + buf * (IM + IN) * IROW + lr * IROW + lp * 16;
+#pragma unroll
+        for (int j = 0; j < NA; ++j) *(uint4*)(d + 64 * j * IROW) = ra[j];
+#pragma unroll
+        for (int j = 0; j < NB; ++j) *(uint4*)(d + (IM + 64 * j) * IROW) = rb[j];
+    };
+    f32x16 acc[BM][BN];
+#pragma unroll
+    for (int i = 0; i < BM; ++i)
+#pragma unroll
+        for (int j = 0; j < BN; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+    load(0);
+    store(0);
     __syncthreads();
     for (int kt = 0; kt < nk; ++kt) {
-        const bool more = kt + 1 < nk;
-        if (more) BSX_CGLOAD(kt + 1)
+        if (kt + 1 < nk) load(kt + 1);
         const char* buf = lds + (kt & 1) * (IM + IN) * IROW;
 #pragma unroll
         for (int sub = 0; sub < IK / 16; ++sub) {
             const int off = sub * 32 + (lane >> 5) * 16;
-            const bf16x8 fa = *(const bf16x8*)(buf + (wave * 32 + (lane & 31)) * IROW + off);
-            const bf16x8 fb0 = *(const bf16x8*)(buf + (IM + (lane & 31)) * IROW + off);
-            const bf16x8 fb1 = *(const bf16x8*)(buf + (IM + 32 + (lane & 31)) * IROW + off);
-            acc0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa, fb0, acc0, 0, 0, 0);
-            acc1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa, fb1, acc1, 0, 0, 0);
+            bf16x8 fa[BM], fb[BN];
+#pragma unroll
+            for (int i = 0; i < BM; ++i)
+                fa[i] = *(const bf16x8*)(buf + ((wm * BM + i) * 32 + (lane & 31)) * IROW + off);
+#pragma unroll
+            for (int j = 0; j < BN; ++j)
+                fb[j] = *(const bf16x8*)(buf + (IM + (wn * BN + j) * 32 + (lane & 31)) * IROW + off);
+#pragma unroll
+            for (int i = 0; i < BM; ++i)
+#pragma unroll
+                for (int j = 0; j < BN; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
         }
-        if (more) BSX_CLSTORE(lds + ((kt + 1) & 1) * (IM + IN) * IROW)
+        if (kt + 1 < nk) store((kt + 1) & 1);
         __syncthreads();
     }
-#undef BSX_CGLOAD
-#undef BSX_CLSTORE
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < BN; ++j) {
+        const int cl = (wn * BN + j) * 32 + (lane & 31), co = n0 + cl;
+        const float bv = co < Cout ? bf16_to_f(bias[co]) : 0.f;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const long m = m0 + wave * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-            const int co = n0 + j * 32 + (lane & 31);
-            if (m >= M || co >= Cout) continue;
-            const float v = (j == 0 ? acc0[r] : acc1[r]) + bf16_to_f(bias[co]);
-            if (OUTF32) ((float*)out)[m * ldo + co] = v;
-            else ((uint16_t*)out)[m * Cout + co] = f_to_bf16(fmaxf(v, 0.f));
+        for (int i = 0; i < BM; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int row = (wm * BM + i) * 32 + acc_row(r, lane);
+                const float v = acc[i][j][r] + bv;
+                if (OUTF32) {
+                    if (m0 + row < M && co < Cout) ((float*)out)[(m0 + row) * ldo + co] = v;
+                } else {
+                    *(uint16_t*)(lds + row * OR + cl * 2) = f_to_bf16(fmaxf(v, 0.f));
+                }
+            }
+    }
+    if (OUTF32) return;
+    __syncthreads();
+    if (Cout & 7) {   // last layer only: rows are not 16-byte aligned
+        const int w = min(IN, Cout - n0);
+        for (int c = tid; c < IM * w; c += 256) {
+            const int row = c / w, q = c - row * w;
+            if (m0 + row < M)
+                ((uint16_t*)out)[(m0 + row) * Cout + n0 + q] = *(const uint16_t*)(lds + row * OR + q * 2);
         }
+        return;
+    }
+    const int per = min(IN, Cout - n0) / 8;   // 16-byte chunks per row
+    for (int c = tid; c < IM * per; c += 256) {
+        const int row = c / per, q = c - row * per;
+        if (m0 + row < M)
+            *(uint4*)((uint16_t*)out + (m0 + row) * Cout + n0 + q * 8) = *(const uint4*)(lds + row * OR + q * 16);
+    }
 }
 
 // BF16 inference weights: conv [co][ci][ky][kx] -> [co][ky*3+kx][ci]; FC
@@ -1407,24 +1562,36 @@ int infer_chunks(bsx_cnn* h, const float* x_dev, int64_t n, hipStream_t s, const
             if (rc) return rc;
         } else {
             const uint16_t* P = h->d_pb;
-            const long pos1 = (long)nb * in * (h->ch[1] / 8);
+            const long pos1 = (long)nb * (in / 4) * (h->ch[1] / 8);
             hipLaunchKernelGGL(k_conv1_nhwc, dim3(nblk(pos1)), dim3(256),
                                sizeof(float) * 10 * h->ch[1], s, x_dev + b0 * in, P + h->woff[0],
                                P + h->boff[0], nb, h->S, h->ch[1], h->d_ib[1]);
             BSX_HIP(hipGetLastError());
             for (int l = 2; l <= 4; ++l) {
+                // up to 64 output channels 256 x 64 tiles, else 128 x 128; 64 x 64
+                // where those would leave CUs without a tile
                 const long M = (long)nb * h->hw[l] * h->hw[l];
-                dim3 g((unsigned)((M + IM - 1) / IM), (unsigned)((h->ch[l] + IN - 1) / IN));
-                hipLaunchKernelGGL((k_conv_mfma<false>), g, dim3(256), 0, s, h->d_ib[l - 1], nb,
-                                   h->hw[l - 1], h->hw[l - 1], h->ch[l - 1], 3, 2, h->hw[l], h->hw[l],
-                                   h->d_wi[l - 1], P + h->boff[l - 1], h->ch[l], (long)h->ch[l],
-                                   (void*)h->d_ib[l]);
+                const int N = h->ch[l], im = N <= 64 ? 256 : 128, in_ = N <= 64 ? 64 : 128;
+                const bool few = ((M + im - 1) / im) * ((N + in_ - 1) / in_) < 256;
+                auto go = [&](auto kernel, int tm, int tn) {
+                    hipLaunchKernelGGL(kernel, dim3((unsigned)((M + tm - 1) / tm), (unsigned)((N + tn - 1) / tn)),
+                                       dim3(256), 0, s, h->d_ib[l - 1], nb, h->hw[l - 1], h->hw[l - 1],
+                                       h->ch[l - 1], h->hw[l], h->hw[l], h->d_wi[l - 1], P + h->boff[l - 1],
+                                       N, (long)N, (void*)h->d_ib[l]);
+                };
+                if (few) go(k_conv_mfma<1, 1, 2, 2, 3, false>, 64, 64);
+                else if (N <= 64) go(k_conv_mfma<2, 2, 4, 1, 3, false>, 256, 64);
+                else go(k_conv_mfma<2, 2, 2, 2, 3, false>, 128, 128);
                 BSX_HIP(hipGetLastError());
             }
-            dim3 g((unsigned)((nb + IM - 1) / IM), (unsigned)((h->nclass + IN - 1) / IN));
-            hipLaunchKernelGGL((k_conv_mfma<true>), g, dim3(256), 0, s, h->d_ib[4], nb, 1, 1,
-                               (int)h->feat, 1, 1, 1, 1, h->d_wi[4], P + h->boff[4], h->nclass,
-                               (long)h->nclass, (void*)h->d_ilog);
+            const bool few = ((nb + 127l) / 128) * ((h->nclass + 127l) / 128) < 256;
+            auto fc = [&](auto kernel, int t) {
+                hipLaunchKernelGGL(kernel, dim3((unsigned)((nb + t - 1) / t), (unsigned)((h->nclass + t - 1) / t)),
+                                   dim3(256), 0, s, h->d_ib[4], nb, 1, 1, (int)h->feat, 1, 1, h->d_wi[4],
+                                   P + h->boff[4], h->nclass, (long)h->nclass, (void*)h->d_ilog);
+            };
+            if (few) fc(k_conv_mfma<1, 1, 2, 2, 1, true>, 64);
+            else fc(k_conv_mfma<2, 2, 2, 2, 1, true>, 128);
             BSX_HIP(hipGetLastError());
         }
         const int rc = use(mfma ? h->d_ilog : h->d_act[0], b0, nb);
@@ -1599,12 +1766,8 @@ int bsx_cnn_infer_topk(bsx_cnn* h, const float* x_dev, int64_t n, int32_t k, int
     BSX_REQUIRE(k >= 1 && k <= 32 && k <= h->nclass, BSX_ERR_ARG, "bsx_cnn_infer_topk: k %d out of range", k);
     hipStream_t s = (hipStream_t)stream;
     return infer_chunks(h, x_dev, n, s, "bsx_cnn_infer_topk", [&](const float* lg, int64_t b0, int nb) {
-        if (k <= 16)
-            hipLaunchKernelGGL(k_row_topk<16>, dim3(nb), dim3(256), 0, s, lg, h->nclass, k,
-                               cls_dev + b0 * k, prob_dev + b0 * k);
-        else
-            hipLaunchKernelGGL(k_row_topk<32>, dim3(nb), dim3(256), 0, s, lg, h->nclass, k,
-                               cls_dev + b0 * k, prob_dev + b0 * k);
+        hipLaunchKernelGGL(k_row_topk, dim3(nblk(nb, 4)), dim3(256), 0, s, lg, (long)nb, h->nclass, k,
+                           cls_dev + b0 * k, prob_dev + b0 * k);
         BSX_HIP(hipGetLastError());
         return BSX_OK;
     });
@@ -1643,19 +1806,11 @@ int bsx_cnn_match_topk(bsx_cnn* h, const float* p_dev, int64_t n, const float* r
     for (int64_t b0 = 0; b0 < n; b0 += chunk) {
         const int nb = (int)std::min<int64_t>(chunk, n - b0);
         // scores = P R^T / tau: the rows' softmax over the references
-        dim3 g((m + 63) / 64, (nb + 63) / 64);
-        hipLaunchKernelGGL((k_sgemm<float>), g, dim3(256), 0, s, nb, m, d, p_dev + b0 * d, (long)d,
-                           1l, r_dev, 1l, (long)d, (const float*)nullptr, h->d_match, (long)m);
+        hipLaunchKernelGGL(k_scores32, dim3((m + 127) / 128, (nb + 127) / 128), dim3(256), 0, s, nb, m, d,
+                           p_dev + b0 * d, r_dev, 1.f / tau, h->d_match);
         BSX_HIP(hipGetLastError());
-        hipLaunchKernelGGL(k_scale, dim3(nblk((long)nb * m)), dim3(256), 0, s, h->d_match,
-                           (long)nb * m, 1.f / tau);
-        BSX_HIP(hipGetLastError());
-        if (k <= 16)
-            hipLaunchKernelGGL(k_row_topk<16>, dim3(nb), dim3(256), 0, s, h->d_match, m, k,
-                               cls_dev + b0 * k, prob_dev + b0 * k);
-        else
-            hipLaunchKernelGGL(k_row_topk<32>, dim3(nb), dim3(256), 0, s, h->d_match, m, k,
-                               cls_dev + b0 * k, prob_dev + b0 * k);
+        hipLaunchKernelGGL(k_row_topk, dim3(nblk(nb, 4)), dim3(256), 0, s, h->d_match, (long)nb, m, k,
+                           cls_dev + b0 * k, prob_dev + b0 * k);
         BSX_HIP(hipGetLastError());
     }
     return BSX_OK;

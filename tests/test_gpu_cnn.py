@@ -125,6 +125,54 @@ def test_pair_gradients_tile_edges(S, ch, d, B):
     assert np.array_equal(g, again.cpu().numpy())      # sums in a fixed order
 
 
+@pytest.mark.parametrize("S,ch,ncls,B", [(8, (32, 32, 32, 32), 5, 3), (24, (32, 96, 64, 4), 200, 37),
+                                         (32, (64, 160, 32, 36), 130, 130)])
+def test_bf16_inference_tile_edges(S, ch, ncls, B):
+    """Matrix-core inference at the edges of its tiles (positions, channels and
+    classes that are no multiples of 64 or 128, a last layer whose rows are not
+    16-byte aligned): probabilities against the FP64 forward of the BF16-rounded
+    weights with BF16 activations (1e-3)."""
+    say(f"inference S={S} ch={ch} classes={ncls} batch={B}")
+    net = ProposalNet(S, ncls, ch, max_batch=B, seed=9)
+    x = np.random.default_rng(S).normal(size=(B, S, S)).astype(np.float32)
+    k = min(5, ncls)
+    cls, prob = (t.cpu().numpy() for t in net.topk(torch.as_tensor(x).cuda(), k))
+    ol, _ = cnn_ref.forward(bf16_round(net.params().cpu().numpy()), x.astype(np.float64), S, ch, ncls,
+                            round_act=bf16_round)
+    e = np.exp(ol - ol.max(axis=1, keepdims=True))
+    pr = e / e.sum(axis=1, keepdims=True)
+    np.testing.assert_allclose(prob, np.take_along_axis(pr, cls, 1), atol=1e-3)
+    assert np.all(prob[:, -1] >= np.sort(pr, axis=1)[:, -k] - 1e-3)
+
+
+@pytest.mark.parametrize("m,k", [(5, 5), (40, 32), (63, 8), (64, 16), (1021, 16), (9000, 32)])
+def test_row_topk_against_sort(m, k):
+    """The k best references by cosine over rows shorter and longer than a
+    wavefront, with tied scores (repeated references: the lower index first) and
+    rows of equal scores throughout; probabilities against an FP64 softmax."""
+    net = EmbeddingNet(8, 16, (8, 8, 8, 8), max_batch=4)
+    rng = np.random.default_rng(m)
+    r = rng.normal(size=(m, 16)).astype(np.float32)
+    r[m // 2:] = r[: m - m // 2]                       # every score twice
+    p = rng.normal(size=(7, 16)).astype(np.float32)
+    p[3] = 0                                           # all scores equal
+    say(f"row top-k m={m} k={k}")
+    cls, prob = (t.cpu().numpy() for t in net.match_topk(torch.as_tensor(p).cuda(), torch.as_tensor(r).cuda(), k, 0.5))
+    sc = p.astype(np.float64) @ r.T.astype(np.float64) / 0.5
+    sm = np.exp(sc - sc.max(axis=1, keepdims=True))
+    sm /= sm.sum(axis=1, keepdims=True)
+    for i in range(len(p)):
+        assert len(set(cls[i])) == k
+        np.testing.assert_allclose(prob[i], sm[i, cls[i]], rtol=1e-4)
+        np.testing.assert_allclose(sc[i, cls[i]], np.sort(sc[i])[::-1][:k], atol=1e-4)
+    assert list(cls[3]) == list(range(k))
+    for i in (0, 1, 2):      # a repeated pair: the lower index comes first
+        pos = {c: q for q, c in enumerate(cls[i])}
+        for c in cls[i]:
+            if c >= m // 2 and c - m // 2 in pos and np.array_equal(r[c], r[c - m // 2]):
+                assert pos[c - m // 2] < pos[c]
+
+
 @pytest.mark.parametrize("ch", [(8, 8, 16, 8), (32, 64, 32, 64)])
 def test_training_reduces_loss_and_bf16_inference(ch):
     """Adam memorises a fixed batch; BF16 inference (VALU path for small
