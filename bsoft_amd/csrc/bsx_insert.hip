@@ -550,7 +550,7 @@ __device__ __forceinline__ void interp_emit(float* __restrict__ acc, const Recon
                                             const double m[3], bool inband, double w, float fr,
                                             float fi, int kk, int merge, unsigned keybase,
                                             const BinCtx& bc, int bin = 1, bool flush = false) {
-    if (FAST || K.interp < 2) {
+    if (FAST == 1 || FAST == 2 || (!FAST && K.interp < 2)) {
         const double fx = floor(m[0] + 0.5), fy = floor(m[1] + 0.5), fz = floor(m[2] + 0.5);
         double ww = w;
         if (FAST == 2 || (!FAST && K.interp == 1)) {   // weighted nearest neighbour
@@ -575,10 +575,16 @@ __device__ __forceinline__ void interp_emit(float* __restrict__ acc, const Recon
                                 make_emit<FOM>(keybase + rec_index32(jx, jy, jz, K.NT), kk,
                                                inband, fr, fi, ww, bin),
                                 bc);
-            // staged pair entries: at most one per thread and corner, so the
-            // list is flushed after every second corner (workgroup-uniform:
-            // only the sample's own emission, which every thread makes, asks)
-            if (MODE == MODE_FILL && flush && bc.st.on && (corner & 1)) stage_flush(bc);
+            // staged pair entries: at most one per thread and corner, so the list
+            // is flushed once it could not take another corner's
+            // (workgroup-uniform: only the sample's own emission, which every
+            // thread makes, asks)
+            if (MODE == MODE_FILL && flush && bc.st.on) {
+                __syncthreads();
+                const bool full = *bc.st.nent > BSX_STAGE_CAP - (int)blockDim.x;
+                __syncthreads();   // every wave has read the count
+                if (full) stage_flush(bc);
+            }
         }
     }
 }
@@ -696,7 +702,7 @@ __device__ __forceinline__ void insert_pair(float* __restrict__ acc, const Recon
         // same weights (floor(-m) = -floor(m) - 1 and 1 - dx; a coordinate
         // that is an integer only swaps a zero-weight corner)
         bool sym = km == -k;
-        if (FAST || K.interp < 2) {
+        if (FAST == 1 || FAST == 2 || (!FAST && K.interp < 2)) {
 #pragma unroll
             for (int q = 0; q < 3; ++q) sym = sym && floor(-m[q] + 0.5) == -floor(m[q] + 0.5);
         }
@@ -713,13 +719,15 @@ __device__ __forceinline__ void insert_pair(float* __restrict__ acc, const Recon
 }
 
 // Column tasks: task = (particle, x) with x in [0, FT/2]; G tasks per WG.
-// The nearest-neighbour specialisations (FAST 1: nearest, 2: weighted
-// nearest, both with pair entries and staging, no Ewald) are held to 5 waves
-// per SIMD (at most 96 VGPRs): their 31.7 KB of LDS allows 5 workgroups per
-// CU, and one register more would round the allocation up to 104 and allow
-// only 4 (the weighted one spills 12 B for it).
+// The specialisations (FAST 1: nearest, 2: weighted nearest, 3: trilinear, with
+// pair entries and staging, no Ewald) are held to 5 waves per SIMD (at most 96
+// VGPRs): their 31.7 KB of LDS allows 5 workgroups per CU, and one register
+// more would round the allocation up to 104 and allow only 4 (the weighted one
+// spills 12 B for it); with the FOM sums (35.8 KB) and for trilinear insertion to
+// 4. Generic kernel (167 VGPRs) against the specialised ones, per batch: FOM sums
+// of 128^2 particles 1,151 -> 889 us, trilinear insertion of 90^2 ones 836 -> 734.
 template <int FT, bool FOM, int MODE, int FAST = 0>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FAST ? 5 : 1)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FAST ? (FOM || FAST == 3 ? 4 : 5) : 1)))
 void k_cols(const float2* __restrict__ inter,
                                               const float* __restrict__ bkg,
                                               const PartDev* __restrict__ recs, int nb, int box,
@@ -806,7 +814,7 @@ void k_cols(const float2* __restrict__ inter,
             ei = er * sd + ei * c;
             er = nr;
         }
-        if (MODE == MODE_FILL && staged && (r & 1) == 1) stage_flush(bc);
+        if (MODE == MODE_FILL && staged && (FAST == 3 ? r == 7 : (r & 1) == 1)) stage_flush(bc);
     }
 }
 
@@ -840,13 +848,15 @@ int insert_batch(bsx_recon* h, const float* imgs, int64_t p0, int nb, hipStream_
     };
     if (!h->binned) {
         h->K.fom ? go(k_cols<FT, true, MODE_DIRECT>) : go(k_cols<FT, false, MODE_DIRECT>);
-    } else if (h->K.fom) {
-        go(k_cols<FT, true, MODE_FILL>);
-    } else if (h->K.pairs && h->K.interp < 2 && !h->K.ewald && NT == 256) {
-        // nearest-neighbour pair entries with LDS staging: the specialised kernels
-        h->K.interp == 0 ? go(k_cols<FT, false, MODE_FILL, 1>) : go(k_cols<FT, false, MODE_FILL, 2>);
+    } else if (h->K.ewald || NT != 256) {
+        h->K.fom ? go(k_cols<FT, true, MODE_FILL>) : go(k_cols<FT, false, MODE_FILL>);
     } else {
-        go(k_cols<FT, false, MODE_FILL>);
+        // pair entries with LDS staging: the specialised kernels
+        switch (h->K.interp) {
+            case 0: h->K.fom ? go(k_cols<FT, true, MODE_FILL, 1>) : go(k_cols<FT, false, MODE_FILL, 1>); break;
+            case 1: h->K.fom ? go(k_cols<FT, true, MODE_FILL, 2>) : go(k_cols<FT, false, MODE_FILL, 2>); break;
+            default: h->K.fom ? go(k_cols<FT, true, MODE_FILL, 3>) : go(k_cols<FT, false, MODE_FILL, 3>);
+        }
     }
     BSX_HIP(hipGetLastError());
     return mark(h, s, h->binned ? KT_FILL : KT_DIRECT);

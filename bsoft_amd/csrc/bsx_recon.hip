@@ -283,9 +283,12 @@ __device__ __forceinline__ void lds_fadd2(float2* p, float x, float y) {
 // add the tile partial to the volume — a plain read-modify-write when the bin
 // is a single piece, float atomics per touched record for multi-piece bins.
 // Each thread keeps 8 entry loads in flight before its LDS adds. FOM: the
-// entries' (sum w|F|^2, sum w^2) come from bins2 and the records hold 5 floats.
+// entries' (sum w|F|^2, sum w^2) come from bins2 and the records hold 5 floats,
+// 80 KB of LDS, so that one workgroup fits a CU: 1024 threads of 4 loads
+// (674 -> 648 us a batch
+// of 2,048 particles against 512 threads of 8).
 template <bool FOM>
-__global__ __launch_bounds__(512) void k_tile_accum(const int* __restrict__ fill,
+__global__ __launch_bounds__(FOM ? 1024 : 512) void k_tile_accum(const int* __restrict__ fill,
                                                     const int* __restrict__ chunks, int maxc,
                                                     int piece_len, const int* __restrict__ poff,
                                                     const int* __restrict__ pbin, int nbins,
@@ -293,6 +296,7 @@ __global__ __launch_bounds__(512) void k_tile_accum(const int* __restrict__ fill
                                                     const float2* __restrict__ bins2,
                                                     float* __restrict__ acc) {
     constexpr int RS = FOM ? 5 : 3;                 // floats per record
+    constexpr int TN = FOM ? 1024 : 512;            // threads
     constexpr int PC = BSX_PIECE_MAX / BSX_CHUNK;   // chunks per piece, at most
     const int pcn = piece_len / BSX_CHUNK;
     const int piece = blockIdx.x;
@@ -318,7 +322,7 @@ __global__ __launch_bounds__(512) void k_tile_accum(const int* __restrict__ fill
         if (FOM) spw[i] = make_float2(0.f, 0.f);
     }
     __syncthreads();
-    constexpr int U = 8;
+    constexpr int U = FOM ? 4 : 8;
     const int stride = blockDim.x;
     for (int e0 = beg + threadIdx.x; e0 < end; e0 += U * stride) {
         float4 v[U];
@@ -345,13 +349,13 @@ __global__ __launch_bounds__(512) void k_tile_accum(const int* __restrict__ fill
     if (single) {
         // the tile's 4096 RS floats as float4: all loads, then all stores
         float4* g4 = reinterpret_cast<float4*>(g);
-        constexpr int NV = 1024 * RS / 512;
+        constexpr int NV = 1024 * RS / TN;
         float4 cur[NV];
 #pragma unroll
-        for (int u = 0; u < NV; ++u) cur[u] = g4[threadIdx.x + u * 512];
+        for (int u = 0; u < NV; ++u) cur[u] = g4[threadIdx.x + u * TN];
 #pragma unroll
         for (int u = 0; u < NV; ++u) {
-            const int f = 4 * (threadIdx.x + u * 512);
+            const int f = 4 * (threadIdx.x + u * TN);
             float add[4];
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
@@ -363,7 +367,7 @@ __global__ __launch_bounds__(512) void k_tile_accum(const int* __restrict__ fill
             cur[u].y += add[1];
             cur[u].z += add[2];
             cur[u].w += add[3];
-            g4[threadIdx.x + u * 512] = cur[u];
+            g4[threadIdx.x + u * TN] = cur[u];
         }
     } else {
         for (int li = threadIdx.x; li < 4096; li += blockDim.x) {
@@ -1096,7 +1100,7 @@ static int run_batch(bsx_recon* h, const float* imgs, int64_t p0, int nb, hipStr
     BSX_HIP(hipGetLastError());
     if ((r = tmark(h, s, KT_SCAN))) return r;
     if (h->K.fom)
-        hipLaunchKernelGGL(k_tile_accum<true>, dim3(maxpieces), dim3(512), 0, s, h->fill,
+        hipLaunchKernelGGL(k_tile_accum<true>, dim3(maxpieces), dim3(1024), 0, s, h->fill,
                            h->chunks, h->maxc, h->piece, h->poff, h->pbin, h->nbins, h->bins,
                            h->bins2, h->xacc);
     else
