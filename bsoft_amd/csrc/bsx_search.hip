@@ -1750,10 +1750,12 @@ int run_exhaustive(bsx_search* h, const uint16_t* A, int64_t nrows, int32_t* can
     const int64_t rblocks = round_up(nrows, GM4) / GM4;
     const int ntiles = (int)(round_up(h->nviews, GN4) / GN4);
     // enough segments to give the chip >= 1024 workgroups (one per CU at a
-    // time), at least 4 tiles each
+    // time), at least 4 tiles each; few particles: shorter segments, a workgroup
+    // for every CU (150 particles against 269 tiles: 64 workgroups of 5 tiles took
+    // 253 us, 135 of 2 take 107)
     int nseg = (int)std::max<int64_t>(1, std::min<int64_t>(ntiles / 4 > 0 ? ntiles / 4 : 1,
                                                            (1024 + rblocks - 1) / rblocks));
-    nseg = std::min(nseg, 64);
+    nseg = std::max(std::min(nseg, 64), (int)std::min<int64_t>(ntiles, 256 / rblocks));
     const int tps = (ntiles + nseg - 1) / nseg;
     nseg = (ntiles + tps - 1) / tps;
     const int64_t need = rblocks * GM4 * nseg * 4 * T;

@@ -175,6 +175,26 @@ def test_gemm_topk_row_blocks_and_k_steps():
     assert parities == {0, 1}
 
 
+@pytest.mark.parametrize("nview", [100, 256, 700, 1153])
+def test_few_particles_in_short_segments(setup64, nview):
+    """Few particles split the views into segments of as little as one tile:
+    three particles searched alone have the same candidates and the same
+    scores, bit for bit, as among 1,100, whose segments are longer."""
+    n, R, bm, vol, ft, ps = setup64
+    mats = search.view_matrices(synth.uniform_views(nview, np.random.default_rng(nview)))
+    say(f"short segments views={nview}")
+    out = []
+    for count in (3, 1100):
+        pick = np.arange(count) % 3
+        s = search.Search(n, R, 1.5, topk=16)
+        s.set_reference(ft, mats)
+        s.stage(ps.images[pick].cuda().contiguous(), ps.parts[pick])
+        cand, score = s.exhaustive()
+        out.append((cand[:3].cpu().numpy(), score[:3].cpu().numpy()))
+    assert np.array_equal(out[0][0], out[1][0])
+    assert np.array_equal(out[0][1], out[1][1])
+
+
 def test_rescore_and_score_mats_match_reference_frc(setup64):
     n, R, bm, vol, ft, ps = setup64
     views = search.views_c1(10.0, angle_step_deg=45.0)
