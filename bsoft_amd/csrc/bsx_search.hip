@@ -1749,15 +1749,32 @@ int run_exhaustive(bsx_search* h, const uint16_t* A, int64_t nrows, int32_t* can
     const int T = h->p.topk <= 8 ? 8 : 16;
     const int64_t rblocks = round_up(nrows, GM4) / GM4;
     const int ntiles = (int)(round_up(h->nviews, GN4) / GN4);
-    // enough segments to give the chip >= 1024 workgroups (one per CU at a
-    // time), at least 4 tiles each; few particles: shorter segments, a workgroup
-    // for every CU (150 particles against 269 tiles: 64 workgroups of 5 tiles took
-    // 253 us, 135 of 2 take 107)
-    int nseg = (int)std::max<int64_t>(1, std::min<int64_t>(ntiles / 4 > 0 ? ntiles / 4 : 1,
-                                                           (1024 + rblocks - 1) / rblocks));
-    nseg = std::max(std::min(nseg, 64), (int)std::min<int64_t>(ntiles, 256 / rblocks));
-    const int tps = (ntiles + nseg - 1) / nseg;
-    nseg = (ntiles + tps - 1) / tps;
+    // Segments of views: one workgroup a CU at a time and 32 CUs an XCD, each XCD
+    // taking an eighth of the workgroups, so the whole takes
+    // ceil(ceil(workgroups / 8) / 32) rounds of (tiles + about half a tile for the
+    // first loads and the filling of the lists). The fewest segments of the
+    // smallest product: 1,024 workgroups or 64 segments whatever the tiles made
+    // 51 tiles of 10 row blocks x 1,060 tiles where 42 suffice, and 10 of
+    // 5 x 269 where 6 do (whole searches with a 64^3 map: 1,200 particles against
+    // 230,940 views 1,433 -> 907 us, 5,000 against 68,520 1,011 -> 868; 25,000
+    // particles of 96^2 3,301 -> 2,565). Up to 2,048 workgroups, which bounds the
+    // lists, and 256 segments, where the tiles of few particles take a CU each
+    // (150 against 269 tiles: 253 -> 107 us in this kernel); under a memory cap no
+    // more than 64 segments and about 1,024 workgroups of 4 tiles need.
+    int nmax = (int)std::min<int64_t>(ntiles, std::min<int64_t>(256, 1 + 2048 / rblocks));
+    if (h->p.mem_cap > 0)
+        nmax = (int)std::min<int64_t>(std::min(64, std::max(1, ntiles / 4)), (1024 + rblocks - 1) / rblocks);
+    int nseg = 1, tps = ntiles;
+    int64_t least = INT64_MAX;
+    for (int n = 1; n <= nmax; ++n) {
+        const int per = (ntiles + n - 1) / n, used = (ntiles + per - 1) / per;
+        const int64_t rounds = ((rblocks * used + 7) / 8 + 31) / 32;
+        if (rounds * (2 * per + 1) < least) {
+            least = rounds * (2 * per + 1);
+            nseg = used;
+            tps = per;
+        }
+    }
     const int64_t need = rblocks * GM4 * nseg * 4 * T;
     int rc = grow(h, &h->d_pscore, &h->pscore_cap, need, "top-k partials");
     if (!rc) rc = grow(h, &h->d_pidx, &h->pidx_cap, need, "top-k partials");
