@@ -273,48 +273,21 @@ __global__ __launch_bounds__(256) void k_lib_build(
 // through LDS in two 128-row halves (rows of 260 floats, so b128 row reads
 // stay conflict-free); thread t folds row t % 128 of the half, columns
 // 64 (t / 128) .. + 63, into its running top-T list, 4 columns at a time
-// against the list's T-th value and against the row's bound. The top-T lists
-// come out per (row, segment, column quarter).
+// against the list's T-th value. The top-T lists come out per (row,
+// segment, column quarter).
 constexpr int GM4 = 256, GN4 = 256;
 constexpr int GSTAGE4 = (GM4 + GN4) * 128;        // bytes per pipeline stage
 constexpr int CROW4 = GN4 + 4;
 constexpr int GEMM4_LDS = (2 * GSTAGE4 > 128 * CROW4 * 4) ? 2 * GSTAGE4 : 128 * CROW4 * 4;
-
-// A row's bound: a score that T views of the row are known to reach, as an
-// unsigned key in the order of the floats, shared by the row's lists of every
-// segment. A list on its own takes some 8 (1 + ln(n / 8)) of its n columns, and a
-// wave goes through the insertion when any of its 64 rows has one, which with
-// lists of 1,000 columns is almost always. Whole searches without and with the
-// bounds: 1,200 particles against 230,940 views of a 64^3 map 907 -> 795 us,
-// 5,000 against 68,520 868 -> 724, 25,000 of 96^2 2,565 -> 2,413; 5,000 of 128^2
-// (K = 1,792), where the products are most of it, 4,985 -> 4,984. Views below it are in no top-T list,
-// views that equal it may be (the lower index wins), so the lists take what is
-// above the float just below the bound; -0 counts as 0.
-constexpr unsigned BOUND_NONE = 0x007FFFFFu;   // -infinity
-__device__ __forceinline__ unsigned bound_key(float v) {
-    const unsigned u = __float_as_uint(v + 0.f);
-    return (u & 0x80000000u) ? ~u : u | 0x80000000u;
-}
-__device__ __forceinline__ float below_bound(unsigned key) {
-    if (key <= BOUND_NONE) return -INFINITY;
-    const unsigned b = key - (key == 0x80000000u ? 2 : 1);
-    return __uint_as_float((b & 0x80000000u) ? b ^ 0x80000000u : ~b);
-}
-__global__ void k_no_bounds(unsigned* __restrict__ rbound, int64_t n) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) rbound[i] = BOUND_NONE;
-}
 
 template <int T>
 __global__ __launch_bounds__(512) void k_gemm_topk4(const uint16_t* __restrict__ A,
                                                     const uint16_t* __restrict__ B, int Kp,
                                                     int ncols, int tiles_per_seg, int ntiles,
                                                     int rblocks, int nseg,
-                                                    unsigned* __restrict__ rbound,
                                                     float* __restrict__ pscore,
                                                     int* __restrict__ pidx) {
     __shared__ __attribute__((aligned(16))) char lds[GEMM4_LDS];
-    __shared__ float quarter[4][128];
     typedef __attribute__((address_space(3))) void* lds_ptr;
     // XCD-aware order: hardware block b runs on XCD b % 8; logical block
     // L = (b % 8) * per + b / 8 gives each XCD a contiguous range, row blocks
@@ -338,18 +311,17 @@ __global__ __launch_bounds__(512) void k_gemm_topk4(const uint16_t* __restrict__
 #pragma unroll
         for (int q = 0; q < T; ++q) { best[hh][q] = -INFINITY; bidx[hh][q] = -1; }
     const int nk = Kp / GK;
-    // this wave's load instructions: A rows 32 w .. + 31, B rows 32 w .. + 31;
-    // row 8 i + (lane >> 3) takes its chunks in the same order for every i
-    const int lofs = (lane >> 3) * Kp + ((lane & 7) ^ (lane >> 3)) * 8;
-    const size_t wrow = (size_t)__builtin_amdgcn_readfirstlane(wave) * 32 * Kp;
-    const uint16_t* const arow = A + row0 * Kp + wrow;
-    // this lane's chunk of K sub-step 0 in rows wm 64 + (lane & 31) of A and wn 128 + ..
-    // of B: sub-step ks is 2 ks chunks away under the XOR, row + 32 i 4096 i bytes
-    const int slot = ((lane >> 5) ^ (lane & 7)) << 4;
-    const int aofs = (wm * 64 + (lane & 31)) * 128 + slot;
-    const int bofs = GM4 * 128 + (wn * 128 + (lane & 31)) * 128 + slot;
+    // this wave's load instructions: A rows 32 w .. + 31, B rows 32 w .. + 31
+    const uint16_t* asrc[4];
+    const uint16_t* bsrc[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int r = 8 * (wave * 4 + q) + (lane >> 3);
+        asrc[q] = A + (row0 + r) * Kp + ((lane & 7) ^ (r & 7)) * 8;
+        bsrc[q] = B + (size_t)r * Kp + ((lane & 7) ^ (r & 7)) * 8;
+    }
     for (int t = t0; t < t1; ++t) {
-        const uint16_t* const brow = B + (size_t)t * GN4 * Kp + wrow;
+        const size_t cofs = (size_t)t * GN4 * Kp;
         f32x16 acc[2][4];
 #pragma unroll
         for (int i = 0; i < 2; ++i)
@@ -357,31 +329,40 @@ __global__ __launch_bounds__(512) void k_gemm_topk4(const uint16_t* __restrict__
             for (int j = 0; j < 4; ++j)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-        auto stage = [&](int kt) {
-            char* base = lds + (kt & 1) * GSTAGE4 + wave * 4096;
+        auto stage = [&](int buf, size_t k0) {
+            char* base = lds + buf * GSTAGE4;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const size_t o = (size_t)8 * q * Kp + (size_t)kt * GK;
-                __builtin_amdgcn_global_load_lds(arow + o + lofs, (lds_ptr)(base + q * 1024), 16, 0, 0);
-                __builtin_amdgcn_global_load_lds(brow + o + lofs, (lds_ptr)(base + GM4 * 128 + q * 1024),
+                __builtin_amdgcn_global_load_lds(asrc[q] + k0, (lds_ptr)(base + (wave * 4 + q) * 1024),
+                                                 16, 0, 0);
+                __builtin_amdgcn_global_load_lds(bsrc[q] + cofs + k0,
+                                                 (lds_ptr)(base + GM4 * 128 + (wave * 4 + q) * 1024),
                                                  16, 0, 0);
             }
         };
-        stage(0);
+        stage(0, 0);
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
         for (int kt = 0; kt < nk; ++kt) {
             // buffer (kt + 1) & 1 was read in step kt - 1, which every wave
             // has left (barrier at its end)
-            if (kt + 1 < nk) stage(kt + 1);
-            const char* buf = lds + (kt & 1) * GSTAGE4;
+            if (kt + 1 < nk) stage((kt + 1) & 1, (size_t)(kt + 1) * GK);
+            const char* abuf = lds + (kt & 1) * GSTAGE4;
+            const char* bbuf = abuf + GM4 * 128;
 #pragma unroll
             for (int ks = 0; ks < GK / 16; ++ks) {
+                const int c = ks * 2 + (lane >> 5);
                 bf16x8 fa[2], fb[4];
 #pragma unroll
-                for (int i = 0; i < 2; ++i) fa[i] = *(const bf16x8*)(buf + (aofs ^ (ks << 5)) + i * 4096);
+                for (int i = 0; i < 2; ++i) {
+                    const int ra = wm * 64 + i * 32 + (lane & 31);
+                    fa[i] = *(const bf16x8*)(abuf + ra * 128 + ((c ^ (ra & 7)) << 4));
+                }
 #pragma unroll
-                for (int j = 0; j < 4; ++j) fb[j] = *(const bf16x8*)(buf + (bofs ^ (ks << 5)) + j * 4096);
+                for (int j = 0; j < 4; ++j) {
+                    const int rb = wn * 128 + j * 32 + (lane & 31);
+                    fb[j] = *(const bf16x8*)(bbuf + rb * 128 + ((c ^ (rb & 7)) << 4));
+                }
 #pragma unroll
                 for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -395,9 +376,6 @@ __global__ __launch_bounds__(512) void k_gemm_topk4(const uint16_t* __restrict__
         float* C = (float*)lds;
 #pragma unroll
         for (int hh = 0; hh < 2; ++hh) {
-            unsigned* const bound = rbound + row0 + hh * 128 + my_row;
-            const unsigned known = rbound ? __hip_atomic_load(bound, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                                          : BOUND_NONE;
             if ((wm >> 1) == hh) {
 #pragma unroll
                 for (int i = 0; i < 2; ++i)
@@ -414,16 +392,14 @@ __global__ __launch_bounds__(512) void k_gemm_topk4(const uint16_t* __restrict__
             const float* cr = C + my_row * CROW4 + my_q * 64;
             const int cbase = t * GN4 + my_q * 64;
             const int jmax = min(64, ncols - cbase);
-            const float below = below_bound(known);
-            float cut = fmaxf(best[hh][T - 1], below);
             for (int j = 0; j < jmax; j += 4) {
                 const float4 v4 = *(const float4*)(cr + j);
-                if (fmaxf(fmaxf(v4.x, v4.y), fmaxf(v4.z, v4.w)) > cut) {
+                if (fmaxf(fmaxf(v4.x, v4.y), fmaxf(v4.z, v4.w)) > best[hh][T - 1]) {
                     const float vv[4] = {v4.x, v4.y, v4.z, v4.w};
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         const float v = vv[e];
-                        if (j + e < jmax && v > cut) {
+                        if (j + e < jmax && v > best[hh][T - 1]) {
                             best[hh][T - 1] = v;
                             bidx[hh][T - 1] = cbase + j + e;
 #pragma unroll
@@ -433,18 +409,11 @@ __global__ __launch_bounds__(512) void k_gemm_topk4(const uint16_t* __restrict__
                                     const int ti = bidx[hh][q]; bidx[hh][q] = bidx[hh][q - 1]; bidx[hh][q - 1] = ti;
                                 }
                             }
-                            cut = fmaxf(best[hh][T - 1], below);
                         }
                     }
                 }
             }
-            quarter[my_q][my_row] = best[hh][T / 4 - 1];
             __syncthreads();
-            if (my_q == 0 && rbound) {   // T / 4 scores in each quarter are no less than the least of these
-                const float least = fminf(fminf(quarter[0][my_row], quarter[1][my_row]),
-                                          fminf(quarter[2][my_row], quarter[3][my_row]));
-                if (bound_key(least) > known) atomicMax(bound, bound_key(least));
-            }
         }
     }
 #pragma unroll
@@ -1471,8 +1440,7 @@ struct bsx_search {
     float* d_ktab = nullptr;
     float* d_pscore = nullptr;
     int* d_pidx = nullptr;
-    int64_t pscore_cap = 0, pidx_cap = 0, rbound_cap = 0;
-    unsigned* d_rbound = nullptr;   // bounds of the rows' top lists
+    int64_t pscore_cap = 0, pidx_cap = 0;
     int64_t bytes = 0;
 };
 
@@ -1618,7 +1586,7 @@ int bsx_search_destroy(bsx_search* h) {
     if (!h) return BSX_OK;
     void* ptrs[] = {h->d_hk,   h->d_ring,    h->d_lib,    h->d_lbf,    h->d_fp,
                     h->d_ctf,  h->d_pbf,     h->d_spec,   h->d_sp,
-                    h->d_ktab, h->d_pscore,  h->d_pidx, h->d_rbound,  h->d_libmats, h->d_lmats,
+                    h->d_ktab, h->d_pscore,  h->d_pidx,   h->d_libmats, h->d_lmats,
                     h->d_lfrc, h->d_sub,     h->d_members, h->d_mcount, h->d_counts,
                     h->d_cursors, h->d_pairs, h->d_items, h->d_cube,
                     h->d_rv,   h->d_rvi};
@@ -1810,23 +1778,15 @@ int run_exhaustive(bsx_search* h, const uint16_t* A, int64_t nrows, int32_t* can
     const int64_t need = rblocks * GM4 * nseg * 4 * T;
     int rc = grow(h, &h->d_pscore, &h->pscore_cap, need, "top-k partials");
     if (!rc) rc = grow(h, &h->d_pidx, &h->pidx_cap, need, "top-k partials");
-    // Bounds from the third tile of a segment on: with two, one tile has no bound
-    // yet, and they gain nothing (150 particles: 183 us a search without, 184 with
-    // them). Under a memory cap what the lists take is all there may be.
-    const bool bounds = tps > 2 && h->p.mem_cap <= 0;
-    if (!rc && bounds) rc = grow(h, &h->d_rbound, &h->rbound_cap, rblocks * GM4, "score bounds");
     if (rc) return rc;
-    if (bounds)
-        hipLaunchKernelGGL(k_no_bounds, dim3((unsigned)rblocks), dim3(GM4), 0, s, h->d_rbound, rblocks * GM4);
-    unsigned* const rb = bounds ? h->d_rbound : nullptr;
     BSX_REQUIRE(rblocks * nseg < (1ll << 31) - 8, BSX_ERR_ARG, "bsx_search_exhaustive: too many particles");
     const dim3 grid((unsigned)(8 * ((rblocks * nseg + 7) / 8)));
     if (T == 8)
         hipLaunchKernelGGL((k_gemm_topk4<8>), grid, dim3(512), 0, s, A, h->d_lbf, h->Kp,
-                           (int)h->nviews, tps, ntiles, (int)rblocks, nseg, rb, h->d_pscore, h->d_pidx);
+                           (int)h->nviews, tps, ntiles, (int)rblocks, nseg, h->d_pscore, h->d_pidx);
     else
         hipLaunchKernelGGL((k_gemm_topk4<16>), grid, dim3(512), 0, s, A, h->d_lbf, h->Kp,
-                           (int)h->nviews, tps, ntiles, (int)rblocks, nseg, rb, h->d_pscore, h->d_pidx);
+                           (int)h->nviews, tps, ntiles, (int)rblocks, nseg, h->d_pscore, h->d_pidx);
     BSX_HIP(hipGetLastError());
     const unsigned mg = (unsigned)((nrows + 3) / 4);
     if (T == 8)

@@ -195,31 +195,6 @@ def test_few_particles_in_short_segments(setup64, nview):
     assert np.array_equal(out[0][1], out[1][1])
 
 
-@pytest.mark.parametrize("topk", [3, 8, 16])
-@pytest.mark.parametrize("npart,nview,repeat", [(5, 90, 1), (600, 1153, 3), (1100, 1153, 30)])
-def test_row_bounds_change_no_list(setup64, npart, nview, repeat, topk):
-    """The bounds that the segments of a row share drop only what no top list
-    holds: candidates and scores equal, bit for bit, those without them (under
-    a memory cap), also among repeated views, whose scores tie, and again in a
-    second search, which starts from no bounds."""
-    n, R, bm, vol, ft, ps = setup64
-    mats = np.tile(search.view_matrices(synth.uniform_views(nview, np.random.default_rng(nview))),
-                   (repeat, 1, 1))
-    say(f"bounds particles={npart} views={len(mats)} topk={topk}")
-    pick = np.arange(npart) % len(ps.parts)
-    out = []
-    for cap in (0, 8 << 30):
-        s = search.Search(n, R, 1.5, topk=topk, mem_cap=cap)
-        s.set_reference(ft, mats)
-        s.stage(ps.images[pick].cuda().contiguous(), ps.parts[pick])
-        for _ in range(2):
-            cand, score = s.exhaustive()
-            out.append((cand.cpu().numpy(), score.cpu().numpy()))
-    for c, v in out[1:]:
-        assert np.array_equal(c, out[0][0])
-        assert np.array_equal(v, out[0][1])
-
-
 def test_rescore_and_score_mats_match_reference_frc(setup64):
     n, R, bm, vol, ft, ps = setup64
     views = search.views_c1(10.0, angle_step_deg=45.0)
