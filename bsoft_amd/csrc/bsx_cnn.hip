@@ -787,13 +787,17 @@ __global__ __launch_bounds__(256) void k_softmax_ce(const float* __restrict__ lo
 
 // The k largest logits of a row (k <= 32) as classes and softmax probabilities,
 // best first (ties: lower class; NaN and -inf are never taken, missing places
-// -1 and 0). One wavefront per row, two passes over it: the lanes' maxima, the
+// -1 and 0). W wavefronts per row, two passes over it: the lanes' maxima, the
 // k-th largest of which bounds the k-th value from below, then the exponential
-// sum and the few values that reach the bound (ROWCAP of them; a row with more,
-// e.g. of equal values, takes k passes). Bound by reading the row: 16,384 rows of
-// 4,368 took 388 us with 16 block-wide arg-max rounds over per-thread lists, now
-// 179 us.
-constexpr int ROWCAP = 192;
+// sum and the values that reach the bound, listed in LDS. Before a list could
+// overflow (values equal to the bound, or large ones on fewer than k lanes) it is
+// cut to its k best, whose last one is the new bound: the classes come in
+// ascending order, so that a later equal value never belongs to them. Bound by
+// reading the row: 16,384 x 4,368 179 us (388 with 16 block-wide arg-max rounds over
+// per-thread lists). Rows of equal values, the whole call with its scores: 1 x 2^20
+// 0.6 ms, 16,384 x 4,368 0.8 ms; with a pass for each of 16 places once a list
+// was full they took 46.8 and 1.5 ms.
+constexpr int ROWCAP = 256;   // listed values of a wavefront
 
 __device__ __forceinline__ unsigned long long logit_key(float v, int c) {
     const unsigned u = __float_as_uint(v + 0.f);   // -0 counts as 0
@@ -808,17 +812,45 @@ __device__ __forceinline__ unsigned long long wave_max64(unsigned long long m) {
     }
     return m;
 }
+// LDS written by lanes of this wavefront before is read by others after.
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+// The k largest of the keys x (Q a lane, all different, 0: none), largest first,
+// to out[0..k); returns the k-th, 0 if there are fewer.
+template <int Q>
+__device__ __forceinline__ unsigned long long wave_best(unsigned long long (&x)[Q], int k, int lane,
+                                                        unsigned long long* out) {
+    unsigned long long m = 0;
+    for (int r = 0; r < k; ++r) {
+        m = x[0];
+#pragma unroll
+        for (int q = 1; q < Q; ++q) m = x[q] > m ? x[q] : m;
+        m = wave_max64(m);
+        if (lane == 0) out[r] = m;
+#pragma unroll
+        for (int q = 0; q < Q; ++q) x[q] = x[q] == m ? 0 : x[q];
+    }
+    return m;
+}
 
-__global__ __launch_bounds__(256) void k_row_topk(const float* __restrict__ logits, long n, int C, int k,
-                                                  int* __restrict__ cls, float* __restrict__ prob) {
-    __shared__ unsigned long long list[4][ROWCAP];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const long b = (long)blockIdx.x * 4 + wave;
-    if (b >= n) return;   // a whole wavefront; no workgroup barrier below
+template <int W>
+__global__ __launch_bounds__(W > 4 ? 64 * W : 256) void k_row_topk(const float* __restrict__ logits, long n,
+                                                                   int C, int k, int* __restrict__ cls,
+                                                                   float* __restrict__ prob) {
+    constexpr int ROWS = W >= 4 ? 1 : 4 / W;   // rows per workgroup
+    __shared__ unsigned long long list[ROWS * W][ROWCAP];
+    __shared__ float red[3][W];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, part = wave % W;
+    const long b = (long)blockIdx.x * ROWS + wave / W;
+    if (b >= n) return;   // whole wavefronts; with W > 1 a workgroup has one row
     const float* l = logits + b * C;
+    unsigned long long* mine = list[wave];
     float lm = -INFINITY;
 #pragma unroll 4
-    for (int c = lane; c < C; c += 64) lm = fmaxf(lm, l[c]);
+    for (int c = part * 64 + lane; c < C; c += 64 * W) lm = fmaxf(lm, l[c]);
     float mx = lm;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
@@ -832,46 +864,71 @@ __global__ __launch_bounds__(256) void k_row_topk(const float* __restrict__ logi
         const unsigned long long has = __ballot(left == m);
         if (lane == __builtin_ctzll(has | (1ull << 63))) left = -INFINITY;
     }
+    if (W > 1) {   // every wavefront's bound is one of the row
+        if (lane == 0) {
+            red[0][part] = mx;
+            red[1][part] = bound;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            mx = fmaxf(mx, red[0][w]);
+            bound = fmaxf(bound, red[1][w]);
+        }
+    }
     float se = 0.f;
     int cnt = 0;
-    for (int c0 = 0; c0 < C; c0 += 64) {
+    unsigned long long above = 0;   // keys up to this one are out of the running
+    auto cut = [&]() {
+        unsigned long long x[ROWCAP / 64];
+        wave_lds_sync();
+#pragma unroll
+        for (int q = 0; q < ROWCAP / 64; ++q) x[q] = lane + 64 * q < cnt ? mine[lane + 64 * q] : 0;
+        wave_lds_sync();
+        above = wave_best(x, k, lane, mine);
+        wave_lds_sync();
+        cnt = min(cnt, k);
+    };
+    for (int c0 = part * 64; c0 < C; c0 += 64 * W) {
         const int c = c0 + lane;
         const float v = c < C ? l[c] : -INFINITY;
         if (c < C) se += expf(v - mx);
-        const bool in = v >= bound && v > -INFINITY;
-        const unsigned long long has = __ballot(in);
-        if (has) {
-            const int at = cnt + __popcll(has & ((1ull << lane) - 1ull));
-            if (in && at < ROWCAP) list[wave][at] = logit_key(v, c);
+        bool in = v >= bound && v > -INFINITY;
+        if (__ballot(in)) {
+            const unsigned long long key = logit_key(v, c);
+            in = in && key > above;
+            const unsigned long long has = __ballot(in);
+            if (in) mine[cnt + __popcll(has & ((1ull << lane) - 1ull))] = key;
             cnt += __popcll(has);
+            if (cnt > ROWCAP - 64) cut();
         }
     }
     se = wave_add(se);
-    __builtin_amdgcn_wave_barrier();
-    unsigned long long last = ~0ull;
-    for (int r = 0; r < k; ++r) {
-        // the largest key below the last one taken
-        unsigned long long m = 0;
-        if (cnt <= ROWCAP) {
-            for (int i = lane; i < cnt; i += 64) {
-                const unsigned long long x = list[wave][i];
-                m = (x < last && x > m) ? x : m;
-            }
-        } else {
-            for (int c = lane; c < C; c += 64) {
-                const float v = l[c];
-                const unsigned long long x = v > -INFINITY ? logit_key(v, c) : 0;
-                m = (x < last && x > m) ? x : m;
-            }
+    cut();
+    if (W > 1) {
+        if (lane == 0) red[2][part] = se;
+        __syncthreads();
+        if (wave) return;
+        se = 0.f;
+#pragma unroll
+        for (int w = 0; w < W; ++w) se += red[2][w];
+        constexpr int Q = W > 1 ? W / 2 : 1;   // 64 Q >= W * 32
+        unsigned long long x[Q];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int i = lane + 64 * q;
+            x[q] = i < W * k ? list[i / k][i % k] : 0;
         }
-        m = wave_max64(m);
-        last = m;
-        if (lane == 0) {
-            const unsigned o = (unsigned)(m >> 32);
-            const float v = __uint_as_float((o & 0x80000000u) ? o & 0x7fffffffu : ~o);
-            cls[b * k + r] = m ? (int)~(unsigned)m : -1;
-            prob[b * k + r] = m ? expf(v - mx) / se : 0.f;
-        }
+        wave_lds_sync();
+        (void)wave_best(x, k, lane, mine);
+        wave_lds_sync();
+    }
+    if (lane < k) {
+        const unsigned long long m = mine[lane];
+        const unsigned o = (unsigned)(m >> 32);
+        const float v = __uint_as_float((o & 0x80000000u) ? o & 0x7fffffffu : ~o);
+        cls[b * k + lane] = m ? (int)~(unsigned)m : -1;
+        prob[b * k + lane] = m ? expf(v - mx) / se : 0.f;
     }
 }
 
@@ -1283,6 +1340,26 @@ struct Rng {
     double uniform() { return ((next() >> 11) + 0.5) * (1.0 / 9007199254740992.0); }
     double normal() { return sqrt(-2 * log(uniform())) * cos(2 * M_PI * uniform()); }
 };
+
+// The k best of each of n rows of C logits. One wavefront reads a row in about
+// 4 us a thousand logits, which few long rows wait for; several share it where
+// the rows leave CUs idle and their reading outweighs the 5 us (4 wavefronts) and
+// 20 us (16) that a row's join takes, or 2 x and 8 x the rows a CU holds (scores of
+// 16 values and the top 16, 1 / 4 / 16 wavefronts a row): 16 x 65,536 295 / 98 / 60 us,
+// 16 x 16,384 88 / 44 / 45, 16 x 1,200 26 / 27 / 40; 256 x 4,368 42 / 33 / 44,
+// 512 x 4,368 44 / 39 / 70, 1,024 x 4,368 48 / 54 / 118; 512 x 65,536 471 / 170 / 125,
+// 1,024 x 65,536 530 / 229 / 223; 2,048 x 16,384 161 / 123 / 243, 4,096 x 16,384
+// 222 / 220 / 468.
+int row_topk(const float* logits, long n, int C, int k, int* cls, float* prob, hipStream_t s) {
+    auto go = [&](auto kernel, int rows, int threads) {
+        hipLaunchKernelGGL(kernel, dim3(nblk(n, rows)), dim3(threads), 0, s, logits, n, C, k, cls, prob);
+    };
+    if (C >= 32768 && n <= 512) go(k_row_topk<16>, 1, 1024);
+    else if ((C >= 4096 && n <= 256) || (C >= 16384 && n <= 2048)) go(k_row_topk<4>, 1, 256);
+    else go(k_row_topk<1>, 4, 256);
+    BSX_HIP(hipGetLastError());
+    return BSX_OK;
+}
 
 // Shares that a sum over `steps` stages is split into so that some 512
 // workgroups (two per CU) run, with at least 4 stages a share.
@@ -1766,10 +1843,7 @@ int bsx_cnn_infer_topk(bsx_cnn* h, const float* x_dev, int64_t n, int32_t k, int
     BSX_REQUIRE(k >= 1 && k <= 32 && k <= h->nclass, BSX_ERR_ARG, "bsx_cnn_infer_topk: k %d out of range", k);
     hipStream_t s = (hipStream_t)stream;
     return infer_chunks(h, x_dev, n, s, "bsx_cnn_infer_topk", [&](const float* lg, int64_t b0, int nb) {
-        hipLaunchKernelGGL(k_row_topk, dim3(nblk(nb, 4)), dim3(256), 0, s, lg, (long)nb, h->nclass, k,
-                           cls_dev + b0 * k, prob_dev + b0 * k);
-        BSX_HIP(hipGetLastError());
-        return BSX_OK;
+        return row_topk(lg, nb, h->nclass, k, cls_dev + b0 * k, prob_dev + b0 * k, s);
     });
 }
 
@@ -1809,9 +1883,8 @@ int bsx_cnn_match_topk(bsx_cnn* h, const float* p_dev, int64_t n, const float* r
         hipLaunchKernelGGL(k_scores32, dim3((m + 127) / 128, (nb + 127) / 128), dim3(256), 0, s, nb, m, d,
                            p_dev + b0 * d, r_dev, 1.f / tau, h->d_match);
         BSX_HIP(hipGetLastError());
-        hipLaunchKernelGGL(k_row_topk, dim3(nblk(nb, 4)), dim3(256), 0, s, h->d_match, (long)nb, m, k,
-                           cls_dev + b0 * k, prob_dev + b0 * k);
-        BSX_HIP(hipGetLastError());
+        const int rc = row_topk(h->d_match, nb, m, k, cls_dev + b0 * k, prob_dev + b0 * k, s);
+        if (rc) return rc;
     }
     return BSX_OK;
 }

@@ -173,6 +173,63 @@ def test_row_topk_against_sort(m, k):
                 assert pos[c - m // 2] < pos[c]
 
 
+@pytest.mark.parametrize("n,m,k", [(1, 4095, 16), (1, 4096, 16), (256, 4097, 32), (257, 4097, 5), (3, 16384, 32),
+                                   (2, 32767, 16), (5, 32768, 32), (1, 70001, 1)])
+def test_row_topk_orders_ties_and_extremes(n, m, k):
+    """The k best of rows on both sides of every line of the rule that shares a
+    row among wavefronts, whose values fill and overflow the kept lists: random,
+    all equal, seven values over and over, ascending, large ones on two lanes
+    only, and with NaN and infinities. Classes by value, equal ones by index."""
+    rng = np.random.default_rng(m)
+    v = rng.normal(size=m).astype(np.float32)
+    lanes = np.where(np.arange(m) % 1024 < 2, 10 + np.arange(m) * 1e-3, v).astype(np.float32)
+    odd = v.copy()
+    odd[rng.integers(m, size=40)] = np.nan
+    odd[rng.integers(m, size=40)] = np.inf
+    odd[: m - 20] = np.where(rng.random(m - 20) < 0.5, -np.inf, odd[: m - 20])
+    few = np.full(m, -np.inf, dtype=np.float32)
+    few[[m // 2, m - 1]] = 1, 2
+    rows = {"random": v, "equal": np.zeros(m, np.float32), "signed zeros": np.where(v > 0, 0.0, -0.0).astype(np.float32),
+            "seven": v[np.arange(m) % 7], "ascending": np.sort(v), "descending": np.sort(v)[::-1].copy(),
+            "two lanes": lanes, "odd": odd, "few": few}
+    net = EmbeddingNet(8, 8, (8, 8, 8, 8), max_batch=4)
+    p = torch.zeros((n, 8), device="cuda")
+    p[:, 0] = 1
+    for name, row in rows.items():
+        say(f"row top-k n={n} m={m} k={k} {name}")
+        r = torch.zeros((m, 8), device="cuda")
+        r[:, 0] = torch.as_tensor(row).cuda()
+        cls, prob = (t.cpu().numpy() for t in net.match_topk(p, r, k, 1.0))
+        take = np.flatnonzero(row > -np.inf)
+        want = take[np.lexsort((take, -row[take]))][:k]
+        want = np.concatenate([want, np.full(k - len(want), -1, int)])
+        assert np.array_equal(cls, np.tile(want, (n, 1))), name
+        if np.all(np.isfinite(row)):
+            e = np.exp(row.astype(np.float64) - row.max())
+            np.testing.assert_allclose(prob, np.tile((e / e.sum())[want], (n, 1)), rtol=1e-4)
+
+
+def test_row_topk_of_equal_values_takes_one_pass():
+    """Rows of equal values are no slower than others by more than a factor of
+    three (a pass over the row for each of 16 places took 11 times as long)."""
+    net = EmbeddingNet(8, 64, (8, 8, 8, 8), max_batch=4)
+    r = torch.randn((1 << 19, 64), device="cuda", generator=torch.Generator("cuda").manual_seed(1))
+
+    def best(p):
+        took = []
+        for _ in range(6):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            net.match_topk(p, r, 16, 1.0)
+            b.record()
+            b.synchronize()
+            took.append(a.elapsed_time(b))
+        return min(took[1:])
+
+    say("row top-k of equal values")
+    assert best(torch.zeros((1, 64), device="cuda")) <= 3 * best(r[:1].contiguous())
+
+
 @pytest.mark.parametrize("ch", [(8, 8, 16, 8), (32, 64, 32, 64)])
 def test_training_reduces_loss_and_bf16_inference(ch):
     """Adam memorises a fixed batch; BF16 inference (VALU path for small
