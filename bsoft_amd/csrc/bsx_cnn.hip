@@ -795,7 +795,7 @@ __global__ __launch_bounds__(256) void k_softmax_ce(const float* __restrict__ lo
 // ascending order, so that a later equal value never belongs to them. Bound by
 // reading the row: 16,384 x 4,368 179 us (388 with 16 block-wide arg-max rounds over
 // per-thread lists). Rows of equal values, the whole call with its scores: 1 x 2^20
-// 0.6 ms, 16,384 x 4,368 0.8 ms; with a pass for each of 16 places once a list
+// 0.6 ms, 16,384 x 4,368 0.4 ms; with a pass for each of 16 places once a list
 // was full they took 46.8 and 1.5 ms.
 constexpr int ROWCAP = 256;   // listed values of a wavefront
 
