@@ -41,6 +41,7 @@ using namespace bsx;
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16;
+typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4;
 
 namespace {
 
@@ -442,12 +443,11 @@ __global__ void k_route_count(const int* __restrict__ cls, int64_t n, int k, int
 struct GroupItem {
     int cls, p0, np, pad_;
 };
-constexpr int RM = 64, RN = 64;   // routed pairs x member views of a grouped GEMM tile
 
 // Exclusive sums of the class counts (the fill's cursors) and the list of work
-// items, up to RM routed pairs of one class each: one workgroup, so that the
+// items, up to `rm` routed pairs of one class each: one workgroup, so that the
 // host need not see the counts. nitems: the number of items.
-__global__ __launch_bounds__(1024) void k_route_scan(const int* __restrict__ counts, int nclass,
+__global__ __launch_bounds__(1024) void k_route_scan(const int* __restrict__ counts, int nclass, int rm,
                                                      int* __restrict__ cursors,
                                                      GroupItem* __restrict__ items,
                                                      int* __restrict__ nitems) {
@@ -458,7 +458,7 @@ __global__ __launch_bounds__(1024) void k_route_scan(const int* __restrict__ cou
     int np = 0, ni = 0;
     for (int c = c0; c < c1; ++c) {
         np += counts[c];
-        ni += (counts[c] + RM - 1) / RM;
+        ni += (counts[c] + rm - 1) / rm;
     }
     sp[tid] = np;
     si[tid] = ni;
@@ -474,7 +474,7 @@ __global__ __launch_bounds__(1024) void k_route_scan(const int* __restrict__ cou
     for (int c = c0; c < c1; ++c) {
         const int n = counts[c];
         cursors[c] = p;
-        for (int q = 0; q < n; q += RM) items[i++] = GroupItem{c, p + q, min(RM, n - q), 0};
+        for (int q = 0; q < n; q += rm) items[i++] = GroupItem{c, p + q, min(rm, n - q), 0};
         p += n;
     }
     if (tid == 1023) *nitems = si[1023];
@@ -495,23 +495,30 @@ __global__ void k_route_fill(const int* __restrict__ cls, int64_t n, int k, int 
     for (int q = 0; q < T; ++q) { pscore[t * T + q] = -INFINITY; pidx[t * T + q] = -1; }
 }
 
-// One workgroup (4 waves of 32 x 32) per work item: up to 64 routed pairs of one
-// class against the class's member views, 64 a tile. At 4-degree views in
-// 15-degree classes a class has some 53 members and, for 8,000 particles x 16
-// proposals, some 29 pairs, and every view's row is read about once: reading the
-// rows bounds it (1.3 GB there), so that tiles are small (four workgroups a CU
-// keep loads in flight) and rows beyond the pairs or members are not read.
-// 128 x 128 tiles took 417 us, these 226 us (3.7 TB/s of lines). The per-pair top T over the
-// members goes to pscore/pidx[(particle * k + slot) * T + q].
-template <int T>
+// One workgroup (2 x 2 waves of BM x BM blocks of 32 x 32) per work item: up to
+// 64 BM routed pairs of one class against the class's member views, 64 BM a tile.
+// At 4-degree views in 15-degree classes a class has some 53 members and, for 8,000
+// particles x 16 proposals, some 29 pairs, and every view's row is read about once:
+// reading the rows bounds it (1.3 GB there), so that tiles are small (BM 1: four
+// workgroups a CU keep loads in flight). 128 x 128 tiles took 417 us, these 226 us
+// (3.7 TB/s of lines). Where classes are crowded an item walks many tiles one after
+// the other, each step of which takes about as long for 128 x 128 products as for
+// 64 x 64: BM 2, whose waves read four times for four products instead of two for one
+// (20 classes of 1,000 members, 10,000 x 5 pairs, radius 32: a search of 1,249 us with BM 1
+// and 873 with BM 2). The per-pair top T over the members goes to
+// pscore/pidx[(particle * k + slot) * T + q].
+template <int T, int BM>
 __global__ __launch_bounds__(256) void k_gemm_grouped(
     const uint16_t* __restrict__ A, const uint16_t* __restrict__ B, int Kp,
     const GroupItem* __restrict__ items, const int* __restrict__ nitems, const int* __restrict__ pairs,
     int k, const int* __restrict__ members, const int* __restrict__ mcount, int maxm,
     float* __restrict__ pscore, int* __restrict__ pidx) {
+    constexpr int RM = 64 * BM, RN = 64 * BM;   // pairs x member views of a tile
+    constexpr int LD = 2 * BM;                  // staged rows per thread, A and B each
+    constexpr int PARTS = 256 / RM, PC = RN / PARTS;   // epilogue: threads per row, columns of each
     constexpr int CR = RN + 1;   // floats per epilogue row
     constexpr int STAGE = (RM + RN) * LROW;
-    static_assert(RM * CR * 4 <= 2 * STAGE && RM * 4 * T * 8 <= 2 * STAGE, "epilogue fits the staging buffers");
+    static_assert(RM * CR * 4 <= 2 * STAGE && RM * PARTS * T * 8 <= 2 * STAGE, "epilogue fits the staging buffers");
     __shared__ __attribute__((aligned(16))) char lds[2 * STAGE];
     __shared__ int scol[RN];
     if ((int)blockIdx.x >= *nitems) return;
@@ -519,75 +526,93 @@ __global__ __launch_bounds__(256) void k_gemm_grouped(
     const int wm = wave >> 1, wn = wave & 1;
     const GroupItem it = items[blockIdx.x];
     const int nm = mcount[it.cls];
-    const int my_row = tid & (RM - 1), my_q = tid >> 6;   // epilogue: row, column quarter
+    const int my_row = tid & (RM - 1), my_q = tid / RM;   // epilogue: row, part of its columns
     float best[T];
     int bidx[T];
 #pragma unroll
     for (int q = 0; q < T; ++q) { best[q] = -INFINITY; bidx[q] = -1; }
     const int nk = Kp / GK;
-    // staging: 64 rows of 8 16-byte chunks, A and B, two rows per thread each
+    // staging: RM rows of 8 16-byte chunks, A and B; rows beyond the pairs or members
+    // repeat the last one (products with them are never read), so that the loads
+    // need no masks and the stages no zeros
     const int ld_row = tid >> 3, ld_part = tid & 7;
-    const uint16_t* pa[2];
+    const uint16_t* pa[LD];
 #pragma unroll
-    for (int q = 0; q < 2; ++q) {
-        const int r = ld_row + 32 * q;
-        pa[q] = r < it.np ? A + (size_t)(pairs[it.p0 + r] / k) * Kp + ld_part * 8 : nullptr;
-    }
+    for (int q = 0; q < LD; ++q)
+        pa[q] = A + (size_t)(pairs[it.p0 + min(ld_row + 32 * q, it.np - 1)] / k) * Kp + ld_part * 8;
     const int own = my_row < it.np ? pairs[it.p0 + my_row] : -1;
-    const bool mine_a = wm * 32 < it.np;
+    // whether this wavefront's blocks hold something (small tiles: uniform, or
+    // the products would be masked)
+    const int uw = __builtin_amdgcn_readfirstlane(wave);
+    const bool mine_a = BM > 1 || (uw >> 1) * 32 < it.np;
     for (int t0 = 0; t0 < nm; t0 += RN) {
         __syncthreads();   // the epilogue before has been read
-        if (tid < RN) scol[tid] = t0 + tid < nm ? members[(size_t)it.cls * maxm + t0 + tid] : -1;
+        if (tid < RN) scol[tid] = members[(size_t)it.cls * maxm + min(t0 + tid, nm - 1)];
         __syncthreads();
-        const uint16_t* pb[2];
+        const uint16_t* pb[LD];
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const int v = scol[ld_row + 32 * q];
-            pb[q] = v >= 0 ? B + (size_t)v * Kp + ld_part * 8 : nullptr;
-        }
-        const bool mine = mine_a && t0 + wn * 32 < nm;   // this wave's block holds something
-        f32x16 acc;
+        for (int q = 0; q < LD; ++q) pb[q] = B + (size_t)scol[ld_row + 32 * q] * Kp + ld_part * 8;
+        const bool mine = mine_a && (BM > 1 || t0 + (uw & 1) * 32 < nm);
+        f32x16 acc[BM][BM];
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-        uint4 ra[2], rb[2];
-        auto load = [&](int k0) {
+        for (int i = 0; i < BM; ++i)
 #pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                ra[q] = pa[q] ? *(const uint4*)(pa[q] + k0) : make_uint4(0, 0, 0, 0);
-                rb[q] = pb[q] ? *(const uint4*)(pb[q] + k0) : make_uint4(0, 0, 0, 0);
-            }
-        };
-        auto store = [&](int buf) {
-            char* d = lds + buf * STAGE + ld_row * LROW + ld_part * 16;
+            for (int j = 0; j < BM; ++j)
 #pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                *(uint4*)(d + 32 * q * LROW) = ra[q];
-                *(uint4*)(d + (RM + 32 * q) * LROW) = rb[q];
-            }
-        };
-        load(0);
-        store(0);
+                for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+        u32x4 ra[LD], rb[LD];   // vector type: structs that live across the branches end up in scratch memory
+        char* const st = lds + ld_row * LROW + ld_part * 16;
+#define BSX_GLOAD(K0)                                                \
+    _Pragma("unroll") for (int q = 0; q < LD; ++q) {                 \
+        ra[q] = *(const u32x4*)(pa[q] + (K0));                       \
+        rb[q] = *(const u32x4*)(pb[q] + (K0));                       \
+    }
+#define BSX_GSTORE(D)                                                \
+    _Pragma("unroll") for (int q = 0; q < LD; ++q) {                 \
+        *(u32x4*)((D) + 32 * q * LROW) = ra[q];                      \
+        *(u32x4*)((D) + (RM + 32 * q) * LROW) = rb[q];               \
+    }
+        BSX_GLOAD(0)
+        BSX_GSTORE(st)
         __syncthreads();
         for (int kt = 0; kt < nk; ++kt) {
-            if (kt + 1 < nk) load((kt + 1) * GK);
+            const bool more = kt + 1 < nk;
+            if (more) { BSX_GLOAD((kt + 1) * GK) }
             if (mine) {
-                const char* fa = lds + (kt & 1) * STAGE + (wm * 32 + (lane & 31)) * LROW + (lane >> 5) * 16;
-                const char* fb = lds + (kt & 1) * STAGE + (RM + wn * 32 + (lane & 31)) * LROW + (lane >> 5) * 16;
+                const char* fa = lds + (kt & 1) * STAGE + (wm * 32 * BM + (lane & 31)) * LROW + (lane >> 5) * 16;
+                const char* fb = lds + (kt & 1) * STAGE + (RM + wn * 32 * BM + (lane & 31)) * LROW + (lane >> 5) * 16;
 #pragma unroll
-                for (int ks = 0; ks < GK / 16; ++ks)
-                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)(fa + ks * 32),
-                                                                  *(const bf16x8*)(fb + ks * 32), acc, 0, 0, 0);
+                for (int ks = 0; ks < GK / 16; ++ks) {
+                    bf16x8 va[BM], vb[BM];
+#pragma unroll
+                    for (int i = 0; i < BM; ++i) {
+                        va[i] = *(const bf16x8*)(fa + i * 32 * LROW + ks * 32);
+                        vb[i] = *(const bf16x8*)(fb + i * 32 * LROW + ks * 32);
+                    }
+#pragma unroll
+                    for (int i = 0; i < BM; ++i)
+#pragma unroll
+                        for (int j = 0; j < BM; ++j)
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[i], vb[j], acc[i][j], 0, 0, 0);
+                }
             }
-            if (kt + 1 < nk) store((kt + 1) & 1);
+            if (more) { BSX_GSTORE(st + ((kt + 1) & 1) * STAGE) }
             __syncthreads();
         }
+#undef BSX_GLOAD
+#undef BSX_GSTORE
         float* C = (float*)lds;
 #pragma unroll
-        for (int r = 0; r < 16; ++r)
-            C[(wm * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * CR + wn * 32 + (lane & 31)] = acc[r];
+        for (int i = 0; i < BM; ++i)
+#pragma unroll
+            for (int j = 0; j < BM; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    C[((wm * BM + i) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * CR +
+                      (wn * BM + j) * 32 + (lane & 31)] = acc[i][j][r];
         __syncthreads();
         if (own >= 0)
-            for (int j = my_q * (RN / 4); j < min((my_q + 1) * (RN / 4), nm - t0); ++j) {
+            for (int j = my_q * PC; j < min((my_q + 1) * PC, nm - t0); ++j) {
                 const float v = C[my_row * CR + j];
                 if (v > best[T - 1]) {
                     best[T - 1] = v;
@@ -602,10 +627,10 @@ __global__ __launch_bounds__(256) void k_gemm_grouped(
                 }
             }
     }
-    // combine the four column quarters of each row into the row's list
+    // combine the parts of each row into the row's list
     __syncthreads();
     float* xs = (float*)lds;
-    int* xi = (int*)(lds + RM * 4 * T * sizeof(float));
+    int* xi = (int*)(lds + RM * PARTS * T * sizeof(float));
 #pragma unroll
     for (int q = 0; q < T; ++q) {
         xs[(my_q * T + q) * RM + my_row] = best[q];
@@ -613,7 +638,7 @@ __global__ __launch_bounds__(256) void k_gemm_grouped(
     }
     __syncthreads();
     if (my_q != 0 || own < 0) return;
-    for (int e = T; e < 4 * T; ++e) {
+    for (int e = T; e < PARTS * T; ++e) {
         const float v = xs[e * RM + my_row];
         const int id = xi[e * RM + my_row];
         if (id >= 0 && v > best[T - 1]) {
@@ -1428,6 +1453,7 @@ struct bsx_search {
     int* d_members = nullptr;
     int64_t members_cap = 0;
     int* d_mcount = nullptr;
+    int64_t tiles64 = 0, tiles128 = 0;   // tiles of 64 and 128 members over all classes
     int64_t mcount_cap = 0;
     int* d_counts = nullptr;
     int64_t counts_cap = 0;
@@ -1864,6 +1890,11 @@ int bsx_search_set_classes(bsx_search* h, const int32_t* members, int32_t nclass
     BSX_HIP(hipMemcpy(h->d_mcount, cnt.data(), sizeof(int) * nclasses, hipMemcpyHostToDevice));
     h->nclass = nclasses;
     h->maxm = maxm;
+    h->tiles64 = h->tiles128 = 0;
+    for (int m : cnt) {
+        h->tiles64 += (m + 63) / 64;
+        h->tiles128 += (m + 127) / 128;
+    }
     return BSX_OK;
 }
 
@@ -1885,27 +1916,37 @@ int bsx_search_proposed(bsx_search* h, const int32_t* cls_dev, int32_t k, int32_
     if (!rc) rc = grow(h, &h->d_pidx, &h->pidx_cap, n * k * T, "proposal partials");
     if (rc) return rc;
     const unsigned g = (unsigned)((n * k + 255) / 256);
-    const int64_t most = h->nclass + n * k / RM;   // items: sum over classes of ceil(pairs / RM)
+    // 128 x 128 tiles for long products of classes that fill them, i.e. whose members
+    // take at most two thirds of the number of 64 x 64 tiles (55 % and some 500 or
+    // 2,048 members a class for shorter products). Whole calls with 20,000 views,
+    // 128 against 64, for 2 to 2,000 pairs a class: Kp 4,992 (radius 40) 53 members 1.29 to 0.90,
+    // 80 0.68 to 0.77, 190 0.72 to 0.92, 4,000 0.66 to 0.69; 1,792 53 members 1.17 to 0.98, 80 0.84 to 0.90,
+    // 190 0.89 to 1.03, 4,000 0.72 to 0.81; 1,280 190 0.94 to 1.06, 500 0.80 to 0.98;
+    // 832 500 0.83 to 1.05, 1,150 0.84 to 1.13, 4,000 0.80 to 0.93; 448 500 0.95 to 1.15.
+    const int64_t t64 = h->tiles64, t128 = h->tiles128, nc = h->nclass;
+    const bool wide = h->Kp >= 1536 ? 3 * t128 <= 2 * t64
+                                    : 20 * t128 <= 11 * t64 && ((h->Kp >= 1152 && t64 >= 8 * nc) ||
+                                                                (h->Kp >= 768 && t64 >= 32 * nc));
+    const int rm = wide ? 128 : 64;
+    const int64_t most = h->nclass + n * k / rm;   // items: sum over classes of ceil(pairs / rm)
     rc = grow(h, &h->d_items, &h->items_cap, most + 1, "work items");
     if (rc) return rc;
     int* nitems = (int*)(h->d_items + most);
     BSX_HIP(hipMemsetAsync(h->d_counts, 0, sizeof(int) * h->nclass, s));
     hipLaunchKernelGGL(k_route_count, dim3(g), dim3(256), 0, s, cls_dev, n, k, h->nclass, h->d_counts);
     BSX_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_route_scan, dim3(1), dim3(1024), 0, s, h->d_counts, h->nclass, h->d_cursors,
+    hipLaunchKernelGGL(k_route_scan, dim3(1), dim3(1024), 0, s, h->d_counts, h->nclass, rm, h->d_cursors,
                        h->d_items, nitems);
     BSX_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_route_fill, dim3(g), dim3(256), 0, s, cls_dev, n, k, h->nclass, T, h->d_cursors,
                        h->d_pairs, h->d_pscore, h->d_pidx);
     BSX_HIP(hipGetLastError());
-    if (T == 8)
-        hipLaunchKernelGGL((k_gemm_grouped<8>), dim3((unsigned)most), dim3(256), 0, s, h->d_pbf, h->d_lbf,
-                           h->Kp, h->d_items, nitems, h->d_pairs, k, h->d_members, h->d_mcount, h->maxm,
-                           h->d_pscore, h->d_pidx);
-    else
-        hipLaunchKernelGGL((k_gemm_grouped<16>), dim3((unsigned)most), dim3(256), 0, s, h->d_pbf, h->d_lbf,
-                           h->Kp, h->d_items, nitems, h->d_pairs, k, h->d_members, h->d_mcount, h->maxm,
-                           h->d_pscore, h->d_pidx);
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)most), dim3(256), 0, s, h->d_pbf, h->d_lbf, h->Kp, h->d_items,
+                           nitems, h->d_pairs, k, h->d_members, h->d_mcount, h->maxm, h->d_pscore, h->d_pidx);
+    };
+    if (T == 8) wide ? go(k_gemm_grouped<8, 2>) : go(k_gemm_grouped<8, 1>);
+    else wide ? go(k_gemm_grouped<16, 2>) : go(k_gemm_grouped<16, 1>);
     BSX_HIP(hipGetLastError());
     const unsigned mg = (unsigned)((n + 3) / 4);
     if (T == 8)

@@ -361,6 +361,45 @@ def test_proposed_tiles_of_pairs_and_members(setup64, npart, topk):
             assert score[i][kk - 1] >= np.sort(A[i] @ B[allowed].T)[::-1][kk - 1] - 2e-4
 
 
+@pytest.mark.parametrize("npart,topk", [(1, 16), (127, 8), (300, 16), (129, 3)])
+def test_proposed_wide_tiles(setup64, npart, topk):
+    """The 128 x 128 tiles of long products of crowded classes at their edges:
+    0 to 257 member views, fewer or more pairs of a class than a tile has rows;
+    the top-k of the exact BF16 products (FP32 accumulation: 1e-4)."""
+    n, _, bm, vol, ft, ps = setup64
+    R = 24
+    rng = np.random.default_rng(npart)
+    sizes = [0, 1, 65, 127, 129, 257]
+    mats = search.view_matrices(synth.uniform_views(sum(sizes), rng))
+    members = np.full((len(sizes), max(sizes)), -1, dtype=np.int32)
+    order, at = rng.permutation(len(mats)), 0
+    for c, m in enumerate(sizes):
+        members[c, :m] = order[at:at + m]
+        at += m
+    rep = np.arange(npart) % len(ps.parts)
+    say(f"wide proposed tiles particles={npart} topk={topk}")
+    s = search.Search(n, R, 1.5, topk=topk)
+    assert s.kdim >= 1536 and 3 * sum(-(-m // 128) for m in sizes) <= 2 * sum(-(-m // 64) for m in sizes)
+    s.set_reference(ft, mats)
+    s.set_classes(members)
+    s.stage(ps.images[torch.as_tensor(rep)].cuda().contiguous(), ps.parts[rep])
+    cls = np.stack([rng.permutation(len(sizes))[:3] for _ in range(npart)]).astype(np.int32)
+    cls[:, 0] = np.where(rng.random(npart) < 0.5, 5, cls[:, 0])    # a crowded class
+    cls[cls[:, 1] == cls[:, 0], 1] = -1
+    cls[cls[:, 2] == cls[:, 0], 2] = 99                            # no such class
+    cand, score = (t.cpu().numpy() for t in s.proposed(torch.as_tensor(cls)))
+    A, B = bf16_to_f32(s.particle_data()[2]), bf16_to_f32(s.library_data()[1])
+    for i in range(npart):
+        allowed = np.concatenate([members[c][members[c] >= 0] for c in cls[i] if 0 <= c < len(sizes)])
+        kk = min(topk, len(allowed))
+        assert np.all(cand[i][:kk] >= 0) and np.all(cand[i][kk:] == -1)
+        assert len(set(cand[i][:kk])) == kk and set(cand[i][:kk]) <= set(allowed)
+        np.testing.assert_allclose(score[i][:kk], A[i] @ B[cand[i][:kk]].T, atol=1e-4)
+        if kk:
+            assert np.all(np.diff(score[i][:kk]) <= 0)
+            assert score[i][kk - 1] >= np.sort(A[i] @ B[allowed].T)[::-1][kk - 1] - 2e-4
+
+
 def _fit_setup(snr, seed, ctf=True):
     n, R = 64, 16
     rng = np.random.default_rng(seed)
