@@ -1453,7 +1453,7 @@ struct bsx_search {
     int* d_members = nullptr;
     int64_t members_cap = 0;
     int* d_mcount = nullptr;
-    int64_t tiles64 = 0, tiles128 = 0;   // tiles of 64 and 128 members over all classes
+    int64_t members = 0, tiles64 = 0, tiles128 = 0;   // of all classes; tiles of 64 and 128 members
     int64_t mcount_cap = 0;
     int* d_counts = nullptr;
     int64_t counts_cap = 0;
@@ -1890,8 +1890,9 @@ int bsx_search_set_classes(bsx_search* h, const int32_t* members, int32_t nclass
     BSX_HIP(hipMemcpy(h->d_mcount, cnt.data(), sizeof(int) * nclasses, hipMemcpyHostToDevice));
     h->nclass = nclasses;
     h->maxm = maxm;
-    h->tiles64 = h->tiles128 = 0;
+    h->members = h->tiles64 = h->tiles128 = 0;
     for (int m : cnt) {
+        h->members += m;
         h->tiles64 += (m + 63) / 64;
         h->tiles128 += (m + 127) / 128;
     }
@@ -1918,15 +1919,17 @@ int bsx_search_proposed(bsx_search* h, const int32_t* cls_dev, int32_t k, int32_
     const unsigned g = (unsigned)((n * k + 255) / 256);
     // 128 x 128 tiles for long products of classes that fill them, i.e. whose members
     // take at most two thirds of the number of 64 x 64 tiles (55 % and some 500 or
-    // 2,048 members a class for shorter products). Whole calls with 20,000 views,
-    // 128 against 64, for 2 to 2,000 pairs a class: Kp 4,992 (radius 40) 53 members 1.29 to 0.90,
-    // 80 0.68 to 0.77, 190 0.72 to 0.92, 4,000 0.66 to 0.69; 1,792 53 members 1.17 to 0.98, 80 0.84 to 0.90,
-    // 190 0.89 to 1.03, 4,000 0.72 to 0.81; 1,280 190 0.94 to 1.06, 500 0.80 to 0.98;
-    // 832 500 0.83 to 1.05, 1,150 0.84 to 1.13, 4,000 0.80 to 0.93; 448 500 0.95 to 1.15.
+    // 2,048 members a class for shorter products), or that have 150 pairs a class.
+    // Whole calls with 20,000 views, 128 against 64, for 2 to 2,000 pairs a class: Kp 4,992
+    // (radius 40) 53 members 1.29 to 0.90, 80 0.68 to 0.77, 190 0.72 to 0.92, 4,000 0.66 to 0.69;
+    // 1,792 53 members 1.17 to 0.98, 80 0.84 to 0.90, 190 0.89 to 1.03, 4,000 0.72 to 0.81;
+    // 1,280 190 0.94 to 1.06, 500 0.80 to 0.98; 832 500 0.83 to 1.05, 1,150 0.84 to 1.13, 4,000
+    // 0.80 to 0.93; 448 500 0.95 to 1.15.
     const int64_t t64 = h->tiles64, t128 = h->tiles128, nc = h->nclass;
-    const bool wide = h->Kp >= 1536 ? 3 * t128 <= 2 * t64
-                                    : 20 * t128 <= 11 * t64 && ((h->Kp >= 1152 && t64 >= 8 * nc) ||
-                                                                (h->Kp >= 768 && t64 >= 32 * nc));
+    const bool wide = (h->Kp >= 1536 && 3 * t128 <= 2 * t64) ||
+                      (20 * t128 <= 11 * t64 &&
+                       ((h->Kp >= 1152 && t64 >= 8 * nc) || (h->Kp >= 768 && t64 >= 32 * nc))) ||
+                      (h->Kp >= 2048 && n * k >= 150 * nc && h->members > 40 * nc);
     const int rm = wide ? 128 : 64;
     const int64_t most = h->nclass + n * k / rm;   // items: sum over classes of ceil(pairs / rm)
     rc = grow(h, &h->d_items, &h->items_cap, most + 1, "work items");
