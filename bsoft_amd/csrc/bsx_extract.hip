@@ -7,6 +7,7 @@
 //        FSI_Kernel, include/FSI_Kernel.h:28-68), centre shift as project()
 //   k_fsc            : FP64 shell sums of Bimage::fsc (Bimage_resolution.cpp:330-406)
 //   k_frc_pairs      : img_recip_space_fom, fom_type 0 (src/mg/mg_refine.cpp:660-781)
+#include <algorithm>
 #include <climits>
 #include <cmath>
 #include <cstring>
@@ -416,27 +417,32 @@ static int extract_launch(const float* ft_dev, int n, double sampling, const dou
     const double inv = 1.0 / (n * sampling), rs = n * sampling;
     const double maxs2 = 1.0 / (resolution * resolution);
     const int tiles = (n + 7) / 8;
-    BSX_REQUIRE((long long)tiles * tiles * nviews < (1ll << 31) - 8, BSX_ERR_ARG,
-                "section extraction: %lld views of %d x %d are too many", (long long)nviews, n, n);
-    const int ntile = (int)(tiles * tiles * nviews);
     const float2* ft = (const float2*)ft_dev;
-    float2* out = (float2*)out_dev;
-    switch (kernel_width) {
+    // a launch takes fewer than 2^32 threads; at most 2^23 tiles of up to 256 each
+    // go into one, so that any number of views is accepted
+    const int64_t per = std::max<int64_t>(1, (1ll << 23) / ((int64_t)tiles * tiles));
+    for (int64_t v0 = 0; v0 < nviews; v0 += per) {
+        const int nv = (int)std::min(per, nviews - v0);
+        const int ntile = tiles * tiles * nv;
+        const double* m = dmats + 9 * v0;
+        float2* out = (float2*)out_dev + v0 * n * n;
+        switch (kernel_width) {
 // LDS boxes from width 5 on (see k_extract); cap holds the largest box of an 8 x 8
 // patch over random rotations (37 KB at W = 8, four workgroups per CU)
 #define BSX_EXT(W) case W: { \
-        constexpr int WPT = W >= 8 ? 4 : W >= 5 ? 2 : 0; \
-        constexpr int cap = WPT ? (W + 10) * (W + 9) * (W + 7) + 64 : 0; \
-        constexpr size_t lds = WPT ? sizeof(float2) * cap : sizeof(float) * (FSI_NDIV + 1) * W; \
-        const int nblk = WPT ? ntile : (ntile + 3) / 4; \
-        hipLaunchKernelGGL((k_extract<W, WPT>), dim3((unsigned)((nblk + 7) / 8 * 8)), dim3(WPT ? 64 * WPT : 256), \
-                           lds, s, ft, n, dmats, inv, rs, maxs2, center, tiles, (int)nviews, nblk, cap, dtab, out); \
-        break; }
-        BSX_EXT(1) BSX_EXT(2) BSX_EXT(3) BSX_EXT(4) BSX_EXT(5)
-        BSX_EXT(6) BSX_EXT(7) BSX_EXT(8) BSX_EXT(9) BSX_EXT(10)
+            constexpr int WPT = W >= 8 ? 4 : W >= 5 ? 2 : 0; \
+            constexpr int cap = WPT ? (W + 10) * (W + 9) * (W + 7) + 64 : 0; \
+            constexpr size_t lds = WPT ? sizeof(float2) * cap : sizeof(float) * (FSI_NDIV + 1) * W; \
+            const int nblk = WPT ? ntile : (ntile + 3) / 4; \
+            hipLaunchKernelGGL((k_extract<W, WPT>), dim3((unsigned)((nblk + 7) / 8 * 8)), dim3(WPT ? 64 * WPT : 256), \
+                               lds, s, ft, n, m, inv, rs, maxs2, center, tiles, nv, nblk, cap, dtab, out); \
+            break; }
+            BSX_EXT(1) BSX_EXT(2) BSX_EXT(3) BSX_EXT(4) BSX_EXT(5)
+            BSX_EXT(6) BSX_EXT(7) BSX_EXT(8) BSX_EXT(9) BSX_EXT(10)
 #undef BSX_EXT
+        }
+        BSX_HIP(hipGetLastError());
     }
-    BSX_HIP(hipGetLastError());
     return BSX_OK;
 }
 

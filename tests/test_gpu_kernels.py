@@ -158,6 +158,22 @@ def test_sections_of_every_tile_path(n, width):
         assert np.abs(out[i] - ref).max() <= 1e-5 * np.abs(ref).max()
 
 
+@pytest.mark.parametrize("n,width,views", [(256, 8, 16385), (24, 3, 65535)])
+def test_sections_of_very_many_views(n, width, views):
+    """More sections than one launch has threads for (2^32 threads from 16,385
+    sections of 256^2 on), and the most views that are accepted: sections at both
+    ends and on both sides of every launch equal those of a call of their own."""
+    rng = np.random.default_rng(views)
+    ft = torch.randn((n, n, n), dtype=torch.complex64, device="cuda", generator=torch.Generator("cuda").manual_seed(n))
+    some = synth.view_to_matrix(synth.uniform_views(7, rng))
+    pick = np.arange(views) % 7
+    say(f"sections n={n} width={width} views={views}")
+    out = recon.central_sections(ft, some[pick], 1.5, 3.0, width, 2, True)
+    want = recon.central_sections(ft, some, 1.5, 3.0, width, 2, True)
+    for v in (0, 1, views // 2 - 1, views // 2, 8191, 8192, 16383, views - 2, views - 1):
+        assert torch.equal(torch.view_as_real(out[v]), torch.view_as_real(want[pick[v]])), v
+
+
 def test_workspaces_shared_by_threads_and_streams():
     """Calls without a handle keep their workspaces between calls: four threads,
     each on a stream of its own and with sizes of its own, get the results of
