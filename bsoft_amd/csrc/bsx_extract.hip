@@ -26,16 +26,18 @@ using namespace bsx;
 // sample, each voxel of the box is used about 10 times.
 // WPT > 0: the box is loaded into LDS once (rows of 16 or 32 lanes), the taps are
 // read from there in the order and precision of fsi_sample, and the wavefronts
-// share the tap planes, whose sums are added in order. A box beyond `cap` voxels
-// (matrices that are no rotations) is sampled from memory.
+// share the tap planes, whose sums are added in order. Where a box is beyond `cap`
+// voxels (matrices that are no rotations) they read their planes from memory: 200
+// sections of 128^2 by a matrix that stretches the plane twofold at W = 10 take 3.6 ms
+// (3.7 with one thread a pixel, 16.1 with the tile sampled by one wavefront alone).
 // WPT 0: narrow kernels (at W = 4 a voxel is used about twice) take the taps from
 // memory, four tiles a workgroup with the kernel table in LDS.
 // Whole calls with the map transform, 200 sections of 128^2, before (one thread a
-// pixel of a row, taps from memory) and now: W = 3 341 / 336 us, 4 525 / 465,
-// 5 802 / 493, 6 999 / 616, 8 1,936 / 987; 50 sections of 256^2: 604 / 535,
-// 847 / 669, 1,181 / 635, 1,432 / 752, 2,715 / 1,104. LDS reads bound it at W = 8
-// (busy 55 %, 60 % of that bank conflicts: the lanes' boxes start anywhere); one
-// and two wavefronts a tile at W = 8: 1,100 and 1,025 us, four at W = 6: 651.
+// pixel of a row, taps from memory) and now: W = 3 322 / 183 us, 4 520 / 317,
+// 5 803 / 337, 6 1,016 / 414, 8 1,989 / 699; 50 sections of 256^2: 589 / 282,
+// 869 / 414, 1,234 / 415, 1,502 / 499, 2,845 / 830. LDS reads bound it at W = 8 (the
+// lanes' boxes start anywhere, so that they meet in banks); when whole calls took
+// 967 us with four wavefronts a tile there, they took 1,100 with one and 1,025 with two.
 struct __attribute__((packed, aligned(4))) Float4u {
     float v[4];
 };
@@ -113,6 +115,9 @@ __global__ __launch_bounds__(WPT ? 64 * WPT : 256) __attribute__((amdgpu_waves_p
             }
             const int sx = n[0] | 1;   // odd row stride: rows start in different banks
             fits = fits && sx * n[1] * n[2] <= cap;
+            float pr[PW], pi[PW];   // sums over this wavefront's tap planes
+#pragma unroll
+            for (int q = 0; q < PW; ++q) pr[q] = pi[q] = 0.f;
             if (fits) {
                 // this lane's kernel weights, in flight together with the box
                 float wx[WD], wy[WD], wz[PW];
@@ -159,9 +164,6 @@ __global__ __launch_bounds__(WPT ? 64 * WPT : 256) __attribute__((amdgpu_waves_p
                     }
                 }
                 __syncthreads();
-                float pr[PW], pi[PW];
-#pragma unroll
-                for (int q = 0; q < PW; ++q) pr[q] = pi[q] = 0.f;
                 if (band) {
                     const float2* t = box + (((int)fl[2] - HW - lo[2] + wave * PW) * n[1] + (int)fl[1] - HW - lo[1]) * sx +
                                       (int)fl[0] - HW - lo[0];
@@ -183,25 +185,50 @@ __global__ __launch_bounds__(WPT ? 64 * WPT : 256) __attribute__((amdgpu_waves_p
                         }
                     }
                 }
-                // plane sums of every wavefront, added in the order of the planes
-                __syncthreads();
-                if (wave)
+            } else if (band) {
+                // from memory, with one periodic wrap or more
+                const float* kx = ktab + ((int)((m[0] - fl[0]) * FSI_NDIV + 0.5)) * WD;
+                const float* ky = ktab + ((int)((m[1] - fl[1]) * FSI_NDIV + 0.5)) * WD;
+                const float* kz = ktab + ((int)((m[2] - fl[2]) * FSI_NDIV + 0.5)) * WD;
+                int jx[WD];
 #pragma unroll
-                    for (int q = 0; q < PW; ++q) box[((wave - 1) * PW + q) * 64 + lane] = make_float2(pr[q], pi[q]);
-                __syncthreads();
-                if (wave) return;
+                for (int e = 0; e < WD; ++e) jx[e] = wrap_index((int)fl[0] - HW + e, N);
 #pragma unroll
                 for (int q = 0; q < PW; ++q) {
-                    vr += pr[q];
-                    vi += pi[q];
+                    const int z2 = wave * PW + q;
+                    if (z2 >= WD) break;
+                    const float2* plane = ft + (size_t)wrap_index((int)fl[2] - HW + z2, N) * N * N;
+                    const float kzz = kz[z2];
+#pragma unroll 1
+                    for (int y2 = 0; y2 < WD; ++y2) {
+                        const float2* row = plane + (size_t)wrap_index((int)fl[1] - HW + y2, N) * N;
+                        const float w = ky[y2] * kzz;
+#pragma unroll
+                        for (int e = 0; e < WD; ++e) {
+                            const float kw = kx[e] * w;
+                            const float2 a = row[jx[e]];
+                            pr[q] = fmaf(a.x, kw, pr[q]);
+                            pi[q] = fmaf(a.y, kw, pi[q]);
+                        }
+                    }
                 }
-                for (int q = 0; q < WD - PW; ++q) {
-                    const float2 p = box[q * 64 + lane];
-                    vr += p.x;
-                    vi += p.y;
-                }
-            } else if (band && wave == 0) {
-                fsi_sample<WD>(ft, N, m, ktab, vr, vi);
+            }
+            // plane sums of every wavefront, added in the order of the planes
+            __syncthreads();
+            if (wave)
+#pragma unroll
+                for (int q = 0; q < PW; ++q) box[((wave - 1) * PW + q) * 64 + lane] = make_float2(pr[q], pi[q]);
+            __syncthreads();
+            if (wave) return;
+#pragma unroll
+            for (int q = 0; q < PW; ++q) {
+                vr += pr[q];
+                vi += pi[q];
+            }
+            for (int q = 0; q < WD - PW; ++q) {
+                const float2 p = box[q * 64 + lane];
+                vr += p.x;
+                vi += p.y;
             }
         }
         if (wave) return;
@@ -427,8 +454,9 @@ static int extract_launch(const float* ft_dev, int n, double sampling, const dou
         const double* m = dmats + 9 * v0;
         float2* out = (float2*)out_dev + v0 * n * n;
         switch (kernel_width) {
-// LDS boxes from width 5 on (see k_extract); cap holds the largest box of an 8 x 8
-// patch over random rotations (37 KB at W = 8, four workgroups per CU)
+// LDS boxes from width 5 on (see k_extract); cap holds the boxes of 8 x 8 patches of
+// rotations: the largest of 10^7 random ones at W = 8 had 4,590 voxels, cap is 4,654
+// (37 KB, four workgroups per CU); 1 to 2 % above the largest at the other widths
 #define BSX_EXT(W) case W: { \
             constexpr int WPT = W >= 8 ? 4 : W >= 5 ? 2 : 0; \
             constexpr int cap = WPT ? (W + 10) * (W + 9) * (W + 7) + 64 : 0; \

@@ -158,6 +158,49 @@ def test_sections_of_every_tile_path(n, width):
         assert np.abs(out[i] - ref).max() <= 1e-5 * np.abs(ref).max()
 
 
+@pytest.mark.parametrize("n,width", [(24, 5), (40, 6), (33, 7), (48, 8), (64, 9), (96, 10), (2, 8), (3, 5), (10, 10)])
+def test_sections_of_boxes_beyond_lds(n, width):
+    """Sections whose taps do not fit an LDS box (matrices that stretch the
+    plane; maps smaller than the kernel, with several periodic wraps) are
+    shared among a tile's wavefronts like the others: against the FP64 oracle,
+    FP32 rounding (1e-5 of the maximum)."""
+    rng = np.random.default_rng(n + width)
+    ft = (rng.normal(size=(n, n, n)) + 1j * rng.normal(size=(n, n, n))).astype(np.complex64)
+    mats = np.array([[[1, 1, 0], [1, -1, 0], [1, 1, 0]], [[1, -1, 1], [-1, 1, 1], [1, 1, 1]],
+                     [[0, 1, 0], [1, 0, 0], [0, 0, 1]]], dtype=float)
+    say(f"sections beyond LDS n={n} width={width}")
+    out = recon.central_sections(torch.as_tensor(ft).cuda(), mats, 1.5, 1.5, width, 2, True).cpu().numpy()
+    o = Oracle(64)
+    for i, m in enumerate(mats):
+        ref = o.central_section(ft, 1.5, m, 1.5, width, 2, 1)
+        assert np.abs(out[i] - ref).max() <= 1e-5 * np.abs(ref).max()
+
+
+def test_sections_beyond_lds_take_no_longer_than_their_taps():
+    """Sections of matrices that stretch the plane, whose taps come from memory,
+    take at most eight times as long as those of rotations at width 10 (12
+    times with one of a tile's wavefronts at work)."""
+    ft = torch.randn((128, 128, 128), dtype=torch.complex64, device="cuda")
+    wide = np.tile(np.array([[1, 1, 0], [1, -1, 0], [1, 1, 0]], dtype=float), (200, 1, 1))
+    rot = synth.view_to_matrix(synth.uniform_views(200, np.random.default_rng(1)))
+
+    def best(mats):
+        took = []
+        for _ in range(6):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            recon.central_sections(ft, mats, 1.5, 3.0, 10, 2)
+            b.record()
+            b.synchronize()
+            took.append(a.elapsed_time(b))
+        return min(took[1:])
+
+    say("sections beyond LDS, time")
+    w, r = best(wide), best(rot)
+    say(f"  {w:.3f} ms against {r:.3f} ms")
+    assert w <= 8 * r
+
+
 @pytest.mark.parametrize("n,width,views", [(256, 8, 16385), (24, 3, 65535)])
 def test_sections_of_very_many_views(n, width, views):
     """More sections than one launch has threads for (2^32 threads from 16,385
