@@ -1281,11 +1281,11 @@ struct bsx_cnn {
     float* d_gact[5] = {};
     float* d_loss = nullptr;
     // training: conv weights of layers 2-4 reordered for k_conv32 (forward,
-    // data gradient), and the shares of split sums; sized for max_batch
+    // data gradient), and the shares of split sums, sized for every batch up to
+    // max_batch, so that no step allocates
     float* d_wt[2] = {};
     long wt_ofs[5] = {};
     float* d_part = nullptr;
-    long part_cap = 0;
     long step = 0;
     // MFMA inference: permuted BF16 weights of layers 2-4 and the FC; NHWC
     // BF16 activations of layers 1-4 and FP32 logits, sized for chunks larger
@@ -1372,19 +1372,6 @@ int shares(long tiles, long steps) {
 // counts keep the direct kernels.
 bool conv32_ok(const bsx_cnn* h, int l) { return l >= 2 && h->ch[l - 1] % TK == 0 && h->ch[l] % TK == 0; }
 
-int reserve_part(bsx_cnn* h, long n, hipStream_t s) {
-    if (n <= h->part_cap) return BSX_OK;
-    if (h->d_part) {
-        BSX_HIP(hipStreamSynchronize(s));
-        (void)hipFree(h->d_part);
-    }
-    h->d_part = nullptr;
-    h->part_cap = 0;
-    BSX_HIP(hipMalloc(&h->d_part, sizeof(float) * n));
-    h->part_cap = n;
-    return BSX_OK;
-}
-
 // Shares of a k_gemm32 product, and the K range of each.
 int gemm32_shares(int M, int N, int K, int* kper) {
     const int z = shares(((N + 63) / 64) * (long)((M + 63) / 64), (K + TK - 1) / TK);
@@ -1400,27 +1387,30 @@ dim3 dw_grid(const bsx_cnn* h, int l, int B) {
     return dim3(t.x, t.y, shares((long)t.x * t.y, ((long)B * Ho * Ho + 15) / 16));
 }
 
-// One buffer for every split sum of a training step of B inputs (pairs: B / 2
-// pairs of them), so that the step allocates once.
-int reserve_training(bsx_cnn* h, int B, bool pairs, hipStream_t s) {
+// Values of the largest split sum of a forward or training step of up to
+// h->maxb inputs or h->maxb / 2 pairs. A smaller batch may need more than a larger
+// one (fewer tiles, more shares), so every batch is looked at.
+long part_values(const bsx_cnn* h) {
     const int C = h->nclass, F = (int)h->feat;
     long n = 0;
-    for (int l = 1; l <= 4; ++l)
-        if (l == 1 || conv32_ok(h, l))
-            n = std::max(n, ((long)h->ch[l] * h->ch[l - 1] * 9 + h->ch[l]) * dw_grid(h, l, B).z);
     auto product = [&](int M, int N, int K) {
         int kper;
         const int nz = gemm32_shares(M, N, K, &kper);
         if (nz > 1) n = std::max(n, (long)M * N * nz);
     };
-    product(B, C, F);
-    product(C, F, B);
-    product(B, F, C);
-    if (pairs) {
-        product(B / 2, B / 2, C);
-        product(B / 2, C, B / 2);
+    for (int B = 1; B <= h->maxb; ++B) {
+        for (int l = 1; l <= 4; ++l)
+            if (l == 1 || conv32_ok(h, l))
+                n = std::max(n, ((long)h->ch[l] * h->ch[l - 1] * 9 + h->ch[l]) * dw_grid(h, l, B).z);
+        product(B, C, F);
+        product(C, F, B);
+        product(B, F, C);
+        if (B % 2 == 0) {
+            product(B / 2, B / 2, C);
+            product(B / 2, C, B / 2);
+        }
     }
-    return reserve_part(h, n, s);
+    return n;
 }
 
 // C = A B (+ bias) on k_gemm32, K split over shares where C has few tiles.
@@ -1435,8 +1425,6 @@ int gemm32(bsx_cnn* h, int M, int N, int K, const float* A, long am, long ak, co
         return BSX_OK;
     }
     const long n = (long)M * N;
-    const int rc = reserve_part(h, n * nz, s);
-    if (rc) return rc;
     hipLaunchKernelGGL(k_gemm32, dim3(g.x, g.y, nz), dim3(256), 0, s, M, N, K, A, am, ak, B, bk, bn,
                        (const float*)nullptr, h->d_part, kper);
     BSX_HIP(hipGetLastError());
@@ -1534,7 +1522,6 @@ int backward_body(bsx_cnn* h, const float* x, int B, hipStream_t s) {
             // weights and biases are neighbours in the parameter vector
             const dim3 tiles = dw_grid(h, l, B);
             const int nz = (int)tiles.z;
-            if ((rc = reserve_part(h, n * nz, s))) return rc;
             if (l == 1)
                 hipLaunchKernelGGL(k_conv1_32_dw, dim3(nz, tiles.y), dim3(256), 0, s, h->d_gact[1], in,
                                    h->d_part, B, H, Cout, (B + nz - 1) / nz);
@@ -1749,6 +1736,8 @@ int bsx_cnn_create(bsx_cnn** out, int32_t in_size, const int32_t* channels, int3
     for (float*& q : h->d_wt)
         if ((e = hipMalloc(&q, sizeof(float) * (h->wt_ofs[4] + (long)h->ch[4] * h->ch[3] * 9))) != hipSuccess)
             return fail(e, "training weights");
+    if ((e = hipMalloc(&h->d_part, sizeof(float) * std::max(1l, part_values(h)))) != hipSuccess)
+        return fail(e, "training sums");
     for (int l = 1; l < 4; ++l)
         if ((e = hipMalloc(&h->d_wi[l], sizeof(uint16_t) * h->ch[l + 1] * h->ch[l] * 9)) != hipSuccess)
             return fail(e, "inference weights");
@@ -1808,8 +1797,7 @@ int bsx_cnn_gradients(bsx_cnn* h, const float* x_dev, const int32_t* labels_dev,
     BSX_REQUIRE(batch >= 1 && batch <= h->maxb, BSX_ERR_ARG,
                 "bsx_cnn_gradients: batch %d out of 1..%d", batch, h->maxb);
     hipStream_t s = (hipStream_t)stream;
-    int rc = reserve_training(h, batch, false, s);
-    if (!rc) rc = forward<float>(h, x_dev, batch, h->d_p, s);
+    int rc = forward<float>(h, x_dev, batch, h->d_p, s);
     if (!rc) rc = backward(h, x_dev, labels_dev, batch, s);
     if (rc) return rc;
     if (grad_dev)
@@ -1916,8 +1904,7 @@ int bsx_cnn_pair_gradients(bsx_cnn* h, const float* x_dev, int32_t batch, float 
     float* P = S + (long)B * B;
     float* Q = P + (long)B * B;
     float* dS = Q + (long)B * B;
-    int rc = reserve_training(h, B2, true, s);
-    if (!rc) rc = forward<float>(h, x_dev, B2, h->d_p, s);
+    int rc = forward<float>(h, x_dev, B2, h->d_p, s);
     if (rc) return rc;
     hipLaunchKernelGGL(k_unit_rows, dim3(nblk(B2, 4)), dim3(256), 0, s, h->d_act[0], (long)B2, d, U, nrm);
     BSX_HIP(hipGetLastError());

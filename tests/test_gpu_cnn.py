@@ -145,6 +145,35 @@ def test_bf16_inference_tile_edges(S, ch, ncls, B):
     assert np.all(prob[:, -1] >= np.sort(pr, axis=1)[:, -k] - 1e-3)
 
 
+@pytest.mark.parametrize("S,ch,ncls,batch", [(16, (16, 32, 32, 16), 10, 3), (32, (32, 64, 128, 128), 70, 60),
+                                            (16, (8, 12, 16, 32), 4, 17)])
+def test_first_calls_of_a_network_under_capture(S, ch, ncls, batch):
+    """A network's first forward pass and its first gradients can be recorded
+    into graphs (no call allocates): every replay, with other inputs and eager
+    work in between, gives what a second network computes."""
+    say(f"capture S={S} ch={ch} classes={ncls} batch={batch}")
+    gen = torch.Generator("cuda").manual_seed(S + batch)
+    xs = [torch.randn((batch, S, S), device="cuda", generator=gen) for _ in range(4)]
+    labels = torch.randint(ncls, (batch,), device="cuda", generator=gen).int()
+    net, ref = (ProposalNet(S, ncls, ch, max_batch=64, seed=5) for _ in range(2))
+    x = xs[0].clone()
+    torch.cuda.synchronize()
+    graphs = []
+    for call in (lambda: (net.forward(x),), lambda: net.gradients(x, labels)):
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            out = call()
+        graphs.append((g, out))
+    for v in xs:
+        x.copy_(v)
+        for (g, out), want in zip(graphs, ((ref.forward(v),), ref.gradients(v, labels))):
+            g.replay()
+            torch.cuda.synchronize()
+            for a, b in zip(out, want):
+                assert torch.equal(a, b)
+        ref.topk(v, 2)
+
+
 @pytest.mark.parametrize("m,k", [(5, 5), (40, 32), (63, 8), (64, 16), (1021, 16), (9000, 32)])
 def test_row_topk_against_sort(m, k):
     """The k best references by cosine over rows shorter and longer than a
