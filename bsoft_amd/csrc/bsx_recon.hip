@@ -1079,6 +1079,15 @@ __global__ __launch_bounds__(256) void k_sym_op(const float* __restrict__ in,
     out[v] = acc;
 }
 
+// Whether calls on the stream are being recorded into a graph (or the runtime does
+// not say: the legacy stream while another one records).
+static bool recording(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
+}
+
 // Insertion of one batch: rows and fill, then for binned entries the piece
 // table, the tile pass and the clearing of the bins.
 static int run_batch(bsx_recon* h, const float* imgs, int64_t p0, int nb, hipStream_t s) {
@@ -1312,13 +1321,16 @@ int bsx_recon_destroy(bsx_recon* h) {
 int bsx_recon_reset(bsx_recon* h, void* stream) {
     BSX_REQUIRE(h, BSX_ERR_ARG, "null handle");
     const long long n = (long long)h->acc_elems;
-    const bool x = h->binned && h->xdirty, b = h->binned && h->bins_dirty;
+    // a recorded reset clears everything: what is clean now need not be when the
+    // graph is replayed, and nothing is cleared before
+    const bool rec = recording((hipStream_t)stream);
+    const bool x = h->binned && (rec || h->xdirty), b = h->binned && (rec || h->bins_dirty);
     hipLaunchKernelGGL(k_reset, dim3((unsigned)std::min(2048LL, (n / 4 + 255) / 256)), dim3(256), 0,
                        (hipStream_t)stream, (unsigned*)h->acc, n, (unsigned*)h->xacc, x ? n : 0,
                        (unsigned*)h->fill, b ? (long long)h->nbins : 0, (unsigned*)h->chunks,
                        b ? (long long)h->nbins * h->maxc : 0, (unsigned*)h->pool);
     BSX_HIP(hipGetLastError());
-    h->xdirty = h->bins_dirty = false;
+    if (!rec) h->xdirty = h->bins_dirty = false;
     h->inserted[0] = h->inserted[1] = 0;
     return BSX_OK;
 }
@@ -1995,15 +2007,17 @@ int bsx_recon_kernel_times(const bsx_recon* h, double* ms, int n) {
 }
 
 // Brings the binned accumulator into the volume records (stream-ordered after
-// the inserts) where entries were binned since the last fold.
+// the inserts) where entries were binned since the last fold; a recorded fold
+// always, since its graph may be replayed after any insert.
 static int fold(bsx_recon* h, hipStream_t s) {
-    if (!h->binned || !h->xdirty) return BSX_OK;
+    const bool rec = recording(s);
+    if (!h->binned || !(rec || h->xdirty)) return BSX_OK;
     const long long n3 = (long long)h->K.N * h->K.N * h->K.N;
     const long long nrec = (long long)h->K.NT * h->K.NT * h->K.NT * 4096;
     hipLaunchKernelGGL(k_fold, dim3(2048), dim3(256), 0, s, h->acc, h->xacc, n3, h->K.N, h->K.NT,
                        nrec, h->p.nhalves, h->K.pairs, h->K.stride);
     BSX_HIP(hipGetLastError());
-    h->xdirty = false;
+    if (!rec) h->xdirty = false;
     return BSX_OK;
 }
 

@@ -624,6 +624,60 @@ def test_two_d_reconstruction(interp, tilted):
     assert abs(g.friedel - st.friedel) <= 1e-3 * st.friedel + 1e-5 * np.abs(ftc).max()
 
 
+@pytest.mark.parametrize("first", [False, True])
+def test_reset_recorded_in_a_graph(first):
+    """A reset recorded into a graph clears what inserts leave, whether the
+    handle was empty or not when it was recorded, and on every replay, with the
+    program's own inserts, resets and finishes in between."""
+    rng = np.random.default_rng(3)
+    ps = synth.make_particles(synth.make_blob_map(32, 8, rng), 40, 32, rng, seed=3)
+    imgs = ps.images.cuda().contiguous()
+    r, ref = (Reconstruction(32, 32, 64, 1.5, ctf_action=1) for _ in range(2))
+    ref.insert(imgs, ps.parts)
+    want = ref.finish().map
+    say(f"recorded reset, inserts before: {first}")
+    if first:
+        r.insert(imgs, ps.parts)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        r.reset()
+    for _ in range(3):
+        r.insert(imgs, ps.parts)
+        g.replay()
+        r.insert(imgs, ps.parts)
+        assert (r.finish().map - want).abs().max() <= 1e-5 * want.abs().max()
+        torch.cuda.synchronize()
+        r.reset()
+        r.insert(imgs, ps.parts)
+        assert (r.finish().map - want).abs().max() <= 1e-5 * want.abs().max()
+
+
+def test_accumulators_recorded_in_a_graph():
+    """Reading the sums (bsx_recon_accumulators, no allocation), recorded while
+    the handle was empty, gives the sums of the inserts before each replay."""
+    rng = np.random.default_rng(4)
+    ps = synth.make_particles(synth.make_blob_map(32, 8, rng), 40, 32, rng, seed=4)
+    imgs = ps.images.cuda().contiguous()
+    r, ref = (Reconstruction(32, 32, 64, 1.5, ctf_action=1) for _ in range(2))
+    planes = torch.zeros((5, 32, 32, 32), device="cuda")
+    say("recorded accumulators")
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        abi.call("bsx_recon_accumulators", r.h, 0, planes.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    for half in (imgs[:25], imgs[25:]):
+        part = ps.parts[:25] if len(half) == 25 else ps.parts[25:]
+        r.insert(half.contiguous(), part)
+        ref.insert(half.contiguous(), part)
+        g.replay()
+        torch.cuda.synchronize()
+        want = ref.accumulators(0)
+        for a, b in zip(planes[:3], want[:3]):
+            assert (a - b).abs().max() <= 1e-5 * b.abs().max()
+    assert (r.finish().map - ref.finish().map).abs().max() <= 1e-5 * ref.finish().map.abs().max()
+
+
 @pytest.mark.parametrize("size,flags,interp", [(32, 0, 0), (24, abi.BSX_FLAG_FOM, 0), (32, abi.BSX_FLAG_2D, 1),
                                                (48, 0, 2)])
 def test_finish_insert_and_reset_in_any_order(size, flags, interp):
