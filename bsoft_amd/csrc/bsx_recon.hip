@@ -1079,10 +1079,11 @@ __global__ __launch_bounds__(256) void k_sym_op(const float* __restrict__ in,
     out[v] = acc;
 }
 
-// Whether calls on the stream are being recorded into a graph (or the runtime does
-// not say: the legacy stream while another one records).
+// Whether calls on the stream are being recorded into a graph. The legacy default
+// stream cannot be recorded, so that calls on it do not pay for the question (2 us).
 static bool recording(hipStream_t s) {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (!s) return false;
     if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
     (void)hipGetLastError();
     return true;
