@@ -110,6 +110,7 @@ _dp = C.POINTER(C.c_double)
 SIGNATURES = {
     "bsx_last_error": ([], C.c_char_p),
     "bsx_version": ([C.POINTER(C.c_int), C.POINTER(C.c_int)], C.c_int),
+    "bsx_release_workspaces": ([], C.c_int),
     "bsx_device_info": ([C.c_char_p, C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_int64)], C.c_int),
     "bsx_part_ft_size": ([C.c_int, C.c_double, C.c_int], C.c_int),
     "bsx_recon_create": ([C.POINTER(_vp), C.POINTER(ReconParams)], C.c_int),

@@ -18,7 +18,7 @@ LIB = os.path.join(HERE, "libbsx.so")
 # minutes to compile, so each transform size is a unit of its own)
 UNITS = [("bsx_insert.hip", f"bsx_insert_{ft}", [f"-DBSX_INSERT_FT={ft}"])
          for ft in (512, 256, 128, 64, 32)]
-UNITS += [(f"{n}.hip", n, []) for n in ("bsx_search", "bsx_recon", "bsx_fft", "bsx_extract", "bsx_cnn")]
+UNITS += [(f"{n}.hip", n, []) for n in ("bsx_search", "bsx_recon", "bsx_fft", "bsx_extract", "bsx_cnn", "bsx_mem")]
 HEADERS = ["bsx_internal.h", "bsx_fft_dev.h", "bsx_common.h"]
 UNIT_HEADERS = {"bsx_insert.hip": ["bsx_insert.h"], "bsx_recon.hip": ["bsx_insert.h"]}
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

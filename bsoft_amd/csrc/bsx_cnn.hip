@@ -1607,11 +1607,11 @@ int infer_chunks(bsx_cnn* h, const float* x_dev, int64_t n, hipStream_t s, const
             h->d_ilog = nullptr;
             h->icap = 0;
             for (int l = 1; l < 5; ++l)
-                if (hipMalloc(&h->d_ib[l], sizeof(uint16_t) * act_size(h, l, chunk)) != hipSuccess) {
+                if (device_malloc(&h->d_ib[l], sizeof(uint16_t) * act_size(h, l, chunk)) != hipSuccess) {
                     set_error("%s: inference activations (%d particles)", who, chunk);
                     return BSX_ERR_NOMEM;
                 }
-            if (hipMalloc(&h->d_ilog, sizeof(float) * (size_t)chunk * h->nclass) != hipSuccess) {
+            if (device_malloc(&h->d_ilog, sizeof(float) * (size_t)chunk * h->nclass) != hipSuccess) {
                 set_error("%s: logits (%d particles)", who, chunk);
                 return BSX_ERR_NOMEM;
             }
@@ -1721,27 +1721,27 @@ int bsx_cnn_create(bsx_cnn** out, int32_t in_size, const int32_t* channels, int3
         return BSX_ERR_NOMEM;
     };
     hipError_t e;
-    if ((e = hipMalloc(&h->d_p, sizeof(float) * o)) != hipSuccess) return fail(e, "parameters");
-    if ((e = hipMalloc(&h->d_g, sizeof(float) * o)) != hipSuccess) return fail(e, "gradients");
-    if ((e = hipMalloc(&h->d_m, sizeof(float) * o)) != hipSuccess) return fail(e, "moments");
-    if ((e = hipMalloc(&h->d_v, sizeof(float) * o)) != hipSuccess) return fail(e, "moments");
-    if ((e = hipMalloc(&h->d_pb, sizeof(uint16_t) * o)) != hipSuccess) return fail(e, "bf16 copy");
-    if ((e = hipMalloc(&h->d_loss, sizeof(float) * max_batch)) != hipSuccess) return fail(e, "loss");
+    if ((e = device_malloc(&h->d_p, sizeof(float) * o)) != hipSuccess) return fail(e, "parameters");
+    if ((e = device_malloc(&h->d_g, sizeof(float) * o)) != hipSuccess) return fail(e, "gradients");
+    if ((e = device_malloc(&h->d_m, sizeof(float) * o)) != hipSuccess) return fail(e, "moments");
+    if ((e = device_malloc(&h->d_v, sizeof(float) * o)) != hipSuccess) return fail(e, "moments");
+    if ((e = device_malloc(&h->d_pb, sizeof(uint16_t) * o)) != hipSuccess) return fail(e, "bf16 copy");
+    if ((e = device_malloc(&h->d_loss, sizeof(float) * max_batch)) != hipSuccess) return fail(e, "loss");
     for (int l = 0; l < 5; ++l) {
         const long n = act_size(h, l, max_batch);
-        if ((e = hipMalloc(&h->d_act[l], sizeof(float) * n)) != hipSuccess) return fail(e, "activations");
-        if ((e = hipMalloc(&h->d_gact[l], sizeof(float) * n)) != hipSuccess) return fail(e, "activations");
+        if ((e = device_malloc(&h->d_act[l], sizeof(float) * n)) != hipSuccess) return fail(e, "activations");
+        if ((e = device_malloc(&h->d_gact[l], sizeof(float) * n)) != hipSuccess) return fail(e, "activations");
     }
     for (int l = 2; l <= 4; ++l) h->wt_ofs[l] = l == 2 ? 0 : h->wt_ofs[l - 1] + (long)h->ch[l - 1] * h->ch[l - 2] * 9;
     for (float*& q : h->d_wt)
-        if ((e = hipMalloc(&q, sizeof(float) * (h->wt_ofs[4] + (long)h->ch[4] * h->ch[3] * 9))) != hipSuccess)
+        if ((e = device_malloc(&q, sizeof(float) * (h->wt_ofs[4] + (long)h->ch[4] * h->ch[3] * 9))) != hipSuccess)
             return fail(e, "training weights");
-    if ((e = hipMalloc(&h->d_part, sizeof(float) * std::max(1l, part_values(h)))) != hipSuccess)
+    if ((e = device_malloc(&h->d_part, sizeof(float) * std::max(1l, part_values(h)))) != hipSuccess)
         return fail(e, "training sums");
     for (int l = 1; l < 4; ++l)
-        if ((e = hipMalloc(&h->d_wi[l], sizeof(uint16_t) * h->ch[l + 1] * h->ch[l] * 9)) != hipSuccess)
+        if ((e = device_malloc(&h->d_wi[l], sizeof(uint16_t) * h->ch[l + 1] * h->ch[l] * 9)) != hipSuccess)
             return fail(e, "inference weights");
-    if ((e = hipMalloc(&h->d_wi[4], sizeof(uint16_t) * h->feat * nclasses)) != hipSuccess)
+    if ((e = device_malloc(&h->d_wi[4], sizeof(uint16_t) * h->feat * nclasses)) != hipSuccess)
         return fail(e, "inference weights");
     if ((e = hipMemcpy(h->d_p, p.data(), sizeof(float) * o, hipMemcpyHostToDevice)) != hipSuccess ||
         (e = hipMemset(h->d_m, 0, sizeof(float) * o)) != hipSuccess ||
@@ -1862,7 +1862,7 @@ int bsx_cnn_match_topk(bsx_cnn* h, const float* p_dev, int64_t n, const float* r
         if (h->d_match) (void)hipFree(h->d_match);
         h->d_match = nullptr;
         h->match_cap = 0;
-        BSX_HIP(hipMalloc(&h->d_match, sizeof(float) * chunk * m));
+        BSX_HIP(device_malloc(&h->d_match, sizeof(float) * chunk * m));
         h->match_cap = chunk * m;
     }
     for (int64_t b0 = 0; b0 < n; b0 += chunk) {
@@ -1893,7 +1893,7 @@ int bsx_cnn_pair_gradients(bsx_cnn* h, const float* x_dev, int32_t batch, float 
         if (h->d_nce) (void)hipFree(h->d_nce);
         h->d_nce = nullptr;
         h->nce_cap = 0;
-        BSX_HIP(hipMalloc(&h->d_nce, sizeof(float) * need));
+        BSX_HIP(device_malloc(&h->d_nce, sizeof(float) * need));
         h->nce_cap = need;
     }
     float* U = h->d_nce;

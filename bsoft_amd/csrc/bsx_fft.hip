@@ -27,89 +27,6 @@ void set_error(const char* fmt, ...) {
 }
 const char* last_error() { return g_err; }
 
-// -------------------------------------------------------------- workspaces
-namespace {
-struct Kept {
-    void* p;
-    size_t bytes;
-    int dev;
-    bool pinned;
-    uint64_t used;
-};
-std::mutex kept_mu;
-std::vector<Kept> kept;
-uint64_t kept_clock = 0;
-
-void buffer_free(void* p, bool pinned) {
-    if (pinned) (void)hipHostFree(p);
-    else (void)hipFree(p);
-}
-}  // namespace
-
-hipError_t Scratch::get(size_t bytes) {
-    hipError_t e = hipGetDevice(&dev_);
-    if (e != hipSuccess) return e;
-    bytes = (bytes + 255) / 256 * 256;
-    {
-        // the smallest kept buffer that fits and is not far too large
-        std::lock_guard<std::mutex> g(kept_mu);
-        int at = -1;
-        for (int i = 0; i < (int)kept.size(); ++i)
-            if (kept[i].dev == dev_ && kept[i].pinned == pinned_ && kept[i].bytes >= bytes &&
-                kept[i].bytes <= 4 * bytes + (1 << 20) && (at < 0 || kept[i].bytes < kept[at].bytes))
-                at = i;
-        if (at >= 0) {
-            p_ = kept[at].p;
-            bytes_ = kept[at].bytes;
-            kept.erase(kept.begin() + at);
-            return hipSuccess;
-        }
-    }
-    auto alloc = [&]() { return pinned_ ? hipHostMalloc(&p_, bytes, hipHostMallocDefault) : hipMalloc(&p_, bytes); };
-    e = alloc();
-    if (e != hipSuccess) {
-        std::vector<Kept> all;
-        {
-            std::lock_guard<std::mutex> g(kept_mu);
-            all.swap(kept);
-        }
-        for (const Kept& k : all) buffer_free(k.p, k.pinned);
-        (void)hipGetLastError();
-        e = alloc();
-    }
-    if (e != hipSuccess) p_ = nullptr;
-    bytes_ = bytes;
-    return e;
-}
-
-void Scratch::release() {
-    constexpr size_t MOST = 512u << 20;
-    if (!p_ || bytes_ > MOST) return;   // freed by the destructor
-    std::vector<Kept> out;
-    {
-        std::lock_guard<std::mutex> g(kept_mu);
-        kept.push_back(Kept{p_, bytes_, dev_, pinned_, ++kept_clock});
-        p_ = nullptr;
-        for (;;) {
-            size_t sum = 0, n = 0, at = kept.size();
-            for (size_t i = 0; i < kept.size(); ++i) {
-                if (kept[i].pinned != pinned_) continue;
-                sum += kept[i].bytes;
-                ++n;
-                if (at == kept.size() || kept[i].used < kept[at].used) at = i;
-            }
-            if (sum <= MOST && n <= 16) break;
-            out.push_back(kept[at]);
-            kept.erase(kept.begin() + at);
-        }
-    }
-    for (const Kept& k : out) buffer_free(k.p, k.pinned);
-}
-
-Scratch::~Scratch() {
-    if (p_) buffer_free(p_, pinned_);
-}
-
 // ---------------------------------------------------------------- twiddles
 const float2* twiddles(int n, hipStream_t s) {
     static std::mutex mu;
@@ -126,7 +43,7 @@ const float2* twiddles(int n, hipStream_t s) {
         h[a] = make_float2((float)cos(ang), (float)sin(ang));
     }
     float2* d = nullptr;
-    if (hipMalloc(&d, sizeof(float2) * n) != hipSuccess) return nullptr;
+    if (device_malloc(&d, sizeof(float2) * n) != hipSuccess) return nullptr;
     if (hipMemcpyAsync(d, h.data(), sizeof(float2) * n, hipMemcpyHostToDevice, s) != hipSuccess)
         return nullptr;
     if (hipStreamSynchronize(s) != hipSuccess) return nullptr;

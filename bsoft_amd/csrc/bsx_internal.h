@@ -32,12 +32,26 @@ const char* last_error();
         }                                                                               \
     } while (0)
 
-// ---- workspaces of calls without a handle (bsx_fft.hip) ----
-// A device (or pinned host) buffer for one call. Allocating and freeing on every
-// call cost more than the kernels of small calls and stalled large ones for
-// milliseconds, so a buffer that its call has finished with is kept for the next
-// one: at most 16 buffers and 512 MB of each kind, the least recently used going
-// first, all of them given back when an allocation fails. release() says that the
+// ---- memory (bsx_mem.hip) ----
+// Every device and pinned allocation of the library: where memory has run out, the
+// workspaces below are given back before it fails.
+hipError_t device_malloc(void** p, size_t bytes);
+hipError_t pinned_malloc(void** p, size_t bytes);
+template <class T> hipError_t device_malloc(T** p, size_t bytes) {
+    return device_malloc((void**)p, bytes);
+}
+template <class T> hipError_t pinned_malloc(T** p, size_t bytes) {
+    return pinned_malloc((void**)p, bytes);
+}
+// Frees the workspaces that no call is using; returns their number.
+int release_workspaces();
+
+// Workspaces of calls without a handle: a device (or pinned host) buffer for one
+// call. Allocating and freeing on every call cost more than the kernels of small
+// calls and stalled large ones for milliseconds, so a buffer that its call has
+// finished with is kept for the next one: at most 16 buffers and 512 MB of each
+// kind, the least recently used going first, all of them given back when an
+// allocation of the library fails and by bsx_release_workspaces. release() says that the
 // call's stream has been waited for, i.e. that nothing uses the buffer any more, so
 // any thread may take it for any stream; a buffer that is destroyed without it
 // (an error return) is freed, which waits for the device.

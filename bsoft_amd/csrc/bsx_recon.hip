@@ -1255,21 +1255,21 @@ int bsx_recon_create(bsx_recon** out, const bsx_recon_params* p) {
         delete h;
         return BSX_ERR_NOMEM;
     }
-    bool ok = hipMalloc(&h->acc, h->acc_elems * sizeof(float)) == hipSuccess &&
-              hipMalloc(&h->inter, inter_bytes) == hipSuccess &&
-              hipMalloc(&h->nonfinite, sizeof(int)) == hipSuccess;
-    if (ok && bins2_bytes) ok = hipMalloc(&h->bins2, bins2_bytes) == hipSuccess;
+    bool ok = device_malloc(&h->acc, h->acc_elems * sizeof(float)) == hipSuccess &&
+              device_malloc(&h->inter, inter_bytes) == hipSuccess &&
+              device_malloc(&h->nonfinite, sizeof(int)) == hipSuccess;
+    if (ok && bins2_bytes) ok = device_malloc(&h->bins2, bins2_bytes) == hipSuccess;
     if (ok && h->binned)
-        ok = hipMalloc(&h->bins, bins_bytes) == hipSuccess &&
-             hipMalloc(&h->xacc, h->acc_elems * sizeof(float)) == hipSuccess &&
-             hipMalloc(&h->fill, sizeof(int) * h->nbins) == hipSuccess &&
-             hipMalloc(&h->chunks, sizeof(int) * (size_t)h->nbins * h->maxc) == hipSuccess &&
-             hipMalloc(&h->pool, sizeof(int) * 2) == hipSuccess &&
-             hipMalloc(&h->poff, sizeof(int) * (h->nbins + 1)) == hipSuccess &&
-             hipMalloc(&h->pbin, sizeof(int) * ((size_t)h->nbins +
+        ok = device_malloc(&h->bins, bins_bytes) == hipSuccess &&
+             device_malloc(&h->xacc, h->acc_elems * sizeof(float)) == hipSuccess &&
+             device_malloc(&h->fill, sizeof(int) * h->nbins) == hipSuccess &&
+             device_malloc(&h->chunks, sizeof(int) * (size_t)h->nbins * h->maxc) == hipSuccess &&
+             device_malloc(&h->pool, sizeof(int) * 2) == hipSuccess &&
+             device_malloc(&h->poff, sizeof(int) * (h->nbins + 1)) == hipSuccess &&
+             device_malloc(&h->pbin, sizeof(int) * ((size_t)h->nbins +
                                                 (size_t)h->npool * BSX_CHUNK / BSX_PIECE_MIN + 1)) ==
                  hipSuccess &&
-             hipMalloc(&h->entries, sizeof(unsigned long long)) == hipSuccess;
+             device_malloc(&h->entries, sizeof(unsigned long long)) == hipSuccess;
     if (!ok) {
         set_error("device allocation of %zu bytes failed", h->bytes);
         bsx_recon_destroy(h);
@@ -1419,9 +1419,9 @@ static int insert_prepare(bsx_recon* h, const bsx_particle* parts, int64_t n, hi
             set_error("particle records (%lld bytes) exceed the device-memory cap", (long long)extra);
             return BSX_ERR_NOMEM;
         }
-        if (hipMalloc(&h->recs, sizeof(PartDev) * n) != hipSuccess ||
-            hipMalloc(&h->bkg, sizeof(float) * n) != hipSuccess ||
-            (rescale && hipMalloc(&h->resc, sizeof(double2) * n) != hipSuccess)) {
+        if (device_malloc(&h->recs, sizeof(PartDev) * n) != hipSuccess ||
+            device_malloc(&h->bkg, sizeof(float) * n) != hipSuccess ||
+            (rescale && device_malloc(&h->resc, sizeof(double2) * n) != hipSuccess)) {
             h->recs_cap = 0;
             set_error("allocation of %lld particle records failed", (long long)n);
             return BSX_ERR_NOMEM;
@@ -1434,7 +1434,7 @@ static int insert_prepare(bsx_recon* h, const bsx_particle* parts, int64_t n, hi
         if (h->hrecs) BSX_HIP(hipHostFree(h->hrecs));
         h->hrecs = nullptr;
         h->hrecs_cap = 0;
-        BSX_HIP(hipHostMalloc((void**)&h->hrecs, sizeof(PartDev) * n, hipHostMallocDefault));
+        BSX_HIP(pinned_malloc(&h->hrecs, sizeof(PartDev) * n));
         h->hrecs_cap = n;
     }
     // Insertion order: by plane orientation (normal folded to one hemisphere,
@@ -1810,9 +1810,9 @@ static int symmetrize_impl(const float* in_dev, float* out_dev, int32_t n, int32
         if (dm) (void)hipFree(dm);
         if (part) (void)hipFree(part);
     };
-    hipError_t e = hipMalloc((void**)&dm, sizeof(double) * mats.size());
-    if (e == hipSuccess) e = hipMalloc((void**)&part, sizeof(double) * (2 * nblk + 1));
-    if (e == hipSuccess && ops.size() > 1) e = hipMalloc((void**)&tmp, sizeof(float) * total);
+    hipError_t e = device_malloc(&dm, sizeof(double) * mats.size());
+    if (e == hipSuccess) e = device_malloc(&part, sizeof(double) * (2 * nblk + 1));
+    if (e == hipSuccess && ops.size() > 1) e = device_malloc(&tmp, sizeof(float) * total);
     if (e != hipSuccess) {
         release();
         BSX_REQUIRE(false, BSX_ERR_DEVICE, "bsx_symmetrize: device allocation failed (%s)",
@@ -2090,7 +2090,7 @@ int bsx_recon_stats(bsx_recon* h, int imap, int nmaps, double resolution, double
     const int nblk = 1024;
     const int m = (int)(6 * nr1);
     double* part = nullptr;
-    BSX_HIP(hipMalloc((void**)&part, sizeof(double) * ((size_t)nblk * m + m)));
+    BSX_HIP(device_malloc(&part, sizeof(double) * ((size_t)nblk * m + m)));
     double* dsum = part + (size_t)nblk * m;
     const long long n3 = (long long)N * N * nz;
     const long long nrec = (long long)h->K.NT * h->K.NT * h->K.NT * 4096;
@@ -2366,8 +2366,8 @@ int bsx_recon_group_run(bsx_recon_group* g, const float* const* imgs_dev,
     // finish buffers (allocated outside any capture)
     for (bsx_recon* h : g->hs) {
         const size_t n3 = (size_t)h->K.N * h->K.N * h->K.nz;
-        if (!h->gvol) BSX_HIP(hipMalloc((void**)&h->gvol, sizeof(float2) * n3));
-        if (!h->gfin) BSX_HIP(hipMalloc((void**)&h->gfin, 64));
+        if (!h->gvol) BSX_HIP(device_malloc(&h->gvol, sizeof(float2) * n3));
+        if (!h->gfin) BSX_HIP(device_malloc(&h->gfin, 64));
     }
     // a run that stops half-way leaves its members to be cleared
     for (bsx_recon* h : g->hs) h->xdirty = h->bins_dirty = h->binned;

@@ -1485,7 +1485,7 @@ int grow(bsx_search* h, T** ptr, int64_t* cap, int64_t need, const char* what) {
         *ptr = nullptr;
         *cap = 0;
     }
-    hipError_t e = hipMalloc((void**)ptr, sizeof(T) * (size_t)need);
+    hipError_t e = device_malloc(ptr, sizeof(T) * (size_t)need);
     if (e != hipSuccess) {
         *ptr = nullptr;
         set_error("bsx_search: allocation of %lld bytes for %s failed: %s",

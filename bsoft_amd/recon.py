@@ -41,6 +41,12 @@ def _stream(stream=None):
     return C.c_void_p(s.cuda_stream)
 
 
+def release_workspaces() -> None:
+    """Free the workspaces that calls without a handle keep for the next one
+    (at most 512 MB of device and of pinned host memory each)."""
+    call("bsx_release_workspaces")
+
+
 def part_ft_size(xsize: int, scale: float = 1.0, pad_factor: int = 2) -> int:
     """part_ft_size (mg_reconstruct.cpp:38-64): transform size of padded particles."""
     return abi.lib().bsx_part_ft_size(int(xsize), float(scale), int(pad_factor))

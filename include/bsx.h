@@ -120,6 +120,13 @@ const char* bsx_last_error(void);
 
 /* Library / device information. */
 int bsx_version(int* major, int* minor);
+
+/* Calls without a handle (FSC, sections, finish, ...) keep their workspaces for
+ * the next one, at most 16 buffers and 512 MB of device and of pinned host memory
+ * each; they are also given back when an allocation of the library would fail.
+ * This frees those that no call is using, on every device, which waits for the
+ * devices (for callers that allocate device memory by other means). */
+int bsx_release_workspaces(void);
 int bsx_device_info(char* name, int name_len, int* cu_count, int64_t* hbm_bytes);
 
 /* ---- sizes ---- */

@@ -217,6 +217,22 @@ def test_sections_of_very_many_views(n, width, views):
         assert torch.equal(torch.view_as_real(out[v]), torch.view_as_real(want[pick[v]])), v
 
 
+def test_workspaces_given_back():
+    """release_workspaces frees what earlier calls kept, so that other users of
+    the device get it; the calls after it give the same values."""
+    rng = np.random.default_rng(5)
+    v = [torch.as_tensor(rng.normal(size=(192, 192, 192)).astype(np.float32)).cuda() for _ in range(2)]
+    say("workspaces given back")
+    one = bresolve.fsc_dpr(*v, 1.5)
+    torch.cuda.synchronize()
+    kept = torch.cuda.mem_get_info()[0]
+    recon.release_workspaces()
+    # the two half transforms of the call
+    assert torch.cuda.mem_get_info()[0] - kept >= 2 * 96 * 192 * 192 * 8
+    for a, b in zip(one, bresolve.fsc_dpr(*v, 1.5)):
+        np.testing.assert_allclose(a, b, rtol=1e-9, atol=1e-12)
+
+
 def test_workspaces_shared_by_threads_and_streams():
     """Calls without a handle keep their workspaces between calls: four threads,
     each on a stream of its own and with sizes of its own, get the results of
