@@ -2230,12 +2230,19 @@ int bsx_search_cnn_input(bsx_search* h, int32_t S, float* out_dev, void* stream)
         if (i > 0) gidx[(size_t)((-kk + S) % S) * S + (-hh + S) % S] = -i - 1;
     }
     hipStream_t s = (hipStream_t)stream;
+    // the table is a workspace, but counts towards the memory cap during the call
+    const int64_t S2 = (int64_t)S * S, tab_bytes = (int64_t)sizeof(int) * S2;
+    BSX_REQUIRE(h->p.mem_cap <= 0 || h->bytes + tab_bytes <= h->p.mem_cap, BSX_ERR_NOMEM,
+                "bsx_search: network input table needs %lld more bytes over the memory cap %lld",
+                (long long)tab_bytes, (long long)h->p.mem_cap);
     Scratch tab;
-    BSX_HIP(tab.get(sizeof(int) * S * S));
+    BSX_REQUIRE(tab.get(tab_bytes) == hipSuccess, BSX_ERR_NOMEM,
+                "bsx_search: allocation of %lld bytes for network input table failed", (long long)tab_bytes);
     int* dg = tab.as<int>();
-    const int64_t S2 = (int64_t)S * S;
     const int64_t chunk = std::max<int64_t>(1, std::min<int64_t>(n, (256ll << 20) / (8 * S2)));
+    h->bytes += tab_bytes;
     int rc = grow(h, &h->d_spec, &h->spec_cap, chunk * S2, "network input grids");
+    h->bytes -= tab_bytes;
     if (rc == BSX_OK &&
         hipMemcpyAsync(dg, gidx.data(), sizeof(int) * S2, hipMemcpyHostToDevice, s) != hipSuccess) {
         set_error("bsx_search_cnn_input: table upload failed");

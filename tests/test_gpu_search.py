@@ -12,7 +12,7 @@ import numpy as np
 import pytest
 import torch
 
-from bsoft_amd import search, synth
+from bsoft_amd import abi, search, synth
 from bsoft_amd.recon import central_sections, map_transform
 from oracle import search_ref as sr
 from oracle.oracle import Oracle
@@ -359,6 +359,36 @@ def test_proposed_tiles_of_pairs_and_members(setup64, npart, topk):
         if kk:
             assert np.all(np.diff(score[i][:kk]) <= 0)
             assert score[i][kk - 1] >= np.sort(A[i] @ B[allowed].T)[::-1][kk - 1] - 2e-4
+
+
+def test_network_input_within_memory_cap(setup64):
+    """The network's inputs are made where the memory cap has room for their
+    grids and for the table of grid points, and refused a byte below."""
+    n, R, bm, vol, ft, ps = setup64
+    S, npart = 32, 3
+    imgs = ps.images[:npart].cuda().contiguous()
+
+    def staged(cap):
+        s = search.Search(n, R, 1.5, mem_cap=cap)
+        s.stage(imgs, ps.parts[:npart])
+        return s
+
+    lo, hi = 1, 1 << 30                       # the least cap that staging takes
+    while lo < hi:
+        mid = (lo + hi) // 2
+        try:
+            staged(mid)
+            hi = mid
+        except abi.BsxError as e:
+            assert e.code == abi.BSX_ERR_NOMEM
+            lo = mid + 1
+    need = lo + 8 * npart * S * S + 4 * S * S
+    say(f"memory cap: staging {lo}, with network inputs {need}")
+    want = staged(0).cnn_input(S)
+    assert torch.equal(staged(need).cnn_input(S), want)
+    with pytest.raises(abi.BsxError) as e:
+        staged(need - 1).cnn_input(S)
+    assert e.value.code == abi.BSX_ERR_NOMEM
 
 
 @pytest.mark.parametrize("npart,topk", [(1, 16), (127, 8), (300, 16), (129, 3)])
