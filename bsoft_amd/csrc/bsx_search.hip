@@ -1785,25 +1785,30 @@ int run_exhaustive(bsx_search* h, const uint16_t* A, int64_t nrows, int32_t* can
     // 230,940 views 1,433 -> 907 us, 5,000 against 68,520 1,011 -> 868; 25,000
     // particles of 96^2 3,301 -> 2,565). Up to 2,048 workgroups, which bounds the
     // lists, and 256 segments, where the tiles of few particles take a CU each
-    // (150 against 269 tiles: 253 -> 107 us in this kernel); under a memory cap no
-    // more than 64 segments and about 1,024 workgroups of 4 tiles need.
+    // (150 against 269 tiles: 253 -> 107 us in this kernel); under a memory cap, or
+    // where there is no memory for more, what 64 segments and about 1,024 workgroups
+    // of 4 tiles need.
+    const int nfew = (int)std::min<int64_t>(std::min(64, std::max(1, ntiles / 4)), (1024 + rblocks - 1) / rblocks);
     int nmax = (int)std::min<int64_t>(ntiles, std::min<int64_t>(256, 1 + 2048 / rblocks));
-    if (h->p.mem_cap > 0)
-        nmax = (int)std::min<int64_t>(std::min(64, std::max(1, ntiles / 4)), (1024 + rblocks - 1) / rblocks);
-    int nseg = 1, tps = ntiles;
-    int64_t least = INT64_MAX;
-    for (int n = 1; n <= nmax; ++n) {
-        const int per = (ntiles + n - 1) / n, used = (ntiles + per - 1) / per;
-        const int64_t rounds = ((rblocks * used + 7) / 8 + 31) / 32;
-        if (rounds * (2 * per + 1) < least) {
-            least = rounds * (2 * per + 1);
-            nseg = used;
-            tps = per;
+    if (h->p.mem_cap > 0) nmax = nfew;
+    int nseg = 1, tps = ntiles, rc = BSX_OK;
+    for (;;) {
+        int64_t least = INT64_MAX;
+        for (int n = 1; n <= nmax; ++n) {
+            const int per = (ntiles + n - 1) / n, used = (ntiles + per - 1) / per;
+            const int64_t rounds = ((rblocks * used + 7) / 8 + 31) / 32;
+            if (rounds * (2 * per + 1) < least) {
+                least = rounds * (2 * per + 1);
+                nseg = used;
+                tps = per;
+            }
         }
+        const int64_t need = rblocks * GM4 * nseg * 4 * T;
+        rc = grow(h, &h->d_pscore, &h->pscore_cap, need, "top-k partials");
+        if (!rc) rc = grow(h, &h->d_pidx, &h->pidx_cap, need, "top-k partials");
+        if (rc != BSX_ERR_NOMEM || nmax <= nfew) break;
+        nmax = nfew;   // no memory for the longer lists: with as few as under a cap
     }
-    const int64_t need = rblocks * GM4 * nseg * 4 * T;
-    int rc = grow(h, &h->d_pscore, &h->pscore_cap, need, "top-k partials");
-    if (!rc) rc = grow(h, &h->d_pidx, &h->pidx_cap, need, "top-k partials");
     if (rc) return rc;
     BSX_REQUIRE(rblocks * nseg < (1ll << 31) - 8, BSX_ERR_ARG, "bsx_search_exhaustive: too many particles");
     const dim3 grid((unsigned)(8 * ((rblocks * nseg + 7) / 8)));
