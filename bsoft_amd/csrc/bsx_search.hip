@@ -510,8 +510,8 @@ __global__ void k_route_fill(const int* __restrict__ cls, int64_t n, int k, int 
 template <int T, int BM>
 __global__ __launch_bounds__(256) void k_gemm_grouped(
     const uint16_t* __restrict__ A, const uint16_t* __restrict__ B, int Kp,
-    const GroupItem* __restrict__ items, const int* __restrict__ nitems, const int* __restrict__ pairs,
-    int k, const int* __restrict__ members, const int* __restrict__ mcount, int maxm,
+    const GroupItem* __restrict__ items, int item0, const int* __restrict__ nitems,
+    const int* __restrict__ pairs, int k, const int* __restrict__ members, const int* __restrict__ mcount, int maxm,
     float* __restrict__ pscore, int* __restrict__ pidx) {
     constexpr int RM = 64 * BM, RN = 64 * BM;   // pairs x member views of a tile
     constexpr int LD = 2 * BM;                  // staged rows per thread, A and B each
@@ -521,10 +521,11 @@ __global__ __launch_bounds__(256) void k_gemm_grouped(
     static_assert(RM * CR * 4 <= 2 * STAGE && RM * PARTS * T * 8 <= 2 * STAGE, "epilogue fits the staging buffers");
     __shared__ __attribute__((aligned(16))) char lds[2 * STAGE];
     __shared__ int scol[RN];
-    if ((int)blockIdx.x >= *nitems) return;
+    const int item = item0 + (int)blockIdx.x;
+    if (item >= *nitems) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
-    const GroupItem it = items[blockIdx.x];
+    const GroupItem it = items[item];
     const int nm = mcount[it.cls];
     const int my_row = tid & (RM - 1), my_q = tid / RM;   // epilogue: row, part of its columns
     float best[T];
@@ -1768,6 +1769,22 @@ int bsx_search_stage(bsx_search* h, const float* imgs_dev, const bsx_particle* p
 
 namespace {
 
+// The best of each particle's nlist lists, 2^24 particles a launch (fewer than 2^32
+// threads).
+int topk_merge(bsx_search* h, int T, int nlist, int64_t n, int32_t* cand_dev, float* score_dev, hipStream_t s) {
+    const int topk = h->p.topk;
+    for (int64_t p0 = 0; p0 < n; p0 += 1 << 24) {
+        const int64_t nb = std::min<int64_t>(1 << 24, n - p0), at = p0 * nlist * T;
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3((unsigned)((nb + 3) / 4)), dim3(256), 0, s, h->d_pscore + at,
+                               h->d_pidx + at, nlist, nb, topk, cand_dev + p0 * topk, score_dev + p0 * topk);
+        };
+        T == 8 ? go(k_topk_merge<8>) : go(k_topk_merge<16>);
+        BSX_HIP(hipGetLastError());
+    }
+    return BSX_OK;
+}
+
 // GEMM + top-k of `nrows` BF16 rows at A (allocated to a multiple of GM4 rows)
 // against the whole library.
 int run_exhaustive(bsx_search* h, const uint16_t* A, int64_t nrows, int32_t* cand_dev,
@@ -1819,15 +1836,7 @@ int run_exhaustive(bsx_search* h, const uint16_t* A, int64_t nrows, int32_t* can
         hipLaunchKernelGGL((k_gemm_topk4<16>), grid, dim3(512), 0, s, A, h->d_lbf, h->Kp,
                            (int)h->nviews, tps, ntiles, (int)rblocks, nseg, h->d_pscore, h->d_pidx);
     BSX_HIP(hipGetLastError());
-    const unsigned mg = (unsigned)((nrows + 3) / 4);
-    if (T == 8)
-        hipLaunchKernelGGL((k_topk_merge<8>), dim3(mg), dim3(256), 0, s, h->d_pscore, h->d_pidx,
-                           4 * nseg, nrows, h->p.topk, cand_dev, score_dev);
-    else
-        hipLaunchKernelGGL((k_topk_merge<16>), dim3(mg), dim3(256), 0, s, h->d_pscore, h->d_pidx,
-                           4 * nseg, nrows, h->p.topk, cand_dev, score_dev);
-    BSX_HIP(hipGetLastError());
-    return BSX_OK;
+    return topk_merge(h, T, 4 * nseg, nrows, cand_dev, score_dev, s);
 }
 
 __global__ void k_gather_rows(const uint16_t* __restrict__ src, const int* __restrict__ rows,
@@ -1936,7 +1945,8 @@ int bsx_search_proposed(bsx_search* h, const int32_t* cls_dev, int32_t k, int32_
                        ((h->Kp >= 1152 && t64 >= 8 * nc) || (h->Kp >= 768 && t64 >= 32 * nc))) ||
                       (h->Kp >= 2048 && n * k >= 150 * nc && h->members > 40 * nc);
     const int rm = wide ? 128 : 64;
-    const int64_t most = h->nclass + n * k / rm;   // items: sum over classes of ceil(pairs / rm)
+    // items: sum over the classes that have pairs of ceil(pairs / rm)
+    const int64_t most = std::min<int64_t>(h->nclass, n * k) + n * k / rm;
     rc = grow(h, &h->d_items, &h->items_cap, most + 1, "work items");
     if (rc) return rc;
     int* nitems = (int*)(h->d_items + most);
@@ -1949,21 +1959,17 @@ int bsx_search_proposed(bsx_search* h, const int32_t* cls_dev, int32_t k, int32_
     hipLaunchKernelGGL(k_route_fill, dim3(g), dim3(256), 0, s, cls_dev, n, k, h->nclass, T, h->d_cursors,
                        h->d_pairs, h->d_pscore, h->d_pidx);
     BSX_HIP(hipGetLastError());
-    auto go = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3((unsigned)most), dim3(256), 0, s, h->d_pbf, h->d_lbf, h->Kp, h->d_items,
-                           nitems, h->d_pairs, k, h->d_members, h->d_mcount, h->maxm, h->d_pscore, h->d_pidx);
+    auto go = [&](auto kernel) {   // launches of fewer than 2^32 threads
+        for (int64_t i0 = 0; i0 < most; i0 += 1 << 23)
+            hipLaunchKernelGGL(kernel, dim3((unsigned)std::min<int64_t>(1 << 23, most - i0)), dim3(256), 0, s,
+                               h->d_pbf, h->d_lbf, h->Kp, h->d_items, (int)i0, nitems, h->d_pairs, k,
+                               h->d_members, h->d_mcount, h->maxm, h->d_pscore, h->d_pidx);
     };
     if (T == 8) wide ? go(k_gemm_grouped<8, 2>) : go(k_gemm_grouped<8, 1>);
     else wide ? go(k_gemm_grouped<16, 2>) : go(k_gemm_grouped<16, 1>);
     BSX_HIP(hipGetLastError());
-    const unsigned mg = (unsigned)((n + 3) / 4);
-    if (T == 8)
-        hipLaunchKernelGGL((k_topk_merge<8>), dim3(mg), dim3(256), 0, s, h->d_pscore, h->d_pidx, k,
-                           n, h->p.topk, cand_dev, score_dev);
-    else
-        hipLaunchKernelGGL((k_topk_merge<16>), dim3(mg), dim3(256), 0, s, h->d_pscore, h->d_pidx, k,
-                           n, h->p.topk, cand_dev, score_dev);
-    BSX_HIP(hipGetLastError());
+    rc = topk_merge(h, T, k, n, cand_dev, score_dev, s);
+    if (rc) return rc;
     // complete on return: the partial lists are shared with calls on other streams
     BSX_HIP(hipStreamSynchronize(s));
     return BSX_OK;
