@@ -30,6 +30,9 @@ def bf16_to_f32(x: torch.Tensor) -> np.ndarray:
     return u.view(np.float32).astype(np.float64)
 
 
+SPLIT_CAP = 1 << 34   # a memory cap with room for everything: segments of four tiles or more
+
+
 @pytest.fixture(scope="module")
 def setup64():
     n, R = 64, 14
@@ -90,15 +93,17 @@ def test_library_matches_extraction_and_oracle(setup64):
         assert np.all(np.abs(lr - orow) <= 2.0 ** -8 * np.abs(orow) + 1e-7)
 
 
+@pytest.mark.parametrize("cap", [0, SPLIT_CAP])
 @pytest.mark.parametrize("topk", [8, 16, 3])
-def test_gemm_topk_exact_on_bf16_rows(setup64, topk):
+def test_gemm_topk_exact_on_bf16_rows(setup64, topk, cap):
     """The GEMM scores are the FP32-accumulated dot products of the BF16 rows
-    and the selected views are the top-k of those products."""
+    and the selected views are the top-k of those products, with 54 segments of
+    one tile and (under a memory cap) with lists carried over five tiles."""
     n, R, bm, vol, ft, ps = setup64
     views = search.views_c1(6.0, angle_step_deg=30.0)   # 1154 x 12 views: ragged last tile
     mats = search.view_matrices(views)
-    say(f"gemm views={len(mats)} topk={topk}")
-    s = search.Search(n, R, 1.5, topk=topk)
+    say(f"gemm views={len(mats)} topk={topk} cap={cap}")
+    s = search.Search(n, R, 1.5, topk=topk, mem_cap=cap)
     s.set_reference(ft, mats)
     s.stage(ps.images.cuda().contiguous(), ps.parts)
     cand, score = s.exhaustive()
@@ -142,11 +147,12 @@ def test_topk_merge_ties_and_short_lists(setup64, npart, nview, repeat, topk):
         assert np.all(cand[i][len(want):] == -1) and np.all(np.isneginf(score[i][len(want):]))
 
 
-def test_gemm_topk_row_blocks_and_k_steps():
+@pytest.mark.parametrize("cap", [0, SPLIT_CAP])
+def test_gemm_topk_row_blocks_and_k_steps(cap):
     """The GEMM over more than one 256-row block (300 particles) and disk
     radii whose K = 2(Nd - 1), rounded up to 64, gives both odd and even
-    numbers of 64-deep K steps: every row's top-8 are the top-8 of the exact
-    BF16 products."""
+    numbers of 64-deep K steps, in segments of one tile and of several (under a
+    memory cap): every row's top-8 are the top-8 of the exact BF16 products."""
     n = 64
     rng = np.random.default_rng(29)
     bm = synth.make_blob_map(n, 30, rng)
@@ -155,7 +161,7 @@ def test_gemm_topk_row_blocks_and_k_steps():
     mats = search.view_matrices(search.views_c1(8.0, angle_step_deg=45.0))
     parities = set()
     for R in (10, 11, 14, 16):   # 5, 6, 10 and 13 K steps
-        s = search.Search(n, R, 1.5, topk=8)
+        s = search.Search(n, R, 1.5, topk=8, mem_cap=cap)
         s.set_reference(ft, mats)
         s.stage(ps.images.cuda().contiguous(), ps.parts)
         cand, score = s.exhaustive()
@@ -175,24 +181,26 @@ def test_gemm_topk_row_blocks_and_k_steps():
     assert parities == {0, 1}
 
 
-@pytest.mark.parametrize("nview", [100, 256, 700, 1153])
+@pytest.mark.parametrize("nview", [100, 256, 700, 1153, 13848])
 def test_few_particles_in_short_segments(setup64, nview):
-    """Few particles split the views into segments of as little as one tile:
-    three particles searched alone have the same candidates and the same
-    scores, bit for bit, as among 1,100, whose segments are longer."""
+    """Few particles split the views into segments of as little as one tile of
+    256, under a memory cap into ones of four tiles or more: three particles
+    searched alone have the same candidates and the same scores, bit for bit,
+    either way (1,153 views: five segments and one), and as among 1,100."""
     n, R, bm, vol, ft, ps = setup64
     mats = search.view_matrices(synth.uniform_views(nview, np.random.default_rng(nview)))
     say(f"short segments views={nview}")
     out = []
-    for count in (3, 1100):
+    for count, cap in ((3, 0), (3, SPLIT_CAP), (1100, SPLIT_CAP), (1100, 0)):
         pick = np.arange(count) % 3
-        s = search.Search(n, R, 1.5, topk=16)
+        s = search.Search(n, R, 1.5, topk=16, mem_cap=cap)
         s.set_reference(ft, mats)
         s.stage(ps.images[pick].cuda().contiguous(), ps.parts[pick])
         cand, score = s.exhaustive()
         out.append((cand[:3].cpu().numpy(), score[:3].cpu().numpy()))
-    assert np.array_equal(out[0][0], out[1][0])
-    assert np.array_equal(out[0][1], out[1][1])
+    for cand, score in out[1:]:
+        assert np.array_equal(out[0][0], cand)
+        assert np.array_equal(out[0][1], score)
 
 
 def test_rescore_and_score_mats_match_reference_frc(setup64):
