@@ -175,12 +175,12 @@ __global__ __launch_bounds__(256) void k_conv_bwd_weight(const float* __restrict
 }
 
 // ------------------------------------------------------------------ GEMM
-// C[m][n] = sum_k A[m*am + k*ak] * B[k*bk + n*bn] (+ bias[n]); 64x64 tiles,
+// C[m][n] = sum_k A[m*am + k*ak] * B[k*bk + n*bn] (+ bias[n]) with BF16 B and bias
+// (inference of networks that the matrix-core kernels do not take); 64x64 tiles,
 // K step 16 through LDS, 4x4 outputs per thread, edges guarded.
-template <typename TB>
 __global__ __launch_bounds__(256) void k_sgemm(int M, int N, int K, const float* __restrict__ A,
-                                               long am, long ak, const TB* __restrict__ Bm, long bk,
-                                               long bn, const TB* __restrict__ bias,
+                                               long am, long ak, const uint16_t* __restrict__ Bm,
+                                               long bk, long bn, const uint16_t* __restrict__ bias,
                                                float* __restrict__ Cm, long ldc) {
     __shared__ float As[16][64 + 4];
     __shared__ float Bs[16][64 + 4];
@@ -1439,7 +1439,7 @@ int forward_fc(bsx_cnn* h, int B, const float* W, const float* bias, hipStream_t
 }
 int forward_fc(bsx_cnn* h, int B, const uint16_t* W, const uint16_t* bias, hipStream_t s) {
     const int F = (int)h->feat, C = h->nclass;
-    hipLaunchKernelGGL((k_sgemm<uint16_t>), dim3((C + 63) / 64, (B + 63) / 64), dim3(256), 0, s, B, C, F,
+    hipLaunchKernelGGL(k_sgemm, dim3((C + 63) / 64, (B + 63) / 64), dim3(256), 0, s, B, C, F,
                        h->d_act[4], (long)F, 1l, W, 1l, (long)F, bias, h->d_act[0], (long)C);
     BSX_HIP(hipGetLastError());
     return BSX_OK;

@@ -33,9 +33,7 @@ struct alignas(16) PartDev {
 
 struct ReconConst {
     int N, ft, box, stride, interp, ctf_mode, fom, nhalves;   // ctf_mode 0 none 1 flip 2 apply 3 wiener
-    int merge, ewald, NT, pairs;                              // NT: 16^3 tiles per edge
-    // pairs: binned entries stand for a sample and its Friedel mate (value
-    // at v, conjugate at -v), folded into the volume by k_fold
+    int merge, ewald, NT;                                     // NT: 16^3 tiles per edge
     double mins2, maxs2, mscale, shi2, wiener;
     // z extent: a 2D map (breconstruct -TwoD) has one plane (nz = 1) and z
     // real size 1 (particle_reconstruct sets the z sampling to 1,

@@ -137,8 +137,7 @@ struct Emit {
     float re, im, w, p, w2;
 };
 
-// Fill-pass staging in LDS (nearest / weighted-nearest insertion without
-// Ewald): a workgroup appends its merged entries to a dense LDS list (one
+// Fill-pass staging in LDS: a workgroup appends its merged entries to a dense LDS list (one
 // 16-B record each; a wavefront takes its slots with one LDS atomic) and
 // counts them per bin in a small LDS hash table; at each flush one integer
 // atomic per (workgroup, bin) reserves the bin range (at most two chunks)
@@ -157,7 +156,6 @@ struct Stage {
     int* hcnt;       // entries per hash slot
     int4* hinfo;     // at a flush, per hash slot: reserved base, chunks of the
                      // range start and end, bin
-    int on;
     float2* ent2;    // FOM: (sum w|F|^2, sum w^2) of each entry, else null
 };
 
@@ -169,7 +167,7 @@ struct BinCtx {
     float* acc;      // volume records (3 floats), target of the atomic fallback
     int npool;       // chunks in the pool
     int maxc;        // chunks per bin
-    Stage st;        // fill-pass staging (st.on = 0: reserve per wavefront)
+    Stage st;        // fill-pass staging
     float2* bins2;   // FOM: (sum w|F|^2, sum w^2) of each pool entry, else null
     int stride;      // floats per volume record (3, or 5 with the FOM sums)
 };
@@ -376,9 +374,8 @@ __device__ __forceinline__ void merge_step(Emit& e, int& pk, int lg) {
 // equal and their sample rows differ by exactly d, so the samples between lie
 // on one straight segment and equal keys are contiguous (a periodic revisit
 // would need a segment longer than N-1 voxels, excluded on the host). The
-// first lane of each run then either adds to the volume with atomics
-// (MODE_DIRECT) or reserves a bin slot: lanes of a wavefront are grouped by
-// bin with ballots and one integer atomic per (wavefront, bin).
+// first lane of each run then adds to the volume with atomics (MODE_DIRECT, and
+// samples without a pair entry) or appends to the workgroup's list.
 template <int MG, bool FOM, int MODE, int FAST = 0>
 __device__ __forceinline__ void emit(float* __restrict__ acc, int stride, int merge, Emit e,
                                      const BinCtx& bc) {
@@ -412,42 +409,7 @@ __device__ __forceinline__ void emit(float* __restrict__ acc, int stride, int me
         }
         return;
     }
-    const bool out = out0;   // lanes still here hold binned entries
-    if (FAST || bc.st.on) {
-        stage_append(bc, out, e.key, e.re, e.im, e.w, e.p, e.w2);
-        return;
-    }
-    // per wavefront: one reservation per bin, all issued before any chunk
-    // lookup waits on them
-    const int bin = (int)((unsigned)e.key >> 12);
-    const int lane = __lane_id();
-    unsigned long long active = __ballot(out);
-    int mybase = 0, myleader = lane, myrank = 0, mycnt = 0;
-    while (active) {
-        const int leader = __builtin_ctzll(active);
-        const int b0 = __shfl(bin, leader, 64);
-        const bool mine = out && bin == b0;
-        const unsigned long long m = __ballot(mine);
-        if (lane == leader) {
-            mycnt = __popcll(m);
-            mybase = atomicAdd(bc.fill + b0, mycnt);
-        }
-        if (mine) {
-            myleader = leader;
-            myrank = __popcll(m & ((1ull << lane) - 1ull));
-        }
-        active &= ~m;
-    }
-    int myc0 = -1, myc1 = -1;   // this lane leads its bin's group: resolve its chunks
-    range_chunks(bc, bin, mybase, mycnt, mycnt > 0, myc0, myc1);
-    const int base = __shfl(mybase, myleader, 64);
-    const int c0 = __shfl(myc0, myleader, 64);
-    const int c1 = __shfl(myc1, myleader, 64);
-    if (out) {
-        const int pos = base + myrank;
-        put_entry(bc, pos / BSX_CHUNK == base / BSX_CHUNK ? c0 : c1, pos, e.re, e.im, e.w, e.key,
-                  e.p, e.w2);
-    }
+    stage_append(bc, out0, e.key, e.re, e.im, e.w, e.p, e.w2);   // lanes still here hold binned entries
 }
 
 template <bool FOM>
@@ -579,7 +541,7 @@ __device__ __forceinline__ void interp_emit(float* __restrict__ acc, const Recon
             // is flushed once it could not take another corner's
             // (workgroup-uniform: only the sample's own emission, which every
             // thread makes, asks)
-            if (MODE == MODE_FILL && flush && bc.st.on) {
+            if (MODE == MODE_FILL && flush) {
                 __syncthreads();
                 const bool full = *bc.st.nent > BSX_STAGE_CAP - (int)blockDim.x;
                 __syncthreads();   // every wave has read the count
@@ -604,10 +566,10 @@ __device__ __forceinline__ void coords(const ReconConst& K, const PartDev& P, do
 // same emits (excluded samples carry incl = 0), so shuffles and ballots stay
 // uniform.
 //
-// With K.pairs (binned insertion; the Ewald offsets have their own branch)
-// a sample whose mate lands on exactly the opposite voxels (-v for v:
+// In the fill pass (the Ewald offsets have their own branch) a sample whose mate
+// lands on exactly the opposite voxels (-v for v:
 // nearest neighbour all but exact .5 ties, trilinear always) is emitted
-// once, as pair entries at v that k_fold later also adds, conjugated, at
+// once, as pair entries at v that the fold later also adds, conjugated, at
 // -v. Samples without such a mate (the x = 0 and x = FT/2
 // columns, the Nyquist row, ties) add to the volume directly, and the mate
 // of a tie is emitted on its own, as before.
@@ -631,13 +593,13 @@ __device__ __forceinline__ void insert_pair(float* __restrict__ acc, const Recon
     } else {
         coords(K, P, s0, s1, mz0, m);
     }
-    if (!FAST && K.ewald) {
+    if (!FAST && (MODE == MODE_FILL || K.ewald)) {   // the general fill serves Ewald insertion only
         // two emissions per frequency, at +mz0 (A) and -mz0 (B). Off the
         // Nyquist row the mate's emissions at +mz0 and -mz0 lie at exactly
         // -B and -A with the conjugate value, so with pair entries A stands
         // for the mate's -mz0 emission and B for its +mz0 one (where the
         // nearest voxels mirror too); the others are computed in full.
-        const bool pr = MODE == MODE_FILL && K.pairs;
+        constexpr bool pr = MODE == MODE_FILL;
         double mb[3];
         coords(K, P, s0, s1, -mz0, mb);
         bool sa = pr && km == -k, sb = sa;
@@ -653,7 +615,7 @@ __device__ __forceinline__ void insert_pair(float* __restrict__ acc, const Recon
         interp_emit<MG, FOM, MODE, FAST>(acc, K, mb, inband, w, fr, fi, (int)k, merge, keybase, bc,
                                          mirror && sb ? 1 : 0, pr);
         // staged nearest-neighbour entries: at most two per thread here
-        if (MODE == MODE_FILL && pr && bc.st.on && K.interp < 2) stage_flush(bc);
+        if (pr && K.interp < 2) stage_flush(bc);
         double t0, t1, t2, tw;
         float gr, gi;
         const bool ib = sample_value<MODE>(K, P, mirror, -h, km, make_float2(F.x, -F.y), &t0,
@@ -697,12 +659,12 @@ __device__ __forceinline__ void insert_pair(float* __restrict__ acc, const Recon
                                 &tw, &gr, &gi);
         coords(K, P, t0, t1, 0.0, mm);
     }
-    if (FAST || (MODE == MODE_FILL && K.pairs)) {
+    if (FAST) {
         // trilinear: the mate's corners are the sample's negated, with the
         // same weights (floor(-m) = -floor(m) - 1 and 1 - dx; a coordinate
         // that is an integer only swaps a zero-weight corner)
         bool sym = km == -k;
-        if (FAST == 1 || FAST == 2 || (!FAST && K.interp < 2)) {
+        if (FAST < 3) {
 #pragma unroll
             for (int q = 0; q < 3; ++q) sym = sym && floor(-m[q] + 0.5) == -floor(m[q] + 0.5);
         }
@@ -764,11 +726,9 @@ void k_cols(const float2* __restrict__ inter,
     // staging (pair entries: at most one binned emission per thread and
     // round, so 2 rounds fit the list; the 512-entry list keeps the LDS of a
     // workgroup under 32 KB, 5 workgroups per CU)
-    const bool staged = FAST || (MODE == MODE_FILL && K.pairs && NT == 256 &&
-                                 2 * NT <= BSX_STAGE_CAP);
-    bc.st = Stage{st_ent, &st_nent, st_hkey, st_hcnt, st_hinfo, staged ? 1 : 0,
-                  FOM ? st_ent2 : nullptr};
-    if (staged) {
+    static_assert(NT == 256 && 2 * NT <= BSX_STAGE_CAP, "two rounds fit the list");
+    bc.st = Stage{st_ent, &st_nent, st_hkey, st_hcnt, st_hinfo, FOM ? st_ent2 : nullptr};
+    if (MODE == MODE_FILL) {
         if (tid < BSX_STAGE_HASH) {
             st_hkey[tid] = -1;
             st_hcnt[tid] = 0;
@@ -814,7 +774,7 @@ void k_cols(const float2* __restrict__ inter,
             ei = er * sd + ei * c;
             er = nr;
         }
-        if (MODE == MODE_FILL && staged && (FAST == 3 ? r == 7 : (r & 1) == 1)) stage_flush(bc);
+        if (MODE == MODE_FILL && (FAST == 3 ? r == 7 : (r & 1) == 1)) stage_flush(bc);
     }
 }
 
@@ -848,10 +808,10 @@ int insert_batch(bsx_recon* h, const float* imgs, int64_t p0, int nb, hipStream_
     };
     if (!h->binned) {
         h->K.fom ? go(k_cols<FT, true, MODE_DIRECT>) : go(k_cols<FT, false, MODE_DIRECT>);
-    } else if (h->K.ewald || NT != 256) {
+    } else if (h->K.ewald) {
         h->K.fom ? go(k_cols<FT, true, MODE_FILL>) : go(k_cols<FT, false, MODE_FILL>);
     } else {
-        // pair entries with LDS staging: the specialised kernels
+        // specialised on the interpolation
         switch (h->K.interp) {
             case 0: h->K.fom ? go(k_cols<FT, true, MODE_FILL, 1>) : go(k_cols<FT, false, MODE_FILL, 1>); break;
             case 1: h->K.fom ? go(k_cols<FT, true, MODE_FILL, 2>) : go(k_cols<FT, false, MODE_FILL, 2>); break;

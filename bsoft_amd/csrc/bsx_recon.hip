@@ -646,13 +646,13 @@ __global__ void k_stats_sum(const double* __restrict__ part, int nblocks, int m,
 
 // Folds the binned accumulator X into the volume records S (3 floats per
 // record, both in the tiled layout, `nrec` records per half) and clears X.
-// pairs = 0: X holds plain sums, S += X. pairs = 1: an X record at v stands
-// for the same sums at v and their conjugates at -v (mod N), so
+// A binned entry stands for a sample and its Friedel mate: an X record at v for
+// the same sums at v and their conjugates at -v (mod N), so
 // S(v) += X(v) + conj(X(-v)) and the weight W(v) += Xw(v) + Xw(-v). One
 // thread per voxel pair {v, -v}; linear order decides which voxel of the
 // pair handles it.
 __global__ void k_fold(float* __restrict__ S, float* __restrict__ X, long long n3, int N, int NT,
-                       long long nrec, int nhalves, int pairs, int rs) {
+                       long long nrec, int nhalves, int rs) {
     for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n3 * nhalves;
          i += (long long)gridDim.x * blockDim.x) {
         const int half = (int)(i / n3);
@@ -661,13 +661,6 @@ __global__ void k_fold(float* __restrict__ S, float* __restrict__ X, long long n
         float* s = S + (size_t)half * nrec * rs;
         float* xa = X + (size_t)half * nrec * rs;
         const size_t rv = (size_t)rec_index(x, y, z, NT) * rs;
-        if (!pairs) {
-            for (int c = 0; c < rs; ++c) {
-                s[rv + c] += xa[rv + c];
-                xa[rv + c] = 0.f;
-            }
-            continue;
-        }
         const long mx = x ? N - x : 0, my = y ? N - y : 0, mz = z ? N - z : 0;
         const long long jm = mx + (long long)N * (my + (long long)N * mz);
         if (jm < j) continue;
@@ -1211,7 +1204,6 @@ int bsx_recon_create(bsx_recon** out, const bsx_recon_params* p) {
     K.shi2 = 1.0 / (h->hi_res * h->hi_res);          // img_ctf_calculate hires
     K.ewald = (p->flags & BSX_FLAG_EWALD) ? 1 : 0;
     K.merge = 0;
-    K.pairs = h->binned ? 1 : 0;
     const size_t ntile = (size_t)K.NT * K.NT * K.NT;
     const size_t nrec = ntile * 4096;   // records incl. tile padding
     h->acc_elems = nrec * K.stride * p->nhalves;
@@ -2016,7 +2008,7 @@ static int fold(bsx_recon* h, hipStream_t s) {
     const long long n3 = (long long)h->K.N * h->K.N * h->K.N;
     const long long nrec = (long long)h->K.NT * h->K.NT * h->K.NT * 4096;
     hipLaunchKernelGGL(k_fold, dim3(2048), dim3(256), 0, s, h->acc, h->xacc, n3, h->K.N, h->K.NT,
-                       nrec, h->p.nhalves, h->K.pairs, h->K.stride);
+                       nrec, h->p.nhalves, h->K.stride);
     BSX_HIP(hipGetLastError());
     if (!rec) h->xdirty = false;
     return BSX_OK;
