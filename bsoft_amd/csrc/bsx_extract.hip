@@ -35,8 +35,8 @@ using namespace bsx;
 // Whole calls with the map transform, 200 sections of 128^2, before (one thread a
 // pixel of a row, taps from memory) and now: W = 3 322 / 183 us, 4 520 / 317,
 // 5 803 / 337, 6 1,016 / 414, 8 1,989 / 699; 50 sections of 256^2: 589 / 282,
-// 869 / 414, 1,234 / 415, 1,502 / 499, 2,845 / 830. LDS reads bound it at W = 8 (the
-// lanes' boxes start anywhere, so that they meet in banks); when whole calls took
+// 869 / 414, 1,234 / 415, 1,502 / 499, 2,845 / 830. LDS reads bound it at W = 8 (busy
+// 71 %, 61 % of that conflicts: the lanes' taps start anywhere and meet in banks); when whole calls took
 // 967 us with four wavefronts a tile there, they took 1,100 with one and 1,025 with two.
 struct __attribute__((packed, aligned(4))) Float4u {
     float v[4];

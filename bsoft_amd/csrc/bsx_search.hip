@@ -500,8 +500,8 @@ __global__ void k_route_fill(const int* __restrict__ cls, int64_t n, int k, int 
 // At 4-degree views in 15-degree classes a class has some 53 members and, for 8,000
 // particles x 16 proposals, some 29 pairs, and every view's row is read about once:
 // reading the rows bounds it (1.3 GB there), so that tiles are small (BM 1: four
-// workgroups a CU keep loads in flight). 128 x 128 tiles took 417 us, these 226 us
-// (3.7 TB/s of lines). Where classes are crowded an item walks many tiles one after
+// workgroups a CU keep loads in flight). 128 x 128 tiles took 417 us, these 222 us
+// (1.06 GB from HBM, 4.8 TB/s). Where classes are crowded an item walks many tiles one after
 // the other, each step of which takes about as long for 128 x 128 products as for
 // 64 x 64: BM 2, whose waves read four times for four products instead of two for one
 // (20 classes of 1,000 members, 10,000 x 5 pairs, radius 32: a search of 1,249 us with BM 1
