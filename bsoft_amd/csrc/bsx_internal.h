@@ -54,7 +54,7 @@ int release_workspaces();
 // allocation of the library fails and by bsx_release_workspaces. release() says that the
 // call's stream has been waited for, i.e. that nothing uses the buffer any more, so
 // any thread may take it for any stream; a buffer that is destroyed without it
-// (an error return) is freed, which waits for the device.
+// (an error return) is freed once the device is idle.
 class Scratch {
 public:
     explicit Scratch(bool pinned = false) : pinned_(pinned) {}
@@ -70,6 +70,7 @@ private:
     size_t bytes_ = 0;
     int dev_ = 0;
     bool pinned_;
+    bool idle_ = false;   // released
 };
 
 // ---- FFT launchers (bsx_fft.hip) ----

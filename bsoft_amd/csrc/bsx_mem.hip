@@ -84,6 +84,7 @@ hipError_t Scratch::get(size_t bytes) {
 }
 
 void Scratch::release() {
+    idle_ = true;
     if (!p_ || bytes_ > MOST) return;   // freed by the destructor
     Kept out[COUNT + 1];
     int nout = 0;
@@ -109,7 +110,9 @@ void Scratch::release() {
 }
 
 Scratch::~Scratch() {
-    if (p_) buffer_free(p_, pinned_);
+    if (!p_) return;
+    if (!idle_) (void)hipDeviceSynchronize();   // freeing pinned memory need not wait for copies from it
+    buffer_free(p_, pinned_);
 }
 
 }  // namespace bsx

@@ -15,6 +15,7 @@ hipError_t hipFree(void* p);
 hipError_t hipHostMalloc(void** p, size_t bytes, unsigned flags);
 hipError_t hipHostFree(void* p);
 hipError_t hipGetDevice(int* dev);
+hipError_t hipDeviceSynchronize(void);
 hipError_t hipGetLastError(void);
 const char* hipGetErrorString(hipError_t e);
 }

@@ -13,6 +13,7 @@
 static std::mutex mu;
 static std::map<void*, size_t> live[2];   // device, pinned
 static size_t used[2], calls;
+static std::atomic<int> waits{0};   // for the device
 static char* next_address = (char*)0x1000;
 static const size_t MB = 1u << 20, CAPACITY = 1000 * MB;
 
@@ -43,6 +44,7 @@ hipError_t hipFree(void* p) { return give(0, p); }
 hipError_t hipHostMalloc(void** p, size_t bytes, unsigned) { return take(1, p, bytes); }
 hipError_t hipHostFree(void* p) { return give(1, p); }
 hipError_t hipGetDevice(int* dev) { *dev = 0; return hipSuccess; }
+hipError_t hipDeviceSynchronize(void) { ++waits; return hipSuccess; }
 hipError_t hipGetLastError(void) { return hipSuccess; }
 const char* hipGetErrorString(hipError_t) { return ""; }
 }
@@ -80,6 +82,19 @@ int main() {
             CHECK(a.get(1 * MB) == hipSuccess && a.as<void>() != first);
         }                        // not released: freed
         CHECK(used[pinned] == 100 * MB);
+        // a buffer that its call has not released may be in use by the device
+        const int seen = waits;
+        {
+            Scratch a(pinned);
+            CHECK(a.get(600 * MB) == hipSuccess);
+        }
+        CHECK(waits == seen + 1);
+        {
+            Scratch a(pinned);   // released, but too large to keep
+            CHECK(a.get(600 * MB) == hipSuccess);
+            a.release();
+        }
+        CHECK(waits == seen + 1 && used[pinned] == 100 * MB);
     }
     // an allocation that does not fit beside the kept buffers takes their place
     void* p = nullptr;
